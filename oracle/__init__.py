@@ -29,10 +29,10 @@ _ip = C.POINTER(C.c_int)
 
 
 def build(ref: bool | None = None) -> None:
-    """Compile liboracle.so (and oracle/_ref when the reference tree exists)."""
+    """Compile liboracle.so (and oracle/_ref when the reference's sources are there)."""
     subprocess.run(["make", "-s", "-C", HERE, "liboracle.so"], check=True)
     if ref is None:
-        ref = os.path.isdir(REF_DIR)
+        ref = os.path.exists(os.path.join(REF_DIR, "src", "m_util_r8.f"))
     if ref:
         subprocess.run(["make", "-s", "-C", HERE, "ref"], check=True)
 
