@@ -17,6 +17,7 @@
 #include <vector>
 
 #include "pmg_kernels.h"
+#include "pmg_sweep_launch.h"
 #include "pamr_mg_gpu.h"
 
 extern "C" int pmg_net_reserve(pmg_net *N, long long points);
@@ -288,45 +289,6 @@ T *ucur(Level &Lv) { LevelArrays<T> &A = arrays<T>(Lv); return curbuf<T>(Lv) ? A
 template <typename T>
 T *uoth(Level &Lv) { LevelArrays<T> &A = arrays<T>(Lv); return curbuf<T>(Lv) ? A.u : A.ua; }
 
-// sweep tile variants (TX, TY, NT, planes in flight, LDS ring planes)
-#define PMG_SWEEP_VARIANTS(X)                                                                                   \
-  X(0, 64, 8, 256, 1, 4) X(1, 64, 16, 512, 1, 4) X(2, 32, 16, 512, 1, 4) X(3, 128, 8, 512, 1, 4)             \
-  X(4, 64, 32, 512, 1, 4) X(5, 128, 16, 1024, 1, 4) X(6, 128, 16, 1024, 2, 4) X(7, 64, 16, 512, 2, 4)        \
-  X(8, 128, 8, 512, 2, 4) X(9, 128, 16, 1024, 2, 5) X(10, 128, 16, 1024, 1, 5) X(11, 128, 8, 512, 1, 5)
-constexpr int kNumSweepVariants = 12;
-
-template <typename T, int OP, bool EX, bool P2, bool RHS0>
-int launch_sweep_v(pmg_solver *S, int variant, SweepP<T> P) {
-  P.zchunk = std::max(1, std::min(P.zchunk, P.nz - 2));
-  int tx = 64, ty = 8;
-  switch (variant) {
-#define PMG_TXY(V, TXV, TYV, NTV, PFV, RGV) case V: tx = TXV; ty = TYV; break;
-    PMG_SWEEP_VARIANTS(PMG_TXY)
-#undef PMG_TXY
-    default: return -1;
-  }
-  dim3 grid(((P.nx - 2 + tx - 1) / tx) * ((P.ny - 2 + ty - 1) / ty) * ((P.nz - 2 + P.zchunk - 1) / P.zchunk));
-  P.nb = (int)grid.x;
-  if (P.nb > S->ws.cap) return -3;
-  switch (variant) {
-#define PMG_LSW(V, TXV, TYV, NTV, PFV, RGV)                                                         \
-  case V:                                                                                           \
-    hipLaunchKernelGGL((k_sweep<T, OP, EX, P2, RHS0, TXV, TYV, NTV, PFV, RGV>), grid, dim3(NTV), 0, \
-                       S->stream, P);                                                               \
-    break;
-    PMG_SWEEP_VARIANTS(PMG_LSW)
-#undef PMG_LSW
-  }
-  PMG_HOST_CHECK(hipGetLastError());
-  return 0;
-}
-
-template <typename T, int OP, bool EX>
-int launch_sweep(pmg_solver *S, int v, SweepP<T> P, bool p2, bool rhs0) {
-  if (p2) return rhs0 ? launch_sweep_v<T, OP, EX, true, true>(S, v, P) : launch_sweep_v<T, OP, EX, true, false>(S, v, P);
-  return rhs0 ? launch_sweep_v<T, OP, EX, false, true>(S, v, P) : launch_sweep_v<T, OP, EX, false, false>(S, v, P);
-}
-
 // two sweeps in one pass (temporal blocking), 64 x 16 tiles, 1024 threads,
 // on levels with at least kSweep2MinN points per side
 constexpr int kSweep2MinN = 65;
@@ -389,8 +351,8 @@ int sweeps(pmg_solver *S, int L, int n, int slot, bool rhs0) {
       else rc = S->do_ex ? launch_sweep2<T, 1, true>(S, Q, p2, rhs0) : launch_sweep2<T, 1, false>(S, Q, p2, rhs0);
       done += 2;
     } else {
-      if (S->op == 0) rc = S->do_ex ? launch_sweep<T, 0, true>(S, variant, P, p2, rhs0) : launch_sweep<T, 0, false>(S, variant, P, p2, rhs0);
-      else rc = S->do_ex ? launch_sweep<T, 1, true>(S, variant, P, p2, rhs0) : launch_sweep<T, 1, false>(S, variant, P, p2, rhs0);
+      if (S->op == 0) rc = S->do_ex ? launch_sweep<T, 0, true>(S->stream, variant, P, p2, rhs0) : launch_sweep<T, 0, false>(S->stream, variant, P, p2, rhs0);
+      else rc = S->do_ex ? launch_sweep<T, 1, true>(S->stream, variant, P, p2, rhs0) : launch_sweep<T, 1, false>(S->stream, variant, P, p2, rhs0);
       done += 1;
     }
     if (rc) return rc;
