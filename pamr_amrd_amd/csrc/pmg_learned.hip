@@ -6,13 +6,13 @@
 // u += s * h^2 * N(r/s) and keeps the step only when the FP64 residual says
 // it contracts (pmg_solver's learned mode).
 //
-// Kernels are implicit GEMMs on the MFMA units: every layer is computed as a
-// 16 -> 16 channel convolution in BF16 with FP32 accumulation
-// (v_mfma_f32_16x16x16_bf16): a wavefront owns 16 consecutive points of an
-// x row and all 16 output channels, and accumulates the 27 taps as 27 MFMAs
-// with K = 16 input channels.  Layer 1's single input channel and layer 3's
-// single output channel are zero-padded to 16 (their padding rows/columns
-// stay exactly zero under training).  Activations are channel-last BF16
+// Kernels are implicit GEMMs on the MFMA units in BF16 with FP32 accumulation,
+// the same ones for inference and training (their epilogues differ): tiles of
+// (x, y) columns marching z with the input planes in LDS.  The hidden layer
+// has 16 channels and tap pairs along K, layer 1 the taps of its one input
+// channel along K, layer 3 the taps of its one output channel as columns.
+// The master weights are padded to 16 x 16 channels per tap (the padding
+// stays exactly zero under training).  Activations are channel-last BF16
 // [point][16]; pre-activations FP32.
 //
 // Training kernels: backward-data is the same convolution with flipped taps
@@ -36,6 +36,10 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 constexpr int NC = 16;      // channels (padded)
 constexpr int NTAP = 27;
+
+// master layout per layer: W[tap][ci][co] (27*256 floats) then bias[co]
+// (16 floats), i.e. 28 rows of 256 with the bias in row 27, entries 0..15
+constexpr int LAYER_FLOATS = (NTAP + 1) * 256;
 
 __host__ __device__ inline uint16_t f2bf(float f) {
   uint32_t u;
@@ -99,144 +103,152 @@ __global__ __launch_bounds__(64) void k_mfma32_probe(const uint16_t *A, const ui
   for (int i = 0; i < 4; i++) D[(4 * g + i) * 16 + m] = acc[i];
 }
 
-// ---------------------------------------------------------------------------
-// 16 -> 16 convolution.  Grid (ceil(nx/16), ceil(ny/4), nz*nb), 4 waves per
-// block, one x row segment of 16 points per wave.
-//   EPI 0: z = conv + bias -> Z (fp32), A = bf16(gelu(z))
-//   EPI 1: z = conv + bias -> Z (fp32) only (last layer)
-//   EPI 2: backward data: v = conv * gelu'(aux) -> Z (fp32), A = bf16(v)
-// Wf: weight fragments [27][64 lanes][4] bf16 (B operand order).
-// ---------------------------------------------------------------------------
-template <int EPI>
-__global__ __launch_bounds__(256) void k_conv16(const uint16_t *__restrict__ X,
-                                                const uint16_t *__restrict__ Wf,
-                                                const float *__restrict__ bias,
-                                                const float *__restrict__ aux,
-                                                float *__restrict__ Zout,
-                                                uint16_t *__restrict__ Aout, Geom g) {
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int x0 = blockIdx.x * 16, y = blockIdx.y * 4 + w;
-  const int z = blockIdx.z % g.nz, b = blockIdx.z / g.nz;
-  if (y >= g.ny) return;  // uniform per wave; no block barrier below
-  const int m = lane & 15, grp = lane >> 4;
-  const size_t box = (size_t)g.nx * g.ny * g.nz;
-  const uint16_t *Xb = X + (size_t)b * box * NC;
-  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 3
-  for (int tap = 0; tap < NTAP; tap++) {
-    const int dx = tap % 3 - 1, dy = (tap / 3) % 3 - 1, dz = tap / 9 - 1;
-    const int xx = x0 + m + dx, yy = y + dy, zz = z + dz;
-    bf16x4 a = {0, 0, 0, 0};
-    if (xx >= 0 && xx < g.nx && yy >= 0 && yy < g.ny && zz >= 0 && zz < g.nz)
-      a = *(const bf16x4 *)(Xb + (((size_t)zz * g.ny + yy) * g.nx + xx) * NC + 4 * grp);
-    const bf16x4 bw = *(const bf16x4 *)(Wf + ((size_t)tap * 64 + lane) * 4);
-    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bw, acc, 0, 0, 0);
-  }
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int xx = x0 + 4 * grp + i;
-    if (xx >= g.nx) continue;
-    const size_t pp = (size_t)b * box + ((size_t)z * g.ny + y) * g.nx + xx;
-    const size_t p = pp * NC + m;
-    float v = acc[i];
-    if constexpr (EPI == 0) {
-      v += bias[m];
-      Zout[p] = v;
-      Aout[p] = f2bf(gelu_f(v));
-    } else if constexpr (EPI == 1) {
-      Zout[p] = v + bias[m];
-    } else {
-      v *= gelu_grad_f(aux[p]);
-      Zout[p] = v;
-      Aout[p] = f2bf(v);
-    }
-  }
+// two floats to two BF16 in one word, rounded to nearest even (one instruction)
+__device__ inline unsigned pk_bf16(float lo, float hi) {
+  typedef float f2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+  const b2 r = __builtin_convertvector(f2{lo, hi}, b2);
+  unsigned w;
+  __builtin_memcpy(&w, &r, 4);
+  return w;
 }
 
 // GELU (tanh form) through the logistic function: 0.5 x (1 + tanh u) =
-// x / (1 + e^(-2u)), u = k (x + 0.044715 x^3); the inference epilogues use it
-// (the training kernels keep tanhf; the two agree to FP32 rounding)
+// x / (1 + e^(-2u)), u = k (x + 0.044715 x^3), with the constants folded
+// into the power of two; the inference epilogues use it (the training
+// kernels keep tanhf; the two agree to FP32 rounding).  The epilogue's vector
+// instructions, not the matrix units or LDS, bounded the hidden layer: with
+// the IEEE division and a software rounding to BF16 it took 0.27 of its
+// 0.61 ms at 257^3.
 __device__ inline float gelu_fast(float x) {
-  const float k = 0.7978845608028654f;
-  const float u = k * (x + 0.044715f * x * x * x);
-  return x / (1.0f + __expf(-2.0f * u));
+  const float c1 = -2.0f * 0.7978845608028654f * 1.4426950408889634f, c2 = c1 * 0.044715f;
+  const float e = __builtin_amdgcn_exp2f(x * fmaf(c2, x * x, c1));
+  return x * __builtin_amdgcn_rcpf(1.0f + e);
 }
 
 // Stores one MFMA result tile of BF16 activations channel-last: lane (m, grp)
-// holds channel m of points 4grp + i (v[i], i = 0..3); after a shuffle lane L
-// holds channels 4(L%4) .. +3 of point L/4 and writes them as one 8-byte store,
-// so the wave writes 16 points x 32 B contiguously.  `row` is the element
-// offset of the group's point 0, `npts` how many of its 16 points exist.
-__device__ inline void store_act16(uint16_t *__restrict__ Aout, size_t row, int npts, const uint16_t (&v)[4]) {
+// holds channel m of points 4grp + i (w01: points 0, 1, w23: points 2, 3);
+// after a shuffle lane L holds channels 4(L%4) .. +3 of point L/4 and writes
+// them as one 8-byte store, so the wave writes 16 points x 32 B contiguously.
+// `row` is the element offset of the group's point 0, `npts` how many of its
+// 16 points exist.
+__device__ inline void store_act16(uint16_t *__restrict__ Aout, size_t row, int npts, unsigned w01, unsigned w23) {
   const int L = threadIdx.x & 63;
-  const unsigned w01 = (unsigned)v[0] | ((unsigned)v[1] << 16), w23 = (unsigned)v[2] | ((unsigned)v[3] << 16);
   const int p = L >> 2, c0 = (L & 3) * 4, i = p & 3, sg = p >> 2;
-  unsigned out[2];
+  unsigned h[4];
 #pragma unroll
   for (int k = 0; k < 4; k++) {
     const int src = (c0 + k) + 16 * sg;
     const unsigned a = (unsigned)__builtin_amdgcn_ds_bpermute(src * 4, (int)w01);
     const unsigned b = (unsigned)__builtin_amdgcn_ds_bpermute(src * 4, (int)w23);
-    const unsigned word = i < 2 ? a : b;
-    const unsigned h = (i & 1) ? (word >> 16) : (word & 0xffffu);
-    if (k & 1) out[k >> 1] |= h << 16;
-    else out[k >> 1] = h;
+    h[k] = i < 2 ? a : b;
   }
-  if (p < npts) *(uint2 *)(Aout + (row + (size_t)p) * NC + c0) = make_uint2(out[0], out[1]);
+  // the low or the high half of each word, by the point's parity
+  const unsigned sel = (i & 1) ? 0x07060302u : 0x05040100u;
+  if (p < npts)
+    *(uint2 *)(Aout + (row + (size_t)p) * NC + c0) =
+        make_uint2(__builtin_amdgcn_perm(h[1], h[0], sel), __builtin_amdgcn_perm(h[3], h[2], sel));
 }
 
-// Hidden and last layer of the inference path with the input staged in LDS:
-// a block owns a CTX x CTY tile of (x, y) columns and marches ZC planes in
-// z, keeping a ring of 4 input planes (tile plus a 1-point halo, 16 BF16
-// channels = 32 B per point, zero outside the box) in LDS.  Wave w computes
-// rows 2w, 2w+1 of the tile, two 16-point segments each.  The 27 taps go in
-// pairs through the K = 32 MFMA (14 per segment and plane, the last pair
-// padded with zeros): lanes 0-31 read 16 channel bytes of the pair's first
-// tap, lanes 32-63 of its second, as one 16-byte LDS read each; the 14 weight
-// fragments stay in registers.  One barrier per plane: plane z+2 is stored
-// into the slot plane z-2 left at the start of step z, plane z+3 is fetched
-// into registers, and step z reads z-1..z+1.
-//   EPI 3: A = bf16(gelu(conv + bias));  EPI 4: Z[p] = conv + bias, channel 0
+// What a convolution tile does with its sums v (lane (m, grp): channel m of
+// points 4grp + i of a 16-point segment starting at element `row`):
+//   EPI 0: z = v + bias -> Z (FP32), A = bf16(gelu(z))          (training)
+//   EPI 2: A = bf16(v * gelu'(aux))                             (backward data)
+//   EPI 3: A = bf16(gelu(v + bias))                             (inference)
+template <int EPI>
+__device__ __forceinline__ void conv_epilogue(floatx4 v, float bias, const float *__restrict__ aux,
+                                              float *__restrict__ Z, uint16_t *__restrict__ A, size_t row, int npts) {
+  const int lane = threadIdx.x & 63, m = lane & 15, grp = lane >> 4;
+  float o[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const size_t p = (row + 4 * grp + i) * NC + m;
+    const bool in = 4 * grp + i < npts;
+    if constexpr (EPI == 0) {
+      const float z = v[i] + bias;
+      if (in) Z[p] = z;
+      o[i] = gelu_f(z);
+    } else if constexpr (EPI == 2) {
+      o[i] = in ? v[i] * gelu_grad_f(aux[p]) : 0.f;
+    } else {
+      o[i] = gelu_fast(v[i] + bias);
+    }
+  }
+  store_act16(A, row, npts, pk_bf16(o[0], o[1]), pk_bf16(o[2], o[3]));
+}
+
+// The 16 -> 16 convolutions with the input staged in LDS: a block owns a
+// CTX x CTY tile of (x, y) columns and marches ZC planes in z, keeping a ring
+// of 4 input planes (tile plus a 1-point halo, 16 BF16 channels = 32 B per
+// point, zero outside the box) in LDS.  Wave w computes rows 2w, 2w+1 of the
+// tile, two 16-point segments each.  The 27 taps go in pairs through the K =
+// 32 MFMA (14 per segment and plane, the last pair padded with zeros): lanes
+// 0-31 read 16 channel bytes of the pair's first tap, lanes 32-63 of its
+// second, as one 16-byte LDS read each; the 14 weight fragments stay in
+// registers.  One barrier per plane: plane z+2 is stored into the slot plane
+// z-2 left at the start of step z, plane z+3 is fetched into registers, and
+// step z reads z-1..z+1.  The fetches are unconditional (positions outside
+// the box read element 0 and are stored as zero), so they stay in flight
+// across the step.
 constexpr int CTX = 32, CTY = 8, CLX = CTX + 2, CLY = CTY + 2;
 constexpr int CCHUNK = CLY * CLX * 2;                  // 16-byte chunks per staged plane
 constexpr int CLOAD = (CCHUNK + 255) / 256;            // per thread
 constexpr int NPAIR = (NTAP + 1) / 2;                  // tap pairs of the K = 32 form
-template <int EPI, int ZC>
+
+struct ConvTile {
+  int x0, y0, z0, z1, b;
+};
+__device__ __forceinline__ ConvTile conv_tile(const Geom &g, int tx_, int ty_, int zc_) {
+  const int ntx = (g.nx + tx_ - 1) / tx_, nty = (g.ny + ty_ - 1) / ty_, nzc = (g.nz + zc_ - 1) / zc_;
+  int t = blockIdx.x;
+  ConvTile c;
+  c.x0 = (t % ntx) * tx_;
+  t /= ntx;
+  c.y0 = (t % nty) * ty_;
+  t /= nty;
+  c.z0 = (t % nzc) * zc_;
+  c.b = t / nzc;
+  c.z1 = min(g.nz, c.z0 + zc_);
+  return c;
+}
+inline unsigned conv_blocks(const Geom &g, int tx_, int ty_, int zc_) {
+  return (unsigned)((size_t)((g.nx + tx_ - 1) / tx_) * ((g.ny + ty_ - 1) / ty_) * ((g.nz + zc_ - 1) / zc_) * g.nb);
+}
+
+template <int EPI>
 __global__ __launch_bounds__(256) void k_conv16_tile(const uint16_t *__restrict__ X,
                                                      const uint16_t *__restrict__ Wp,
-                                                     const float *__restrict__ bias, float *__restrict__ Zout,
-                                                     uint16_t *__restrict__ Aout, Geom g) {
+                                                     const float *__restrict__ bias, const float *__restrict__ aux,
+                                                     float *__restrict__ Zout, uint16_t *__restrict__ Aout, Geom g,
+                                                     int zc) {
   __shared__ uint4 sX[4][CLY][CLX][2];
-  const int ntx = (g.nx + CTX - 1) / CTX, nty = (g.ny + CTY - 1) / CTY, nzc = (g.nz + ZC - 1) / ZC;
-  int t = blockIdx.x;
-  const int tx = t % ntx;
-  t /= ntx;
-  const int ty = t % nty;
-  t /= nty;
-  const int zc = t % nzc, b = t / nzc;
-  const int x0 = tx * CTX, y0 = ty * CTY, z0 = zc * ZC, z1 = min(g.nz, z0 + ZC);
+  const ConvTile T = conv_tile(g, CTX, CTY, zc);
+  const int x0 = T.x0, y0 = T.y0, z0 = T.z0, z1 = T.z1;
   const size_t box = (size_t)g.nx * g.ny * g.nz;
-  const uint16_t *Xb = X + (size_t)b * box * NC;
+  const uint16_t *Xb = X + (size_t)T.b * box * NC;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m = lane & 15, grp = lane >> 4;
   uint4 reg[CLOAD];
-  auto fetch = [&](int k) {
+  int off[CLOAD];  // element offset of this thread's chunks within a plane, or -1
 #pragma unroll
-    for (int q = 0; q < CLOAD; q++) {
-      const int idx = (int)threadIdx.x + q * 256;
-      reg[q] = make_uint4(0u, 0u, 0u, 0u);
-      if (idx >= CCHUNK || k < 0 || k >= g.nz) continue;
-      const int ly = idx / (CLX * 2), rem = idx % (CLX * 2), lx = rem >> 1, h = rem & 1;
-      const int gx = x0 - 1 + lx, gy = y0 - 1 + ly;
-      if (gx >= 0 && gx < g.nx && gy >= 0 && gy < g.ny)
-        reg[q] = ((const uint4 *)(Xb + (((size_t)k * g.ny + gy) * g.nx + gx) * NC))[h];
-    }
+  for (int q = 0; q < CLOAD; q++) {
+    const int idx = (int)threadIdx.x + q * 256;
+    const int ly = idx / (CLX * 2), rem = idx % (CLX * 2), lx = rem >> 1, h = rem & 1;
+    const int gx = x0 - 1 + lx, gy = y0 - 1 + ly;
+    off[q] = (idx < CCHUNK && gx >= 0 && gx < g.nx && gy >= 0 && gy < g.ny) ? (gy * g.nx + gx) * NC + 8 * h : -1;
+  }
+  const size_t plane = (size_t)g.nx * g.ny * NC;
+  auto fetch = [&](int k) {
+    const uint16_t *Xk = Xb + (k >= 0 && k < g.nz ? (size_t)k * plane : 0);
+#pragma unroll
+    for (int q = 0; q < CLOAD; q++) reg[q] = *(const uint4 *)(Xk + (off[q] < 0 ? 0 : off[q]));
   };
   auto store = [&](int k) {
     uint4 *S = &sX[k & 3][0][0][0];
+    const bool kin = k >= 0 && k < g.nz;
 #pragma unroll
     for (int q = 0; q < CLOAD; q++) {
       const int idx = (int)threadIdx.x + q * 256;
-      if (idx < CCHUNK) S[idx] = reg[q];
+      if (idx < CCHUNK) S[idx] = kin && off[q] >= 0 ? reg[q] : make_uint4(0u, 0u, 0u, 0u);
     }
   };
   // the 14 weight fragments stay in registers for the whole march
@@ -244,7 +256,7 @@ __global__ __launch_bounds__(256) void k_conv16_tile(const uint16_t *__restrict_
 #pragma unroll
   for (int pr = 0; pr < NPAIR; pr++) wk[pr] = *(const bf16x8 *)(Wp + ((size_t)pr * 64 + lane) * 8);
   const int half = grp & 1, second = grp >> 1;  // channel half; first or second tap of the pair
-  const float bm = bias[EPI == 3 ? m : 0];
+  const float bm = EPI == 2 ? 0.f : bias[m];
   fetch(z0 - 1);
   store(z0 - 1);
   fetch(z0);
@@ -269,6 +281,7 @@ __global__ __launch_bounds__(256) void k_conv16_tile(const uint16_t *__restrict_
 #pragma unroll
       for (int q = 0; q < 4; q++) {
         const int r = 2 * w + (q >> 1), sg = q & 1;
+        // (the weights of the tap past the 27th are zero, and so is its operand)
         bf16x8 a = *(const bf16x8 *)&sX[slot][r + 1 + dy][16 * sg + m + 1 + dx][half];
         if (!live) a = bf16x8{};
         acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, wk[pr], acc[q], 0, 0, 0);
@@ -276,70 +289,74 @@ __global__ __launch_bounds__(256) void k_conv16_tile(const uint16_t *__restrict_
     }
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-      const int y = y0 + 2 * w + (q >> 1);
-      if (y >= g.ny) continue;  // uniform per wave
-      const int xs = x0 + 16 * (q & 1);
-      const size_t row = (size_t)b * box + ((size_t)z * g.ny + y) * g.nx + xs;
-      if constexpr (EPI == 3) {
-        uint16_t v[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) v[i] = f2bf(gelu_fast(acc[q][i] + bm));
-        store_act16(Aout, row, min(16, g.nx - xs), v);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const int xx = xs + 4 * grp + i;
-          if (m == 0 && xx < g.nx) Zout[row + 4 * grp + i] = acc[q][i] + bm;
-        }
-      }
+      const int y = y0 + 2 * w + (q >> 1), xs = x0 + 16 * (q & 1);
+      if (y >= g.ny || xs >= g.nx) continue;  // uniform per wave
+      conv_epilogue<EPI>(acc[q], bm, aux, Zout, Aout, (size_t)T.b * box + ((size_t)z * g.ny + y) * g.nx + xs,
+                         min(16, g.nx - xs));
     }
     __syncthreads();
   }
 }
 
-// Layer 1 of the inference path on the same tiles: the plane tile of
-// bf16(scale * x) (one channel, 2 B per point, zero outside the box) is staged
-// in a 4-plane LDS ring; lane (m, grp) gathers its taps 8grp + j from LDS for
-// one K = 32 MFMA whose K is the 27 taps (5 zero).
-template <int ZC>
-__global__ __launch_bounds__(256) void k_conv_in_tile(const float *__restrict__ x, float scale,
+// Convolutions of one input channel (layer 1, and the backward data of layer
+// 3) on the same tiles: the plane tile of bf16(scale * x) (zero outside the
+// box) is staged in a 4-plane LDS ring, each word holding the point and its
+// east neighbour, so that two words two apart are the four points x-1 .. x+2.
+// One K = 16 MFMA per dz: lane group grp takes dy = grp - 1 (the fourth group is
+// zero), its four K slots dx = -1, 0, 1 (the fourth is zero): one LDS
+// instruction per operand, where 27 taps laid along K took eight 2-byte reads
+// and their packing.
+template <typename TIN, int EPI>
+__global__ __launch_bounds__(256) void k_conv_in_tile(const TIN *__restrict__ x, float scale,
                                                       const uint16_t *__restrict__ Wfi,
-                                                      const float *__restrict__ bias, uint16_t *__restrict__ Aout,
-                                                      Geom g) {
-  __shared__ uint16_t sx[4][CLY][CLX];
-  const int ntx = (g.nx + CTX - 1) / CTX, nty = (g.ny + CTY - 1) / CTY, nzc = (g.nz + ZC - 1) / ZC;
-  int t = blockIdx.x;
-  const int tx = t % ntx;
-  t /= ntx;
-  const int ty = t % nty;
-  t /= nty;
-  const int zc = t % nzc, b = t / nzc;
-  const int x0 = tx * CTX, y0 = ty * CTY, z0 = zc * ZC, z1 = min(g.nz, z0 + ZC);
+                                                      const float *__restrict__ bias, const float *__restrict__ aux,
+                                                      float *__restrict__ Zout, uint16_t *__restrict__ Aout, Geom g,
+                                                      int zc) {
+  constexpr int LXW = CTX + 4;  // words per row: x0-1 .. x0+CTX (+ padding)
+  // one row more than the tile and its halo, for the reads of the fourth lane group
+  __shared__ uint32_t sx[4][CLY + 1][LXW];
+  const ConvTile T = conv_tile(g, CTX, CTY, zc);
+  const int x0 = T.x0, y0 = T.y0, z0 = T.z0, z1 = T.z1;
   const size_t box = (size_t)g.nx * g.ny * g.nz;
-  const float *xb = x + (size_t)b * box;
+  const TIN *xb = x + (size_t)T.b * box;
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m = lane & 15, grp = lane >> 4;
   constexpr int NPT = CLY * CLX, NLD = (NPT + 255) / 256;
-  uint16_t reg[NLD];
-  auto fetch = [&](int k) {
+  TIN reg[NLD];
+  int off[NLD], lds[NLD];
 #pragma unroll
-    for (int q = 0; q < NLD; q++) {
-      const int idx = (int)threadIdx.x + q * 256;
-      reg[q] = 0;
-      if (idx >= NPT || k < 0 || k >= g.nz) continue;
-      const int ly = idx / CLX, lx = idx % CLX, gx = x0 - 1 + lx, gy = y0 - 1 + ly;
-      if (gx >= 0 && gx < g.nx && gy >= 0 && gy < g.ny) reg[q] = f2bf(xb[((size_t)k * g.ny + gy) * g.nx + gx] * scale);
-    }
+  for (int q = 0; q < NLD; q++) {
+    const int idx = (int)threadIdx.x + q * 256;
+    const int ly = idx / CLX, lx = idx % CLX, gx = x0 - 1 + lx, gy = y0 - 1 + ly;
+    off[q] = (idx < NPT && gx >= 0 && gx < g.nx && gy >= 0 && gy < g.ny) ? gy * g.nx + gx : -1;
+    lds[q] = idx < NPT ? ly * LXW + lx : -1;
+  }
+  for (int q = (int)threadIdx.x; q < 4 * (CLY + 1) * LXW; q += 256) (&sx[0][0][0])[q] = 0u;
+  __syncthreads();
+  const size_t plane = (size_t)g.nx * g.ny;
+  auto fetch = [&](int k) {
+    const TIN *xk = xb + (k >= 0 && k < g.nz ? (size_t)k * plane : 0);
+#pragma unroll
+    for (int q = 0; q < NLD; q++) reg[q] = xk[off[q] < 0 ? 0 : off[q]];
   };
   auto store = [&](int k) {
-    uint16_t *S = &sx[k & 3][0][0];
+    uint16_t *S = (uint16_t *)&sx[k & 3][0][0];
+    const bool kin = k >= 0 && k < g.nz;
 #pragma unroll
     for (int q = 0; q < NLD; q++) {
-      const int idx = (int)threadIdx.x + q * 256;
-      if (idx < NPT) S[idx] = reg[q];
+      if (lds[q] < 0) continue;
+      uint16_t v;
+      if constexpr (std::is_same<TIN, float>::value) v = (uint16_t)pk_bf16(reg[q] * scale, 0.f);
+      else v = reg[q];
+      if (!(kin && off[q] >= 0)) v = 0;
+      S[2 * lds[q]] = v;                              // low half of its own word
+      if (lds[q] % LXW > 0) S[2 * lds[q] - 1] = v;    // high half of the west neighbour's
     }
   };
-  const bf16x8 bw = *(const bf16x8 *)(Wfi + (size_t)lane * 8);
-  const float bm = bias[m];
+  bf16x4 bw[3];
+#pragma unroll
+  for (int d = 0; d < 3; d++) bw[d] = *(const bf16x4 *)(Wfi + ((size_t)d * 64 + lane) * 4);
+  const float bm = EPI == 2 ? 0.f : bias[m];
+  const uint32_t live = grp < 3 ? ~0u : 0u;
   fetch(z0 - 1);
   store(z0 - 1);
   fetch(z0);
@@ -353,99 +370,390 @@ __global__ __launch_bounds__(256) void k_conv_in_tile(const float *__restrict__ 
     fetch(z + 3);
 #pragma unroll
     for (int q = 0; q < 4; q++) {
-      const int r = 2 * w + (q >> 1), sg = q & 1;
-      uint16_t av[8];
-#pragma unroll
-      for (int j = 0; j < 8; j++) {
-        const int tap = 8 * grp + j;
-        av[j] = 0;
-        if (tap < NTAP) {
-          const int dx = tap % 3 - 1, dy = (tap / 3) % 3 - 1, dz = tap / 9 - 1;
-          av[j] = sx[(z + dz) & 3][r + 1 + dy][16 * sg + m + 1 + dx];
-        }
-      }
-      bf16x8 a;
-      __builtin_memcpy(&a, av, 16);
+      const int r = 2 * w + (q >> 1), sg = q & 1, y = y0 + r, xs = x0 + 16 * sg;
       floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bw, acc, 0, 0, 0);
-      const int y = y0 + r;
-      if (y < g.ny) {  // uniform per wave
-        const int xs = x0 + 16 * sg;
-        uint16_t v[4];
 #pragma unroll
-        for (int i = 0; i < 4; i++) v[i] = f2bf(gelu_fast(acc[i] + bm));
-        store_act16(Aout, (size_t)b * box + ((size_t)z * g.ny + y) * g.nx + xs, min(16, g.nx - xs), v);
+      for (int d = 0; d < 3; d++) {
+        // LDS column lx is the point x0 - 1 + lx: the four points from x-1 on
+        const uint32_t *S = &sx[(z + d - 1) & 3][r + grp][16 * sg + m];
+        const uint32_t aw[2] = {S[0] & live, S[2] & live & 0xffffu};
+        bf16x4 a;
+        __builtin_memcpy(&a, aw, 8);
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bw[d], acc, 0, 0, 0);
       }
+      if (y < g.ny && xs < g.nx)  // uniform per wave
+        conv_epilogue<EPI>(acc, bm, aux, Zout, Aout, (size_t)T.b * box + ((size_t)z * g.ny + y) * g.nx + xs,
+                           min(16, g.nx - xs));
     }
     __syncthreads();
   }
 }
 
-// ---------------------------------------------------------------------------
-// Weight gradient: dW[tap][ci][co] = sum_p X[p+off(tap)][ci] * dZ[p][co];
-// tap 27 is the bias (input channel 0 == 1).  Grid (nchunk, 28): block
-// (chunk, tap), 4 waves each summing every 4th group of 16 points of the
-// chunk with MFMA (M = ci, N = co, K = points), then a fixed-order fold of
-// the 4 waves into partial[chunk][tap][16][16].
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(256) void k_conv16_wgrad(const uint16_t *__restrict__ X,
-                                                      const uint16_t *__restrict__ dZ,
-                                                      float *__restrict__ partial, Geom g,
-                                                      int chunk) {
-  __shared__ float red[4][256];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int tap = blockIdx.y;
-  const int m = lane & 15, grp = lane >> 4;
-  const int dx = tap % 3 - 1, dy = (tap / 3) % 3 - 1, dz = tap / 9 - 1;
+// The last layer (16 -> 1): out[q] = sum_tap G[q + off(tap)][tap] with
+// G[p][tap] = sum_ci A[p][ci] w3[ci][tap], a product of every point's 16
+// channels with the 16 x 27 weights: two K = 16 MFMAs per 16 points instead
+// of the 14 of K = 32 that padding the single output channel to 16 takes, and
+// the activations go from global memory straight into the operand registers
+// (each input point is read once per tile, 8 bytes a lane, contiguous).  G of
+// one input plane (OIX x OIY points) lies in LDS tap by tap; every output
+// column then adds its 27 values to the three running sums of the output
+// planes z-1, z, z+1.  At 257^3: 0.34 -> 0.13 ms.
+constexpr int OIX = 32, OIY = 12, OTX = OIX - 2, OTY = OIY - 2;
+constexpr int OPTS = OIX * OIY, OSEG = OPTS / 16 / 4;  // segments per wave
+constexpr int OSTR = OPTS + 16;                        // LDS words per tap (16 mod 64: conflict-free 16-byte writes)
+static_assert(OPTS % 64 == 0, "whole segments per wave");
+__global__ __launch_bounds__(256) void k_conv_out_tile(const uint16_t *__restrict__ X,
+                                                       const uint16_t *__restrict__ Wo,
+                                                       const float *__restrict__ bias, float *__restrict__ out, Geom g,
+                                                       int zc) {
+  __shared__ float sG[NTAP * OSTR];
+  const ConvTile T = conv_tile(g, OTX, OTY, zc);
   const size_t box = (size_t)g.nx * g.ny * g.nz;
-  const size_t total = box * g.nb;
-  const size_t p0 = (size_t)blockIdx.x * chunk;
-  const size_t p1 = p0 + chunk < total ? p0 + chunk : total;
-  floatx4 acc = {0.f, 0.f, 0.f, 0.f};
-  for (size_t base = p0 + 16 * w; base < p1; base += 64) {
-    bf16x4 a = {0, 0, 0, 0}, bb = {0, 0, 0, 0};
+  const uint16_t *Xb = X + (size_t)T.b * box * NC;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m = lane & 15, grp = lane >> 4;
+  // input segment s of this wave: 16 points of row (w * OSEG + s) / 2
+  uint2 reg[OSEG];
+  int off[OSEG];
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const size_t p = base + 4 * grp + j;
-      if (p >= p1) continue;
-      bb[j] = (short)dZ[p * NC + m];
-      if (tap == NTAP) {
-        a[j] = (short)(m == 0 ? 0x3f80 : 0);  // bf16(1.0) on channel 0
-      } else {
-        const size_t q = p % box;
-        const size_t bidx = p / box;
-        const int x = (int)(q % g.nx), y = (int)((q / g.nx) % g.ny), z = (int)(q / ((size_t)g.nx * g.ny));
-        const int xx = x + dx, yy = y + dy, zz = z + dz;
-        if (xx >= 0 && xx < g.nx && yy >= 0 && yy < g.ny && zz >= 0 && zz < g.nz)
-          a[j] = (short)X[(bidx * box + ((size_t)zz * g.ny + yy) * g.nx + xx) * NC + m];
+  for (int s = 0; s < OSEG; s++) {
+    const int seg = w * OSEG + s, gy = T.y0 - 1 + seg / 2, gx = T.x0 - 1 + 16 * (seg & 1) + m;
+    off[s] = gx >= 0 && gx < g.nx && gy >= 0 && gy < g.ny ? (gy * g.nx + gx) * NC + 4 * grp : -1;
+  }
+  const size_t plane = (size_t)g.nx * g.ny * NC;
+  auto fetch = [&](int k) {
+    const uint16_t *Xk = Xb + (k >= 0 && k < g.nz ? (size_t)k * plane : 0);
+#pragma unroll
+    for (int s = 0; s < OSEG; s++) reg[s] = *(const uint2 *)(Xk + (off[s] < 0 ? 0 : off[s]));
+  };
+  const bf16x4 w0 = *(const bf16x4 *)(Wo + (size_t)lane * 4), w1 = *(const bf16x4 *)(Wo + (size_t)(64 + lane) * 4);
+  // output columns of this thread
+  constexpr int NOUT = (OTX * OTY + 255) / 256;
+  float sum[NOUT][3];
+  int col[NOUT];  // LDS position of the column's own point, or -1
+#pragma unroll
+  for (int o = 0; o < NOUT; o++) {
+    const int q = (int)threadIdx.x + o * 256, ox = q % OTX, oy = q / OTX;
+    col[o] = q < OTX * OTY && T.x0 + ox < g.nx && T.y0 + oy < g.ny ? (oy + 1) * OIX + ox + 1 : -1;
+    sum[o][0] = sum[o][1] = sum[o][2] = 0.f;
+  }
+  const float b0 = bias[0];
+  fetch(T.z0 - 1);
+  for (int k = T.z0 - 1; k <= T.z1; k++) {
+    const bool kin = k >= 0 && k < g.nz;
+    bf16x4 a[OSEG];
+#pragma unroll
+    for (int s = 0; s < OSEG; s++) {
+      const uint2 v = kin && off[s] >= 0 ? reg[s] : make_uint2(0u, 0u);
+      __builtin_memcpy(&a[s], &v, 8);
+    }
+    if (k < T.z1) fetch(k + 1);
+    __syncthreads();  // the sums of the plane before have read sG
+#pragma unroll
+    for (int s = 0; s < OSEG; s++) {
+      const floatx4 zero = {0.f, 0.f, 0.f, 0.f};
+      const floatx4 g0 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[s], w0, zero, 0, 0, 0);
+      const floatx4 g1 = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[s], w1, zero, 0, 0, 0);
+      // lane (m, grp): points 4grp .. 4grp+3 of taps m and 16 + m
+      float *S = &sG[m * OSTR + (w * OSEG + s) * 16 + 4 * grp];
+      *(floatx4 *)S = g0;
+      if (16 + m < NTAP) *(floatx4 *)(S + 16 * OSTR) = g1;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int o = 0; o < NOUT; o++) {
+      if (col[o] < 0) continue;
+      // input plane k is at dz = +1 of output plane k-1, 0 of k, -1 of k+1
+#pragma unroll
+      for (int dz = -1; dz <= 1; dz++) {
+        float v = sum[o][1 - dz];
+#pragma unroll
+        for (int dy = -1; dy <= 1; dy++)
+#pragma unroll
+          for (int dx = -1; dx <= 1; dx++)
+            v += sG[((dz + 1) * 9 + (dy + 1) * 3 + dx + 1) * OSTR + col[o] + dy * OIX + dx];
+        sum[o][1 - dz] = v;
+      }
+      if (k - 1 >= T.z0) {  // plane k-1 is complete
+        const int q = (int)threadIdx.x + o * 256;
+        out[(size_t)T.b * box + ((size_t)(k - 1) * g.ny + T.y0 + q / OTX) * g.nx + T.x0 + q % OTX] = sum[o][0] + b0;
+      }
+      sum[o][0] = sum[o][1];
+      sum[o][1] = sum[o][2];
+      sum[o][2] = 0.f;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Weight gradients: dW[tap][ci][co] = sum_p X[p+off(tap)][ci] * dZ[p][co], and
+// the bias gradient sum_p dZ[p][co] as row 27.  A GEMM per tap with the points
+// along K.  A block owns a WTX x WTY tile of (x, y) columns and marches zc
+// planes, one 32-point row of dZ per wave and step against the 9 rows of X
+// around it, all 27 taps accumulated in registers -- so every point of X and
+// dZ is read from memory once per tile, where one workgroup per tap read
+// both 28 times, 2 bytes at a time (0.70 -> 0.02 ms for 16 crops of 32^3).
+// The operands want 8 consecutive points of one channel per lane, the arrays
+// are channel-last: the planes are transposed on their way into LDS
+// ([row][channel][x], two points per word).  The taps dx = -1 and +1 of a row
+// come from the aligned 8 points and their outer neighbours by five funnel
+// shifts.  Row strides of 28 and 20 words spread the 16 channels over the
+// banks.  The waves' sums are added in wave order, one partial per block.
+//   XCH: 16 -- X is BF16 [P][16]; 1 -- X is FP32 [P] (the network's input,
+//   rounded to BF16): the taps themselves are the rows of A (27 of 32, row 27
+//   all ones for the bias), one LDS row per point row and dx.
+//   ZCH: 16 -- dZ is BF16 [P][16]; 1 -- BF16 [P], the single output channel.
+// ---------------------------------------------------------------------------
+constexpr int WTX = 32, WTY = 8, WLY = WTY + 2;
+constexpr int WXS = 56, WZS = 40;  // 2-byte elements per (row, channel) of the X and dZ planes
+
+// words of channels c .. c+7 of two neighbouring points, one word per channel
+__device__ __forceinline__ void put_pair(uint16_t *S, int stride, const uint4 &p, const uint4 &q) {
+  const unsigned pw[4] = {p.x, p.y, p.z, p.w}, qw[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    *(unsigned *)(S + (2 * c) * stride) = __builtin_amdgcn_perm(qw[c], pw[c], 0x05040100u);
+    *(unsigned *)(S + (2 * c + 1) * stride) = __builtin_amdgcn_perm(qw[c], pw[c], 0x07060302u);
+  }
+}
+
+template <int ZCH>
+__global__ __launch_bounds__(256) void k_wgrad_tile(const uint16_t *__restrict__ X, const uint16_t *__restrict__ dZ,
+                                                    float *__restrict__ partial, Geom g, int zc) {
+  // X planes k-1, k, k+1 and the plane being filled share 4 slots
+  extern __shared__ __align__(16) unsigned char wsm[];
+  uint16_t *sX = (uint16_t *)wsm;                          // [4][WLY][16][WXS]
+  uint16_t *sZ = sX + 4 * WLY * NC * WXS;                  // [2][WTY][16][WZS]
+  const ConvTile T = conv_tile(g, WTX, WTY, zc);
+  const size_t box = (size_t)g.nx * g.ny * g.nz;
+  const uint16_t *Xb = X + (size_t)T.b * box * NC;
+  const uint16_t *Zb = dZ + (size_t)T.b * box * ZCH;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m = lane & 15, grp = lane >> 4;
+  const uint4 zero4 = make_uint4(0u, 0u, 0u, 0u);
+  // staging tasks: a pair of points (x even relative to the tile) of one row, 8 channels
+  constexpr int XPAIR = WTX / 2 + 2, NXT = (WLY * XPAIR * 2 + 255) / 256;
+  uint4 xp[NXT], xq[NXT], zp, zq;
+  auto fetch_x = [&](int k) {
+    const bool kin = k >= 0 && k < g.nz;
+#pragma unroll
+    for (int t = 0; t < NXT; t++) {
+      const int idx = (int)threadIdx.x + t * 256, h = idx & 1, pr = (idx >> 1) % XPAIR, row = (idx >> 1) / XPAIR;
+      const int gy = T.y0 - 1 + row, gx = T.x0 - 2 + 2 * pr;
+      const bool ok = kin && row < WLY && gy >= 0 && gy < g.ny;
+      const size_t at = ok ? (((size_t)k * g.ny + gy) * g.nx) * NC + 8 * h : 0;
+      xp[t] = ok && gx >= 0 && gx < g.nx ? *(const uint4 *)(Xb + at + (size_t)gx * NC) : zero4;
+      xq[t] = ok && gx + 1 >= 0 && gx + 1 < g.nx ? *(const uint4 *)(Xb + at + (size_t)(gx + 1) * NC) : zero4;
+    }
+  };
+  auto store_x = [&](int k) {
+    uint16_t *S = sX + (size_t)(k & 3) * WLY * NC * WXS;
+#pragma unroll
+    for (int t = 0; t < NXT; t++) {
+      const int idx = (int)threadIdx.x + t * 256, h = idx & 1, pr = (idx >> 1) % XPAIR, row = (idx >> 1) / XPAIR;
+      if (row < WLY) put_pair(S + ((size_t)row * NC + 8 * h) * WXS + 6 + 2 * pr, WXS, xp[t], xq[t]);
+    }
+  };
+  auto fetch_z = [&](int k) {
+    if constexpr (ZCH == 16) {
+      const int h = threadIdx.x & 1, pr = (threadIdx.x >> 1) % (WTX / 2), row = (threadIdx.x >> 1) / (WTX / 2);
+      const int gy = T.y0 + row, gx = T.x0 + 2 * pr;
+      const bool ok = k < T.z1 && gy < g.ny;
+      const size_t at = ok ? (((size_t)k * g.ny + gy) * g.nx) * NC + 8 * h : 0;
+      zp = ok && gx < g.nx ? *(const uint4 *)(Zb + at + (size_t)gx * NC) : zero4;
+      zq = ok && gx + 1 < g.nx ? *(const uint4 *)(Zb + at + (size_t)(gx + 1) * NC) : zero4;
+    } else {
+      const int x = threadIdx.x % WTX, row = threadIdx.x / WTX, gy = T.y0 + row, gx = T.x0 + x;
+      const bool ok = k < T.z1 && gy < g.ny && gx < g.nx;
+      zp.x = ok ? Zb[((size_t)k * g.ny + gy) * g.nx + gx] : 0u;
+    }
+  };
+  auto store_z = [&](int k) {
+    uint16_t *S = sZ + (size_t)(k & 1) * WTY * NC * WZS;
+    if constexpr (ZCH == 16) {
+      const int h = threadIdx.x & 1, pr = (threadIdx.x >> 1) % (WTX / 2), row = (threadIdx.x >> 1) / (WTX / 2);
+      put_pair(S + ((size_t)row * NC + 8 * h) * WZS + 2 * pr, WZS, zp, zq);
+    } else {
+      S[(size_t)(threadIdx.x / WTX) * NC * WZS + threadIdx.x % WTX] = (uint16_t)zp.x;
+    }
+  };
+  static_assert(WTX * WTY == 256, "one dZ task per thread");
+  floatx4 acc[NTAP + 1];
+#pragma unroll
+  for (int t = 0; t <= NTAP; t++) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
+  bf16x8 ones = {};
+  if (m == 0)
+    for (int j = 0; j < 8; j++) ones[j] = (__bf16)1.0f;
+  auto u4 = [](unsigned a, unsigned b, unsigned c, unsigned d) {
+    const unsigned v[4] = {a, b, c, d};
+    bf16x8 r;
+    __builtin_memcpy(&r, v, 16);
+    return r;
+  };
+  fetch_x(T.z0 - 1);
+  store_x(T.z0 - 1);
+  fetch_x(T.z0);
+  store_x(T.z0);
+  fetch_x(T.z0 + 1);
+  store_x(T.z0 + 1);
+  fetch_z(T.z0);
+  store_z(T.z0);
+  __syncthreads();
+  for (int k = T.z0; k < T.z1; k++) {
+    // the next planes' loads are in flight through this step's products and go
+    // into slots that no wave reads in it
+    fetch_x(k + 2);
+    fetch_z(k + 1);
+#pragma unroll
+    for (int rr = 0; rr < WTY / 4; rr++) {
+      const int row = w * (WTY / 4) + rr;
+      bf16x8 bz = *(const bf16x8 *)(sZ + ((size_t)((k & 1) * WTY + row) * NC + (ZCH == 16 ? m : 0)) * WZS + 8 * grp);
+      if (ZCH == 1 && m != 0) bz = bf16x8{};
+      acc[NTAP] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, bz, acc[NTAP], 0, 0, 0);
+#pragma unroll
+      for (int dzy = 0; dzy < 9; dzy++) {
+        const int slot = (k + dzy / 3 - 1) & 3, xr = row + dzy % 3;
+        const uint16_t *S = sX + ((size_t)(slot * WLY + xr) * NC + m) * WXS + 8 + 8 * grp;
+        const uint4 v = *(const uint4 *)S;
+        const unsigned wl = *(const unsigned *)(S - 2), wr = *(const unsigned *)(S + 8);
+        const unsigned a0 = __builtin_amdgcn_alignbit(v.x, wl, 16), a1 = __builtin_amdgcn_alignbit(v.y, v.x, 16),
+                       a2 = __builtin_amdgcn_alignbit(v.z, v.y, 16), a3 = __builtin_amdgcn_alignbit(v.w, v.z, 16),
+                       a4 = __builtin_amdgcn_alignbit(wr, v.w, 16);
+        acc[3 * dzy] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(u4(a0, a1, a2, a3), bz, acc[3 * dzy], 0, 0, 0);
+        acc[3 * dzy + 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(u4(v.x, v.y, v.z, v.w), bz, acc[3 * dzy + 1], 0, 0, 0);
+        acc[3 * dzy + 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(u4(a1, a2, a3, a4), bz, acc[3 * dzy + 2], 0, 0, 0);
       }
     }
-    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bb, acc, 0, 0, 0);
+    store_x(k + 2);
+    store_z(k + 1);
+    __syncthreads();
   }
-  // lane holds D[ci = 4*grp + i][co = m]
+  // lane holds D[ci = 4grp + i][co = m]; the waves' sums in wave order
+  float *red = (float *)wsm;
+  for (int ww = 0; ww < 4; ww++) {
+    if (w == ww) {
 #pragma unroll
-  for (int i = 0; i < 4; i++) red[w][(4 * grp + i) * 16 + m] = acc[i];
+      for (int t = 0; t <= NTAP; t++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          float *r = red + t * 256 + (4 * grp + i) * 16 + m;
+          *r = ww == 0 ? acc[t][i] : *r + acc[t][i];
+        }
+    }
+    __syncthreads();
+  }
+  float *out = partial + (size_t)blockIdx.x * LAYER_FLOATS;
+  for (int e = threadIdx.x; e < LAYER_FLOATS; e += 256) out[e] = red[e];
+}
+constexpr size_t kWgradLds = (4 * (size_t)WLY * NC * WXS + 2 * (size_t)WTY * NC * WZS) * sizeof(uint16_t);
+static_assert(kWgradLds >= LAYER_FLOATS * sizeof(float), "the wave sums reuse the planes' LDS");
+
+// layer 1: the taps are the rows of A (two MFMAs per 32 points)
+__global__ __launch_bounds__(256) void k_wgrad_in_tile(const float *__restrict__ x, const uint16_t *__restrict__ dZ,
+                                                       float *__restrict__ partial, Geom g, int zc) {
+  constexpr int XS = 40;  // elements per row; copy d holds the points shifted by d - 1
+  __shared__ __align__(16) uint16_t sX[4][3][WLY][XS];
+  __shared__ __align__(16) uint16_t sZ[2][WTY][NC][WZS];
+  __shared__ float red[2 * 256];
+  const ConvTile T = conv_tile(g, WTX, WTY, zc);
+  const size_t box = (size_t)g.nx * g.ny * g.nz;
+  const float *xb = x + (size_t)T.b * box;
+  const uint16_t *Zb = dZ + (size_t)T.b * box * NC;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m = lane & 15, grp = lane >> 4;
+  const uint4 zero4 = make_uint4(0u, 0u, 0u, 0u);
+  constexpr int LXP = WTX + 2, NXT = (WLY * LXP + 255) / 256;
+  auto stage_x = [&](int k) {
+    float v[NXT];
+#pragma unroll
+    for (int t = 0; t < NXT; t++) {
+      const int idx = (int)threadIdx.x + t * 256, row = idx / LXP, gy = T.y0 - 1 + row, gx = T.x0 - 1 + idx % LXP;
+      v[t] = k >= 0 && k < g.nz && row < WLY && gy >= 0 && gy < g.ny && gx >= 0 && gx < g.nx
+                 ? xb[((size_t)k * g.ny + gy) * g.nx + gx] : 0.f;
+    }
+#pragma unroll
+    for (int t = 0; t < NXT; t++) {
+      const int idx = (int)threadIdx.x + t * 256, row = idx / LXP, lx = idx % LXP;
+      if (row >= WLY) continue;
+      const uint16_t h = (uint16_t)pk_bf16(v[t], 0.f);
+      // the point x0 - 1 + lx is element p + (d - 1) of copy d at p = lx - d
+#pragma unroll
+      for (int d = 0; d < 3; d++)
+        if (lx - d >= 0 && lx - d < WTX) sX[k & 3][d][row][lx - d] = h;
+    }
+  };
+  auto stage_z = [&](int k) {
+    const int h = threadIdx.x & 1, pr = (threadIdx.x >> 1) % (WTX / 2), row = (threadIdx.x >> 1) / (WTX / 2);
+    const int gy = T.y0 + row, gx = T.x0 + 2 * pr;
+    const bool ok = k < T.z1 && gy < g.ny;
+    const size_t at = ok ? (((size_t)k * g.ny + gy) * g.nx) * NC + 8 * h : 0;
+    const uint4 p = ok && gx < g.nx ? *(const uint4 *)(Zb + at + (size_t)gx * NC) : zero4;
+    const uint4 q = ok && gx + 1 < g.nx ? *(const uint4 *)(Zb + at + (size_t)(gx + 1) * NC) : zero4;
+    put_pair(&sZ[k & 1][row][8 * h][2 * pr], WZS, p, q);
+  };
+  floatx4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  bf16x8 ones;
+  for (int j = 0; j < 8; j++) ones[j] = (__bf16)1.0f;
+  stage_x(T.z0 - 1);
+  stage_x(T.z0);
+  stage_x(T.z0 + 1);
+  stage_z(T.z0);
   __syncthreads();
-  const int e = threadIdx.x;  // 256 entries
-  const float v = ((red[0][e] + red[1][e]) + red[2][e]) + red[3][e];
-  partial[((size_t)blockIdx.x * (NTAP + 1) + tap) * 256 + e] = v;
+  for (int k = T.z0; k < T.z1; k++) {
+    if (k + 1 < T.z1) {
+      stage_x(k + 2);
+      stage_z(k + 1);
+    }
+#pragma unroll
+    for (int rr = 0; rr < WTY / 4; rr++) {
+      const int row = w * (WTY / 4) + rr;
+      const bf16x8 bz = *(const bf16x8 *)&sZ[k & 1][row][m][8 * grp];
+#pragma unroll
+      for (int h = 0; h < 2; h++) {
+        const int tap = 16 * h + m, tp = tap < NTAP ? tap : 0;
+        bf16x8 a = *(const bf16x8 *)&sX[(k + tp / 9 - 1) & 3][tp % 3][row + (tp / 3) % 3][8 * grp];
+        if (tap >= NTAP) a = tap == NTAP ? ones : bf16x8{};
+        acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bz, acc[h], 0, 0, 0);
+      }
+    }
+    __syncthreads();
+  }
+  for (int ww = 0; ww < 4; ww++) {
+    if (w == ww)
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          float *r = red + (16 * h + 4 * grp + i) * 16 + m;
+          *r = ww == 0 ? acc[h][i] : *r + acc[h][i];
+        }
+    __syncthreads();
+  }
+  // only input channel 0 (row 0 of every tap, and the bias row) has gradients
+  float *out = partial + (size_t)blockIdx.x * LAYER_FLOATS;
+  for (int e = threadIdx.x; e < LAYER_FLOATS; e += 256) out[e] = e % 256 < 16 ? red[(e / 256) * 16 + e % 256] : 0.f;
 }
 
-// fold partials over chunks (fixed order) -> grad[28][256]
-__global__ __launch_bounds__(256) void k_fold_wgrad(const float *__restrict__ partial,
-                                                    float *__restrict__ grad, int nchunk) {
-  const int tap = blockIdx.x, e = threadIdx.x;
+// fold of the blocks' partials -> grad[28][256]: a block takes 64 entries, its
+// 16 waves every 16th partial (64 neighbouring words a load), then the waves'
+// sums in order (deterministic for a fixed launch shape)
+__global__ __launch_bounds__(1024) void k_fold_wgrad(const float *__restrict__ partial, float *__restrict__ grad,
+                                                     int nblk) {
+  __shared__ float red[16][64];
+  const int e = blockIdx.x * 64 + (threadIdx.x & 63), w = threadIdx.x >> 6;
   float s = 0.f;
-  for (int c = 0; c < nchunk; c++) s += partial[((size_t)c * (NTAP + 1) + tap) * 256 + e];
-  grad[tap * 256 + e] = s;
+  for (int c = w; c < nblk; c += 16) s += partial[(size_t)c * LAYER_FLOATS + e];
+  red[w][threadIdx.x & 63] = s;
+  __syncthreads();
+  if (w == 0) {
+    for (int c = 1; c < 16; c++) s += red[c][threadIdx.x];
+    grad[e] = s;
+  }
 }
 
-// loss = 0.5 * mean over counted points of (Z[p][0] - T[p])^2 ; dZ[p][0] =
-// (Z - T)/count (bf16), other channels 0.  Points within `margin` of a box
+// loss = 0.5 * mean over counted points of (Y[p] - T[p])^2; dY[p] =
+// (Y - T)/count (bf16).  Points within `margin` of a box
 // face are not counted.  Per-block partial sums of the squared error.
-__global__ __launch_bounds__(256) void k_loss(const float *__restrict__ Z, const float *__restrict__ T,
+__global__ __launch_bounds__(256) void k_loss(const float *__restrict__ Y, const float *__restrict__ T,
                                               const float *__restrict__ W, const double *__restrict__ wcount,
-                                              uint16_t *__restrict__ dZ, double *__restrict__ part,
+                                              uint16_t *__restrict__ dY, double *__restrict__ part,
                                               Geom g, int margin, double inv_count) {
   // W (optional): per-point weights 0/1 on top of the margin rule; the
   // mean then runs over the weighted points, whose count *wcount holds
@@ -462,12 +770,10 @@ __global__ __launch_bounds__(256) void k_loss(const float *__restrict__ Z, const
     if (W) on = on && W[p] != 0.f;
     float d = 0.f;
     if (on) {
-      d = Z[p * NC] - T[p];
+      d = Y[p] - T[p];
       e2 = (double)d * (double)d;
     }
-    dZ[p * NC] = f2bf((float)(d * inv_count));
-#pragma unroll
-    for (int c = 1; c < NC; c++) dZ[p * NC + c] = 0;
+    dY[p] = f2bf((float)(d * inv_count));
   }
   red[threadIdx.x] = e2;
   __syncthreads();
@@ -514,22 +820,6 @@ __global__ __launch_bounds__(256) void k_fold_d(const double *__restrict__ part,
   if (threadIdx.x == 0) out[0] = red[0];
 }
 
-// input packing: X[p][0] = bf16(src[p] * scale), channels 1..15 = 0
-template <typename TS>
-__global__ __launch_bounds__(256) void k_pack_input(const TS *__restrict__ src, uint16_t *__restrict__ X,
-                                                    size_t n, float scale) {
-  const size_t p = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (p >= n) return;
-  bf16x4 v = {0, 0, 0, 0};
-  v[0] = (short)f2bf((float)src[p] * scale);
-  const bf16x4 zero = {0, 0, 0, 0};
-  bf16x4 *d = (bf16x4 *)(X + p * NC);
-  d[0] = v;
-  d[1] = zero;
-  d[2] = zero;
-  d[3] = zero;
-}
-
 // Adam on FP32 master weights (only the entries `mask` marks trainable)
 __global__ __launch_bounds__(256) void k_adam(float *__restrict__ w, float *__restrict__ m1,
                                               float *__restrict__ m2, const float *__restrict__ gr,
@@ -545,40 +835,39 @@ __global__ __launch_bounds__(256) void k_adam(float *__restrict__ w, float *__re
   w[i] -= lr * (a / c1) / (sqrtf(b / c2) + eps);
 }
 
-// master layout per layer: W[tap][ci][co] (27*256 floats) then bias[co]
-// (16 floats), i.e. 28 rows of 256 with the bias in row 27, entries 0..15
-constexpr int LAYER_FLOATS = (NTAP + 1) * 256;
-
-// fragments: forward Wf[tap][lane][j] = W[tap][4*(lane/16)+j][lane%16];
-// backward-data (flipped taps, transposed): Wb[tap][lane][j] =
-// W[26-tap][lane%16][4*(lane/16)+j]
-__global__ __launch_bounds__(256) void k_pack_frags(const float *__restrict__ W, uint16_t *__restrict__ Wf,
-                                                    uint16_t *__restrict__ Wb) {
-  const int idx = blockIdx.x * 256 + threadIdx.x;  // over 27*64*4
-  if (idx >= NTAP * 64 * 4) return;
-  const int tap = idx / 256, lane = (idx / 4) % 64, j = idx % 4;
-  const int m = lane & 15, grp = lane >> 4;
-  Wf[idx] = f2bf(W[tap * 256 + (4 * grp + j) * 16 + m]);
-  Wb[idx] = f2bf(W[(26 - tap) * 256 + m * 16 + (4 * grp + j)]);
-}
-
-// inference fragments for the K = 32 MFMA.  Layer 1 (K = taps of input
-// channel 0): Wfi[lane][j] = W[tap = 8(lane/16) + j][ci 0][co lane%16], 0 past
-// tap 26.  Hidden / last layer (K = a tap pair x 16 channels):
-// Wp[pr][lane][j] = W[tap = 2 pr + (lane/16)/2][ci = 8((lane/16)%2) + j][co lane%16]
-__global__ __launch_bounds__(256) void k_pack_frags_in(const float *__restrict__ W, uint16_t *__restrict__ Wfi) {
-  const int idx = blockIdx.x * 256 + threadIdx.x;  // over 64*8
-  if (idx >= 64 * 8) return;
-  const int lane = idx / 8, j = idx % 8;
-  const int tap = 8 * (lane >> 4) + j;
-  Wfi[idx] = tap < NTAP ? f2bf(W[tap * 256 + (lane & 15)]) : (uint16_t)0;
-}
-__global__ __launch_bounds__(256) void k_pack_frags_pair(const float *__restrict__ W, uint16_t *__restrict__ Wp) {
-  const int idx = blockIdx.x * 256 + threadIdx.x;  // over NPAIR*64*8
-  if (idx >= NPAIR * 64 * 8) return;
-  const int pr = idx / 512, lane = (idx / 8) % 64, j = idx % 8, grp = lane >> 4;
-  const int tap = 2 * pr + (grp >> 1), ci = 8 * (grp & 1) + j;
-  Wp[idx] = tap < NTAP ? f2bf(W[tap * 256 + ci * 16 + (lane & 15)]) : (uint16_t)0;
+// MFMA weight fragments of all three layers, packed by one launch
+// (lane l: m = l%16, grp = l/16):
+//   wfi   layer 1, one input channel (K = 16 per dz): [dz][lane][j] =
+//         W1[tap (dx = j-1, dy = grp-1, dz)][ci 0][co m], 0 for j = 3 or grp = 3
+//   wbi   backward data of layer 3, the same with flipped taps and the single
+//         output channel as input: W3[26 - tap][ci m][co 0]
+//   wp2   layer 2, tap pairs (K = 32): [pr][lane][j] =
+//         W2[2 pr + grp/2][ci 8(grp%2) + j][co m], 0 past tap 26
+//   wpb2  its backward data: W2[26 - tap][ci m][co 8(grp%2) + j]
+//   wo3   layer 3 with the taps as columns (K = 16 channels): [h][lane][j] =
+//         W3[tap 16 h + m][ci 4 grp + j][co 0], 0 past tap 26
+constexpr int FR_IN = 3 * 64 * 4, FR_PAIR = NPAIR * 64 * 8, FR_OUT = 2 * 64 * 4;
+constexpr int FR_WFI = 0, FR_WBI = FR_WFI + FR_IN, FR_WP2 = FR_WBI + FR_IN, FR_WPB2 = FR_WP2 + FR_PAIR,
+              FR_WO3 = FR_WPB2 + FR_PAIR, FR_TOTAL = FR_WO3 + FR_OUT;
+__global__ __launch_bounds__(256) void k_pack_frags(const float *__restrict__ W, uint16_t *__restrict__ F) {
+  const int idx = blockIdx.x * 256 + threadIdx.x;
+  if (idx >= FR_TOTAL) return;
+  const float *W1 = W, *W2 = W + LAYER_FLOATS, *W3 = W + 2 * LAYER_FLOATS;
+  float v = 0.f;
+  if (idx < FR_WP2) {
+    const int q = idx % FR_IN, d = q / 256, lane = (q / 4) % 64, j = q % 4, m = lane & 15, grp = lane >> 4;
+    const int tap = d * 9 + grp * 3 + j;
+    if (j < 3 && grp < 3) v = idx < FR_WBI ? W1[tap * 256 + m] : W3[(26 - tap) * 256 + m * 16];
+  } else if (idx < FR_WO3) {
+    const int q = (idx - FR_WP2) % FR_PAIR, pr = q / 512, lane = (q / 8) % 64, j = q % 8, m = lane & 15, grp = lane >> 4;
+    const int tap = 2 * pr + (grp >> 1), k = 8 * (grp & 1) + j;
+    if (tap < NTAP) v = idx < FR_WPB2 ? W2[tap * 256 + k * 16 + m] : W2[(26 - tap) * 256 + m * 16 + k];
+  } else {
+    const int q = idx - FR_WO3, h = q / 256, lane = (q / 4) % 64, j = q % 4, m = lane & 15, grp = lane >> 4;
+    const int tap = 16 * h + m;
+    if (tap < NTAP) v = W3[tap * 256 + (4 * grp + j) * 16];
+  }
+  F[idx] = f2bf(v);
 }
 
 // u += coef * Z[p * STRIDE] at interior points of the grid (box = the grid)
@@ -603,14 +892,14 @@ struct pmg_net {
   float *w = nullptr;       // 3 layers * LAYER_FLOATS master weights (device)
   float *m1 = nullptr, *m2 = nullptr, *grad = nullptr;
   uint8_t *mask = nullptr;  // trainable entries
-  uint16_t *wf = nullptr, *wb = nullptr;  // 3 layers * 27*64*4 fragments each
-  uint16_t *wfi = nullptr;                // layer 1 with K = taps (inference path), 64*8
-  uint16_t *wp = nullptr;                 // hidden and last layer, tap pairs: 2 * NPAIR*64*8
+  uint16_t *fr = nullptr;   // weight fragments (k_pack_frags)
   int adam_t = 0;
-  // activation buffers (grown on demand): X0, A1, A2, dA (bf16 [P][16]); Z1, Z2, Z3, dZ (fp32)
+  // training buffers (grown on demand): activations and their gradients (BF16
+  // [P][16]), pre-activations (FP32 [P][16]), output (FP32 [P]) and its
+  // gradient (BF16 [P])
   size_t cap = 0;
-  uint16_t *x0 = nullptr, *a1 = nullptr, *a2 = nullptr, *d16 = nullptr, *d16b = nullptr;
-  float *z1 = nullptr, *z2 = nullptr, *z3 = nullptr, *dz = nullptr;
+  uint16_t *a1 = nullptr, *a2 = nullptr, *d16 = nullptr, *d16b = nullptr, *dy = nullptr;
+  float *z1 = nullptr, *z2 = nullptr, *yt = nullptr;
   // inference buffers (their own capacity: inference allocates no training buffers)
   size_t icap = 0;
   uint16_t *ia1 = nullptr, *ia2 = nullptr;  // bf16 [P][16]
@@ -628,19 +917,21 @@ namespace {
 int net_ensure(pmg_net *N, size_t P) {
   if (P <= N->cap) return 0;
   PMG_HOST_CHECK(hipStreamSynchronize(N->stream));
-  for (void *p : {(void *)N->x0, (void *)N->a1, (void *)N->a2, (void *)N->d16, (void *)N->d16b,
-                  (void *)N->z1, (void *)N->z2, (void *)N->z3, (void *)N->dz})
-    if (p) PMG_HOST_CHECK(hipFree(p));
+  N->cap = 0;
+  for (void **p : {(void **)&N->a1, (void **)&N->a2, (void **)&N->d16, (void **)&N->d16b, (void **)&N->dy,
+                   (void **)&N->z1, (void **)&N->z2, (void **)&N->yt}) {
+    if (*p) PMG_HOST_CHECK(hipFree(*p));
+    *p = nullptr;
+  }
   const size_t b16 = P * NC * sizeof(uint16_t), b32 = P * NC * sizeof(float);
-  PMG_HOST_CHECK(hipMalloc(&N->x0, b16));
   PMG_HOST_CHECK(hipMalloc(&N->a1, b16));
   PMG_HOST_CHECK(hipMalloc(&N->a2, b16));
   PMG_HOST_CHECK(hipMalloc(&N->d16, b16));
   PMG_HOST_CHECK(hipMalloc(&N->d16b, b16));
+  PMG_HOST_CHECK(hipMalloc(&N->dy, P * sizeof(uint16_t)));
   PMG_HOST_CHECK(hipMalloc(&N->z1, b32));
   PMG_HOST_CHECK(hipMalloc(&N->z2, b32));
-  PMG_HOST_CHECK(hipMalloc(&N->z3, b32));
-  PMG_HOST_CHECK(hipMalloc(&N->dz, b32));
+  PMG_HOST_CHECK(hipMalloc(&N->yt, P * sizeof(float)));
   N->cap = P;
   return 0;
 }
@@ -659,85 +950,93 @@ int net_ensure_infer(pmg_net *N, size_t P) {
 
 int net_frags(pmg_net *N) {
   if (N->frags_valid) return 0;
-  for (int l = 0; l < 3; l++) {
-    hipLaunchKernelGGL(k_pack_frags, dim3((NTAP * 256 + 255) / 256), dim3(256), 0, N->stream,
-                       N->w + (size_t)l * LAYER_FLOATS, N->wf + (size_t)l * NTAP * 256,
-                       N->wb + (size_t)l * NTAP * 256);
-  }
-  hipLaunchKernelGGL(k_pack_frags_in, dim3(2), dim3(256), 0, N->stream, N->w, N->wfi);
-  for (int l = 1; l < 3; l++)
-    hipLaunchKernelGGL(k_pack_frags_pair, dim3((NPAIR * 512 + 255) / 256), dim3(256), 0, N->stream,
-                       N->w + (size_t)l * LAYER_FLOATS, N->wp + (size_t)(l - 1) * NPAIR * 512);
+  hipLaunchKernelGGL(k_pack_frags, dim3((FR_TOTAL + 255) / 256), dim3(256), 0, N->stream, N->w, N->fr);
   PMG_HOST_CHECK(hipGetLastError());
   N->frags_valid = true;
   return 0;
 }
 
-dim3 conv_grid(const Geom &g) { return dim3((g.nx + 15) / 16, (g.ny + 3) / 4, g.nz * g.nb); }
+const float *net_bias(const pmg_net *N, int layer) { return N->w + (size_t)layer * LAYER_FLOATS + NTAP * 256; }
 
-// z planes one block of the LDS-tiled inference kernels marches
-constexpr int kTilePlanes = 16;
+// z planes one block of a tiled kernel marches: long marches re-read fewer
+// halo planes, short ones give a small batch enough workgroups -- the longest
+// of 16, 8, 4 that still makes `want` of them
+int conv_zc(const Geom &g, int tx, int ty, unsigned want) {
+  int zc = 16;
+  while (zc > 4 && conv_blocks(g, tx, ty, zc) < want) zc /= 2;
+  return zc;
+}
+constexpr unsigned kConvBlocks = 768;  // three workgroups a CU, what the hidden layer's LDS allows
+constexpr unsigned kWgradBlocks = 256;  // one workgroup a CU (their planes take 92 KB of LDS)
 
-// inference: N(scale * x) into N->y (one FP32 per point).  Layer 1 reads x
-// directly (K = taps), the hidden layer keeps only the BF16 activations, the
-// last layer writes channel 0 only -- no pre-activations are stored
-int net_infer(pmg_net *N, const float *x, float scale, const Geom &g) {
+// inference: N(scale * x) into y (one FP32 per point).  Layer 1 reads x
+// directly, the hidden layer keeps only the BF16 activations, the last layer
+// writes its one channel -- no pre-activations are stored
+int net_infer(pmg_net *N, const float *x, float scale, float *y, const Geom &g) {
   int rc;
   if ((rc = net_frags(N))) return rc;
-  const float *b1 = N->w + 0 * LAYER_FLOATS + NTAP * 256;
-  const float *b2 = N->w + 1 * LAYER_FLOATS + NTAP * 256;
-  const float *b3 = N->w + 2 * LAYER_FLOATS + NTAP * 256;
-  constexpr int TZ = kTilePlanes;
-  const dim3 gt((unsigned)(((g.nx + CTX - 1) / CTX) * ((g.ny + CTY - 1) / CTY) * ((g.nz + TZ - 1) / TZ) * g.nb));
-  hipLaunchKernelGGL(k_conv_in_tile<TZ>, gt, dim3(256), 0, N->stream, x, scale, N->wfi, b1, N->ia1, g);
-  hipLaunchKernelGGL((k_conv16_tile<3, TZ>), gt, dim3(256), 0, N->stream, N->ia1, N->wp, b2, (float *)nullptr,
-                     N->ia2, g);
-  hipLaunchKernelGGL((k_conv16_tile<4, TZ>), gt, dim3(256), 0, N->stream, N->ia2, N->wp + NPAIR * 512, b3, N->y,
-                     (uint16_t *)nullptr, g);
+  const int zc = conv_zc(g, CTX, CTY, kConvBlocks), zo = conv_zc(g, OTX, OTY, kConvBlocks);
+  const dim3 gt(conv_blocks(g, CTX, CTY, zc)), blk(256);
+  hipLaunchKernelGGL((k_conv_in_tile<float, 3>), gt, blk, 0, N->stream, x, scale, N->fr + FR_WFI, net_bias(N, 0),
+                     (const float *)nullptr, (float *)nullptr, N->ia1, g, zc);
+  hipLaunchKernelGGL(k_conv16_tile<3>, gt, blk, 0, N->stream, N->ia1, N->fr + FR_WP2, net_bias(N, 1),
+                     (const float *)nullptr, (float *)nullptr, N->ia2, g, zc);
+  hipLaunchKernelGGL(k_conv_out_tile, dim3(conv_blocks(g, OTX, OTY, zo)), blk, 0, N->stream, N->ia2, N->fr + FR_WO3,
+                     net_bias(N, 2), y, g, zo);
   PMG_HOST_CHECK(hipGetLastError());
   return 0;
 }
 
-// forward of the 3 layers on X0 (already packed); Z3[p][0] is the output
-int net_forward(pmg_net *N, const Geom &g) {
+// training forward of the 3 layers on x into y, keeping pre-activations and
+// activations
+int net_forward(pmg_net *N, const float *x, float *y, const Geom &g) {
   int rc;
   if ((rc = net_frags(N))) return rc;
-  const dim3 gr = conv_grid(g);
-  const float *b1 = N->w + 0 * LAYER_FLOATS + NTAP * 256;
-  const float *b2 = N->w + 1 * LAYER_FLOATS + NTAP * 256;
-  const float *b3 = N->w + 2 * LAYER_FLOATS + NTAP * 256;
-  hipLaunchKernelGGL(k_conv16<0>, gr, dim3(256), 0, N->stream, N->x0, N->wf, b1, (const float *)nullptr,
-                     N->z1, N->a1, g);
-  hipLaunchKernelGGL(k_conv16<0>, gr, dim3(256), 0, N->stream, N->a1, N->wf + NTAP * 256, b2,
-                     (const float *)nullptr, N->z2, N->a2, g);
-  hipLaunchKernelGGL(k_conv16<1>, gr, dim3(256), 0, N->stream, N->a2, N->wf + 2 * NTAP * 256, b3,
-                     (const float *)nullptr, N->z3, (uint16_t *)nullptr, g);
+  const int zc = conv_zc(g, CTX, CTY, kConvBlocks), zo = conv_zc(g, OTX, OTY, kConvBlocks);
+  const dim3 gt(conv_blocks(g, CTX, CTY, zc)), blk(256);
+  hipLaunchKernelGGL((k_conv_in_tile<float, 0>), gt, blk, 0, N->stream, x, 1.0f, N->fr + FR_WFI, net_bias(N, 0),
+                     (const float *)nullptr, N->z1, N->a1, g, zc);
+  hipLaunchKernelGGL(k_conv16_tile<0>, gt, blk, 0, N->stream, N->a1, N->fr + FR_WP2, net_bias(N, 1),
+                     (const float *)nullptr, N->z2, N->a2, g, zc);
+  hipLaunchKernelGGL(k_conv_out_tile, dim3(conv_blocks(g, OTX, OTY, zo)), blk, 0, N->stream, N->a2, N->fr + FR_WO3,
+                     net_bias(N, 2), y, g, zo);
   PMG_HOST_CHECK(hipGetLastError());
   return 0;
 }
 
-int net_wgrad(pmg_net *N, const Geom &g, const uint16_t *X, const uint16_t *dZ, float *grad_out) {
-  const size_t total = (size_t)g.nx * g.ny * g.nz * g.nb;
-  const int chunk = 4096;
-  const int nchunk = (int)((total + chunk - 1) / chunk);
-  const size_t need = (size_t)nchunk * (NTAP + 1) * 256;
+// weight gradients of layer l (0, 1, 2) into N->grad
+int net_wgrad(pmg_net *N, const Geom &g, int l, const float *x) {
+  const int zc = conv_zc(g, WTX, WTY, kWgradBlocks);
+  const unsigned nblk = conv_blocks(g, WTX, WTY, zc);
+  const size_t need = (size_t)nblk * LAYER_FLOATS;
   if (need > N->partial_cap) {
     PMG_HOST_CHECK(hipStreamSynchronize(N->stream));
+    N->partial_cap = 0;
     if (N->partial) PMG_HOST_CHECK(hipFree(N->partial));
+    N->partial = nullptr;
     PMG_HOST_CHECK(hipMalloc(&N->partial, need * sizeof(float)));
     N->partial_cap = need;
   }
-  hipLaunchKernelGGL(k_conv16_wgrad, dim3(nchunk, NTAP + 1), dim3(256), 0, N->stream, X, dZ, N->partial, g,
-                     chunk);
-  hipLaunchKernelGGL(k_fold_wgrad, dim3(NTAP + 1), dim3(256), 0, N->stream, N->partial, grad_out, nchunk);
+  if (l == 0) {
+    hipLaunchKernelGGL(k_wgrad_in_tile, dim3(nblk), dim3(256), 0, N->stream, x, N->d16, N->partial, g, zc);
+  } else if (l == 1) {
+    hipLaunchKernelGGL(k_wgrad_tile<16>, dim3(nblk), dim3(256), kWgradLds, N->stream, N->a1, N->d16b, N->partial, g,
+                       zc);
+  } else {
+    hipLaunchKernelGGL(k_wgrad_tile<1>, dim3(nblk), dim3(256), kWgradLds, N->stream, N->a2, N->dy, N->partial, g, zc);
+  }
+  PMG_HOST_CHECK(hipGetLastError());
+  hipLaunchKernelGGL(k_fold_wgrad, dim3(LAYER_FLOATS / 64), dim3(1024), 0, N->stream, N->partial,
+                     N->grad + (size_t)l * LAYER_FLOATS, (int)nblk);
   PMG_HOST_CHECK(hipGetLastError());
   return 0;
 }
 
 // forward + loss + backward; gradients into N->grad (3 * LAYER_FLOATS)
-int net_loss_backward(pmg_net *N, const Geom &g, const float *T, const float *W, int margin, double *loss_out) {
+int net_loss_backward(pmg_net *N, const Geom &g, const float *x, const float *T, const float *W, int margin,
+                      double *loss_out) {
   int rc;
-  if ((rc = net_forward(N, g))) return rc;
+  if ((rc = net_forward(N, x, N->yt, g))) return rc;
   const size_t total = (size_t)g.nx * g.ny * g.nz * g.nb;
   const int nblk = (int)((total + 255) / 256);
   if ((size_t)nblk > N->lpart_cap) {
@@ -753,22 +1052,22 @@ int net_loss_backward(pmg_net *N, const Geom &g, const float *T, const float *W,
     hipLaunchKernelGGL(k_wcount, dim3(nblk), dim3(256), 0, N->stream, W, g, margin, N->lpart);
     hipLaunchKernelGGL(k_fold_d, dim3(1), dim3(256), 0, N->stream, N->lpart, nblk, N->lsum + 1);
   }
-  hipLaunchKernelGGL(k_loss, dim3(nblk), dim3(256), 0, N->stream, N->z3, T, W, W ? N->lsum + 1 : (const double *)nullptr,
-                     N->d16, N->lpart, g, margin, 1.0 / count);
+  hipLaunchKernelGGL(k_loss, dim3(nblk), dim3(256), 0, N->stream, N->yt, T, W, W ? N->lsum + 1 : (const double *)nullptr,
+                     N->dy, N->lpart, g, margin, 1.0 / count);
   hipLaunchKernelGGL(k_fold_d, dim3(1), dim3(256), 0, N->stream, N->lpart, nblk, N->lsum);
   PMG_HOST_CHECK(hipGetLastError());
-  const dim3 gr = conv_grid(g);
-  // layer 3: dW3 from A2 and dZ3; dZ2 = conv^T(dZ3) * gelu'(Z2)
-  if ((rc = net_wgrad(N, g, N->a2, N->d16, N->grad + 2 * LAYER_FLOATS))) return rc;
-  hipLaunchKernelGGL(k_conv16<2>, gr, dim3(256), 0, N->stream, N->d16, N->wb + 2 * NTAP * 256,
-                     (const float *)nullptr, N->z2, N->dz, N->d16b, g);
+  const int zc = conv_zc(g, CTX, CTY, kConvBlocks);
+  const dim3 gt(conv_blocks(g, CTX, CTY, zc)), blk(256);
+  // layer 3: dW3 from A2 and dY; dZ2 = conv^T(dY) * gelu'(Z2)
+  if ((rc = net_wgrad(N, g, 2, nullptr))) return rc;
+  hipLaunchKernelGGL((k_conv_in_tile<uint16_t, 2>), gt, blk, 0, N->stream, N->dy, 1.0f, N->fr + FR_WBI,
+                     (const float *)nullptr, N->z2, (float *)nullptr, N->d16b, g, zc);
   // layer 2
-  if ((rc = net_wgrad(N, g, N->a1, N->d16b, N->grad + 1 * LAYER_FLOATS))) return rc;
-  hipLaunchKernelGGL(k_conv16<2>, gr, dim3(256), 0, N->stream, N->d16b, N->wb + 1 * NTAP * 256,
-                     (const float *)nullptr, N->z1, N->dz, N->d16, g);
+  if ((rc = net_wgrad(N, g, 1, nullptr))) return rc;
+  hipLaunchKernelGGL(k_conv16_tile<2>, gt, blk, 0, N->stream, N->d16b, N->fr + FR_WPB2, (const float *)nullptr, N->z1,
+                     (float *)nullptr, N->d16, g, zc);
   // layer 1
-  if ((rc = net_wgrad(N, g, N->x0, N->d16, N->grad))) return rc;
-  PMG_HOST_CHECK(hipGetLastError());
+  if ((rc = net_wgrad(N, g, 0, x))) return rc;
   if (loss_out) {
     double l[2];
     PMG_HOST_CHECK(hipMemcpyAsync(l, N->lsum, 2 * sizeof(double), hipMemcpyDeviceToHost, N->stream));
@@ -855,11 +1154,11 @@ pmg_net *pmg_net_create(int hidden, unsigned long long seed) {
   bool ok = hipMalloc(&N->w, nf * 4) == hipSuccess && hipMalloc(&N->m1, nf * 4) == hipSuccess &&
             hipMalloc(&N->m2, nf * 4) == hipSuccess && hipMalloc(&N->grad, nf * 4) == hipSuccess &&
             hipMalloc(&N->mask, nf) == hipSuccess &&
-            hipMalloc(&N->wf, 3 * NTAP * 256 * sizeof(uint16_t)) == hipSuccess &&
-            hipMalloc(&N->wb, 3 * NTAP * 256 * sizeof(uint16_t)) == hipSuccess &&
-            hipMalloc(&N->wfi, 64 * 8 * sizeof(uint16_t)) == hipSuccess &&
-            hipMalloc(&N->wp, 2 * NPAIR * 512 * sizeof(uint16_t)) == hipSuccess &&
+            hipMalloc(&N->fr, FR_TOTAL * sizeof(uint16_t)) == hipSuccess &&
             hipMalloc(&N->lsum, 2 * sizeof(double)) == hipSuccess;
+  // the weight gradients' planes take more LDS than a kernel gets by default
+  for (const void *k : {reinterpret_cast<const void *>(&k_wgrad_tile<1>), reinterpret_cast<const void *>(&k_wgrad_tile<16>)})
+    ok = ok && hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kWgradLds) == hipSuccess;
   if (!ok) { pmg_net_destroy(N); return nullptr; }
   (void)hipMemcpy(N->w, w.data(), nf * 4, hipMemcpyHostToDevice);
   (void)hipMemcpy(N->mask, mask.data(), nf, hipMemcpyHostToDevice);
@@ -872,11 +1171,10 @@ pmg_net *pmg_net_create(int hidden, unsigned long long seed) {
 void pmg_net_destroy(pmg_net *N) {
   if (!N) return;
   if (N->stream) (void)hipStreamSynchronize(N->stream);
-  for (void *p : {(void *)N->w, (void *)N->m1, (void *)N->m2, (void *)N->grad, (void *)N->mask,
-                  (void *)N->wf, (void *)N->wb, (void *)N->x0, (void *)N->a1, (void *)N->a2,
-                  (void *)N->d16, (void *)N->d16b, (void *)N->z1, (void *)N->z2, (void *)N->z3,
-                  (void *)N->dz, (void *)N->ia1, (void *)N->ia2, (void *)N->y, (void *)N->wfi, (void *)N->wp,
-                  (void *)N->partial, (void *)N->lpart, (void *)N->lsum})
+  for (void *p : {(void *)N->w, (void *)N->m1, (void *)N->m2, (void *)N->grad, (void *)N->mask, (void *)N->fr,
+                  (void *)N->a1, (void *)N->a2, (void *)N->d16, (void *)N->d16b, (void *)N->dy, (void *)N->z1,
+                  (void *)N->z2, (void *)N->yt, (void *)N->ia1, (void *)N->ia2, (void *)N->y, (void *)N->partial,
+                  (void *)N->lpart, (void *)N->lsum})
     if (p) (void)hipFree(p);
   if (N->stream) (void)hipStreamDestroy(N->stream);
   delete N;
@@ -937,13 +1235,8 @@ int pmg_net_forward(pmg_net *N, const float *x, float *y, int nx, int ny, int nz
   const size_t P = (size_t)nx * ny * nz * nb;
   if (net_ensure(N, P)) return -1;
   Geom g{nx, ny, nz, nb};
-  hipLaunchKernelGGL(k_pack_input<float>, dim3((unsigned)((P + 255) / 256)), dim3(256), 0, N->stream, x, N->x0,
-                     P, 1.0f);
-  int rc = net_forward(N, g);
+  int rc = net_forward(N, x, y, g);
   if (rc) return rc;
-  // y = channel 0 of Z3
-  PMG_HOST_CHECK(hipMemcpy2DAsync(y, sizeof(float), N->z3, NC * sizeof(float), sizeof(float), P,
-                                  hipMemcpyDeviceToDevice, N->stream));
   PMG_HOST_CHECK(hipStreamSynchronize(N->stream));
   return 0;
 }
@@ -957,9 +1250,7 @@ int pmg_net_loss_grad(pmg_net *N, const float *x, const float *t, int nx, int ny
   const size_t P = (size_t)nx * ny * nz * nb;
   if (net_ensure(N, P)) return -1;
   Geom g{nx, ny, nz, nb};
-  hipLaunchKernelGGL(k_pack_input<float>, dim3((unsigned)((P + 255) / 256)), dim3(256), 0, N->stream, x, N->x0,
-                     P, 1.0f);
-  int rc = net_loss_backward(N, g, t, nullptr, margin, loss);
+  int rc = net_loss_backward(N, g, x, t, nullptr, margin, loss);
   if (rc) return rc;
   std::vector<float> gr(3 * (size_t)LAYER_FLOATS);
   PMG_HOST_CHECK(hipMemcpy(gr.data(), N->grad, gr.size() * 4, hipMemcpyDeviceToHost));
@@ -976,9 +1267,7 @@ int pmg_net_loss_grad_w(pmg_net *N, const float *x, const float *t, const float 
   const size_t P = (size_t)nx * ny * nz * nb;
   if (net_ensure(N, P)) return -1;
   Geom g{nx, ny, nz, nb};
-  hipLaunchKernelGGL(k_pack_input<float>, dim3((unsigned)((P + 255) / 256)), dim3(256), 0, N->stream, x, N->x0,
-                     P, 1.0f);
-  int rc = net_loss_backward(N, g, t, w, margin, loss);
+  int rc = net_loss_backward(N, g, x, t, w, margin, loss);
   if (rc) return rc;
   std::vector<float> gr(3 * (size_t)LAYER_FLOATS);
   PMG_HOST_CHECK(hipMemcpy(gr.data(), N->grad, gr.size() * 4, hipMemcpyDeviceToHost));
@@ -994,9 +1283,7 @@ int pmg_net_train_step_w(pmg_net *N, const float *x, const float *t, const float
   const size_t P = (size_t)nx * ny * nz * nb;
   if (net_ensure(N, P)) return -1;
   Geom g{nx, ny, nz, nb};
-  hipLaunchKernelGGL(k_pack_input<float>, dim3((unsigned)((P + 255) / 256)), dim3(256), 0, N->stream, x, N->x0,
-                     P, 1.0f);
-  int rc = net_loss_backward(N, g, t, w, margin, loss);
+  int rc = net_loss_backward(N, g, x, t, w, margin, loss);
   if (rc) return rc;
   N->adam_t++;
   const float b1 = 0.9f, b2 = 0.999f;
@@ -1016,9 +1303,7 @@ int pmg_net_train_step(pmg_net *N, const float *x, const float *t, int nx, int n
   const size_t P = (size_t)nx * ny * nz * nb;
   if (net_ensure(N, P)) return -1;
   Geom g{nx, ny, nz, nb};
-  hipLaunchKernelGGL(k_pack_input<float>, dim3((unsigned)((P + 255) / 256)), dim3(256), 0, N->stream, x, N->x0,
-                     P, 1.0f);
-  int rc = net_loss_backward(N, g, t, nullptr, margin, loss);
+  int rc = net_loss_backward(N, g, x, t, nullptr, margin, loss);
   if (rc) return rc;
   N->adam_t++;
   const float b1 = 0.9f, b2 = 0.999f;
@@ -1045,7 +1330,7 @@ int pmg_net_correct(pmg_net *N, const float *x, float scale, double *u, double c
   if (net_ensure_infer(N, P)) return -1;
   hipStream_t keep = N->stream;
   N->stream = st;
-  int rc = net_infer(N, x, scale, Geom{nx, ny, nz, 1});
+  int rc = net_infer(N, x, scale, N->y, Geom{nx, ny, nz, 1});
   N->stream = keep;
   if (rc) return rc;
   hipLaunchKernelGGL((k_apply_correction<double, 1>), dim3((nx + 63) / 64, (ny + 3) / 4, nz), dim3(256), 0, st, u,
@@ -1081,7 +1366,7 @@ float *pmg_net_infer_async(pmg_net *N, const float *x, float scale, int nx, int 
   if (net_ensure_infer(N, P)) return nullptr;
   hipStream_t keep = N->stream;
   N->stream = (hipStream_t)stream;
-  const int rc = net_infer(N, x, scale, Geom{nx, ny, nz, nb});
+  const int rc = net_infer(N, x, scale, N->y, Geom{nx, ny, nz, nb});
   N->stream = keep;
   return rc ? nullptr : N->y;
 }
@@ -1090,9 +1375,8 @@ int pmg_net_infer(pmg_net *N, const float *x, float scale, float *y, int nx, int
   if (!N || !x || !y || nx < 1 || ny < 1 || nz < 1 || nb < 1) return -1;
   const size_t P = (size_t)nx * ny * nz * nb;
   if (net_ensure_infer(N, P)) return -1;
-  int rc = net_infer(N, x, scale, Geom{nx, ny, nz, nb});
+  int rc = net_infer(N, x, scale, y, Geom{nx, ny, nz, nb});
   if (rc) return rc;
-  PMG_HOST_CHECK(hipMemcpyAsync(y, N->y, P * sizeof(float), hipMemcpyDeviceToDevice, N->stream));
   PMG_HOST_CHECK(hipStreamSynchronize(N->stream));
   return 0;
 }
