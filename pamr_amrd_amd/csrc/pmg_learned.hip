@@ -55,17 +55,6 @@ __host__ __device__ inline float bf2f(uint16_t b) {
   return f;
 }
 
-__device__ inline float gelu_f(float x) {
-  const float k = 0.7978845608028654f;
-  return 0.5f * x * (1.0f + tanhf(k * (x + 0.044715f * x * x * x)));
-}
-__device__ inline float gelu_grad_f(float x) {
-  const float k = 0.7978845608028654f;
-  const float x2 = x * x;
-  const float t = tanhf(k * (x + 0.044715f * x2 * x));
-  return 0.5f * (1.0f + t) + 0.5f * x * (1.0f - t * t) * k * (1.0f + 3.0f * 0.044715f * x2);
-}
-
 struct Geom {
   int nx, ny, nz, nb;  // box shape and number of boxes (batch)
 };
@@ -113,68 +102,49 @@ __device__ inline unsigned pk_bf16(float lo, float hi) {
   return w;
 }
 
-// GELU (tanh form) through the logistic function: 0.5 x (1 + tanh u) =
-// x / (1 + e^(-2u)), u = k (x + 0.044715 x^3), with the constants folded
-// into the power of two; the inference epilogues use it (the training
-// kernels keep tanhf; the two agree to FP32 rounding).  The epilogue's vector
-// instructions, not the matrix units or LDS, bounded the hidden layer: with
-// the IEEE division and a software rounding to BF16 it took 0.27 of its
-// 0.61 ms at 257^3.
-__device__ inline float gelu_fast(float x) {
+// GELU (tanh form) through the logistic function: 0.5 x (1 + tanh u) = x s(u)
+// with s = 1 / (1 + e^(-2u)), u = k (x + 0.044715 x^3), the constants folded
+// into the power of two.  Its derivative is s + 2 x s (1 - s) u'.  Both are
+// FP32 to a few units in the last place, far below the BF16 they are rounded
+// to.  The epilogue's vector instructions, not the matrix units or LDS,
+// bounded the hidden layer: with the IEEE division, tanhf and a software
+// rounding to BF16 it took 0.27 of its 0.61 ms at 257^3.
+__device__ inline float logistic2(float x) {
   const float c1 = -2.0f * 0.7978845608028654f * 1.4426950408889634f, c2 = c1 * 0.044715f;
-  const float e = __builtin_amdgcn_exp2f(x * fmaf(c2, x * x, c1));
-  return x * __builtin_amdgcn_rcpf(1.0f + e);
+  return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(x * fmaf(c2, x * x, c1)));
+}
+__device__ inline float gelu_f(float x) { return x * logistic2(x); }
+__device__ inline float gelu_grad_f(float x) {
+  const float k2 = 2.0f * 0.7978845608028654f, k6 = k2 * 3.0f * 0.044715f;
+  const float s = logistic2(x);
+  return s + x * s * (1.0f - s) * fmaf(k6, x * x, k2);
 }
 
-// Stores one MFMA result tile of BF16 activations channel-last: lane (m, grp)
-// holds channel m of points 4grp + i (w01: points 0, 1, w23: points 2, 3);
-// after a shuffle lane L holds channels 4(L%4) .. +3 of point L/4 and writes
-// them as one 8-byte store, so the wave writes 16 points x 32 B contiguously.
-// `row` is the element offset of the group's point 0, `npts` how many of its
-// 16 points exist.
-__device__ inline void store_act16(uint16_t *__restrict__ Aout, size_t row, int npts, unsigned w01, unsigned w23) {
-  const int L = threadIdx.x & 63;
-  const int p = L >> 2, c0 = (L & 3) * 4, i = p & 3, sg = p >> 2;
-  unsigned h[4];
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const int src = (c0 + k) + 16 * sg;
-    const unsigned a = (unsigned)__builtin_amdgcn_ds_bpermute(src * 4, (int)w01);
-    const unsigned b = (unsigned)__builtin_amdgcn_ds_bpermute(src * 4, (int)w23);
-    h[k] = i < 2 ? a : b;
-  }
-  // the low or the high half of each word, by the point's parity
-  const unsigned sel = (i & 1) ? 0x07060302u : 0x05040100u;
-  if (p < npts)
-    *(uint2 *)(Aout + (row + (size_t)p) * NC + c0) =
-        make_uint2(__builtin_amdgcn_perm(h[1], h[0], sel), __builtin_amdgcn_perm(h[3], h[2], sel));
-}
-
-// What a convolution tile does with its sums v (lane (m, grp): channel m of
-// points 4grp + i of a 16-point segment starting at element `row`):
-//   EPI 0: z = v + bias -> Z (FP32), A = bf16(gelu(z))          (training)
-//   EPI 2: A = bf16(v * gelu'(aux))                             (backward data)
-//   EPI 3: A = bf16(gelu(v + bias))                             (inference)
+// What a convolution tile does with its sums (they start from the bias).  The products are taken with
+// the weights as the A operand, so lane (m, grp) holds channels 4grp .. +3 of
+// point m of a 16-point segment starting at element `row`: its activations
+// are one 8-byte store and its pre-activations one 16-byte store, channel-last
+// and contiguous over the wave, with no exchange between lanes.
+//   EPI 0: v -> Z (FP32), A = bf16(gelu(v))        (training)
+//   EPI 2: A = bf16(v * gelu'(aux)), no bias       (backward data)
+//   EPI 3: A = bf16(gelu(v))                       (inference)
 template <int EPI>
-__device__ __forceinline__ void conv_epilogue(floatx4 v, float bias, const float *__restrict__ aux,
-                                              float *__restrict__ Z, uint16_t *__restrict__ A, size_t row, int npts) {
+__device__ __forceinline__ void conv_epilogue(floatx4 v, floatx4 aux, float *__restrict__ Z, uint16_t *__restrict__ A,
+                                              size_t row, int npts) {
   const int lane = threadIdx.x & 63, m = lane & 15, grp = lane >> 4;
+  if (m >= npts) return;
+  const int p = m * NC + 4 * grp;
   float o[4];
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const size_t p = (row + 4 * grp + i) * NC + m;
-    const bool in = 4 * grp + i < npts;
-    if constexpr (EPI == 0) {
-      const float z = v[i] + bias;
-      if (in) Z[p] = z;
-      o[i] = gelu_f(z);
-    } else if constexpr (EPI == 2) {
-      o[i] = in ? v[i] * gelu_grad_f(aux[p]) : 0.f;
-    } else {
-      o[i] = gelu_fast(v[i] + bias);
-    }
-  }
-  store_act16(A, row, npts, pk_bf16(o[0], o[1]), pk_bf16(o[2], o[3]));
+  for (int i = 0; i < 4; i++) o[i] = EPI == 2 ? v[i] * gelu_grad_f(aux[i]) : gelu_f(v[i]);
+  if constexpr (EPI == 0) *(floatx4 *)(Z + row * NC + p) = v;
+  *(uint2 *)(A + row * NC + p) = make_uint2(pk_bf16(o[0], o[1]), pk_bf16(o[2], o[3]));
+}
+template <int EPI>
+__device__ __forceinline__ floatx4 conv_aux(const float *__restrict__ aux, size_t row, int npts) {
+  const int lane = threadIdx.x & 63, m = lane & 15, grp = lane >> 4;
+  if constexpr (EPI == 2) return *(const floatx4 *)(aux + row * NC + (m < npts ? m * NC + 4 * grp : 0));
+  else return floatx4{0.f, 0.f, 0.f, 0.f};
 }
 
 // The 16 -> 16 convolutions with the input staged in LDS: a block owns a
@@ -195,12 +165,16 @@ constexpr int CCHUNK = CLY * CLX * 2;                  // 16-byte chunks per sta
 constexpr int CLOAD = (CCHUNK + 255) / 256;            // per thread
 constexpr int NPAIR = (NTAP + 1) / 2;                  // tap pairs of the K = 32 form
 
+// the wave's index in its block, in a scalar register: rows and row addresses
+// are then scalar arithmetic
+__device__ __forceinline__ int wave_ix() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
+
 struct ConvTile {
   int x0, y0, z0, z1, b;
 };
 __device__ __forceinline__ ConvTile conv_tile(const Geom &g, int tx_, int ty_, int zc_) {
   const int ntx = (g.nx + tx_ - 1) / tx_, nty = (g.ny + ty_ - 1) / ty_, nzc = (g.nz + zc_ - 1) / zc_;
-  int t = blockIdx.x;
+  int t = xcd_tile(blockIdx.x, gridDim.x);  // neighbouring tiles share an L2
   ConvTile c;
   c.x0 = (t % ntx) * tx_;
   t /= ntx;
@@ -222,11 +196,13 @@ __global__ __launch_bounds__(256) void k_conv16_tile(const uint16_t *__restrict_
                                                      float *__restrict__ Zout, uint16_t *__restrict__ Aout, Geom g,
                                                      int zc) {
   __shared__ uint4 sX[4][CLY][CLX][2];
+  __shared__ uint4 sZero;  // the operand of the tap past the 27th
+  if (threadIdx.x == 0) sZero = make_uint4(0u, 0u, 0u, 0u);
   const ConvTile T = conv_tile(g, CTX, CTY, zc);
   const int x0 = T.x0, y0 = T.y0, z0 = T.z0, z1 = T.z1;
   const size_t box = (size_t)g.nx * g.ny * g.nz;
   const uint16_t *Xb = X + (size_t)T.b * box * NC;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m = lane & 15, grp = lane >> 4;
+  const int lane = threadIdx.x & 63, w = wave_ix(), m = lane & 15, grp = lane >> 4;
   uint4 reg[CLOAD];
   int off[CLOAD];  // element offset of this thread's chunks within a plane, or -1
 #pragma unroll
@@ -256,7 +232,7 @@ __global__ __launch_bounds__(256) void k_conv16_tile(const uint16_t *__restrict_
 #pragma unroll
   for (int pr = 0; pr < NPAIR; pr++) wk[pr] = *(const bf16x8 *)(Wp + ((size_t)pr * 64 + lane) * 8);
   const int half = grp & 1, second = grp >> 1;  // channel half; first or second tap of the pair
-  const float bm = EPI == 2 ? 0.f : bias[m];
+  const floatx4 bm = EPI == 2 ? floatx4{0.f, 0.f, 0.f, 0.f} : *(const floatx4 *)(bias + 4 * grp);
   fetch(z0 - 1);
   store(z0 - 1);
   fetch(z0);
@@ -268,9 +244,17 @@ __global__ __launch_bounds__(256) void k_conv16_tile(const uint16_t *__restrict_
   for (int z = z0; z < z1; z++) {
     store(z + 2);  // the slot of plane z-2, free since the barrier ending step z-1
     fetch(z + 3);
-    floatx4 acc[4];
+    floatx4 acc[4], ax[4];
+    size_t row[4];
+    int npts[4];  // points of the segment inside the box, 0 when there are none
 #pragma unroll
-    for (int q = 0; q < 4; q++) acc[q] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int q = 0; q < 4; q++) {
+      const int y = y0 + 2 * w + (q >> 1), xs = x0 + 16 * (q & 1);
+      npts[q] = y < g.ny && xs < g.nx ? min(16, g.nx - xs) : 0;
+      row[q] = npts[q] ? (size_t)T.b * box + ((size_t)z * g.ny + y) * g.nx + xs : 0;
+      acc[q] = bm;
+      ax[q] = conv_aux<EPI>(aux, row[q], npts[q]);
+    }
 #pragma unroll
     for (int pr = 0; pr < NPAIR; pr++) {
       const int tap = 2 * pr + second;
@@ -281,19 +265,14 @@ __global__ __launch_bounds__(256) void k_conv16_tile(const uint16_t *__restrict_
 #pragma unroll
       for (int q = 0; q < 4; q++) {
         const int r = 2 * w + (q >> 1), sg = q & 1;
-        // (the weights of the tap past the 27th are zero, and so is its operand)
-        bf16x8 a = *(const bf16x8 *)&sX[slot][r + 1 + dy][16 * sg + m + 1 + dx][half];
-        if (!live) a = bf16x8{};
-        acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, wk[pr], acc[q], 0, 0, 0);
+        const uint4 *S = &sX[slot][r + 1 + dy][16 * sg + m + 1 + dx][half];
+        const bf16x8 a = *(const bf16x8 *)(live ? S : &sZero);
+        acc[q] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wk[pr], a, acc[q], 0, 0, 0);
       }
     }
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const int y = y0 + 2 * w + (q >> 1), xs = x0 + 16 * (q & 1);
-      if (y >= g.ny || xs >= g.nx) continue;  // uniform per wave
-      conv_epilogue<EPI>(acc[q], bm, aux, Zout, Aout, (size_t)T.b * box + ((size_t)z * g.ny + y) * g.nx + xs,
-                         min(16, g.nx - xs));
-    }
+    for (int q = 0; q < 4; q++)
+      if (npts[q]) conv_epilogue<EPI>(acc[q], ax[q], Zout, Aout, row[q], npts[q]);  // uniform per wave
     __syncthreads();
   }
 }
@@ -319,7 +298,7 @@ __global__ __launch_bounds__(256) void k_conv_in_tile(const TIN *__restrict__ x,
   const int x0 = T.x0, y0 = T.y0, z0 = T.z0, z1 = T.z1;
   const size_t box = (size_t)g.nx * g.ny * g.nz;
   const TIN *xb = x + (size_t)T.b * box;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m = lane & 15, grp = lane >> 4;
+  const int lane = threadIdx.x & 63, w = wave_ix(), m = lane & 15, grp = lane >> 4;
   constexpr int NPT = CLY * CLX, NLD = (NPT + 255) / 256;
   TIN reg[NLD];
   int off[NLD], lds[NLD];
@@ -355,7 +334,7 @@ __global__ __launch_bounds__(256) void k_conv_in_tile(const TIN *__restrict__ x,
   bf16x4 bw[3];
 #pragma unroll
   for (int d = 0; d < 3; d++) bw[d] = *(const bf16x4 *)(Wfi + ((size_t)d * 64 + lane) * 4);
-  const float bm = EPI == 2 ? 0.f : bias[m];
+  const floatx4 bm = EPI == 2 ? floatx4{0.f, 0.f, 0.f, 0.f} : *(const floatx4 *)(bias + 4 * grp);
   const uint32_t live = grp < 3 ? ~0u : 0u;
   fetch(z0 - 1);
   store(z0 - 1);
@@ -371,7 +350,11 @@ __global__ __launch_bounds__(256) void k_conv_in_tile(const TIN *__restrict__ x,
 #pragma unroll
     for (int q = 0; q < 4; q++) {
       const int r = 2 * w + (q >> 1), sg = q & 1, y = y0 + r, xs = x0 + 16 * sg;
-      floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+      if (y >= g.ny || xs >= g.nx) continue;  // uniform per wave
+      const int npts = min(16, g.nx - xs);
+      const size_t row = (size_t)T.b * box + ((size_t)z * g.ny + y) * g.nx + xs;
+      const floatx4 ax = conv_aux<EPI>(aux, row, npts);
+      floatx4 acc = bm;
 #pragma unroll
       for (int d = 0; d < 3; d++) {
         // LDS column lx is the point x0 - 1 + lx: the four points from x-1 on
@@ -379,11 +362,9 @@ __global__ __launch_bounds__(256) void k_conv_in_tile(const TIN *__restrict__ x,
         const uint32_t aw[2] = {S[0] & live, S[2] & live & 0xffffu};
         bf16x4 a;
         __builtin_memcpy(&a, aw, 8);
-        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, bw[d], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(bw[d], a, acc, 0, 0, 0);
       }
-      if (y < g.ny && xs < g.nx)  // uniform per wave
-        conv_epilogue<EPI>(acc, bm, aux, Zout, Aout, (size_t)T.b * box + ((size_t)z * g.ny + y) * g.nx + xs,
-                           min(16, g.nx - xs));
+      conv_epilogue<EPI>(acc, ax, Zout, Aout, row, npts);
     }
     __syncthreads();
   }
@@ -397,10 +378,11 @@ __global__ __launch_bounds__(256) void k_conv_in_tile(const TIN *__restrict__ x,
 // (each input point is read once per tile, 8 bytes a lane, contiguous).  G of
 // one input plane (OIX x OIY points) lies in LDS tap by tap; every output
 // column then adds its 27 values to the three running sums of the output
-// planes z-1, z, z+1.  At 257^3: 0.34 -> 0.13 ms.
-constexpr int OIX = 32, OIY = 12, OTX = OIX - 2, OTY = OIY - 2;
+// planes z-1, z, z+1.  At 257^3: 0.34 -> 0.20 ms.
+constexpr int OIX = 32, OIY = 10, OTX = OIX - 2, OTY = OIY - 2;
 constexpr int OPTS = OIX * OIY, OSEG = OPTS / 16 / 4;  // segments per wave
-constexpr int OSTR = OPTS + 16;                        // LDS words per tap (16 mod 64: conflict-free 16-byte writes)
+constexpr int OSTR = OPTS + 4;                         // LDS words per tap (4 mod 64: 16 taps on 64 banks)
+static_assert(OIX * OTY == 256 && OSTR % 64 == 4, "one output column per thread");
 static_assert(OPTS % 64 == 0, "whole segments per wave");
 __global__ __launch_bounds__(256) void k_conv_out_tile(const uint16_t *__restrict__ X,
                                                        const uint16_t *__restrict__ Wo,
@@ -410,9 +392,9 @@ __global__ __launch_bounds__(256) void k_conv_out_tile(const uint16_t *__restric
   const ConvTile T = conv_tile(g, OTX, OTY, zc);
   const size_t box = (size_t)g.nx * g.ny * g.nz;
   const uint16_t *Xb = X + (size_t)T.b * box * NC;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m = lane & 15, grp = lane >> 4;
+  const int lane = threadIdx.x & 63, w = wave_ix(), m = lane & 15, grp = lane >> 4;
   // input segment s of this wave: 16 points of row (w * OSEG + s) / 2
-  uint2 reg[OSEG];
+  uint2 regA[OSEG], regB[OSEG];
   int off[OSEG];
 #pragma unroll
   for (int s = 0; s < OSEG; s++) {
@@ -420,25 +402,23 @@ __global__ __launch_bounds__(256) void k_conv_out_tile(const uint16_t *__restric
     off[s] = gx >= 0 && gx < g.nx && gy >= 0 && gy < g.ny ? (gy * g.nx + gx) * NC + 4 * grp : -1;
   }
   const size_t plane = (size_t)g.nx * g.ny * NC;
-  auto fetch = [&](int k) {
+  auto fetch = [&](int k, uint2 (&reg)[OSEG]) {
     const uint16_t *Xk = Xb + (k >= 0 && k < g.nz ? (size_t)k * plane : 0);
 #pragma unroll
     for (int s = 0; s < OSEG; s++) reg[s] = *(const uint2 *)(Xk + (off[s] < 0 ? 0 : off[s]));
   };
   const bf16x4 w0 = *(const bf16x4 *)(Wo + (size_t)lane * 4), w1 = *(const bf16x4 *)(Wo + (size_t)(64 + lane) * 4);
   // output columns of this thread
-  constexpr int NOUT = (OTX * OTY + 255) / 256;
-  float sum[NOUT][3];
-  int col[NOUT];  // LDS position of the column's own point, or -1
-#pragma unroll
-  for (int o = 0; o < NOUT; o++) {
-    const int q = (int)threadIdx.x + o * 256, ox = q % OTX, oy = q / OTX;
-    col[o] = q < OTX * OTY && T.x0 + ox < g.nx && T.y0 + oy < g.ny ? (oy + 1) * OIX + ox + 1 : -1;
-    sum[o][0] = sum[o][1] = sum[o][2] = 0.f;
-  }
+  // (a row of 32 lanes has 30 columns: neighbouring lanes read neighbouring words)
+  const int ox = (int)threadIdx.x % OIX, oy = (int)threadIdx.x / OIX;
+  const bool mine = ox < OTX && T.x0 + ox < g.nx && T.y0 + oy < g.ny;
+  const float *G = &sG[(oy + 1) * OIX + (ox < OTX ? ox : 0) + 1];
+  float *o = out + (size_t)T.b * box + (mine ? (size_t)(T.y0 + oy) * g.nx + T.x0 + ox : 0);
+  const size_t oplane = (size_t)g.nx * g.ny;
+  float sum[3] = {0.f, 0.f, 0.f};
   const float b0 = bias[0];
-  fetch(T.z0 - 1);
-  for (int k = T.z0 - 1; k <= T.z1; k++) {
+  // two planes in flight: a step is shorter than a load's way from memory
+  auto step = [&](int k, uint2 (&reg)[OSEG]) {
     const bool kin = k >= 0 && k < g.nz;
     bf16x4 a[OSEG];
 #pragma unroll
@@ -446,7 +426,7 @@ __global__ __launch_bounds__(256) void k_conv_out_tile(const uint16_t *__restric
       const uint2 v = kin && off[s] >= 0 ? reg[s] : make_uint2(0u, 0u);
       __builtin_memcpy(&a[s], &v, 8);
     }
-    if (k < T.z1) fetch(k + 1);
+    if (k + 1 < T.z1) fetch(k + 2, reg);
     __syncthreads();  // the sums of the plane before have read sG
 #pragma unroll
     for (int s = 0; s < OSEG; s++) {
@@ -459,28 +439,26 @@ __global__ __launch_bounds__(256) void k_conv_out_tile(const uint16_t *__restric
       if (16 + m < NTAP) *(floatx4 *)(S + 16 * OSTR) = g1;
     }
     __syncthreads();
+    // input plane k is at dz = +1 of output plane k-1, 0 of k, -1 of k+1
 #pragma unroll
-    for (int o = 0; o < NOUT; o++) {
-      if (col[o] < 0) continue;
-      // input plane k is at dz = +1 of output plane k-1, 0 of k, -1 of k+1
+    for (int dz = -1; dz <= 1; dz++) {
+      float v = sum[1 - dz];
 #pragma unroll
-      for (int dz = -1; dz <= 1; dz++) {
-        float v = sum[o][1 - dz];
+      for (int dy = -1; dy <= 1; dy++)
 #pragma unroll
-        for (int dy = -1; dy <= 1; dy++)
-#pragma unroll
-          for (int dx = -1; dx <= 1; dx++)
-            v += sG[((dz + 1) * 9 + (dy + 1) * 3 + dx + 1) * OSTR + col[o] + dy * OIX + dx];
-        sum[o][1 - dz] = v;
-      }
-      if (k - 1 >= T.z0) {  // plane k-1 is complete
-        const int q = (int)threadIdx.x + o * 256;
-        out[(size_t)T.b * box + ((size_t)(k - 1) * g.ny + T.y0 + q / OTX) * g.nx + T.x0 + q % OTX] = sum[o][0] + b0;
-      }
-      sum[o][0] = sum[o][1];
-      sum[o][1] = sum[o][2];
-      sum[o][2] = 0.f;
+        for (int dx = -1; dx <= 1; dx++) v += G[((dz + 1) * 9 + (dy + 1) * 3 + dx + 1) * OSTR + dy * OIX + dx];
+      sum[1 - dz] = v;
     }
+    if (mine && k - 1 >= T.z0) o[(size_t)(k - 1) * oplane] = sum[0] + b0;  // plane k-1 is complete
+    sum[0] = sum[1];
+    sum[1] = sum[2];
+    sum[2] = 0.f;
+  };
+  fetch(T.z0 - 1, regA);
+  fetch(T.z0, regB);
+  for (int k = T.z0 - 1; k <= T.z1; k += 2) {
+    step(k, regA);
+    if (k + 1 <= T.z1) step(k + 1, regB);
   }
 }
 
@@ -491,7 +469,7 @@ __global__ __launch_bounds__(256) void k_conv_out_tile(const uint16_t *__restric
 // planes, one 32-point row of dZ per wave and step against the 9 rows of X
 // around it, all 27 taps accumulated in registers -- so every point of X and
 // dZ is read from memory once per tile, where one workgroup per tap read
-// both 28 times, 2 bytes at a time (0.70 -> 0.02 ms for 16 crops of 32^3).
+// both 28 times, 2 bytes at a time (0.70 -> 0.035 ms for 16 crops of 32^3).
 // The operands want 8 consecutive points of one channel per lane, the arrays
 // are channel-last: the planes are transposed on their way into LDS
 // ([row][channel][x], two points per word).  The taps dx = -1 and +1 of a row
@@ -504,7 +482,12 @@ __global__ __launch_bounds__(256) void k_conv_out_tile(const uint16_t *__restric
 //   ZCH: 16 -- dZ is BF16 [P][16]; 1 -- BF16 [P], the single output channel.
 // ---------------------------------------------------------------------------
 constexpr int WTX = 32, WTY = 8, WLY = WTY + 2;
+constexpr int WGT = 512;  // threads: a wave per tile row, two waves a SIMD (the accumulators' registers)
 constexpr int WXS = 56, WZS = 40;  // 2-byte elements per (row, channel) of the X and dZ planes
+
+// the ci * 16 + co of entry e of a row of a block's partial (lane order: lane
+// l = 16 grp + m holds ci = 4grp + i, co = m as entries 4 l + i)
+__device__ __forceinline__ int wgrad_entry(int e) { return (4 * (e >> 6) + (e & 3)) * 16 + ((e >> 2) & 15); }
 
 // words of channels c .. c+7 of two neighbouring points, one word per channel
 __device__ __forceinline__ void put_pair(uint16_t *S, int stride, const uint4 &p, const uint4 &q) {
@@ -517,7 +500,7 @@ __device__ __forceinline__ void put_pair(uint16_t *S, int stride, const uint4 &p
 }
 
 template <int ZCH>
-__global__ __launch_bounds__(256) void k_wgrad_tile(const uint16_t *__restrict__ X, const uint16_t *__restrict__ dZ,
+__global__ __launch_bounds__(WGT) void k_wgrad_tile(const uint16_t *__restrict__ X, const uint16_t *__restrict__ dZ,
                                                     float *__restrict__ partial, Geom g, int zc) {
   // X planes k-1, k, k+1 and the plane being filled share 4 slots
   extern __shared__ __align__(16) unsigned char wsm[];
@@ -527,55 +510,55 @@ __global__ __launch_bounds__(256) void k_wgrad_tile(const uint16_t *__restrict__
   const size_t box = (size_t)g.nx * g.ny * g.nz;
   const uint16_t *Xb = X + (size_t)T.b * box * NC;
   const uint16_t *Zb = dZ + (size_t)T.b * box * ZCH;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m = lane & 15, grp = lane >> 4;
+  const int lane = threadIdx.x & 63, w = wave_ix(), m = lane & 15, grp = lane >> 4;
   const uint4 zero4 = make_uint4(0u, 0u, 0u, 0u);
   // staging tasks: a pair of points (x even relative to the tile) of one row, 8 channels
-  constexpr int XPAIR = WTX / 2 + 2, NXT = (WLY * XPAIR * 2 + 255) / 256;
-  uint4 xp[NXT], xq[NXT], zp, zq;
+  constexpr int XPAIR = WTX / 2 + 2;
+  static_assert(WLY * XPAIR * 2 <= WGT && WTX * WTY == 256, "one task per thread");
+  struct Pair {
+    uint4 p, q;
+  };
   auto fetch_x = [&](int k) {
-    const bool kin = k >= 0 && k < g.nz;
-#pragma unroll
-    for (int t = 0; t < NXT; t++) {
-      const int idx = (int)threadIdx.x + t * 256, h = idx & 1, pr = (idx >> 1) % XPAIR, row = (idx >> 1) / XPAIR;
-      const int gy = T.y0 - 1 + row, gx = T.x0 - 2 + 2 * pr;
-      const bool ok = kin && row < WLY && gy >= 0 && gy < g.ny;
-      const size_t at = ok ? (((size_t)k * g.ny + gy) * g.nx) * NC + 8 * h : 0;
-      xp[t] = ok && gx >= 0 && gx < g.nx ? *(const uint4 *)(Xb + at + (size_t)gx * NC) : zero4;
-      xq[t] = ok && gx + 1 >= 0 && gx + 1 < g.nx ? *(const uint4 *)(Xb + at + (size_t)(gx + 1) * NC) : zero4;
-    }
+    const int idx = (int)threadIdx.x, h = idx & 1, pr = (idx >> 1) % XPAIR, row = (idx >> 1) / XPAIR;
+    const int gy = T.y0 - 1 + row, gx = T.x0 - 2 + 2 * pr;
+    const bool ok = k >= 0 && k < g.nz && row < WLY && gy >= 0 && gy < g.ny;
+    const size_t at = ok ? (((size_t)k * g.ny + gy) * g.nx) * NC + 8 * h : 0;
+    return Pair{ok && gx >= 0 && gx < g.nx ? *(const uint4 *)(Xb + at + (size_t)gx * NC) : zero4,
+                ok && gx + 1 >= 0 && gx + 1 < g.nx ? *(const uint4 *)(Xb + at + (size_t)(gx + 1) * NC) : zero4};
   };
-  auto store_x = [&](int k) {
+  auto store_x = [&](int k, const Pair &v) {
     uint16_t *S = sX + (size_t)(k & 3) * WLY * NC * WXS;
-#pragma unroll
-    for (int t = 0; t < NXT; t++) {
-      const int idx = (int)threadIdx.x + t * 256, h = idx & 1, pr = (idx >> 1) % XPAIR, row = (idx >> 1) / XPAIR;
-      if (row < WLY) put_pair(S + ((size_t)row * NC + 8 * h) * WXS + 6 + 2 * pr, WXS, xp[t], xq[t]);
-    }
+    const int idx = (int)threadIdx.x, h = idx & 1, pr = (idx >> 1) % XPAIR, row = (idx >> 1) / XPAIR;
+    if (row < WLY) put_pair(S + ((size_t)row * NC + 8 * h) * WXS + 6 + 2 * pr, WXS, v.p, v.q);
   };
+  // dZ: the last 256 threads (those with the fewest X tasks)
+  const int zt = (int)threadIdx.x - (WGT - 256);
   auto fetch_z = [&](int k) {
+    Pair v{zero4, zero4};
+    if (zt < 0) return v;
     if constexpr (ZCH == 16) {
-      const int h = threadIdx.x & 1, pr = (threadIdx.x >> 1) % (WTX / 2), row = (threadIdx.x >> 1) / (WTX / 2);
+      const int h = zt & 1, pr = (zt >> 1) % (WTX / 2), row = (zt >> 1) / (WTX / 2);
       const int gy = T.y0 + row, gx = T.x0 + 2 * pr;
       const bool ok = k < T.z1 && gy < g.ny;
       const size_t at = ok ? (((size_t)k * g.ny + gy) * g.nx) * NC + 8 * h : 0;
-      zp = ok && gx < g.nx ? *(const uint4 *)(Zb + at + (size_t)gx * NC) : zero4;
-      zq = ok && gx + 1 < g.nx ? *(const uint4 *)(Zb + at + (size_t)(gx + 1) * NC) : zero4;
+      if (ok && gx < g.nx) v.p = *(const uint4 *)(Zb + at + (size_t)gx * NC);
+      if (ok && gx + 1 < g.nx) v.q = *(const uint4 *)(Zb + at + (size_t)(gx + 1) * NC);
     } else {
-      const int x = threadIdx.x % WTX, row = threadIdx.x / WTX, gy = T.y0 + row, gx = T.x0 + x;
-      const bool ok = k < T.z1 && gy < g.ny && gx < g.nx;
-      zp.x = ok ? Zb[((size_t)k * g.ny + gy) * g.nx + gx] : 0u;
+      const int gy = T.y0 + zt / WTX, gx = T.x0 + zt % WTX;
+      if (k < T.z1 && gy < g.ny && gx < g.nx) v.p.x = Zb[((size_t)k * g.ny + gy) * g.nx + gx];
     }
+    return v;
   };
-  auto store_z = [&](int k) {
+  auto store_z = [&](int k, const Pair &v) {
+    if (zt < 0) return;
     uint16_t *S = sZ + (size_t)(k & 1) * WTY * NC * WZS;
     if constexpr (ZCH == 16) {
-      const int h = threadIdx.x & 1, pr = (threadIdx.x >> 1) % (WTX / 2), row = (threadIdx.x >> 1) / (WTX / 2);
-      put_pair(S + ((size_t)row * NC + 8 * h) * WZS + 2 * pr, WZS, zp, zq);
+      const int h = zt & 1, pr = (zt >> 1) % (WTX / 2), row = (zt >> 1) / (WTX / 2);
+      put_pair(S + ((size_t)row * NC + 8 * h) * WZS + 2 * pr, WZS, v.p, v.q);
     } else {
-      S[(size_t)(threadIdx.x / WTX) * NC * WZS + threadIdx.x % WTX] = (uint16_t)zp.x;
+      S[(size_t)(zt / WTX) * NC * WZS + zt % WTX] = (uint16_t)v.p.x;
     }
   };
-  static_assert(WTX * WTY == 256, "one dZ task per thread");
   floatx4 acc[NTAP + 1];
 #pragma unroll
   for (int t = 0; t <= NTAP; t++) acc[t] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -588,23 +571,21 @@ __global__ __launch_bounds__(256) void k_wgrad_tile(const uint16_t *__restrict__
     __builtin_memcpy(&r, v, 16);
     return r;
   };
-  fetch_x(T.z0 - 1);
-  store_x(T.z0 - 1);
-  fetch_x(T.z0);
-  store_x(T.z0);
-  fetch_x(T.z0 + 1);
-  store_x(T.z0 + 1);
-  fetch_z(T.z0);
-  store_z(T.z0);
+  {
+    const Pair xa = fetch_x(T.z0 - 1), xb_ = fetch_x(T.z0), xc = fetch_x(T.z0 + 1), za = fetch_z(T.z0);
+    store_x(T.z0 - 1, xa);
+    store_x(T.z0, xb_);
+    store_x(T.z0 + 1, xc);
+    store_z(T.z0, za);
+  }
   __syncthreads();
   for (int k = T.z0; k < T.z1; k++) {
     // the next planes' loads are in flight through this step's products and go
-    // into slots that no wave reads in it
-    fetch_x(k + 2);
-    fetch_z(k + 1);
-#pragma unroll
-    for (int rr = 0; rr < WTY / 4; rr++) {
-      const int row = w * (WTY / 4) + rr;
+    // into slots that no wave reads in it (requesting them two steps ahead
+    // measured 10 % slower)
+    const Pair xn = fetch_x(k + 2), zn = fetch_z(k + 1);
+    {
+      const int row = w;
       bf16x8 bz = *(const bf16x8 *)(sZ + ((size_t)((k & 1) * WTY + row) * NC + (ZCH == 16 ? m : 0)) * WZS + 8 * grp);
       if (ZCH == 1 && m != 0) bz = bf16x8{};
       acc[NTAP] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, bz, acc[NTAP], 0, 0, 0);
@@ -622,29 +603,32 @@ __global__ __launch_bounds__(256) void k_wgrad_tile(const uint16_t *__restrict__
         acc[3 * dzy + 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(u4(a1, a2, a3, a4), bz, acc[3 * dzy + 2], 0, 0, 0);
       }
     }
-    store_x(k + 2);
-    store_z(k + 1);
+    store_x(k + 2, xn);
+    store_z(k + 1, zn);
     __syncthreads();
   }
-  // lane holds D[ci = 4grp + i][co = m]; the waves' sums in wave order
-  float *red = (float *)wsm;
-  for (int ww = 0; ww < 4; ww++) {
-    if (w == ww) {
+  // lane holds D[ci = 4grp + i][co = m]: entry 4 lane + i of a tap's 256.  The
+  // waves' sums meet in LDS a quarter of the rows at a time and are added in
+  // wave order, wave w taking row t0 + w.
+  constexpr int NW = WGT / kWave, QT = (NTAP + 1) / 4;
+  floatx4 *red = (floatx4 *)wsm;
+  float *out = partial + (size_t)blockIdx.x * LAYER_FLOATS;
 #pragma unroll
-      for (int t = 0; t <= NTAP; t++)
+  for (int h = 0; h < 4; h++) {
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-          float *r = red + t * 256 + (4 * grp + i) * 16 + m;
-          *r = ww == 0 ? acc[t][i] : *r + acc[t][i];
-        }
+    for (int t = 0; t < QT; t++) red[(t * NW + w) * kWave + lane] = acc[h * QT + t];
+    __syncthreads();
+    if (w < QT) {
+      floatx4 v = red[w * NW * kWave + lane];
+      for (int ww = 1; ww < NW; ww++) v += red[(w * NW + ww) * kWave + lane];
+      *(floatx4 *)(out + (h * QT + w) * 256 + 4 * lane) = v;
     }
     __syncthreads();
   }
-  float *out = partial + (size_t)blockIdx.x * LAYER_FLOATS;
-  for (int e = threadIdx.x; e < LAYER_FLOATS; e += 256) out[e] = red[e];
 }
 constexpr size_t kWgradLds = (4 * (size_t)WLY * NC * WXS + 2 * (size_t)WTY * NC * WZS) * sizeof(uint16_t);
-static_assert(kWgradLds >= LAYER_FLOATS * sizeof(float), "the wave sums reuse the planes' LDS");
+static_assert(kWgradLds >= (NTAP + 1) / 4 * (WGT / kWave) * kWave * 16, "the wave sums reuse the planes' LDS");
+static_assert((NTAP + 1) % 4 == 0 && WGT / kWave == WTY, "one tile row per wave");
 
 // layer 1: the taps are the rows of A (two MFMAs per 32 points)
 __global__ __launch_bounds__(256) void k_wgrad_in_tile(const float *__restrict__ x, const uint16_t *__restrict__ dZ,
@@ -657,50 +641,61 @@ __global__ __launch_bounds__(256) void k_wgrad_in_tile(const float *__restrict__
   const size_t box = (size_t)g.nx * g.ny * g.nz;
   const float *xb = x + (size_t)T.b * box;
   const uint16_t *Zb = dZ + (size_t)T.b * box * NC;
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, m = lane & 15, grp = lane >> 4;
+  const int lane = threadIdx.x & 63, w = wave_ix(), m = lane & 15, grp = lane >> 4;
   const uint4 zero4 = make_uint4(0u, 0u, 0u, 0u);
   constexpr int LXP = WTX + 2, NXT = (WLY * LXP + 255) / 256;
-  auto stage_x = [&](int k) {
+  struct Vals {
     float v[NXT];
+  };
+  auto fetch_x = [&](int k) {
+    Vals r;
 #pragma unroll
     for (int t = 0; t < NXT; t++) {
       const int idx = (int)threadIdx.x + t * 256, row = idx / LXP, gy = T.y0 - 1 + row, gx = T.x0 - 1 + idx % LXP;
-      v[t] = k >= 0 && k < g.nz && row < WLY && gy >= 0 && gy < g.ny && gx >= 0 && gx < g.nx
-                 ? xb[((size_t)k * g.ny + gy) * g.nx + gx] : 0.f;
+      r.v[t] = k >= 0 && k < g.nz && row < WLY && gy >= 0 && gy < g.ny && gx >= 0 && gx < g.nx
+                   ? xb[((size_t)k * g.ny + gy) * g.nx + gx] : 0.f;
     }
+    return r;
+  };
+  auto store_x = [&](int k, const Vals &r) {
 #pragma unroll
     for (int t = 0; t < NXT; t++) {
       const int idx = (int)threadIdx.x + t * 256, row = idx / LXP, lx = idx % LXP;
       if (row >= WLY) continue;
-      const uint16_t h = (uint16_t)pk_bf16(v[t], 0.f);
+      const uint16_t h = (uint16_t)pk_bf16(r.v[t], 0.f);
       // the point x0 - 1 + lx is element p + (d - 1) of copy d at p = lx - d
 #pragma unroll
       for (int d = 0; d < 3; d++)
         if (lx - d >= 0 && lx - d < WTX) sX[k & 3][d][row][lx - d] = h;
     }
   };
-  auto stage_z = [&](int k) {
-    const int h = threadIdx.x & 1, pr = (threadIdx.x >> 1) % (WTX / 2), row = (threadIdx.x >> 1) / (WTX / 2);
-    const int gy = T.y0 + row, gx = T.x0 + 2 * pr;
-    const bool ok = k < T.z1 && gy < g.ny;
-    const size_t at = ok ? (((size_t)k * g.ny + gy) * g.nx) * NC + 8 * h : 0;
-    const uint4 p = ok && gx < g.nx ? *(const uint4 *)(Zb + at + (size_t)gx * NC) : zero4;
-    const uint4 q = ok && gx + 1 < g.nx ? *(const uint4 *)(Zb + at + (size_t)(gx + 1) * NC) : zero4;
-    put_pair(&sZ[k & 1][row][8 * h][2 * pr], WZS, p, q);
+  struct Pair {
+    uint4 p, q;
   };
+  const int zh = threadIdx.x & 1, zpr = (threadIdx.x >> 1) % (WTX / 2), zrow = (threadIdx.x >> 1) / (WTX / 2);
+  auto fetch_z = [&](int k) {
+    const int gy = T.y0 + zrow, gx = T.x0 + 2 * zpr;
+    const bool ok = k < T.z1 && gy < g.ny;
+    const size_t at = ok ? (((size_t)k * g.ny + gy) * g.nx) * NC + 8 * zh : 0;
+    return Pair{ok && gx < g.nx ? *(const uint4 *)(Zb + at + (size_t)gx * NC) : zero4,
+                ok && gx + 1 < g.nx ? *(const uint4 *)(Zb + at + (size_t)(gx + 1) * NC) : zero4};
+  };
+  auto store_z = [&](int k, const Pair &v) { put_pair(&sZ[k & 1][zrow][8 * zh][2 * zpr], WZS, v.p, v.q); };
   floatx4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
   bf16x8 ones;
   for (int j = 0; j < 8; j++) ones[j] = (__bf16)1.0f;
-  stage_x(T.z0 - 1);
-  stage_x(T.z0);
-  stage_x(T.z0 + 1);
-  stage_z(T.z0);
+  {
+    const Vals xa = fetch_x(T.z0 - 1), xb_ = fetch_x(T.z0), xc = fetch_x(T.z0 + 1);
+    const Pair za = fetch_z(T.z0);
+    store_x(T.z0 - 1, xa);
+    store_x(T.z0, xb_);
+    store_x(T.z0 + 1, xc);
+    store_z(T.z0, za);
+  }
   __syncthreads();
   for (int k = T.z0; k < T.z1; k++) {
-    if (k + 1 < T.z1) {
-      stage_x(k + 2);
-      stage_z(k + 1);
-    }
+    const Vals xn = fetch_x(k + 2);
+    const Pair zn = fetch_z(k + 1);
 #pragma unroll
     for (int rr = 0; rr < WTY / 4; rr++) {
       const int row = w * (WTY / 4) + rr;
@@ -713,6 +708,8 @@ __global__ __launch_bounds__(256) void k_wgrad_in_tile(const float *__restrict__
         acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bz, acc[h], 0, 0, 0);
       }
     }
+    store_x(k + 2, xn);
+    store_z(k + 1, zn);
     __syncthreads();
   }
   for (int ww = 0; ww < 4; ww++) {
@@ -728,7 +725,10 @@ __global__ __launch_bounds__(256) void k_wgrad_in_tile(const float *__restrict__
   }
   // only input channel 0 (row 0 of every tap, and the bias row) has gradients
   float *out = partial + (size_t)blockIdx.x * LAYER_FLOATS;
-  for (int e = threadIdx.x; e < LAYER_FLOATS; e += 256) out[e] = e % 256 < 16 ? red[(e / 256) * 16 + e % 256] : 0.f;
+  for (int e = threadIdx.x; e < LAYER_FLOATS; e += 256) {
+    const int q = wgrad_entry(e % 256);
+    out[e] = q < 16 ? red[(e / 256) * 16 + q] : 0.f;
+  }
 }
 
 // fold of the blocks' partials -> grad[28][256]: a block takes 64 entries, its
@@ -744,7 +744,7 @@ __global__ __launch_bounds__(1024) void k_fold_wgrad(const float *__restrict__ p
   __syncthreads();
   if (w == 0) {
     for (int c = 1; c < 16; c++) s += red[c][threadIdx.x];
-    grad[e] = s;
+    grad[e / 256 * 256 + wgrad_entry(e % 256)] = s;
   }
 }
 
@@ -1020,10 +1020,10 @@ int net_wgrad(pmg_net *N, const Geom &g, int l, const float *x) {
   if (l == 0) {
     hipLaunchKernelGGL(k_wgrad_in_tile, dim3(nblk), dim3(256), 0, N->stream, x, N->d16, N->partial, g, zc);
   } else if (l == 1) {
-    hipLaunchKernelGGL(k_wgrad_tile<16>, dim3(nblk), dim3(256), kWgradLds, N->stream, N->a1, N->d16b, N->partial, g,
+    hipLaunchKernelGGL(k_wgrad_tile<16>, dim3(nblk), dim3(WGT), kWgradLds, N->stream, N->a1, N->d16b, N->partial, g,
                        zc);
   } else {
-    hipLaunchKernelGGL(k_wgrad_tile<1>, dim3(nblk), dim3(256), kWgradLds, N->stream, N->a2, N->dy, N->partial, g, zc);
+    hipLaunchKernelGGL(k_wgrad_tile<1>, dim3(nblk), dim3(WGT), kWgradLds, N->stream, N->a2, N->dy, N->partial, g, zc);
   }
   PMG_HOST_CHECK(hipGetLastError());
   hipLaunchKernelGGL(k_fold_wgrad, dim3(LAYER_FLOATS / 64), dim3(1024), 0, N->stream, N->partial,
