@@ -699,13 +699,25 @@ inline dim3 grid3(int nx, int ny, int nz) {
   const int k = blockIdx.z;                                      \
   if (i >= (nx) || j >= (ny)) return;
 
+// A second field (r1 -> r2, no twin) goes along when the launch has 2 nz2
+// planes: the residual beside u, one launch instead of two.
 template <typename T, int KIND, bool EXC>
 __global__ __launch_bounds__(256) void k_restrict_whole(const T *__restrict__ u1,
                                                         T *__restrict__ u2, T *__restrict__ alt,
+                                                        const T *__restrict__ r1, T *__restrict__ r2,
                                                         const T *__restrict__ chr1, T ex,
                                                         int nx1, int ny1, int nz1, int nx2,
                                                         int ny2, int nz2) {
-  PMG_IJK(nx2, ny2)
+  const int i = blockIdx.x * EX_ + (int)(threadIdx.x % EX_);
+  const int j = blockIdx.y * EY_ + (int)(threadIdx.x / EX_);
+  if (i >= nx2 || j >= ny2) return;
+  int k = blockIdx.z;
+  if (k >= nz2) {
+    k -= nz2;
+    u1 = r1;
+    u2 = r2;
+    alt = nullptr;
+  }
   const size_t q = ix3(i, j, k, nx2, ny2);
   const int i0 = 1 + 2 * i, j0 = 1 + 2 * j, k0 = 1 + 2 * k;
   T v;

@@ -167,14 +167,21 @@ __device__ __forceinline__ T fw_point_ex(const T *u1, const T *chr1, T ex, int n
   T sum = 0;
   int w = 0;
   if (xi && yi && zi) {
-    for (int a = im; a <= ip; a++)
-      for (int b = jm; b <= jp; b++)
-        for (int c = km; c <= kp; c++)
-          if (PMG_CH(a, b, c) != ex) {
-            int ww = w3d(a - im + 1, b - jm + 1, c - km + 1);
-            sum = sum + ww * PMG_U1(a, b, c);
-            w += ww;
-          }
+    // unrolled: constant weights, and all 54 loads in flight together
+    T cv[27], uv[27];
+#pragma unroll
+    for (int q = 0; q < 27; q++) {
+      cv[q] = PMG_CH(im + q / 9, jm + (q / 3) % 3, km + q % 3);
+      uv[q] = PMG_U1(im + q / 9, jm + (q / 3) % 3, km + q % 3);
+    }
+#pragma unroll
+    for (int q = 0; q < 27; q++) {
+      const int ww = (q / 9 == 1 ? 2 : 1) * ((q / 3) % 3 == 1 ? 2 : 1) * (q % 3 == 1 ? 2 : 1);
+      if (cv[q] != ex) {
+        sum = sum + ww * uv[q];
+        w += ww;
+      }
+    }
   } else if (xi && yi) {
     for (int a = im; a <= ip; a++)
       for (int b = jm; b <= jp; b++)

@@ -18,6 +18,7 @@
 
 #include "pmg_kernels.h"
 #include "pmg_sweep_launch.h"
+#include "pmg_small.h"
 #include "pamr_mg_gpu.h"
 
 extern "C" int pmg_net_reserve(pmg_net *N, long long points);
@@ -102,6 +103,7 @@ template <typename T>
 struct LevelArrays {
   T *u = nullptr, *ua = nullptr, *rho = nullptr, *rhs = nullptr, *res = nullptr, *lop = nullptr;
   T *a = nullptr, *c = nullptr;
+  T *sres = nullptr;  // small levels below the finest: the residual on its way to the next level
 };
 
 struct Level {
@@ -112,6 +114,7 @@ struct Level {
   Spacing<float> sp32;
   Box rbox;  // relax/residual box: cmask_bdy box clipped to the interior
   Box cbox;  // child mask box (levels below the finest)
+  bool small = false;  // few enough points for the one-launch legs (pmg_small.h)
   LevelArrays<double> d;
   LevelArrays<float> f;
   int cur[2] = {0, 0};      // ping-pong buffer holding u (0: u, 1: ua), FP64 / FP32,
@@ -137,7 +140,7 @@ struct pmg_solver {
   int lv_variant[2][kMaxLev], lv_zchunk[2][kMaxLev];  // per-level sweep configuration, [0] FP64, [1] FP32
   int use_graph = 1;
   int use_bottom = 1;  // fuse the small bottom levels into one workgroup
-  int bottom_max_n = 17;  // ... those with at most this many points per side
+  int bottom_max_n = 0;   // ... those with at most this many points per side (0: see bottom_top)
   int bottom_lds = 1;     // ... with their arrays in LDS when they fit
   int fp32_exact_bottom = 1;  // FP32 inner cycles: exact sine-transform solve of a 17^3 bottom level
   int use_fused_restrict = 2;  // finest residual + injection in one pass (1: res ring; 2, 3: restriction streamed in z)
@@ -231,6 +234,7 @@ int alloc_level_arrays(pmg_solver *S, Level &Lv, bool f32) {
       PMG_HOST_CHECK(hipMalloc(p, n * sizeof(double)));
       PMG_HOST_CHECK(hipMemsetAsync(*p, 0, n * sizeof(double), S->stream));
     }
+    if (Lv.small) PMG_HOST_CHECK(hipMalloc(&d.sres, n * sizeof(double)));
     if (S->op == 1) {
       for (double **p : {&d.a, &d.c}) {
         PMG_HOST_CHECK(hipMalloc(p, n * sizeof(double)));
@@ -248,6 +252,7 @@ int alloc_level_arrays(pmg_solver *S, Level &Lv, bool f32) {
       PMG_HOST_CHECK(hipMalloc(p, n * sizeof(float)));
       PMG_HOST_CHECK(hipMemsetAsync(*p, 0, n * sizeof(float), S->stream));
     }
+    if (Lv.small) PMG_HOST_CHECK(hipMalloc(&f.sres, n * sizeof(float)));
     if (S->op == 1) {
       for (float **p : {&f.a, &f.c}) {
         PMG_HOST_CHECK(hipMalloc(p, n * sizeof(float)));
@@ -259,7 +264,7 @@ int alloc_level_arrays(pmg_solver *S, Level &Lv, bool f32) {
 
 template <typename T>
 void free_arrays(LevelArrays<T> &A) {
-  for (T **p : {&A.u, &A.ua, &A.rho, &A.rhs, &A.res, &A.lop, &A.a, &A.c}) {
+  for (T **p : {&A.u, &A.ua, &A.rho, &A.rhs, &A.res, &A.lop, &A.a, &A.c, &A.sres}) {
     if (*p) (void)hipFree(*p);
     *p = nullptr;
   }
@@ -311,6 +316,9 @@ int launch_sweep2(pmg_solver *S, SweepP<T> P, bool p2, bool rhs0) {
   if (p2) return rhs0 ? launch_sweep2_v<T, OP, EX, true, true>(S, P) : launch_sweep2_v<T, OP, EX, true, false>(S, P);
   return rhs0 ? launch_sweep2_v<T, OP, EX, false, true>(S, P) : launch_sweep2_v<T, OP, EX, false, false>(S, P);
 }
+
+// the largest level whose legs run as one launch each
+constexpr size_t kSmallPoints = 300000;
 
 // levels where pairs of sweeps run temporally blocked
 bool use_sweep2(const pmg_solver *S, const Level &Lv) {
@@ -423,14 +431,16 @@ int residual(pmg_solver *S, int L, int slot, bool rhs0, bool zero, float *neg32 
 #undef PMG_RS
 }
 
-// restriction of one field from level Lf to Lf-1 (whole grid)
-template <typename T>
-int restrict_field(pmg_solver *S, int Lfine, const T *src, T *dst, T *alt, int kind, bool use_ex) {
-  Level &F = S->lev[Lfine - 1], &Cl = S->lev[Lfine - 2];
+// restriction from level Lfine to Lfine-1 (whole grid): src -> dst (boundary
+// also to alt), and r1 -> r2 in the same launch when given
+template <typename T, bool EXC>
+int restrict_launch(pmg_solver *S, int Lfine, const T *src, T *dst, T *alt, int kind, const T *chr, const T *r1 = nullptr,
+                    T *r2 = nullptr) {
   if (kind == 0) return 0;
-  const size_t n = Cl.size;
-  (void)use_ex;
-#define PMG_RW(K) hipLaunchKernelGGL((k_restrict_whole<T, K, false>), grid3(Cl.n[0], Cl.n[1], Cl.n[2]), dim3(256), 0, S->stream, src, dst, alt, (const T *)nullptr, T(0), F.n[0], F.n[1], F.n[2], Cl.n[0], Cl.n[1], Cl.n[2])
+  Level &F = S->lev[Lfine - 1], &Cl = S->lev[Lfine - 2];
+  dim3 grid = grid3(Cl.n[0], Cl.n[1], Cl.n[2]);
+  if (r1) grid.z *= 2;
+#define PMG_RW(K) hipLaunchKernelGGL((k_restrict_whole<T, K, EXC>), grid, dim3(256), 0, S->stream, src, dst, alt, r1, r2, chr, (T)S->ex, F.n[0], F.n[1], F.n[2], Cl.n[0], Cl.n[1], Cl.n[2])
   if (kind == 1) PMG_RW(1);
   else if (kind == 2) PMG_RW(2);
   else PMG_RW(3);
@@ -439,35 +449,28 @@ int restrict_field(pmg_solver *S, int Lfine, const T *src, T *dst, T *alt, int k
   return 0;
 }
 
-}  // namespace
-
-namespace {
 __global__ void k_chr_bytes(uint8_t *dst, const double *chr, double ex, size_t n) {
   size_t q = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (q < n) dst[q] = chr[q] == ex ? 1 : 0;
 }
 
-int restrict_field_ex64(pmg_solver *S, int Lfine, const double *src, double *dst, double *alt,
-                        int kind) {
-  Level &F = S->lev[Lfine - 1], &Cl = S->lev[Lfine - 2];
-  const size_t n = Cl.size;
-  const double *chrv = F.chrd;
-#define PMG_RWE(K) hipLaunchKernelGGL((k_restrict_whole<double, K, true>), grid3(Cl.n[0], Cl.n[1], Cl.n[2]), dim3(256), 0, S->stream, src, dst, alt, chrv, S->ex, F.n[0], F.n[1], F.n[2], Cl.n[0], Cl.n[1], Cl.n[2])
-  if (kind == 1) PMG_RWE(1);
-  else if (kind == 2) PMG_RWE(2);
-  else PMG_RWE(3);
-#undef PMG_RWE
-  PMG_HOST_CHECK(hipGetLastError());
-  return 0;
+template <typename T>
+int restrict_any(pmg_solver *S, int Lfine, const T *src, T *dst, T *alt, int kind, const T *r1 = nullptr,
+                 T *r2 = nullptr) {
+  if constexpr (std::is_same<T, double>::value) {
+    if (S->do_ex) return restrict_launch<double, true>(S, Lfine, src, dst, alt, kind, S->lev[Lfine - 1].chrd, r1, r2);
+  }
+  return restrict_launch<T, false>(S, Lfine, src, dst, alt, kind, (const T *)nullptr, r1, r2);
 }
 
+// u and f_res of level Lfine injected into the next coarser level
 template <typename T>
-int restrict_any(pmg_solver *S, int Lfine, const T *src, T *dst, T *alt, int kind) {
-  if (kind == 0) return 0;
-  if constexpr (std::is_same<T, double>::value) {
-    if (S->do_ex) return restrict_field_ex64(S, Lfine, src, dst, alt, kind);
-  }
-  return restrict_field<T>(S, Lfine, src, dst, alt, kind, false);
+int inject_u_res(pmg_solver *S, int Lfine, const T *res) {
+  LevelArrays<T> &AC = arrays<T>(S->lev[Lfine - 2]);
+  const T *u = ucur<T>(S->lev[Lfine - 1]);
+  if (S->rop_u == S->rop_res) return restrict_any<T>(S, Lfine, u, AC.u, AC.ua, S->rop_u, res, AC.res);
+  int rc = restrict_any<T>(S, Lfine, u, AC.u, AC.ua, S->rop_u);
+  return rc ? rc : restrict_any<T>(S, Lfine, res, AC.res, (T *)nullptr, S->rop_res);
 }
 
 template <typename T>
@@ -599,16 +602,72 @@ int fold_norms(pmg_solver *S, int slot0, int nslots) {
 // single-workgroup kernel; returns the top level of that range or 0.
 constexpr int kBottomMaxN = 17;
 
+template <typename T>
 int bottom_top(const pmg_solver *S) {
   if (S->do_ex || S->nlev < 3) return 0;
+  // by default the one-launch legs take the levels above 9 points a side (a
+  // 17^3 level is three launches of 5 us there, 50 us as part of the single
+  // workgroup, which takes 9^3 and below into LDS) -- except where the FP32
+  // cycle solves a 17^3 level exactly
+  int mx = S->bottom_max_n;
+  if (mx == 0) mx = S->pre == 2 && S->pst == 2 && !(std::is_same<T, float>::value && S->fp32_exact_bottom && S->op == 0) ? 9 : kBottomMaxN;
+  mx = std::min(kBottomMaxN, mx);
   int Lb = 0;
   for (int L = 1; L < S->nlev && L <= kBotMax; L++) {
     const Level &Lv = S->lev[L - 1];
-    const int mx = std::min(kBottomMaxN, S->bottom_max_n);
     if (Lv.n[0] <= mx && Lv.n[1] <= mx && Lv.n[2] <= mx && Lv.rbox.ok) Lb = L;
     else break;
   }
   return Lb >= 2 ? Lb : 0;
+}
+
+// Levels whose legs run as one launch each (pmg_small.h): V(2,2) cycles, at
+// most kSmallPoints points, above the fused bottom.  Not the finest level
+// while its separate sweeps are being timed, nor where the learned correction
+// sits between its coarse-grid correction and its sweeps.
+template <typename T>
+bool use_small(const pmg_solver *S, int L, int Lb) {
+  const Level &Lv = S->lev[L - 1];
+  if (!Lv.small || L < 2 || L <= Lb || S->pre != 2 || S->pst != 2 || !Lv.rbox.ok || use_sweep2(S, Lv)) return false;
+  if (L == S->nlev && (S->tk_ev || (std::is_same<T, float>::value && S->band.enq_inner))) return false;
+  return small_blocks(Lv.n[0], Lv.n[1], Lv.n[2]) <= S->ws.cap;
+}
+
+template <typename T>
+int small_leg(pmg_solver *S, int L, int leg, int slot) {
+  Level &Lv = S->lev[L - 1];
+  LevelArrays<T> &A = arrays<T>(Lv);
+  const bool fine = L == S->nlev;
+  SmallP<T> P{};
+  P.uin = ucur<T>(Lv); P.uout = uoth<T>(Lv);
+  P.rho = A.rho; P.a = A.a; P.c = A.c; P.rhs = A.rhs; P.res = A.res; P.lop = A.lop;
+  P.res_out = fine ? A.res : A.sres;
+  P.chr = Lv.chr;
+  P.nx = Lv.n[0]; P.ny = Lv.n[1]; P.nz = Lv.n[2];
+  if (leg == 1) {
+    Level &Cl = S->lev[L - 2];
+    LevelArrays<T> &AC = arrays<T>(Cl);
+    P.cu = AC.u; P.clop = AC.lop; P.cres = AC.res;
+    P.cnx = Cl.n[0]; P.cny = Cl.n[1]; P.cnz = Cl.n[2];
+  }
+  P.bx0 = Lv.rbox.lo[0]; P.bx1 = Lv.rbox.hi[0];
+  P.by0 = Lv.rbox.lo[1]; P.by1 = Lv.rbox.hi[1];
+  P.bz0 = Lv.rbox.lo[2]; P.bz1 = Lv.rbox.hi[2];
+  if (Lv.cbox.ok) {
+    P.cx0 = Lv.cbox.lo[0]; P.cx1 = Lv.cbox.hi[0];
+    P.cy0 = Lv.cbox.lo[1]; P.cy1 = Lv.cbox.hi[1];
+    P.cz0 = Lv.cbox.lo[2]; P.cz1 = Lv.cbox.hi[2];
+  } else {
+    P.cx0 = P.cy0 = P.cz0 = 1;
+    P.cx1 = P.cy1 = P.cz1 = 0;
+  }
+  P.w0_r = (T)S->w0_r; P.w0_i = (T)S->w0_i;
+  P.sp = spacing<T>(Lv);
+  P.ws = S->ws;
+  P.slot = slot;
+  const int rc = launch_small<T>(S->stream, leg, P, S->op, S->do_ex != 0, fine);
+  curbuf<T>(Lv) ^= 1;
+  return rc;
 }
 
 // whether the LDS bottom kernel can take lds bytes of dynamic LDS: the
@@ -908,34 +967,45 @@ int timed_sweeps(pmg_solver *S, int L, int n, int slot, bool rhs0) {
 template <typename T>
 int enqueue_vcycle(pmg_solver *S, bool final_residual, int norm_base, double *cnorm, int *citer) {
   const int Lf = S->nlev;
-  const int Lb = S->use_bottom ? bottom_top(S) : 0;
+  const int Lb = S->use_bottom ? bottom_top<T>(S) : 0;
   int rc;
   for (int L = Lf; L >= 1; L--) {
+    const bool small = use_small<T>(S, L, Lb);
     if (L < Lf) {
       LevelArrays<T> &AF = arrays<T>(S->lev[L]);
-      LevelArrays<T> &AC = arrays<T>(S->lev[L - 1]);
-      if (L + 1 == Lf && can_fuse_resid_restrict<T>(S)) {
+      if (use_small<T>(S, L + 1, Lb)) {
+        // its down leg has left the residual
+        if ((rc = inject_u_res<T>(S, L + 1, L + 1 == Lf ? AF.res : AF.sres))) return rc;
+      } else if (L + 1 == Lf && can_fuse_resid_restrict<T>(S)) {
         if ((rc = resid_restrict<T>(S, norm_base + NS_RESID + L))) return rc;
       } else {
         // residual on L+1; the finest level was cleared at the cycle start
         if ((rc = residual<T>(S, L + 1, norm_base + NS_RESID + L, L + 1 == Lf, L + 1 == Lf))) return rc;
         // PAMR_inject(L+1): u and u_res (sources are constant, restricted once)
-        if ((rc = restrict_any<T>(S, L + 1, ucur<T>(S->lev[L]), AC.u, AC.ua, S->rop_u))) return rc;
-        if ((rc = restrict_any<T>(S, L + 1, AF.res, AC.res, (T *)nullptr, S->rop_res))) return rc;
+        if ((rc = inject_u_res<T>(S, L + 1, AF.res))) return rc;
       }
       if (L == Lb) {
         if ((rc = bottom<T>(S, Lb, norm_base, cnorm, citer))) return rc;
         break;
       }
-      if ((rc = lop_rhs<T>(S, L))) return rc;
+      if (!small && (rc = lop_rhs<T>(S, L))) return rc;
     }
     if (L == 1) {
       if ((rc = coarse_solve<T>(S, 1, cnorm, cnorm + 1, citer, S->max_citer))) return rc;
+    } else if (small) {
+      if ((rc = small_leg<T>(S, L, 0, norm_base + NS_RESID + L - 1))) return rc;
     } else {
       if ((rc = timed_sweeps<T>(S, L, S->pre, norm_base + NS_RELAX + L - 1, L == Lf))) return rc;
     }
   }
   for (int L = Lb ? Lb + 1 : 2; L <= Lf; L++) {
+    if (use_small<T>(S, L, Lb)) {
+      // the excision-aware correction of the FP64 cycle runs by itself
+      const bool alone = std::is_same<T, double>::value && S->do_ex;
+      if (alone && (rc = cgc<T>(S, L))) return rc;
+      if ((rc = small_leg<T>(S, L, alone ? 2 : 1, norm_base + NS_RELAX + L - 1))) return rc;
+      continue;
+    }
     if ((rc = cgc<T>(S, L))) return rc;
     if constexpr (std::is_same<T, float>::value) {
       // the learned band correction of the finest level's coarse-grid correction
@@ -1166,6 +1236,7 @@ pmg_solver *pmg_create(int nx, int ny, int nz, const double *bbox, int min_cwidt
     }
     Lv.rbox = b;
     Lv.cbox = cmask_child_box(Lv.n, bbox, bbox, Lv.gdx, bbox);
+    Lv.small = Lv.size <= kSmallPoints;
     if (alloc_level_arrays(S, Lv, false)) { pmg_destroy(S); return nullptr; }
   }
   for (int L = 1; L <= nl; L++) {
@@ -1320,7 +1391,7 @@ int pmg_set_resid_restrict_zchunk(pmg_solver *S, int prec, int czchunk) {
 int pmg_set_bottom_fusion(pmg_solver *S, int on) {
   if (!S || on < 0 || on > kBottomMaxN) return -1;
   S->use_bottom = on ? 1 : 0;
-  S->bottom_max_n = on > 1 ? on : kBottomMaxN;
+  S->bottom_max_n = on > 1 ? on : 0;
   invalidate_graphs(S);
   return 0;
 }
@@ -1424,14 +1495,17 @@ int pmg_init(pmg_solver *S) {
   int rc;
   for (int L = S->nlev; L > 1; L--) {
     Level &F = S->lev[L - 1], &Cl = S->lev[L - 2];
-    if ((rc = restrict_any<double>(S, L, F.d.u, Cl.d.u, nullptr, S->rop_u))) return rc;
-    if ((rc = restrict_any<double>(S, L, F.d.rho, Cl.d.rho, nullptr, S->rop_src))) return rc;
+    if (S->rop_u == S->rop_src) {
+      if ((rc = restrict_any<double>(S, L, F.d.u, Cl.d.u, nullptr, S->rop_u, F.d.rho, Cl.d.rho))) return rc;
+    } else {
+      if ((rc = restrict_any<double>(S, L, F.d.u, Cl.d.u, nullptr, S->rop_u))) return rc;
+      if ((rc = restrict_any<double>(S, L, F.d.rho, Cl.d.rho, nullptr, S->rop_src))) return rc;
+    }
     if (S->op == 1) {
       // the coefficients of the (project-defined) variable-coefficient
       // operator have no excised value: restricted without the excision
       // renormalisation, also when excision is on
-      if ((rc = restrict_field<double>(S, L, F.d.a, Cl.d.a, nullptr, S->rop_src, false))) return rc;
-      if ((rc = restrict_field<double>(S, L, F.d.c, Cl.d.c, nullptr, S->rop_src, false))) return rc;
+      if ((rc = restrict_launch<double, false>(S, L, F.d.a, Cl.d.a, nullptr, S->rop_src, nullptr, F.d.c, Cl.d.c))) return rc;
     }
   }
   for (int L = 1; L <= S->nlev; L++) {
