@@ -330,11 +330,16 @@ class Solver:
     def apply_tuning(self):
         """Per-level sweep tile/z-chunk of the FP64 and the FP32 sweeps from
         the autotuner table (tuning.json): the entry tuned for this operator
-        and excision when there is one, else the plain Poisson entry."""
+        and excision when there is one, else the plain Poisson entry.  The
+        table holds cubes; levels of another shape, and sizes it has not, keep
+        the library's own choice."""
         from .autotune import tuned_level_config
         for lev in range(1, self.nlev + 1):
+            shape = self.shape(lev)
+            if len(set(shape)) > 1:
+                continue
             for pi, prec in enumerate(("f64", "f32")):
-                cfg = tuned_level_config(self.shape(lev)[2], prec, self.op, self.do_ex)
+                cfg = tuned_level_config(shape[2], prec, self.op, self.do_ex)
                 if cfg is not None:
                     _check(self._L.pmg_set_level_sweep_config_prec(self.h, lev, pi, *cfg),
                            "pmg_set_level_sweep_config_prec")

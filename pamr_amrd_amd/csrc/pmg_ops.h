@@ -8,12 +8,6 @@
 
 namespace pmg {
 
-// x/d2, or x*inv when d2 is an exact power of two (then identical bits).
-template <typename T, bool P2>
-__device__ __forceinline__ T divd(T x, T d2, T inv) {
-  if constexpr (P2) return x * inv; else return x / d2;
-}
-
 // a / b rounded to nearest from y = RN(1/b), without a division: q0 =
 // RN(a y) is within 2 ulps of a/b; one correction with the exact remainder
 // (an FMA), q1 = RN(q0 + (a - b q0) y), is faithful; a second one with a
@@ -28,6 +22,53 @@ __device__ __forceinline__ double div_rn(double a, double b, double y) {
   const double q1 = __builtin_fma(r0, y, q0);
   const double r1 = __builtin_fma(-b, q1, a);
   return __builtin_fma(r1, y, q1);
+}
+
+__device__ __forceinline__ float div_rn(float a, float b, float y) {
+  const float q0 = a * y;
+  const float r0 = __builtin_fmaf(-b, q0, a);
+  const float q1 = __builtin_fmaf(r0, y, q0);
+  const float r1 = __builtin_fmaf(-b, q1, a);
+  return __builtin_fmaf(r1, y, q1);
+}
+
+// |v| in [2^-E, 2^E): neither zero nor infinite, NaN or subnormal
+template <int E>
+__device__ __forceinline__ bool mid_range(double v) {
+  return ((unsigned)__double2hiint(v) & 0x7fffffffu) - ((unsigned)(1023 - E) << 20) < ((unsigned)(2 * E) << 20);
+}
+template <int E>
+__device__ __forceinline__ bool mid_range(float v) {
+  return ((unsigned)__float_as_int(v) & 0x7fffffffu) - ((unsigned)(127 - E) << 23) < ((unsigned)(2 * E) << 23);
+}
+
+// x / dx2, y / dy2, z / dz2, rounded as the division rounds.  With spacings
+// whose squares are powers of two (P2) the product with the inverse is that
+// quotient; otherwise div_rn is, while no intermediate leaves the normal
+// range: the first quotient within 2^(+-600) and the inverse within 2^(+-200)
+// (FP32: 60 and 30) keep every remainder's last bit above the smallest
+// subnormal.  Anything else (zeros, tiny, infinite) takes the division itself.
+// 15 FP64 operations for the three instead of about 36: the sweep of a
+// 161 x 97 x 129 grid with 1/160 spacing 33 -> 24 us.
+template <typename T, bool P2>
+__device__ __forceinline__ void div3(T &x, T &y, T &z, const Spacing<T> &sp) {
+  if constexpr (P2) {
+    x = x * sp.idx2;
+    y = y * sp.idy2;
+    z = z * sp.idz2;
+  } else {
+    constexpr int EQ = std::is_same<T, double>::value ? 600 : 60, EI = std::is_same<T, double>::value ? 200 : 30;
+    const bool inv = mid_range<EI>(sp.idx2) && mid_range<EI>(sp.idy2) && mid_range<EI>(sp.idz2);
+    if (inv && mid_range<EQ>(x * sp.idx2) && mid_range<EQ>(y * sp.idy2) && mid_range<EQ>(z * sp.idz2)) {
+      x = div_rn(x, sp.dx2, sp.idx2);
+      y = div_rn(y, sp.dy2, sp.idy2);
+      z = div_rn(z, sp.dz2, sp.idz2);
+    } else {
+      x = x / sp.dx2;
+      y = y / sp.dy2;
+      z = z / sp.dz2;
+    }
+  }
 }
 
 // res / jac of the relaxation update V - res/Jac: with the plain operator
@@ -45,9 +86,8 @@ __device__ __forceinline__ T div_jac(T r, T jac, const Spacing<T> &sp) {
 template <typename T, bool P2>
 __device__ __forceinline__ T lop_poisson(T uc, T ue, T uw, T un, T us, T ut, T ub,
                                          T rho, const Spacing<T> &sp) {
-  T lx = divd<T, P2>((ue - 2 * uc) + uw, sp.dx2, sp.idx2);
-  T ly = divd<T, P2>((un - 2 * uc) + us, sp.dy2, sp.idy2);
-  T lz = divd<T, P2>((ut - 2 * uc) + ub, sp.dz2, sp.idz2);
+  T lx = (ue - 2 * uc) + uw, ly = (un - 2 * uc) + us, lz = (ut - 2 * uc) + ub;
+  div3<T, P2>(lx, ly, lz, sp);
   return ((lx + ly) + lz) - rho;
 }
 
@@ -61,12 +101,13 @@ __device__ __forceinline__ T lop_varcoef(T uc, T ue, T uw, T un, T us, T ut, T u
   T fe = T(0.5) * (ac + ae), fw = T(0.5) * (ac + aw);
   T fn = T(0.5) * (ac + an), fs = T(0.5) * (ac + as);
   T ft = T(0.5) * (ac + at), fb = T(0.5) * (ac + ab);
-  T lx = divd<T, P2>(fe * (ue - uc) - fw * (uc - uw), sp.dx2, sp.idx2);
-  T ly = divd<T, P2>(fn * (un - uc) - fs * (uc - us), sp.dy2, sp.idy2);
-  T lz = divd<T, P2>(ft * (ut - uc) - fb * (uc - ub), sp.dz2, sp.idz2);
-  if (jac)
-    *jac = ((divd<T, P2>(-(fe + fw), sp.dx2, sp.idx2) - divd<T, P2>(fn + fs, sp.dy2, sp.idy2)) -
-            divd<T, P2>(ft + fb, sp.dz2, sp.idz2)) + cc;
+  T lx = fe * (ue - uc) - fw * (uc - uw), ly = fn * (un - uc) - fs * (uc - us), lz = ft * (ut - uc) - fb * (uc - ub);
+  div3<T, P2>(lx, ly, lz, sp);
+  if (jac) {
+    T jx = -(fe + fw), jy = fn + fs, jz = ft + fb;
+    div3<T, P2>(jx, jy, jz, sp);
+    *jac = ((jx - jy) - jz) + cc;
+  }
   return (((lx + ly) + lz) + cc * uc) - rho;
 }
 

@@ -325,6 +325,31 @@ bool use_sweep2(const pmg_solver *S, const Level &Lv) {
   return S->use_sweep2 && Lv.n[0] >= kSweep2MinN && Lv.n[1] >= kSweep2MinN && Lv.n[2] >= kSweep2MinN;
 }
 
+// Tile variant and z chunk of a level that was never tuned, from what the
+// tuned sizes show.  From 200^3 points on: 128 x 16 columns with one
+// 1024-thread workgroup per CU (the variable coefficient's LDS ring: 32 x 16 in
+// FP64, the five-plane 128 x 16 in FP32), the longest march that leaves 256 of
+// them; 64 x 16 where 128 columns would leave more than a sixth of the tile
+// outside.  Below: 32 x 16 columns, the longest march of 64 .. 2 planes that
+// makes 400 workgroups -- fewer leave CUs without work, shorter marches repeat
+// the prologue (129^3: 18.7 us at 8 planes and 512 workgroups, 28.5 at 16 on
+// 64 x 16 tiles; 65^3: 8.3 us at 2 planes, 12.8 at 8).
+void default_sweep(const int *n, int op, int pi, int *variant, int *zchunk) {
+  const size_t size = (size_t)n[0] * n[1] * n[2];
+  int tx = 32, ty = 16, want = 400;
+  *variant = 2;
+  if (size >= 8000000 && !(op == 1 && pi == 0)) {
+    const int w = n[0] - 2, w128 = (w + 127) / 128 * 128;
+    tx = 6 * (w128 - w) > w128 ? 64 : 128;
+    *variant = tx == 64 ? 1 : (op == 1 ? 10 : 5);
+    want = tx == 64 ? 400 : 256;
+  }
+  const int cols = ((n[0] - 2 + tx - 1) / tx) * ((n[1] - 2 + ty - 1) / ty);
+  int z = 64;
+  while (z > 2 && cols * ((n[2] - 2 + z - 1) / z) < want) z /= 2;
+  *zchunk = z;
+}
+
 // n red-black sweeps on level L (ping-pong u <-> ua; odd counts copy back)
 template <typename T>
 int sweeps(pmg_solver *S, int L, int n, int slot, bool rhs0) {
@@ -1239,19 +1264,23 @@ pmg_solver *pmg_create(int nx, int ny, int nz, const double *bbox, int min_cwidt
     Lv.small = Lv.size <= kSmallPoints;
     if (alloc_level_arrays(S, Lv, false)) { pmg_destroy(S); return nullptr; }
   }
-  for (int L = 1; L <= nl; L++) {
-    const int n = S->lev[L - 1].n[2];
-    for (int pi = 0; pi < 2; pi++) {
-      S->lv_variant[pi][L - 1] = 1;
-      S->lv_zchunk[pi][L - 1] = n >= 257 ? 32 : (n >= 129 ? 16 : (n >= 65 ? 8 : 4));
-    }
-  }
+  for (int L = 1; L <= nl; L++)
+    for (int pi = 0; pi < 2; pi++) default_sweep(S->lev[L - 1].n, op, pi, &S->lv_variant[pi][L - 1], &S->lv_zchunk[pi][L - 1]);
   // coarse planes per block of the fused finest residual + injection
   // (streamed kernel), the fastest measured: 6 (FP64) and 4 (FP32) on a
-  // coarse level of 129 planes, 8 and 8 from 257 planes; smaller grids 8
-  if (nl >= 2 && S->lev[nl - 2].n[2] >= 129 && S->lev[nl - 2].n[2] < 257) {
-    S->rr_czchunk[0] = 6;
-    S->rr_czchunk[1] = 4;
+  // coarse level of 129 planes, 8 and 8 from 257 planes.  On smaller grids a
+  // block's march is the time: as many planes as still make 1000 blocks, at
+  // least 2 (161 x 97 x 129 fine points, FP64: 47 us with 8, 18 with 2)
+  if (nl >= 2) {
+    const int *cn = S->lev[nl - 2].n;
+    for (int pi = 0; pi < 2; pi++) {
+      int cz = cn[2] >= 257 ? 8 : (pi ? 4 : 6);
+      if (cn[2] < 129) cz = 8;
+      while (cn[2] < 257 && cz > 2 &&
+             (pi ? resid_restrict_blocks<float>(cn, cz, true) : resid_restrict_blocks<double>(cn, cz, true)) < 1000)
+        cz /= 2;
+      S->rr_czchunk[pi] = cz;
+    }
   }
   // norm workspace sized for the largest launch
   // partial-norm capacity: the largest launch over the finest level
