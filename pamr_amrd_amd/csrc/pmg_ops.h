@@ -205,71 +205,32 @@ __device__ __forceinline__ T fw_point_ex(const T *u1, const T *chr1, T ex, int n
   const int im = i0 - 1, jm = j0 - 1, km = k0 - 1, ip = i0 + 1, jp = j0 + 1, kp = k0 + 1;
   const bool xi = i0 > 1 && i0 <= nx1 - 1, yi = j0 > 1 && j0 <= ny1 - 1,
              zi = k0 > 1 && k0 <= nz1 - 1;
+  (void)im; (void)jm; (void)km; (void)ip; (void)jp; (void)kp;
+  if (!xi && !yi && !zi) return PMG_CH(i0, j0, k0) == ex ? T(0) : PMG_U1(i0, j0, k0);
+  // The full, plane and line stencils are one product of weights: an axis
+  // that does not take part has the point itself with weight 1.  All 54
+  // values are requested together (points of absent axes repeat the centre's
+  // and are not added); as loops over the face stencils, the lanes on a face
+  // held their wavefronts through a chain of dependent loads (31 -> 17 us for
+  // 161 x 97 x 129 fine points).
+  T cv[27], uv[27];
+#pragma unroll
+  for (int q = 0; q < 27; q++) {
+    const int a = xi ? q / 9 - 1 : 0, b = yi ? (q / 3) % 3 - 1 : 0, c = zi ? q % 3 - 1 : 0;
+    cv[q] = PMG_CH(i0 + a, j0 + b, k0 + c);
+    uv[q] = PMG_U1(i0 + a, j0 + b, k0 + c);
+  }
   T sum = 0;
   int w = 0;
-  if (xi && yi && zi) {
-    // unrolled: constant weights, and all 54 loads in flight together
-    T cv[27], uv[27];
 #pragma unroll
-    for (int q = 0; q < 27; q++) {
-      cv[q] = PMG_CH(im + q / 9, jm + (q / 3) % 3, km + q % 3);
-      uv[q] = PMG_U1(im + q / 9, jm + (q / 3) % 3, km + q % 3);
+  for (int q = 0; q < 27; q++) {
+    const int oa = q / 9 - 1, ob = (q / 3) % 3 - 1, oc = q % 3 - 1;
+    const bool in = (xi || oa == 0) && (yi || ob == 0) && (zi || oc == 0);
+    const int ww = (xi && oa == 0 ? 2 : 1) * (yi && ob == 0 ? 2 : 1) * (zi && oc == 0 ? 2 : 1);
+    if (in && cv[q] != ex) {
+      sum = sum + ww * uv[q];
+      w += !xi && !yi ? w3d_kbranch(iloop, oc + 2) : ww;
     }
-#pragma unroll
-    for (int q = 0; q < 27; q++) {
-      const int ww = (q / 9 == 1 ? 2 : 1) * ((q / 3) % 3 == 1 ? 2 : 1) * (q % 3 == 1 ? 2 : 1);
-      if (cv[q] != ex) {
-        sum = sum + ww * uv[q];
-        w += ww;
-      }
-    }
-  } else if (xi && yi) {
-    for (int a = im; a <= ip; a++)
-      for (int b = jm; b <= jp; b++)
-        if (PMG_CH(a, b, k0) != ex) {
-          int ww = w3d(a - im + 1, b - jm + 1, 1);
-          sum = sum + ww * PMG_U1(a, b, k0);
-          w += ww;
-        }
-  } else if (yi && zi) {
-    for (int b = jm; b <= jp; b++)
-      for (int c = km; c <= kp; c++)
-        if (PMG_CH(i0, b, c) != ex) {
-          int ww = w3d(1, b - jm + 1, c - km + 1);
-          sum = sum + ww * PMG_U1(i0, b, c);
-          w += ww;
-        }
-  } else if (xi && zi) {
-    for (int a = im; a <= ip; a++)
-      for (int c = km; c <= kp; c++)
-        if (PMG_CH(a, j0, c) != ex) {
-          int ww = w3d(a - im + 1, 1, c - km + 1);
-          sum = sum + ww * PMG_U1(a, j0, c);
-          w += ww;
-        }
-  } else if (xi) {
-    for (int a = im; a <= ip; a++)
-      if (PMG_CH(a, j0, k0) != ex) {
-        int ww = w3d(a - im + 1, 1, 1);
-        sum = sum + ww * PMG_U1(a, j0, k0);
-        w += ww;
-      }
-  } else if (yi) {
-    for (int b = jm; b <= jp; b++)
-      if (PMG_CH(i0, b, k0) != ex) {
-        int ww = w3d(1, b - jm + 1, 1);
-        sum = sum + ww * PMG_U1(i0, b, k0);
-        w += ww;
-      }
-  } else if (zi) {
-    for (int c = km; c <= kp; c++)
-      if (PMG_CH(i0, j0, c) != ex) {
-        sum = sum + w3d(1, 1, c - km + 1) * PMG_U1(i0, j0, c);
-        w += w3d_kbranch(iloop, c - km + 1);
-      }
-  } else {
-    sum = PMG_U1(i0, j0, k0);
-    w = 1;
   }
   if (w == 0 || PMG_CH(i0, j0, k0) == ex) return T(0);
   return sum / w;

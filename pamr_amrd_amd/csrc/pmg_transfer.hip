@@ -7,6 +7,8 @@
 // nothing written); launch errors return -1.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 #include "pamr_mg_gpu.h"
 
 #include "pmg_ops.h"
@@ -17,19 +19,66 @@ namespace {
 
 constexpr int NT = 256;
 
-inline unsigned nblk(size_t n) { return (unsigned)((n + NT - 1) / NT); }
+// q / d for 0 <= q < 2^31, 1 <= d < 2^31: q * m >> 31 + l with l = ceil(log2
+// d), m = floor(2^(31+l) / d) + 1 (Granlund and Montgomery, "Division by
+// invariant integers using multiplication", PLDI 1994: the error m d - 2^(31+l)
+// <= d <= 2^l times q stays below 2^(31+l)).
+struct Div31 {
+  unsigned m, d;
+  int s;
+  __device__ __forceinline__ int div(int q, int &rem) const {
+    const int t = (int)(((unsigned long long)(unsigned)q * m) >> s);
+    rem = q - t * (int)d;
+    return t;
+  }
+};
+inline Div31 make_div31(int d) {
+  int l = 0;
+  while ((1ll << l) < d) l++;
+  return Div31{(unsigned)((1ull << (31 + l)) / (unsigned)d + 1), (unsigned)d, 31 + l};
+}
+
+// The points of an ni x nj x nk box by one linear index, one per thread: full
+// wavefronts whatever the sides.  The indices come from multiplications: with
+// 64-bit divisions these, not the memory, bounded the kernels (trilinear
+// interpolation onto 161 x 97 x 129 points: 19 us, rows of 64 threads 13 us).
+struct BoxPts {
+  Div31 di, dj;
+  int n, k0;
+};
+template <typename F>
+__device__ __forceinline__ void for_box(const BoxPts &b, const F &f) {
+  const int q = (int)(blockIdx.x * NT + threadIdx.x);
+  if (q >= b.n) return;
+  int i, j;
+  const int t = b.di.div(q, i), k = b.dj.div(t, j);
+  f(i, j, k + b.k0);
+}
+// launch(grid, points) over an ni x nj x nk box, in slabs of whole k planes
+// with fewer than 2^31 points; -1 when one plane has more or a launch fails
+template <typename L>
+int box_launch(int ni, int nj, int nk, const L &launch) {
+  const long long plane = (long long)ni * nj, most = (1ll << 31) - NT;
+  if (plane > most) return -1;
+  const int step = (int)std::min<long long>(nk, most / plane);
+  for (int k0 = 0; k0 < nk; k0 += step) {
+    const BoxPts b{make_div31(ni), make_div31(nj), (int)(plane * std::min(step, nk - k0)), k0};
+    launch(dim3((unsigned)((b.n + NT - 1) / NT)), b);
+    PMG_HOST_CHECK(hipGetLastError());
+  }
+  return 0;
+}
 
 // dmcopy3d, src/m_util_r8.f:20-50
 template <typename T>
 __global__ __launch_bounds__(NT) void k_copy3d(const T *u1, T *u2, int nx1, int ny1, int nx2,
                                                int ny2, int i1, int j1, int k1, int i2, int j2,
                                                int k2, int ni, int nj, int nk, int si1, int sj1,
-                                               int sk1, int si2, int sj2, int sk2) {
-  size_t q = (size_t)blockIdx.x * NT + threadIdx.x;
-  if (q >= (size_t)ni * nj * nk) return;
-  int i = (int)(q % ni), j = (int)((q / ni) % nj), k = (int)(q / ((size_t)ni * nj));
-  u2[ix3(i2 - 1 + i * si2, j2 - 1 + j * sj2, k2 - 1 + k * sk2, nx2, ny2)] =
-      u1[ix3(i1 - 1 + i * si1, j1 - 1 + j * sj1, k1 - 1 + k * sk1, nx1, ny1)];
+                                               int sk1, int si2, int sj2, int sk2, BoxPts bp) {
+  for_box(bp, [&](int i, int j, int k) {
+    u2[ix3(i2 - 1 + i * si2, j2 - 1 + j * sj2, k2 - 1 + k * sk2, nx2, ny2)] =
+        u1[ix3(i1 - 1 + i * si1, j1 - 1 + j * sj1, k1 - 1 + k * sk1, nx1, ny1)];
+  });
 }
 
 // dmfwr3d / dmhwr3d over an ni x nj x nk target segment
@@ -39,19 +88,18 @@ __global__ __launch_bounds__(NT) void k_restrict3d(const T *u1, T *u2, const T *
                                                    int i1, int j1, int k1, int i2, int j2,
                                                    int k2, int ni, int nj, int nk, int si1,
                                                    int sj1, int sk1, int si2, int sj2,
-                                                   int sk2) {
-  size_t q = (size_t)blockIdx.x * NT + threadIdx.x;
-  if (q >= (size_t)ni * nj * nk) return;
-  int i = (int)(q % ni), j = (int)((q / ni) % nj), k = (int)(q / ((size_t)ni * nj));
-  int i0 = i1 + i * si1, j0 = j1 + j * sj1, k0 = k1 + k * sk1;
-  T v;
-  if constexpr (KIND == 3) {
-    if constexpr (EXC) v = fw_point_ex<T>(u1, chr1, ex, nx1, ny1, nz1, i0, j0, k0, i + 1);
-    else v = fw_point<T>(u1, nx1, ny1, nz1, i0, j0, k0);
-  } else {
-    v = hw_point<T, EXC>(u1, chr1, ex, nx1, ny1, nz1, i0, j0, k0);
-  }
-  u2[ix3(i2 - 1 + i * si2, j2 - 1 + j * sj2, k2 - 1 + k * sk2, nx2, ny2)] = v;
+                                                   int sk2, BoxPts bp) {
+  for_box(bp, [&](int i, int j, int k) {
+    const int i0 = i1 + i * si1, j0 = j1 + j * sj1, k0 = k1 + k * sk1;
+    T v;
+    if constexpr (KIND == 3) {
+      if constexpr (EXC) v = fw_point_ex<T>(u1, chr1, ex, nx1, ny1, nz1, i0, j0, k0, i + 1);
+      else v = fw_point<T>(u1, nx1, ny1, nz1, i0, j0, k0);
+    } else {
+      v = hw_point<T, EXC>(u1, chr1, ex, nx1, ny1, nz1, i0, j0, k0);
+    }
+    u2[ix3(i2 - 1 + i * si2, j2 - 1 + j * sj2, k2 - 1 + k * sk2, nx2, ny2)] = v;
+  });
 }
 
 // dminterp3d with ord = 2 and no excision: the three line phases of
@@ -66,30 +114,32 @@ __device__ __forceinline__ T interp_coef(int r, int rho, T *c1) {
   return (T)(1 - sg);
 }
 
-template <typename T>
+// R2: all three ratios are 2 (shifts for the divisions, 0.5 for both weights)
+template <typename T, bool R2>
 __global__ __launch_bounds__(NT) void k_interp3d(const T *u1, T *u2, int nx1, int ny1, int nx2,
                                                  int ny2, int i1, int j1, int k1, int i2,
                                                  int j2, int k2, int ni, int nj, int nk,
                                                  int si1, int sj1, int sk1, int irho, int jrho,
-                                                 int krho) {
+                                                 int krho, BoxPts bp) {
+  if (R2) irho = jrho = krho = 2;
   const int mi = (ni - 1) * irho + 1, mj = (nj - 1) * jrho + 1, mk = (nk - 1) * krho + 1;
-  size_t q = (size_t)blockIdx.x * NT + threadIdx.x;
-  if (q >= (size_t)mi * mj * mk) return;
-  int fi = (int)(q % mi), fj = (int)((q / mi) % mj), fk = (int)(q / ((size_t)mi * mj));
-  int ai = fi / irho, ri = fi % irho, aj = fj / jrho, rj = fj % jrho, ak = fk / krho,
-      rk = fk % krho;
-  auto U = [&](int a, int b, int c) -> T {
-    return u1[ix3(i1 - 1 + a * si1, j1 - 1 + b * sj1, k1 - 1 + c * sk1, nx1, ny1)];
-  };
-  T cx1, cy1, cz1;
-  T cx0 = interp_coef<T>(ri, irho, &cx1), cy0 = interp_coef<T>(rj, jrho, &cy1),
-    cz0 = interp_coef<T>(rk, krho, &cz1);
-  auto X = [&](int b, int c) -> T {
-    return ri == 0 ? U(ai, b, c) : cx0 * U(ai, b, c) + cx1 * U(ai + 1, b, c);
-  };
-  auto Y = [&](int c) -> T { return rj == 0 ? X(aj, c) : cy0 * X(aj, c) + cy1 * X(aj + 1, c); };
-  T v = rk == 0 ? Y(ak) : cz0 * Y(ak) + cz1 * Y(ak + 1);
-  u2[ix3(i2 - 1 + fi, j2 - 1 + fj, k2 - 1 + fk, nx2, ny2)] = v;
+  for_box(bp, [&](int fi, int fj, int fk) {
+    const int ai = fi / irho, ri = fi % irho, aj = fj / jrho, rj = fj % jrho, ak = fk / krho, rk = fk % krho;
+    auto U = [&](int a, int b, int c) -> T {
+      return u1[ix3(i1 - 1 + a * si1, j1 - 1 + b * sj1, k1 - 1 + c * sk1, nx1, ny1)];
+    };
+    T cx1 = T(0.5), cy1 = T(0.5), cz1 = T(0.5), cx0 = T(0.5), cy0 = T(0.5), cz0 = T(0.5);
+    if constexpr (!R2) {
+      cx0 = interp_coef<T>(ri, irho, &cx1);
+      cy0 = interp_coef<T>(rj, jrho, &cy1);
+      cz0 = interp_coef<T>(rk, krho, &cz1);
+    }
+    auto X = [&](int b, int c) -> T {
+      return ri == 0 ? U(ai, b, c) : cx0 * U(ai, b, c) + cx1 * U(ai + 1, b, c);
+    };
+    auto Y = [&](int c) -> T { return rj == 0 ? X(aj, c) : cy0 * X(aj, c) + cy1 * X(aj + 1, c); };
+    u2[ix3(i2 - 1 + fi, j2 - 1 + fj, k2 - 1 + fk, nx2, ny2)] = rk == 0 ? Y(ak) : cz0 * Y(ak) + cz1 * Y(ak + 1);
+  });
 }
 
 // ---- fourth-order interpolation (dminterp3d, ord = 4, no excision) ------
@@ -102,41 +152,24 @@ __global__ __launch_bounds__(NT) void k_interp3d(const T *u1, T *u2, int nx1, in
 // reference's order x, y, z on u2 after the common points were copied.
 template <int AX>
 __global__ __launch_bounds__(NT) void k_interp4(double *u2, int nx2, int ny2, int nz2, int i2, int j2, int k2, int ni,
-                                                int nj, int nk, int irho, int jrho, int krho) {
+                                                int nj, int nk, int irho, int jrho, int krho, BoxPts bp) {
   const int mi = (ni - 1) * irho + 1, mj = (nj - 1) * jrho + 1, mk = (nk - 1) * krho + 1;
-  const size_t q = (size_t)blockIdx.x * NT + threadIdx.x;
-  int fi, fj, fk;  // offsets from (i2, j2, k2); the phase's own axis is the fine one
-  if (AX == 0) {
-    if (q >= (size_t)mi * nj * nk) return;
-    fi = (int)(q % mi);
-    const int line = (int)(q / mi);
-    fj = (line % nj) * jrho;
-    fk = (line / nj) * krho;
-    if (fi % irho == 0) return;
-    auto A = [&](int a) -> double { return u2[ix3(i2 - 1 + a * irho, j2 - 1 + fj, k2 - 1 + fk, nx2, ny2)]; };
-    u2[ix3(i2 - 1 + fi, j2 - 1 + fj, k2 - 1 + fk, nx2, ny2)] = vi4_point(ni, irho, i2, nx2, fi, A);
-  } else if (AX == 1) {
-    if (q >= (size_t)mi * mj * nk) return;
-    fj = (int)(q % mj);
-    const size_t line = q / mj;
-    fi = (int)(line % mi);
-    fk = (int)(line / mi) * krho;
-    if (fj % jrho == 0) return;
-    auto A = [&](int a) -> double { return u2[ix3(i2 - 1 + fi, j2 - 1 + a * jrho, k2 - 1 + fk, nx2, ny2)]; };
-    u2[ix3(i2 - 1 + fi, j2 - 1 + fj, k2 - 1 + fk, nx2, ny2)] = vi4_point(nj, jrho, j2, ny2, fj, A);
-  } else {
-    if (q >= (size_t)mi * mj * mk) return;
-    fk = (int)(q / ((size_t)mi * mj));
-    const size_t rest = q % ((size_t)mi * mj);
-    fi = (int)(rest % mi);
-    fj = (int)(rest / mi);
-    if (fk % krho == 0) return;
-    auto A = [&](int a) -> double { return u2[ix3(i2 - 1 + fi, j2 - 1 + fj, k2 - 1 + a * krho, nx2, ny2)]; };
-    u2[ix3(i2 - 1 + fi, j2 - 1 + fj, k2 - 1 + fk, nx2, ny2)] = vi4_point(nk, krho, k2, nz2, fk, A);
-  }
+  // offsets from (i2, j2, k2); axes behind the phase's own are still coarse
+  for_box(bp, [&](int fi, int fj, int fk) {
+    if (AX < 1) fj *= jrho;
+    if (AX < 2) fk *= krho;
+    const int f = AX == 0 ? fi : (AX == 1 ? fj : fk), rho = AX == 0 ? irho : (AX == 1 ? jrho : krho);
+    if (f % rho == 0) return;
+    auto A = [&](int a) -> double {
+      return u2[ix3(i2 - 1 + (AX == 0 ? a * irho : fi), j2 - 1 + (AX == 1 ? a * jrho : fj),
+                    k2 - 1 + (AX == 2 ? a * krho : fk), nx2, ny2)];
+    };
+    u2[ix3(i2 - 1 + fi, j2 - 1 + fj, k2 - 1 + fk, nx2, ny2)] =
+        AX == 0 ? vi4_point(ni, irho, i2, nx2, f, A) : (AX == 1 ? vi4_point(nj, jrho, j2, ny2, f, A) : vi4_point(nk, krho, k2, nz2, f, A));
+  });
 }
 
-// ---- excision interpolation: one thread per line (dvi2q1d_ex) ----------
+// ---- excision interpolation -------------------------------------------
 // Line view: v(q) for q = 1..n1 (1-based) at stride sv elements.
 template <typename T, typename CHR>
 __device__ void line_vi2q1d_ex(T *v, int i1, int n1, int n, int irho, int s1, int s2,
@@ -278,8 +311,93 @@ struct ChrtCols {
   }
 };
 
+// One line phase of the second-order excised interpolation, one thread per
+// point.  dvi2q1d_ex walks a line: it first replaces the value of every
+// excised anchor that has non-excised neighbours by an extrapolation from
+// them, then interpolates between anchors.  The extrapolations read only
+// non-excised anchors, which it never changes, so each anchor's value -- and
+// each point between two anchors -- follows from the line as it was before:
+// no order along the line is needed.  (A thread per line left most of the
+// chip idle behind a serial walk: 89 + 66 + 131 us for the x, y and z lines of
+// 161 x 97 x 129 points, now 7 + 5 + 9.)  In place on u2: an anchor is written
+// only if its extrapolation succeeded, and no other point reads it then.
+template <typename T, typename CHR>
+__device__ __forceinline__ bool anchor_ex(const T *v, long long i10, long long n1, long long s1, const CHR &chr, int i30,
+                                          int s3, T ex, T &val) {
+#define LV(q) v[(q)-1]
+#define LC(q) chr((q)-1)
+  if (LC(i30) == ex) {
+    if (i10 > 3 * s1 && LC(i30 - s3) != ex && LC(i30 - 2 * s3) != ex && LC(i30 - 3 * s3) != ex)
+      val = 3 * (LV(i10 - s1) - LV(i10 - 2 * s1)) + LV(i10 - 3 * s1);
+    else if (i10 <= (n1 - 3 * s1) && LC(i30 + s3) != ex && LC(i30 + 2 * s3) != ex && LC(i30 + 3 * s3) != ex)
+      val = 3 * (LV(i10 + s1) - LV(i10 + 2 * s1)) + LV(i10 + 3 * s1);
+    else if (i10 > 2 * s1 && LC(i30 - s3) != ex && LC(i30 - 2 * s3) != ex)
+      val = 2 * LV(i10 - s1) - LV(i10 - 2 * s1);
+    else if (i10 <= (n1 - 2 * s1) && LC(i30 + s3) != ex && LC(i30 + 2 * s3) != ex)
+      val = 2 * LV(i10 + s1) - LV(i10 + 2 * s1);
+    else if (i10 > s1 && LC(i30 - s3) != ex)
+      val = LV(i10 - s1);
+    else if (i10 <= (n1 - s1) && LC(i30 + s3) != ex)
+      val = LV(i10 + s1);
+    else {
+      val = LV(i10);
+      return false;
+    }
+    return true;
+  }
+  val = LV(i10);
+  return false;
+#undef LV
+#undef LC
+}
+
+template <typename T, int AX>
+__global__ __launch_bounds__(NT) void k_interp_ex2(T *u2, const T *chr1, T ex, int nx1, int ny1, int nx2, int ny2,
+                                                   int nz2, int i1, int j1, int k1, int i2, int j2, int k2, int ni,
+                                                   int nj, int nk, int si1, int sj1, int sk1, int irho, int jrho,
+                                                   int krho, BoxPts bp) {
+  const int mi = (ni - 1) * irho + 1, mj = (nj - 1) * jrho + 1, mk = (nk - 1) * krho + 1;
+  for_box(bp, [&](int fi, int fj, int fk) {
+    if (AX < 1) fj *= jrho;
+    if (AX < 2) fk *= krho;
+    // the line's column(s) of chr: those of the anchors on either side along
+    // the axes already interpolated (init_chrt / and_chrt)
+    const int ic = i1 + si1 * (fi / irho), jc = j1 + sj1 * (fj / jrho), kc = k1 + sk1 * (fk / krho);
+    const bool oi = AX >= 1 && fi % irho != 0, oj = AX >= 2 && fj % jrho != 0;
+    const size_t stride = AX == 0 ? 1 : (AX == 1 ? (size_t)nx1 : (size_t)nx1 * ny1);
+    const T *c0 = chr1 + ix3(AX == 0 ? 0 : ic - 1, AX == 1 ? 0 : jc - 1, AX == 2 ? 0 : kc - 1, nx1, ny1);
+    const size_t di = si1, dj = (size_t)sj1 * nx1;
+    auto chr = [&](int m) -> T {
+      const T *c = c0 + (size_t)m * stride;
+      bool x = c[0] == ex;
+      if (oi) x = x && c[di] == ex;
+      if (oj) x = x && c[dj] == ex;
+      if (oi && oj) x = x && c[di + dj] == ex;
+      return x ? ex : ex + 1;
+    };
+    // the line itself, at stride s2, its first anchor at 1-based position p0
+    const long long s2 = AX == 0 ? 1 : (AX == 1 ? (long long)nx2 : (long long)nx2 * ny2);
+    const int rho = AX == 0 ? irho : (AX == 1 ? jrho : krho), n2 = AX == 0 ? nx2 : (AX == 1 ? ny2 : nz2);
+    const int o2 = AX == 0 ? i2 : (AX == 1 ? j2 : k2), o1 = AX == 0 ? i1 : (AX == 1 ? j1 : k1);
+    const int so = AX == 0 ? si1 : (AX == 1 ? sj1 : sk1), f = AX == 0 ? fi : (AX == 1 ? fj : fk);
+    T *line = u2 + ix3(AX == 0 ? 0 : i2 - 1 + fi, AX == 1 ? 0 : j2 - 1 + fj, AX == 2 ? 0 : k2 - 1 + fk, nx2, ny2);
+    const long long p0 = 1 + (o2 - 1) * s2, n1 = s2 * (n2 - 1) + 1, s1 = rho * s2;
+    const int a = f / rho, r = f % rho;
+    T v0, v1;
+    const bool changed = anchor_ex(line, p0 + a * s1, n1, s1, chr, o1 + a * so, so, ex, v0);
+    if (r == 0) {
+      if (changed) line[p0 + a * s1 - 1] = v0;
+      return;
+    }
+    anchor_ex(line, p0 + (a + 1) * s1, n1, s1, chr, o1 + (a + 1) * so, so, ex, v1);
+    const double sg = (r * 1.0) / rho;
+    line[p0 + f * s2 - 1] = (T)(1 - sg) * v0 + (T)sg * v1;
+  });
+}
+
+// ---- fourth order with excision: one thread per line -------------------
 // x lines through anchor (j,k): in place on u2
-template <typename T, int ORD>
+template <typename T>
 __global__ void k_interp_ex_x(T *u2, const T *chr1, T ex, int nx1, int ny1, int nx2, int ny2,
                               int i1, int j1, int k1, int i2, int j2, int k2, int ni, int nj,
                               int nk, int si1, int sj1, int sk1, int irho, int jrho, int krho) {
@@ -290,12 +408,11 @@ __global__ void k_interp_ex_x(T *u2, const T *chr1, T ex, int nx1, int ny1, int 
   T *line = u2 + ix3(0, j - 1, k - 1, nx2, ny2);
   ChrtCols<T> cl{{chr1 + ix3(0, j1 + sj1 * (j - j2) / jrho - 1, k1 + sk1 * (k - k2) / krho - 1,
                              nx1, ny1), nullptr, nullptr, nullptr}, 1, ex};
-  if (ORD == 4) line_vi4q1d_ex<T>(line, i2, nx2, ni, irho, irho, 1, cl, i1, si1, ex);
-  else line_vi2q1d_ex<T>(line, i2, nx2, ni, irho, irho, 1, cl, i1, si1, ex);
+  line_vi4q1d_ex<T>(line, i2, nx2, ni, irho, irho, 1, cl, i1, si1, ex);
 }
 
 // y lines for every fine i at anchor k; chrt staged in a per-thread column
-template <typename T, int ORD>
+template <typename T>
 __global__ void k_interp_ex_y(T *u2, const T *chr1, T ex, int nx1, int ny1,
                               int nx2, int ny2, int i1, int j1, int k1, int i2, int j2, int k2,
                               int ni, int nj, int nk, int si1, int sj1, int sk1, int irho,
@@ -311,15 +428,11 @@ __global__ void k_interp_ex_y(T *u2, const T *chr1, T ex, int nx1, int ny1,
                   nullptr, nullptr},
                  (size_t)nx1, ex};
   T *col = u2 + ix3(i - 1, 0, k - 1, nx2, ny2);
-  if (ORD == 4)
-    line_vi4q1d_ex<T>(col, 1 + (j2 - 1) * nx2, nx2 * (ny2 - 1) + 1, nj, jrho, jrho * nx2, nx2, ch, j1, sj1, ex);
-  else
-    line_vi2q1d_ex<T>(col, 1 + (j2 - 1) * nx2, nx2 * (ny2 - 1) + 1, nj, jrho, jrho * nx2, nx2, ch,
-                      j1, sj1, ex);
+  line_vi4q1d_ex<T>(col, 1 + (j2 - 1) * nx2, nx2 * (ny2 - 1) + 1, nj, jrho, jrho * nx2, nx2, ch, j1, sj1, ex);
 }
 
 // z lines for every fine (i,j)
-template <typename T, int ORD>
+template <typename T>
 __global__ void k_interp_ex_z(T *u2, const T *chr1, T ex, int nx1, int ny1,
                               int nz1, int nx2, int ny2, int nz2, int i1, int j1, int k1, int i2,
                               int j2, int k2, int ni, int nj, int nk, int si1, int sj1, int sk1,
@@ -339,11 +452,7 @@ __global__ void k_interp_ex_z(T *u2, const T *chr1, T ex, int nx1, int ny1,
   (void)nz1;
   T *col = u2 + ix3(i - 1, j - 1, 0, nx2, ny2);
   const int s2 = nx2 * ny2;
-  if (ORD == 4)
-    line_vi4q1d_ex<T>(col, (k2 - 1) * s2 + 1, s2 * (nz2 - 1) + 1, nk, krho, krho * s2, s2, ch, k1, sk1, ex);
-  else
-    line_vi2q1d_ex<T>(col, (k2 - 1) * s2 + 1, s2 * (nz2 - 1) + 1, nk, krho, krho * s2, s2, ch, k1,
-                      sk1, ex);
+  line_vi4q1d_ex<T>(col, (k2 - 1) * s2 + 1, s2 * (nz2 - 1) + 1, nk, krho, krho * s2, s2, ch, k1, sk1, ex);
 }
 
 }  // namespace
@@ -360,12 +469,11 @@ int pmg_dmcopy3d(const double *u1, double *u2, int nx1, int ny1, int nz1, int nx
   if (j2 < 1 || (j2 + (nj - 1) * sj2) > ny2) return 0;
   if (k1 < 1 || (k1 + (nk - 1) * sk1) > nz1) return 0;
   if (k2 < 1 || (k2 + (nk - 1) * sk2) > nz2) return 0;
-  size_t n = (size_t)ni * nj * nk;
-  if (n == 0) return 0;
-  hipLaunchKernelGGL(k_copy3d<double>, dim3(nblk(n)), dim3(NT), 0, stream, u1, u2, nx1, ny1,
-                     nx2, ny2, i1, j1, k1, i2, j2, k2, ni, nj, nk, si1, sj1, sk1, si2, sj2, sk2);
-  PMG_HOST_CHECK(hipGetLastError());
-  return 0;
+  if (ni < 1 || nj < 1 || nk < 1) return 0;
+  return box_launch(ni, nj, nk, [&](dim3 grid, const BoxPts &b) {
+    hipLaunchKernelGGL(k_copy3d<double>, grid, dim3(NT), 0, stream, u1, u2, nx1, ny1,
+                       nx2, ny2, i1, j1, k1, i2, j2, k2, ni, nj, nk, si1, sj1, sk1, si2, sj2, sk2, b);
+  });
 }
 
 static int restrict_launch(int kind, const double *u1, double *u2, int nx1, int ny1, int nz1,
@@ -379,22 +487,21 @@ static int restrict_launch(int kind, const double *u1, double *u2, int nx1, int 
   if (j2 < 1 || (j2 + (nj - 1) * sj2) > ny2) return 0;
   if (k1 < 1 || (k1 + (nk - 1) * sk1) > nz1) return 0;
   if (k2 < 1 || (k2 + (nk - 1) * sk2) > nz2) return 0;
-  size_t n = (size_t)ni * nj * nk;
-  if (n == 0) return 0;
+  if (ni < 1 || nj < 1 || nk < 1) return 0;
   const bool ex1 = (do_ex == 1);
   if (ex1 && !chr1) return -1;
 #define PMG_RL(K, E)                                                                           \
-  hipLaunchKernelGGL((k_restrict3d<double, K, E>), dim3(nblk(n)), dim3(NT), 0, stream, u1, u2, \
+  hipLaunchKernelGGL((k_restrict3d<double, K, E>), grid, dim3(NT), 0, stream, u1, u2,          \
                      chr1, ex, nx1, ny1, nz1, nx2, ny2, i1, j1, k1, i2, j2, k2, ni, nj, nk,   \
-                     si1, sj1, sk1, si2, sj2, sk2)
-  if (kind == 3) {
-    if (ex1) PMG_RL(3, true); else PMG_RL(3, false);
-  } else {
-    if (ex1) PMG_RL(2, true); else PMG_RL(2, false);
-  }
+                     si1, sj1, sk1, si2, sj2, sk2, b)
+  return box_launch(ni, nj, nk, [&](dim3 grid, const BoxPts &b) {
+    if (kind == 3) {
+      if (ex1) PMG_RL(3, true); else PMG_RL(3, false);
+    } else {
+      if (ex1) PMG_RL(2, true); else PMG_RL(2, false);
+    }
+  });
 #undef PMG_RL
-  PMG_HOST_CHECK(hipGetLastError());
-  return 0;
 }
 
 int pmg_dmfwr3d(const double *u1, double *u2, int nx1, int ny1, int nz1, int nx2, int ny2,
@@ -436,54 +543,56 @@ int pmg_dminterp3d(double *u1, double *u2, int nx1, int ny1, int nz1, int nx2, i
     std::fprintf(stderr, "pmg_dminterp3d: nmax too small\n");
     return -2;
   }
+  if (ni < 1 || nj < 1 || nk < 1) return 0;
   const int mi = (ni - 1) * irho + 1, mj = (nj - 1) * jrho + 1, mk = (nk - 1) * krho + 1;
   if (ord == 4 && do_ex != 1) {
     int rc = pmg_dmcopy3d(u1, u2, nx1, ny1, nz1, nx2, ny2, nz2, i1, j1, k1, i2, j2, k2, ni, nj, nk, si1, sj1, sk1,
                           irho, jrho, krho, stream);
     if (rc) return rc;
-    size_t n = (size_t)mi * nj * nk;
-    hipLaunchKernelGGL(k_interp4<0>, dim3(nblk(n)), dim3(NT), 0, stream, u2, nx2, ny2, nz2, i2, j2, k2, ni, nj, nk,
-                       irho, jrho, krho);
-    PMG_HOST_CHECK(hipGetLastError());
-    if (nj == 1 && nk == 1) return 0;
-    n = (size_t)mi * mj * nk;
-    hipLaunchKernelGGL(k_interp4<1>, dim3(nblk(n)), dim3(NT), 0, stream, u2, nx2, ny2, nz2, i2, j2, k2, ni, nj, nk,
-                       irho, jrho, krho);
-    PMG_HOST_CHECK(hipGetLastError());
-    if (nk == 1) return 0;
-    n = (size_t)mi * mj * mk;
-    hipLaunchKernelGGL(k_interp4<2>, dim3(nblk(n)), dim3(NT), 0, stream, u2, nx2, ny2, nz2, i2, j2, k2, ni, nj, nk,
-                       irho, jrho, krho);
-    PMG_HOST_CHECK(hipGetLastError());
-    return 0;
+#define PMG_I4(AX, M1, M2)                                                                                         \
+  box_launch(mi, M1, M2, [&](dim3 grid, const BoxPts &b) {                                                         \
+    hipLaunchKernelGGL(k_interp4<AX>, grid, dim3(NT), 0, stream, u2, nx2, ny2, nz2, i2, j2, k2, ni, nj, nk, irho, \
+                       jrho, krho, b);                                                                             \
+  })
+    if ((rc = PMG_I4(0, nj, nk)) || (nj == 1 && nk == 1)) return rc;
+    if ((rc = PMG_I4(1, mj, nk)) || nk == 1) return rc;
+    return PMG_I4(2, mj, mk);
+#undef PMG_I4
   }
   if (do_ex != 1) {
-    size_t n = (size_t)mi * mj * mk;
-    hipLaunchKernelGGL(k_interp3d<double>, dim3(nblk(n)), dim3(NT), 0, stream, u1, u2, nx1,
-                       ny1, nx2, ny2, i1, j1, k1, i2, j2, k2, ni, nj, nk, si1, sj1, sk1, irho,
-                       jrho, krho);
-    PMG_HOST_CHECK(hipGetLastError());
-    return 0;
+    const bool r2 = irho == 2 && jrho == 2 && krho == 2;
+    return box_launch(mi, mj, mk, [&](dim3 grid, const BoxPts &b) {
+      hipLaunchKernelGGL((r2 ? k_interp3d<double, true> : k_interp3d<double, false>), grid, dim3(NT), 0, stream, u1, u2,
+                         nx1, ny1, nx2, ny2, i1, j1, k1, i2, j2, k2, ni, nj, nk, si1, sj1, sk1, irho, jrho, krho, b);
+    });
   }
   if (!chr1) return -1;
-  auto kex_x = ord == 4 ? k_interp_ex_x<double, 4> : k_interp_ex_x<double, 2>;
-  auto kex_y = ord == 4 ? k_interp_ex_y<double, 4> : k_interp_ex_y<double, 2>;
-  auto kex_z = ord == 4 ? k_interp_ex_z<double, 4> : k_interp_ex_z<double, 2>;
   // common points, then the three line phases in place on u2
   int rc = pmg_dmcopy3d(u1, u2, nx1, ny1, nz1, nx2, ny2, nz2, i1, j1, k1, i2, j2, k2, ni, nj, nk,
                         si1, sj1, sk1, irho, jrho, krho, stream);
   if (rc) return rc;
-  hipLaunchKernelGGL(kex_x, dim3((nj * nk + 63) / 64), dim3(64), 0, stream, u2,
+  if (ord == 2) {
+#define PMG_IX2(AX, M1, M2)                                                                                            \
+  box_launch(mi, M1, M2, [&](dim3 grid, const BoxPts &b) {                                                             \
+    hipLaunchKernelGGL((k_interp_ex2<double, AX>), grid, dim3(NT), 0, stream, u2, chr1, ex, nx1, ny1, nx2, ny2, nz2,  \
+                       i1, j1, k1, i2, j2, k2, ni, nj, nk, si1, sj1, sk1, irho, jrho, krho, b);                        \
+  })
+    if ((rc = PMG_IX2(0, nj, nk)) || (nj == 1 && nk == 1)) return rc;
+    if ((rc = PMG_IX2(1, mj, nk)) || nk == 1) return rc;
+    return PMG_IX2(2, mj, mk);
+#undef PMG_IX2
+  }
+  hipLaunchKernelGGL(k_interp_ex_x<double>, dim3((nj * nk + 63) / 64), dim3(64), 0, stream, u2,
                      chr1, ex, nx1, ny1, nx2, ny2, i1, j1, k1, i2, j2, k2, ni, nj, nk, si1, sj1,
                      sk1, irho, jrho, krho);
   PMG_HOST_CHECK(hipGetLastError());
   if (nj == 1 && nk == 1) return 0;
-  hipLaunchKernelGGL(kex_y, dim3((mi * nk + 63) / 64), dim3(64), 0, stream, u2,
+  hipLaunchKernelGGL(k_interp_ex_y<double>, dim3((mi * nk + 63) / 64), dim3(64), 0, stream, u2,
                      chr1, ex, nx1, ny1, nx2, ny2, i1, j1, k1, i2, j2, k2, ni, nj, nk,
                      si1, sj1, sk1, irho, jrho, krho);
   PMG_HOST_CHECK(hipGetLastError());
   if (nk == 1) return 0;
-  hipLaunchKernelGGL(kex_z, dim3((mi * mj + 63) / 64), dim3(64), 0, stream, u2,
+  hipLaunchKernelGGL(k_interp_ex_z<double>, dim3((mi * mj + 63) / 64), dim3(64), 0, stream, u2,
                      chr1, ex, nx1, ny1, nz1, nx2, ny2, nz2, i1, j1, k1, i2, j2, k2,
                      ni, nj, nk, si1, sj1, sk1, irho, jrho, krho);
   PMG_HOST_CHECK(hipGetLastError());
