@@ -517,18 +517,17 @@ int lop_rhs(pmg_solver *S, int L) {
   P.w0_r = (T)S->w0_r;
   P.sp = spacing<T>(Lv);
   const bool p2 = P.sp.pow2 != 0;
-  const dim3 nb = grid3(Lv.n[0], Lv.n[1], Lv.n[2]);
-#define PMG_LO(OPV, EXV, P2V) hipLaunchKernelGGL((k_lop_rhs<T, OPV, EXV, P2V>), nb, dim3(256), 0, S->stream, P)
-  if (S->op == 0) {
-    if (S->do_ex) { if (p2) PMG_LO(0, true, true); else PMG_LO(0, true, false); }
-    else { if (p2) PMG_LO(0, false, true); else PMG_LO(0, false, false); }
-  } else {
-    if (S->do_ex) { if (p2) PMG_LO(1, true, true); else PMG_LO(1, true, false); }
-    else { if (p2) PMG_LO(1, false, true); else PMG_LO(1, false, false); }
-  }
+#define PMG_LO(OPV, EXV, P2V) hipLaunchKernelGGL((k_lop_rhs<T, OPV, EXV, P2V>), grid, dim3(256), 0, S->stream, P, b)
+  return box_launch(Lv.n[0], Lv.n[1], Lv.n[2], [&](dim3 grid, const BoxPts &b) {
+    if (S->op == 0) {
+      if (S->do_ex) { if (p2) PMG_LO(0, true, true); else PMG_LO(0, true, false); }
+      else { if (p2) PMG_LO(0, false, true); else PMG_LO(0, false, false); }
+    } else {
+      if (S->do_ex) { if (p2) PMG_LO(1, true, true); else PMG_LO(1, true, false); }
+      else { if (p2) PMG_LO(1, false, true); else PMG_LO(1, false, false); }
+    }
+  });
 #undef PMG_LO
-  PMG_HOST_CHECK(hipGetLastError());
-  return 0;
 }
 
 extern "C" int pmg_dminterp3d(double *u1, double *u2, int nx1, int ny1, int nz1, int nx2, int ny2,
@@ -545,14 +544,11 @@ int cgc(pmg_solver *S, int L) {
   if (S->iord != 2) return -4;
   bool ex = false;
   if constexpr (std::is_same<T, double>::value) ex = S->do_ex != 0;
-  if (!ex) {
-    hipLaunchKernelGGL(k_cgc_diff<T>, dim3(nblk256(Cl.size)), dim3(256), 0, S->stream, AC.res, AC.u, AC.lop,
-                       (T)S->w0_i, Cl.size);
-    hipLaunchKernelGGL(k_cgc<T>, grid3(Cl.n[0], Cl.n[1], Cl.n[2]), dim3(256), 0, S->stream, ucur<T>(F), uoth<T>(F), AC.res,
-                       F.n[0], F.n[1], F.n[2], Cl.n[0], Cl.n[1], Cl.n[2], (const uint8_t *)F.chr);
-    PMG_HOST_CHECK(hipGetLastError());
-    return 0;
-  }
+  if (!ex)
+    return box_launch(Cl.n[0], Cl.n[1], Cl.n[2], [&](dim3 grid, const BoxPts &b) {
+      hipLaunchKernelGGL(k_cgc<T>, grid, dim3(256), 0, S->stream, ucur<T>(F), uoth<T>(F), AC.u, AC.lop, AC.res,
+                         (T)S->w0_i, F.n[0], F.n[1], F.n[2], Cl.n[0], Cl.n[1], Cl.n[2], (const uint8_t *)F.chr, b);
+    });
   if constexpr (std::is_same<T, double>::value) {
     // excision: coarse res, dminterp3d_ex into the fine res, clear_ex, add
     hipLaunchKernelGGL(k_cgc_diff<double>, dim3(nblk256(Cl.size)), dim3(256), 0, S->stream, AC.res,
@@ -564,9 +560,11 @@ int cgc(pmg_solver *S, int L) {
     if (rc) return rc;
     hipLaunchKernelGGL(k_clear_ex<double>, dim3(nblk256(Cl.size)), dim3(256), 0, S->stream, AC.res,
                        Cl.chr, Cl.size);
-    hipLaunchKernelGGL(k_cgc_add_ex<double>, grid3(F.n[0], F.n[1], F.n[2]), dim3(256), 0, S->stream, ucur<double>(F),
-                       uoth<double>(F), AF.res, F.chr, F.n[0], F.n[1], F.n[2]);
     PMG_HOST_CHECK(hipGetLastError());
+    return box_launch(F.n[0], F.n[1], F.n[2], [&](dim3 grid, const BoxPts &b) {
+      hipLaunchKernelGGL(k_cgc_add_ex<double>, grid, dim3(256), 0, S->stream, ucur<double>(F), uoth<double>(F), AF.res,
+                         F.chr, F.n[0], F.n[1], F.n[2], b);
+    });
   }
   return 0;
 }

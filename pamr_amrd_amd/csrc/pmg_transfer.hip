@@ -19,56 +19,6 @@ namespace {
 
 constexpr int NT = 256;
 
-// q / d for 0 <= q < 2^31, 1 <= d < 2^31: q * m >> 31 + l with l = ceil(log2
-// d), m = floor(2^(31+l) / d) + 1 (Granlund and Montgomery, "Division by
-// invariant integers using multiplication", PLDI 1994: the error m d - 2^(31+l)
-// <= d <= 2^l times q stays below 2^(31+l)).
-struct Div31 {
-  unsigned m, d;
-  int s;
-  __device__ __forceinline__ int div(int q, int &rem) const {
-    const int t = (int)(((unsigned long long)(unsigned)q * m) >> s);
-    rem = q - t * (int)d;
-    return t;
-  }
-};
-inline Div31 make_div31(int d) {
-  int l = 0;
-  while ((1ll << l) < d) l++;
-  return Div31{(unsigned)((1ull << (31 + l)) / (unsigned)d + 1), (unsigned)d, 31 + l};
-}
-
-// The points of an ni x nj x nk box by one linear index, one per thread: full
-// wavefronts whatever the sides.  The indices come from multiplications: with
-// 64-bit divisions these, not the memory, bounded the kernels (trilinear
-// interpolation onto 161 x 97 x 129 points: 19 us, rows of 64 threads 13 us).
-struct BoxPts {
-  Div31 di, dj;
-  int n, k0;
-};
-template <typename F>
-__device__ __forceinline__ void for_box(const BoxPts &b, const F &f) {
-  const int q = (int)(blockIdx.x * NT + threadIdx.x);
-  if (q >= b.n) return;
-  int i, j;
-  const int t = b.di.div(q, i), k = b.dj.div(t, j);
-  f(i, j, k + b.k0);
-}
-// launch(grid, points) over an ni x nj x nk box, in slabs of whole k planes
-// with fewer than 2^31 points; -1 when one plane has more or a launch fails
-template <typename L>
-int box_launch(int ni, int nj, int nk, const L &launch) {
-  const long long plane = (long long)ni * nj, most = (1ll << 31) - NT;
-  if (plane > most) return -1;
-  const int step = (int)std::min<long long>(nk, most / plane);
-  for (int k0 = 0; k0 < nk; k0 += step) {
-    const BoxPts b{make_div31(ni), make_div31(nj), (int)(plane * std::min(step, nk - k0)), k0};
-    launch(dim3((unsigned)((b.n + NT - 1) / NT)), b);
-    PMG_HOST_CHECK(hipGetLastError());
-  }
-  return 0;
-}
-
 // dmcopy3d, src/m_util_r8.f:20-50
 template <typename T>
 __global__ __launch_bounds__(NT) void k_copy3d(const T *u1, T *u2, int nx1, int ny1, int nx2,
