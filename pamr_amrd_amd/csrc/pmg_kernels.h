@@ -582,11 +582,20 @@ __global__ __launch_bounds__(NT) void k_sweep2(SweepP<T> P) {
 // A block owns an RTX x RTY tile of interior (x, y) columns and marches in
 // z: the u plane k (tile + 1-point ring) sits in LDS for the x/y
 // neighbours, u(k-1), u(k), u(k+1) of the own column in registers, so each
-// u value is read from HBM once (plus the ring).
+// u value is read from HBM once (plus the ring); the coefficient a of the
+// variable-coefficient operator likewise.  Every load is unconditional
+// (positions outside read element 0).  With the variable coefficient the next
+// step's values are requested a whole step ahead (257^3: FP64 173 -> 119 us
+// with u in FP32, FP32 110 -> 91); with the plain operator the registers this
+// takes cost more wavefronts in flight than it gains (96 -> 104 us), and the
+// loads stay within the step.
+// UT: the type u is stored in (FP32 for the Krylov solver's preconditioned
+// vectors, whose values are FP32).
 // ---------------------------------------------------------------------------
-template <typename T>
+template <typename T, typename UT = T>
 struct ResidP {
-  const T *u, *rho, *rhs, *a, *c;
+  const UT *u;
+  const T *rho, *rhs, *a, *c;
   const uint8_t *chr;
   T *res;
   float *neg32;  // OUT32 mode: writes (float)(-res) here instead of res
@@ -602,11 +611,12 @@ struct ResidP {
 constexpr int RTX = 64, RTY = 8, RZC = 16;
 constexpr int kResRing = 2 * RTX + 2 * RTY + 4;
 
-template <typename T, int OP, bool EX, bool P2, bool RHS0, bool ZERO, bool OUT32>
-__global__ __launch_bounds__(RTX * RTY) void k_residual(ResidP<T> P) {
+template <typename T, int OP, bool EX, bool P2, bool RHS0, bool ZERO, bool OUT32, typename UT = T>
+__global__ __launch_bounds__(RTX * RTY) void k_residual(ResidP<T, UT> P) {
   __shared__ T sP[RTY + 2][RTX + 2];
+  __shared__ T sA[OP == 1 ? RTY + 2 : 1][RTX + 2];
   const int nx = P.nx, ny = P.ny, nz = P.nz;
-  const size_t sy = nx, sz = (size_t)nx * ny;
+  const size_t sz = (size_t)nx * ny;
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
   const int nty = (ny - 2 + RTY - 1) / RTY, ntx = (nx - 2 + RTX - 1) / RTX;
   const int ty = tile % nty, tx = (tile / nty) % ntx, tz = tile / (nty * ntx);
@@ -628,43 +638,73 @@ __global__ __launch_bounds__(RTX * RTY) void k_residual(ResidP<T> P) {
   }
   const int hi = x0 - 1 + hx, hj = y0 - 1 + hy;
   const bool hvalid = hx >= 0 && hi <= nx - 1 && hj <= ny - 1;
-  const T *__restrict__ u = P.u;
+  const UT *__restrict__ u = P.u;
+  const T *__restrict__ ca = P.a;
+  constexpr bool AHEAD = OP == 1;
+  const size_t pxy = inside ? (size_t)i + (size_t)nx * j : 0, hxy = hvalid ? (size_t)hi + (size_t)nx * hj : 0;
   double s = 0.0, cnt = 0.0;
-  T um = T(0), uc = T(0), up = T(0);
-  if (inside) {
-    um = u[ix3(i, j, z0 - 1, nx, ny)];
-    uc = u[ix3(i, j, z0, nx, ny)];
+  T um = (T)u[pxy + (z0 - 1) * sz], uc = (T)u[pxy + z0 * sz], up = T(0);
+  if constexpr (AHEAD) up = (T)u[pxy + (z0 + 1) * sz];
+  T hv = (T)u[hxy + z0 * sz], am = T(0), ac = T(0), ap = T(0), ha = T(0);
+  if constexpr (OP == 1) {
+    am = ca[pxy + (z0 - 1) * sz];
+    ac = ca[pxy + z0 * sz];
+    ap = ca[pxy + (z0 + 1) * sz];
+    ha = ca[hxy + z0 * sz];
   }
-  T hv = hvalid ? u[ix3(hi, hj, z0, nx, ny)] : T(0);
+  // the point's own data of one step
+  struct Own {
+    T rho, rhs, c;
+    uint8_t x;
+  };
+  auto own = [&](int k) {
+    const size_t p = pxy + k * sz;
+    Own o{T(0), T(0), T(0), 0};
+    if (P.rho) o.rho = P.rho[p];  // no source array: a zero source (FGMRES's operator)
+    if constexpr (!RHS0) o.rhs = P.rhs[p];
+    if constexpr (OP == 1) o.c = P.c[p];
+    if constexpr (EX) o.x = P.chr[p];
+    return o;
+  };
+  Own cur{};
+  if constexpr (AHEAD) cur = own(z0);
   for (int k = z0; k < z1; k++) {
-    const size_t p = ix3(i, j, k, nx, ny);
-    if (inside) up = u[p + sz];
-    T hn = T(0);
-    if (hvalid && k + 1 < nz) hn = u[ix3(hi, hj, k + 1, nx, ny)];
-    T rhov = T(0), rhsv = T(0);
-    bool on = inxy && k >= P.bz0 && k <= P.bz1;
-    if constexpr (EX) { if (interior) on = on && !P.chr[p]; }
-    if (on) {
-      rhov = P.rho ? P.rho[p] : T(0);  // no source array: a zero source (FGMRES's operator)
-      if constexpr (!RHS0) rhsv = P.rhs[p];
+    const size_t p = pxy + k * sz;
+    T un = T(0), an = T(0), han = T(0);
+    Own nxt{};
+    if constexpr (AHEAD) {
+      const int k2 = min(k + 2, nz - 1);
+      un = (T)u[pxy + k2 * sz];
+      an = ca[pxy + k2 * sz];
+      han = ca[hxy + (k + 1) * sz];
+      nxt = own(k + 1);
+    } else {
+      up = (T)u[pxy + (k + 1) * sz];
+      cur = own(k);
     }
+    const T hn = (T)u[hxy + (k + 1) * sz];
+    bool on = inxy && k >= P.bz0 && k <= P.bz1;
+    if constexpr (EX) on = on && !cur.x;
     __syncthreads();  // the previous plane's readers are done
     sP[ly + 1][lx + 1] = uc;
     if (hvalid) sP[hy][hx] = hv;
+    if constexpr (OP == 1) {
+      sA[ly + 1][lx + 1] = ac;
+      if (hvalid) sA[hy][hx] = ha;
+    }
     __syncthreads();
     if (on) {
       T L;
       if constexpr (OP == 0) {
         L = lop_poisson<T, P2>(uc, sP[ly + 1][lx + 2], sP[ly + 1][lx], sP[ly + 2][lx + 1], sP[ly][lx + 1], up, um,
-                               rhov, P.sp);
+                               cur.rho, P.sp);
       } else {
-        const T *__restrict__ a = P.a;
         L = lop_varcoef<T, P2>(uc, sP[ly + 1][lx + 2], sP[ly + 1][lx], sP[ly + 2][lx + 1], sP[ly][lx + 1], up, um,
-                               a[p], a[p + 1], a[p - 1], a[p + sy], a[p - sy], a[p + sz], a[p - sz], P.c[p], rhov,
-                               P.sp, nullptr);
+                               ac, sA[ly + 1][lx + 2], sA[ly + 1][lx], sA[ly + 2][lx + 1], sA[ly][lx + 1], ap, am,
+                               cur.c, cur.rho, P.sp, nullptr);
       }
       T r;
-      if constexpr (RHS0) r = L - T(0); else r = L - rhsv;
+      if constexpr (RHS0) r = L - T(0); else r = L - cur.rhs;
       if constexpr (OUT32) P.neg32[p] = (float)(-r); else P.res[p] = r;
       s += (double)r * (double)r;
       cnt += 1.0;
@@ -676,6 +716,14 @@ __global__ __launch_bounds__(RTX * RTY) void k_residual(ResidP<T> P) {
     um = uc;
     uc = up;
     hv = hn;
+    if constexpr (AHEAD) {
+      up = un;
+      am = ac;
+      ac = ap;
+      ap = an;
+      ha = han;
+      cur = nxt;
+    }
   }
   norm_partial<RTX * RTY>(s, cnt, P.ws, P.slot, blockIdx.x, P.nb);
 }
