@@ -90,28 +90,37 @@ inline Div31 make_div31(int d) {
 constexpr int kPtsThreads = 256;
 struct BoxPts {
   Div31 di, dj;
-  int n, k0;
+  int n, j0, k0;
 };
 template <typename F>
 __device__ __forceinline__ void for_box(const BoxPts &b, const F &f) {
-  const int q = (int)(blockIdx.x * kPtsThreads + threadIdx.x);
-  if (q >= b.n) return;
+  const unsigned q = blockIdx.x * kPtsThreads + threadIdx.x;
+  if (q >= (unsigned)b.n) return;
   int i, j;
-  const int t = b.di.div(q, i), k = b.dj.div(t, j);
-  f(i, j, k + b.k0);
+  const int t = b.di.div((int)q, i), k = b.dj.div(t, j);
+  f(i, j + b.j0, k + b.k0);
 }
-// launch(grid, points) over an ni x nj x nk box, in slabs of whole k planes
-// with fewer than 2^31 points; -1 when one plane has more or a launch fails
+// launch(points) over an ni x nj x nk box, in slabs of whole planes with fewer
+// than 2^31 points -- of whole rows where one plane has more
+template <typename L>
+void box_slabs(int ni, int nj, int nk, const L &launch) {
+  if (ni <= 0 || nj <= 0 || nk <= 0) return;
+  const long long most = (1ll << 31) - 1;
+  const int js = (int)std::min<long long>(nj, most / ni);
+  const int ks = js < nj ? 1 : (int)std::min<long long>(nk, most / ((long long)ni * nj));
+  for (int k0 = 0; k0 < nk; k0 += std::min(ks, nk - k0))
+    for (int j0 = 0; j0 < nj; j0 += std::min(js, nj - j0)) {
+      const int mj = std::min(js, nj - j0), mk = std::min(ks, nk - k0);
+      launch(BoxPts{make_div31(ni), make_div31(mj), ni * mj * mk, j0, k0});
+    }
+}
+// launch(grid, points) with one thread per point
 template <typename L>
 int box_launch(int ni, int nj, int nk, const L &launch) {
-  const long long plane = (long long)ni * nj, most = (1ll << 31) - kPtsThreads;
-  if (plane > most) return -1;
-  const int step = (int)std::min<long long>(nk, most / plane);
-  for (int k0 = 0; k0 < nk; k0 += step) {
-    const BoxPts b{make_div31(ni), make_div31(nj), (int)(plane * std::min(step, nk - k0)), k0};
-    launch(dim3((unsigned)((b.n + kPtsThreads - 1) / kPtsThreads)), b);
-    PMG_HOST_CHECK(hipGetLastError());
-  }
+  box_slabs(ni, nj, nk, [&](const BoxPts &b) {
+    launch(dim3((unsigned)(((long long)b.n + kPtsThreads - 1) / kPtsThreads)), b);
+  });
+  PMG_HOST_CHECK(hipGetLastError());
   return 0;
 }
 
