@@ -33,6 +33,9 @@ constexpr int kSmT = 8, kSmH = 4, kSmR = kSmT + 2 * kSmH, kSmL = kSmR + 2;
 constexpr int kSmNT = kSmR * kSmR * 2, kSmP = kSmR / 2;  // threads; points per thread
 constexpr int kSmC = kSmR / 2 + 2;                       // coarse points per axis around a tile
 
+// the largest level whose legs run as one launch each
+constexpr size_t kSmallPoints = 300000;
+
 template <typename T>
 struct SmallP {
   const T *uin;
@@ -43,7 +46,7 @@ struct SmallP {
   T *res_out;      // down: the residual
   T *lop;          // down, below the finest: written
   const T *cu, *clop;
-  T *cres;         // up with the correction: the coarse level; its f_res gets the correction
+  T *cres;         // up with the correction: the coarse level; its f_res gets the correction (null: not stored)
   const uint8_t *chr;
   int nx, ny, nz, cnx, cny, cnz;
   int bx0, bx1, by0, by1, bz0, bz1;  // relax / residual box
@@ -278,7 +281,7 @@ __global__ __launch_bounds__(kSmNT) void k_small_up(SmallP<T> P) {
       if (a >= 0 && a < P.cnx && b >= 0 && b < P.cny && c >= 0 && c < P.cnz) {
         const size_t p = ix3(a, b, c, P.cnx, P.cny);
         d = (P.cu[p] - P.clop[p]) / P.w0_i;
-        if (own1(a, x0, P.nx) && own1(b, y0, P.ny) && own1(c, z0, P.nz)) P.cres[p] = d;
+        if (P.cres && own1(a, x0, P.nx) && own1(b, y0, P.ny) && own1(c, z0, P.nz)) P.cres[p] = d;
       }
       D[q] = d;
     }

@@ -319,9 +319,6 @@ int launch_sweep2(pmg_solver *S, SweepP<T> P, bool p2, bool rhs0) {
   return rhs0 ? launch_sweep2_v<T, OP, EX, false, true>(S, P) : launch_sweep2_v<T, OP, EX, false, false>(S, P);
 }
 
-// the largest level whose legs run as one launch each
-constexpr size_t kSmallPoints = 300000;
-
 // levels where pairs of sweeps run temporally blocked
 bool use_sweep2(const pmg_solver *S, const Level &Lv) {
   return S->use_sweep2 && Lv.n[0] >= kSweep2MinN && Lv.n[1] >= kSweep2MinN && Lv.n[2] >= kSweep2MinN;
