@@ -38,6 +38,9 @@ struct SweepP {
   NormWs ws;
   int slot;  // norm workspace slot
   int nb;
+  // FP32 only: u is zero everywhere, uin one element holding 0 -- a correction
+  // cycle's first sweep neither reads its guess nor needs it cleared
+  bool zero = false;
 };
 
 // Position of colour-slot q of a sweep phase on plane k.  HALO (pass 0):
@@ -271,7 +274,8 @@ __device__ __forceinline__ void sweep_tile(const SweepP<T> &P, int x0, int y0, i
       const int i = x0 - 2 + lx, j = y0 - 2 + ly;
       const bool ok = k >= 0 && k <= kmax && q < LX * LY && i >= 0 && i < nx && j >= 0 && j < ny;
       const size_t p = ok ? ix3(i, j, k, nx, ny) : 0;
-      ld.u[m] = uin[p];
+      if constexpr (std::is_same<T, float>::value) ld.u[m] = uin[P.zero ? 0 : p];
+      else ld.u[m] = uin[p];
       if constexpr (AR) ld.a[m] = ain[p];
     }
   };

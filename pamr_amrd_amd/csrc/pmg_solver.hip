@@ -149,6 +149,7 @@ struct pmg_solver {
                                // (measured slower than single sweeps; off by default)
   int sweep2_zchunk = 32;
   hipGraphExec_t g64 = nullptr;   // captured FP64 V-cycle
+  float *zero32 = nullptr;        // one element, 0: the FP32 cycles' initial guess
   hipGraphExec_t g32 = nullptr;   // captured mixed-precision outer iteration
   bool fp32_ready = false;
   int last_citer = 0;
@@ -169,7 +170,7 @@ struct pmg_solver {
   float *kryz = nullptr;
   double *kry_red = nullptr;
   double *kry_host = nullptr;
-  hipGraphExec_t gprec = nullptr;  // captured FP32 V-cycle (the preconditioner)
+  hipGraphExec_t gprec = nullptr, gprec_next = nullptr;  // captured FP32 V-cycle (the preconditioner): first, further
   int prec_cycles = 1;             // FP32 V-cycles per preconditioner application
   // kernel timing inside V-cycles (pmg_time_kernel which 3): HIP events
   // around the finest level's FP64 sweep launches of ungraphed cycles
@@ -202,7 +203,7 @@ struct pmg_solver {
     bool enq_inner = false;         // set while an FP32 cycle with it is enqueued
     const double *cur_norm = nullptr;  // RMS of that cycle's finest source (device)
     hipGraphExec_t g32i = nullptr;     // mixed iteration with the in-cycle correction
-    hipGraphExec_t gpreci = nullptr;   // preconditioner with the in-cycle correction
+    hipGraphExec_t gpreci = nullptr, gpreci_next = nullptr;  // preconditioner with the in-cycle correction: first, further cycle
     // training crops taken inside the cycle instead of correcting (pmg_band_sample_inner)
     const double *samp_ustar = nullptr;
     int *samp_org = nullptr;
@@ -350,8 +351,9 @@ void default_sweep(const int *n, int op, int pi, int *variant, int *zchunk) {
 }
 
 // n red-black sweeps on level L (ping-pong u <-> ua; odd counts copy back)
+// zero: u counts as zero, whatever its buffer holds (can_sweep_zero)
 template <typename T>
-int sweeps(pmg_solver *S, int L, int n, int slot, bool rhs0) {
+int sweeps(pmg_solver *S, int L, int n, int slot, bool rhs0, bool zero = false) {
   Level &Lv = S->lev[L - 1];
   LevelArrays<T> &A = arrays<T>(Lv);
   if (n <= 0) return 0;
@@ -374,6 +376,10 @@ int sweeps(pmg_solver *S, int L, int n, int slot, bool rhs0) {
   T *const b0 = ucur<T>(Lv), *const b1 = uoth<T>(Lv);
   while (done < n) {
     P.uin = (launches % 2 == 0) ? b0 : b1;
+    if constexpr (std::is_same<T, float>::value) {
+      P.zero = zero && launches == 0;
+      if (P.zero) P.uin = S->zero32;
+    }
     P.uout = (launches % 2 == 0) ? b1 : b0;
     int rc;
     if (two && n - done >= 2) {
@@ -394,6 +400,18 @@ int sweeps(pmg_solver *S, int L, int n, int slot, bool rhs0) {
   // this cycle read it there, settle() moves it back at the end of the level
   curbuf<T>(Lv) ^= (launches & 1);
   return 0;
+}
+
+// Whether the finest level's first FP32 sweep can take a zero guess as given:
+// it runs as a separate one-sweep launch.  The buffers' faces stay 0 through
+// every cycle (no kernel writes another value there), so their interiors need
+// not be cleared and the sweep reads its source alone: 513^3, 486 -> 443 us of
+// the sweep and the 87 us that clearing took.
+template <typename T>
+bool use_small(const pmg_solver *S, int L, int Lb);
+bool can_sweep_zero(const pmg_solver *S, int Lb) {
+  const Level &F = S->lev[S->nlev - 1];
+  return S->nlev > 1 && S->pre > 0 && F.rbox.ok && !use_sweep2(S, F) && !use_small<float>(S, S->nlev, Lb);
 }
 
 // u back in its primary buffer (both buffers then agree)
@@ -978,11 +996,11 @@ int band_inner(pmg_solver *S);
 // sweeps(), with HIP events around the launches of the finest FP64 level
 // while pmg_time_kernel (which 3) collects in-cycle durations
 template <typename T>
-int timed_sweeps(pmg_solver *S, int L, int n, int slot, bool rhs0) {
+int timed_sweeps(pmg_solver *S, int L, int n, int slot, bool rhs0, bool zero = false) {
   const bool tk = std::is_same<T, double>::value && L == S->nlev && S->tk_ev && n > 0 &&
                   S->tk_n + 2 <= S->tk_cap;
   if (tk) PMG_HOST_CHECK(hipEventRecord(S->tk_ev[S->tk_n], S->stream));
-  const int rc = sweeps<T>(S, L, n, slot, rhs0);
+  const int rc = sweeps<T>(S, L, n, slot, rhs0, zero);
   if (tk) {
     PMG_HOST_CHECK(hipEventRecord(S->tk_ev[S->tk_n + 1], S->stream));
     S->tk_n += 2;
@@ -991,11 +1009,20 @@ int timed_sweeps(pmg_solver *S, int L, int n, int slot, bool rhs0) {
   return rc;
 }
 
+// from_zero (FP32): the cycle starts from u = 0, whatever the buffers hold
 template <typename T>
-int enqueue_vcycle(pmg_solver *S, bool final_residual, int norm_base, double *cnorm, int *citer) {
+int enqueue_vcycle(pmg_solver *S, bool final_residual, int norm_base, double *cnorm, int *citer, bool from_zero = false) {
   const int Lf = S->nlev;
   const int Lb = S->use_bottom ? bottom_top<T>(S) : 0;
   int rc;
+  bool zero = false;
+  if constexpr (std::is_same<T, float>::value) {
+    if (from_zero && !(zero = can_sweep_zero(S, Lb))) {
+      Level &F = S->lev[Lf - 1];
+      hipLaunchKernelGGL(k_fill<float>, dim3(nblk256(F.size)), dim3(256), 0, S->stream, ucur<float>(F), 0.0f, F.size);
+      PMG_HOST_CHECK(hipGetLastError());
+    }
+  }
   for (int L = Lf; L >= 1; L--) {
     const bool small = use_small<T>(S, L, Lb);
     if (L < Lf) {
@@ -1022,7 +1049,7 @@ int enqueue_vcycle(pmg_solver *S, bool final_residual, int norm_base, double *cn
     } else if (small) {
       if ((rc = small_leg<T>(S, L, 0, norm_base + NS_RESID + L - 1))) return rc;
     } else {
-      if ((rc = timed_sweeps<T>(S, L, S->pre, norm_base + NS_RELAX + L - 1, L == Lf))) return rc;
+      if ((rc = timed_sweeps<T>(S, L, S->pre, norm_base + NS_RELAX + L - 1, L == Lf, zero && L == Lf))) return rc;
     }
   }
   for (int L = Lb ? Lb + 1 : 2; L <= Lf; L++) {
@@ -1072,24 +1099,20 @@ int enq_v64(pmg_solver *S) {
 }
 
 // Mixed precision outer iteration (defect correction).  On entry the FP32
-// source of the finest level holds -r (r = L64[u], the FP64 defect) and the
-// FP32 correction e is zero; the graph runs the FP32 V-cycle on A e = -r,
-// adds e to u in FP64 (zeroing e again), and recomputes the FP64 defect of
-// the updated u -- its norm is the convergence test, its negation in FP32
-// the next source.
-__global__ __launch_bounds__(256) void k_add_f32(double *u, float *e, size_t n) {
+// source of the finest level holds -r (r = L64[u], the FP64 defect);
+// the graph runs the FP32 V-cycle on A e = -r from e = 0, adds e to u in FP64,
+// and recomputes the FP64 defect of the updated u -- its norm is the
+// convergence test, its negation in FP32 the next source.
+__global__ __launch_bounds__(256) void k_add_f32(double *u, const float *e, size_t n) {
   size_t q = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (q < n) {
-    u[q] = u[q] + (double)e[q];
-    e[q] = 0.0f;
-  }
+  if (q < n) u[q] = u[q] + (double)e[q];
 }
 
 int enq_mixed(pmg_solver *S) {
   const int Lf = S->nlev;
   Level &F = S->lev[Lf - 1];
   int rc;
-  if ((rc = enqueue_vcycle<float>(S, false, NS_F32, S->d_norms + NS_COARSE + 2, S->d_citer + 1))) return rc;
+  if ((rc = enqueue_vcycle<float>(S, false, NS_F32, S->d_norms + NS_COARSE + 2, S->d_citer + 1, true))) return rc;
   hipLaunchKernelGGL(k_add_f32, dim3(nblk256(F.size)), dim3(256), 0, S->stream, F.d.u, F.f.u, F.size);
   PMG_HOST_CHECK(hipGetLastError());
   if ((rc = residual<double>(S, Lf, NS_OUTER, true, true, F.f.rho))) return rc;
@@ -1098,6 +1121,10 @@ int enq_mixed(pmg_solver *S) {
 
 int ensure_fp32(pmg_solver *S) {
   if (S->fp32_ready) return 0;
+  if (!S->zero32) {
+    PMG_HOST_CHECK(hipMalloc(&S->zero32, 64));
+    PMG_HOST_CHECK(hipMemsetAsync(S->zero32, 0, 64, S->stream));
+  }
   for (int L = 1; L <= S->nlev; L++)
     if (alloc_level_arrays(S, S->lev[L - 1], true)) return -1;
   // coefficients in FP32 on every level (restricted FP64 values rounded)
@@ -1184,24 +1211,27 @@ int enq_mixed_inner(pmg_solver *S) {
   return rc;
 }
 
-int enq_prec_inner(pmg_solver *S) {
+int enq_prec_inner_t(pmg_solver *S, bool from_zero) {
   S->band.enq_inner = true;
   S->band.cur_norm = S->d_norms + NS_PSRC;
-  const int rc = enqueue_vcycle<float>(S, false, NS_F32, S->d_norms + NS_COARSE + 2, S->d_citer + 1);
+  const int rc = enqueue_vcycle<float>(S, false, NS_F32, S->d_norms + NS_COARSE + 2, S->d_citer + 1, from_zero);
   S->band.enq_inner = false;
   return rc;
 }
+int enq_prec_inner(pmg_solver *S) { return enq_prec_inner_t(S, true); }
+int enq_prec_inner_next(pmg_solver *S) { return enq_prec_inner_t(S, false); }
 
 void band_graphs_reset(pmg_solver *S) {
   auto &B = S->band;
-  for (hipGraphExec_t *g : {&B.gdc, &B.gpc, &B.g32i, &B.gpreci})
+  for (hipGraphExec_t *g : {&B.gdc, &B.gpc, &B.g32i, &B.gpreci, &B.gpreci_next})
     if (*g) { (void)hipGraphExecDestroy(*g); *g = nullptr; }
 }
 
 void invalidate_graphs(pmg_solver *S) {
   if (S->g64) { (void)hipGraphExecDestroy(S->g64); S->g64 = nullptr; }
   if (S->g32) { (void)hipGraphExecDestroy(S->g32); S->g32 = nullptr; }
-  if (S->gprec) { (void)hipGraphExecDestroy(S->gprec); S->gprec = nullptr; }
+  for (hipGraphExec_t *g : {&S->gprec, &S->gprec_next})
+    if (*g) { (void)hipGraphExecDestroy(*g); *g = nullptr; }
   band_graphs_reset(S);
 }
 
@@ -1332,6 +1362,7 @@ void pmg_destroy(pmg_solver *S) {
   if (S->ws.slot_nb) (void)hipFree(S->ws.slot_nb);
   if (S->d_norms) (void)hipFree(S->d_norms);
   if (S->d_citer) (void)hipFree(S->d_citer);
+  if (S->zero32) (void)hipFree(S->zero32);
   if (S->d_snap) (void)hipFree(S->d_snap);
   if (S->h_pinned) (void)hipHostFree(S->h_pinned);
   if (S->d_hist) (void)hipFree(S->d_hist);
@@ -1363,6 +1394,11 @@ int pmg_set_params(pmg_solver *S, int pre, int pst, int max_citer, double crtol,
   S->w0_r = w0_r; S->w0_i = w0_i; S->rop_u = rop_u; S->rop_res = rop_res; S->rop_src = rop_src;
   S->iord = interp_ord;
   invalidate_graphs(S);
+  // weights that are no numbers may have left some on the faces of the FP32
+  // correction, which are not cleared otherwise
+  Level &F = S->lev[S->nlev - 1];
+  for (float *p : {F.f.u, F.f.ua})
+    if (p) PMG_HOST_CHECK(hipMemsetAsync(p, 0, F.size * sizeof(float), S->stream));
   return 0;
 }
 
@@ -2189,16 +2225,15 @@ __global__ __launch_bounds__(256) void k_kry_update_dots(double *w, VecPtrs V, i
   }
 }
 
-// v = f * w (in place when they are the same), and the preconditioner's input:
-// FP32 source = v, FP32 solution = 0
-__global__ __launch_bounds__(256) void k_kry_next(double *v, const double *w, double f, float *rho32, float *u32,
+// v = f * w (in place when they are the same), and in FP32 the preconditioner's
+// source
+__global__ __launch_bounds__(256) void k_kry_next(double *v, const double *w, double f, float *rho32,
                                                   size_t n) {
   const size_t q = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (q >= n) return;
   const double x = f * w[q];
   v[q] = x;
   rho32[q] = (float)x;
-  u32[q] = 0.0f;
 }
 
 // u (both sweep buffers) += sum_j y_j Z_j
@@ -2216,6 +2251,10 @@ __global__ __launch_bounds__(256) void k_kry_xupdate(double *u, double *ua, ZPtr
 }
 
 int enq_prec(pmg_solver *S) {
+  return enqueue_vcycle<float>(S, false, NS_F32, S->d_norms + NS_COARSE + 2, S->d_citer + 1, true);
+}
+// a further cycle of one preconditioner application
+int enq_prec_next(pmg_solver *S) {
   return enqueue_vcycle<float>(S, false, NS_F32, S->d_norms + NS_COARSE + 2, S->d_citer + 1);
 }
 
@@ -2414,7 +2453,7 @@ int pmg_solve_fgmres(pmg_solver *S, int m, double rtol, int max_iter, double *hi
     for (int j = 0; j < m && it < max_iter; j++) {
       // V_j normalised, and Z_j = M V_j: the FP32 V-cycle from zero with V_j as
       // its source
-      hipLaunchKernelGGL(k_kry_next, dim3(nb), dim3(256), 0, S->stream, V[j], j == 0 ? w : V[j], next, F.f.rho, F.f.u, n);
+      hipLaunchKernelGGL(k_kry_next, dim3(nb), dim3(256), 0, S->stream, V[j], j == 0 ? w : V[j], next, F.f.rho, n);
       PMG_HOST_CHECK(hipGetLastError());
       // prec_cycles FP32 V-cycles on the source V_j, the first from zero;
       // the band correction (when on) after a single cycle, or between
@@ -2422,8 +2461,11 @@ int pmg_solve_fgmres(pmg_solver *S, int m, double rtol, int max_iter, double *hi
       for (int cyc = 0; cyc < S->prec_cycles; cyc++) {
         if (cyc > 0 && band_on && !B.inner && (rc = capture_or_run(S, &B.gpc, enq_band_pc))) return rc;
         if (band_on && B.inner) {
-          if ((rc = capture_or_run(S, &B.gpreci, enq_prec_inner))) return rc;
-        } else if ((rc = capture_or_run(S, &S->gprec, enq_prec))) {
+          if ((rc = cyc == 0 ? capture_or_run(S, &B.gpreci, enq_prec_inner)
+                             : capture_or_run(S, &B.gpreci_next, enq_prec_inner_next)))
+            return rc;
+        } else if ((rc = cyc == 0 ? capture_or_run(S, &S->gprec, enq_prec)
+                                  : capture_or_run(S, &S->gprec_next, enq_prec_next))) {
           return rc;
         }
       }
