@@ -1624,7 +1624,7 @@ int setup_levels(pmg_amr *A, int op) {
     // all grids of a level share one spacing (dyadic boxes); check it
     for (const HGrid &g : Lv.g)
       for (int d = 0; d < 3; d++)
-        if (g.hdx[d] != Lv.g[0].hdx[d] || g.n[d] < 3) return -1;
+        if (g.hdx[d] != Lv.g[0].hdx[d] || g.n[d] < 3 || g.n[0] > 1 << 24) return -1;
     Lv.sp = spacing_of(Lv.g[0].hdx);
     Lv.sp32 = spacing_of32(Lv.g[0].hdx);
     size_t pool = 0;

@@ -60,11 +60,6 @@ __device__ __forceinline__ bool sweep_pos(int q, int x0, int y0, int k, int pass
   return lx <= OFF + W - 1;
 }
 
-template <typename T>
-__device__ __forceinline__ bool sweep_updatable(const SweepP<T> &P, int i, int j, int k) {
-  return i >= P.bx0 && i <= P.bx1 && j >= P.by0 && j <= P.by1 && k >= P.bz0 && k <= P.bz1;
-}
-
 // The variable-coefficient sweep keeps the coefficient a in an LDS ring of
 // the same shape as u's when both rings fit (its seven reads per point then
 // come from LDS, like u's); otherwise a is read from global memory.
@@ -84,12 +79,6 @@ __device__ __forceinline__ int csx(int lx) {
   return (lx & 1) * (LX / 2) + (lx >> 1);
 }
 
-// Slot of plane k (k >= -2) in an LDS ring of RING planes.
-template <int RING>
-__device__ __forceinline__ int ring_ix(int k) {
-  if constexpr (RING == 4) return k & 3; else return (k + 2 * RING) % RING;
-}
-
 // Flat LDS offset (within a plane) of local position (lx, ly), and the
 // offset from it to its east neighbour in the colour-split row: +LX/2 for an
 // even lx, 1 - LX/2 for an odd one (the west neighbour is one word before
@@ -99,127 +88,61 @@ __device__ __forceinline__ int cs_off(int lx, int ly) { return ly * LX + csx<LX>
 template <int LX>
 __device__ __forceinline__ int cs_east(int lx) { return (lx & 1) ? 1 - LX / 2 : LX / 2; }
 
-// One colour update at flat LDS offset `lo` of plane k (`de`: cs_east).
-// rho/rhs are the values at that point (prefetched by the caller); sA is a's
-// ring (AR).
-template <typename T, int OP, bool P2, bool RHS0, int TX, int TY, bool AR = false, int RING = 4>
-__device__ __forceinline__ T sweep_point(const SweepP<T> &P, T (*sU)[TY + 4][TX + 4], int lo,
-                                         int de, int k, size_t p, T rho, T rhs,
-                                         T (*sA)[TY + 4][TX + 4] = nullptr) {
-  constexpr int LX = TX + 4;
-  T *S0 = &sU[ring_ix<RING>(k)][0][0];
-  const T *Sm = &sU[ring_ix<RING>(k - 1)][0][0];
-  const T *Sp = &sU[ring_ix<RING>(k + 1)][0][0];
-  const int ce = lo + de, cw = ce - 1;
-  const T uc = S0[lo];
-  T jac, L;
-  if constexpr (OP == 0) {
-    L = lop_poisson<T, P2>(uc, S0[ce], S0[cw], S0[lo + LX], S0[lo - LX], Sp[lo], Sm[lo], rho, P.sp);
-    jac = P.sp.jac;
-  } else if constexpr (AR) {
-    const T *A0 = &sA[ring_ix<RING>(k)][0][0];
-    const T *Am = &sA[ring_ix<RING>(k - 1)][0][0];
-    const T *Ap = &sA[ring_ix<RING>(k + 1)][0][0];
-    L = lop_varcoef<T, P2>(uc, S0[ce], S0[cw], S0[lo + LX], S0[lo - LX], Sp[lo], Sm[lo], A0[lo], A0[ce],
-                           A0[cw], A0[lo + LX], A0[lo - LX], Ap[lo], Am[lo], P.c[p], rho, P.sp, &jac);
-  } else {
-    const T *__restrict__ a = P.a;
-    const size_t sy = (size_t)P.nx, sz = (size_t)P.nx * P.ny;
-    L = lop_varcoef<T, P2>(uc, S0[ce], S0[cw], S0[lo + LX], S0[lo - LX], Sp[lo], Sm[lo], a[p], a[p + 1],
-                           a[p - 1], a[p + sy], a[p - sy], a[p + sz], a[p - sz], P.c[p], rho, P.sp, &jac);
-  }
-  T res;
-  if constexpr (RHS0) res = L - T(0); else res = L - rhs;
-  if constexpr (std::is_same<T, float>::value && OP == 0)
-    S0[lo] = uc - res * P.sp.ijac;  // FP32 inner cycles: no IEEE division
-  else
-    S0[lo] = uc - div_jac<T, OP>(res, jac, P.sp);  // FP64: the reference's V - res/Jac, bit for bit
-  return res;
+// Where a block's tile lies in a grid function: `base` is the element of local
+// position (0, 0) on plane 0 -- which may lie before the array, no position
+// outside the grid is ever read -- and 32-bit byte offsets within the tile are
+// added to it, so that a load is a scalar address plus a register and no plane
+// of the march computes one (the empty asm keeps the compiler from widening
+// the offsets to register pairs ahead of the march).
+template <typename V>
+__device__ __forceinline__ V tile_at(const V *base, size_t plane, int k, unsigned &off) {
+  asm volatile("" : "+v"(off));
+  return *reinterpret_cast<const V *>(reinterpret_cast<const char *>(base + plane * (size_t)k) + off);
 }
 
-// Prefetch state of one phase: per slot the point index (or -1) and its
-// rho/rhs values, loaded one step before use.
-template <typename T, int N>
-struct PhaseRegs {
-  long long p[N];
-  int lo[N], fl[N];  // as in SlotTab
-  T rho[N], rhs[N];
-};
+// f(0), f(1), ... as constants, until one returns false
+template <int... J, typename F>
+__device__ __forceinline__ void unrolled(std::integer_sequence<int, J...>, const F &f) {
+  (void)(f(std::integral_constant<int, J>{}) && ...);
+}
 
-// Per-thread slot table of one phase for both plane parities, computed once
-// per block: LDS position (flat colour-split offset `lo`; `fl` = 2 * cs_east
-// + 1 when the slot lies in the tile itself, whose residuals the norm
-// counts), xy offset of the point, and whether the slot is inside the tile
-// region and the updatable x/y range.
+// Per-thread slot table of one phase, computed once per block for both plane
+// parities: LDS byte offsets of the point and of its east neighbour, its byte
+// offset in the tile (a position inside the grid where there is nothing to
+// update), whether there is, and whether the norm counts it (the tile proper).
 template <int N>
 struct SlotTab {
-  int lo[2][N], fl[2][N];
-  int off[2][N];  // i + nx*j, or -1
+  int lo[2][N], ea[2][N];
+  unsigned off[2][N];
+  bool ok[2][N], in[2][N];
 };
 
+// kz: the plane whose parity is entry 0 of the table
 template <typename T, int TX, int TY, int NT, bool HALO, int N>
-__device__ __forceinline__ void slot_table(const SweepP<T> &P, int x0, int y0, int pass, SlotTab<N> &S) {
+__device__ __forceinline__ void slot_table(const SweepP<T> &P, int x0, int y0, int kz, int pass, SlotTab<N> &S) {
 #pragma unroll
-  for (int par = 0; par < 2; par++)
+  for (int e = 0; e < 2; e++)
 #pragma unroll
     for (int m = 0; m < N; m++) {
-      int lx = 0, ly = 0;
-      S.off[par][m] = -1;
-      // plane parity par: the colour test uses (j + k + 3 + pass), k = par mod 2
-      if (!sweep_pos<TX, TY, HALO>(threadIdx.x + m * NT, x0, y0, par, pass, lx, ly)) continue;
+      int lx = 2, ly = 2;
+      const bool slot = sweep_pos<TX, TY, HALO>(threadIdx.x + m * NT, x0, y0, kz + e, pass, lx, ly);
       const int i = x0 - 2 + lx, j = y0 - 2 + ly;
-      S.lo[par][m] = cs_off<TX + 4>(lx, ly);
-      S.fl[par][m] = 2 * cs_east<TX + 4>(lx) + ((lx >= 2 && lx < TX + 2 && ly >= 2 && ly < TY + 2) ? 1 : 0);
-      if (i >= P.bx0 && i <= P.bx1 && j >= P.by0 && j <= P.by1) S.off[par][m] = i + P.nx * j;
+      const bool ok = slot && i >= P.bx0 && i <= P.bx1 && j >= P.by0 && j <= P.by1;
+      if (!ok) lx = ly = 2;
+      S.lo[e][m] = cs_off<TX + 4>(lx, ly) * (int)sizeof(T);
+      S.ea[e][m] = S.lo[e][m] + cs_east<TX + 4>(lx) * (int)sizeof(T);
+      S.off[e][m] = ((unsigned)ly * (unsigned)P.nx + (unsigned)lx) * (unsigned)sizeof(T);
+      S.ok[e][m] = ok;
+      S.in[e][m] = ok && lx >= 2 && lx < TX + 2 && ly >= 2 && ly < TY + 2;
     }
 }
 
-// kpar: the plane whose parity selects the table (k itself, except for the
-// prologue's pass 0 over the tile, which takes the pass-1 table of the plane
-// above: the colours of pass 0 on plane k are those of pass 1 on k + 1).
-template <typename T, bool EX, bool RHS0, int N>
-__device__ __forceinline__ void phase_prefetch_t(const SweepP<T> &P, int k, const SlotTab<N> &S,
-                                                 PhaseRegs<T, N> &R, int kpar) {
-  // the plane parity selects between the two register tables with a
-  // select, not an index (a run-time index would move them to scratch)
-  //
-  // The loads are unconditional (slots outside the region read element 0 and
-  // are marked p = -1): a load behind a branch makes the compiler's wait
-  // counting fall back to waiting for every load in flight, which would
-  // stall each march step on the plane prefetched for the steps after it.
-  const bool odd = (kpar & 1) != 0;
-  const bool zok = k >= P.bz0 && k <= P.bz1;
-  const size_t base = (size_t)k * P.nx * P.ny;
-#pragma unroll
-  for (int m = 0; m < N; m++) {
-    const int off = odd ? S.off[1][m] : S.off[0][m];
-    const bool ok = zok && off >= 0;
-    const size_t p = ok ? base + (size_t)off : 0;
-    bool act = ok;
-    if constexpr (EX) act = act && !P.chr[p];
-    R.p[m] = act ? (long long)p : -1;
-    R.lo[m] = odd ? S.lo[1][m] : S.lo[0][m];
-    R.fl[m] = odd ? S.fl[1][m] : S.fl[0][m];
-    R.rho[m] = P.rho[p];
-    if constexpr (!RHS0) R.rhs[m] = P.rhs[p];
-  }
-}
-
-template <typename T, int OP, bool P2, bool RHS0, int TX, int TY, int N, bool AR, int RING>
-__device__ __forceinline__ void phase_run(const SweepP<T> &P, T (*sU)[TY + 4][TX + 4],
-                                          T (*sA)[TY + 4][TX + 4], int k, const PhaseRegs<T, N> &R, bool count,
-                                          double &s, double &cnt) {
-#pragma unroll
-  for (int m = 0; m < N; m++) {
-    if (R.p[m] < 0) continue;
-    const T res = sweep_point<T, OP, P2, RHS0, TX, TY, AR, RING>(P, sU, R.lo[m], R.fl[m] >> 1, k, (size_t)R.p[m],
-                                                                 R.rho[m], RHS0 ? T(0) : R.rhs[m], sA);
-    if (count && (R.fl[m] & 1)) {
-      s += (double)res * (double)res;
-      cnt += 1.0;
-    }
-  }
-}
+// What a phase needs of its points beside u (and a): loaded a step before use.
+template <typename T, int OP, int N>
+struct PhaseRegs {
+  T rho[N], rhs[N], c[OP == 1 ? N : 1];
+  uint8_t x[N];
+};
 
 // Fused sweep.  Step k finalises plane k: pass 0 on plane k+1 (tile+1),
 // pass 1 on plane k (tile), store plane k.  While a step computes, the u
@@ -231,92 +154,182 @@ __device__ __forceinline__ void phase_run(const SweepP<T> &P, T (*sU)[TY + 4][TX
 // level) kernels.
 // PF: u planes in flight ahead of the march (1: one plane issued per step and
 // committed the next; 2: two, for latency-bound tiles such as FP32).  Planes
-// past z1+1, which no pass of the chunk reads, are not fetched.
+// past z1+1, which no pass of the chunk reads, repeat that plane.
 // RING: LDS planes.  With 4, the slot plane k+3 is committed into is that of
 // plane k-1, which pass 1 on plane k reads, so a step needs three barriers
 // (after pass 0, after pass 1, after the commit).  With 5 the commit touches
 // no slot the step reads: it follows pass 1 directly and one barrier covers
 // both, two barriers per step.
+// A point needs some 15 instructions of arithmetic; address computations and
+// selects between plane parities and ring slots took 110 more of a step's 170.
+// So the march is unrolled over the ring (slots and parities become constants,
+// LDS offsets immediate fields) and an address is a scalar plane plus an offset
+// from the block's tables: 67 a step, and 63 registers instead of 100, two
+// blocks of 1024 threads a CU.  One sweep: FP32 257^3 with variable coefficient
+// and excision 141 -> 100 us, FP32 257^3 77 -> 70 and 129^3 17.6 -> 13.7, FP64
+// 129^3 20.5 -> 19.2.  The largest stay with memory: FP64 257^3 93 -> 92 (4.5
+// TB/s), FP32 513^3 475 -> 455 (3.6 TB/s).
 template <typename T, int OP, bool EX, bool P2, bool RHS0, int TX, int TY, int NT, int PF = 1, int RING = 4>
 __device__ __forceinline__ void sweep_tile(const SweepP<T> &P, int x0, int y0, int z0, int z1, int bid) {
   static_assert(PF == 1 || PF == 2, "prefetch depth");
   static_assert(RING == 4 || RING == 5, "LDS ring");
-  constexpr int LX = TX + 4, LY = TY + 4;
-  constexpr int NLD = (LX * LY + NT - 1) / NT;
+  constexpr int LX = TX + 4, LY = TY + 4, PL = LX * LY;
+  constexpr int NLD = (PL + NT - 1) / NT, NST = (TX * TY + NT - 1) / NT;
   constexpr int N0 = (((TX + 3) / 2) * (TY + 2) + NT - 1) / NT;
   constexpr int N1 = (((TX + 1) / 2) * TY + NT - 1) / NT;
   constexpr bool AR = sweep_a_ring<T, OP, TX, TY, RING>();
-  __shared__ T sU[RING][LY][LX];
-  __shared__ T sAbuf[AR ? RING * LY * LX : 1];
-  T(*sA)[LY][LX] = AR ? reinterpret_cast<T(*)[LY][LX]>(sAbuf) : nullptr;
+  constexpr bool F32 = std::is_same<T, float>::value;
+  constexpr int B = (int)sizeof(T);
+  // steps unrolled: a multiple of both parities, of the register sets of planes
+  // in flight and, for one plane in flight, of the ring
+  constexpr int U = PF == 1 ? (RING == 4 ? 4 : 10) : 6;
+  __shared__ T sU[RING * PL];
+  __shared__ T sAbuf[AR ? RING * PL : 1];
+  char *const lu = reinterpret_cast<char *>(sU), *const la = reinterpret_cast<char *>(sAbuf);
+  auto L = [](char *p, int byte) -> T & { return *reinterpret_cast<T *>(p + byte); };
   const int nx = P.nx, ny = P.ny, nz = P.nz;
-  const T *__restrict__ uin = P.uin;
-  const T *__restrict__ ain = P.a;
-  T *__restrict__ uout = P.uout;
-  double s = 0.0, cnt = 0.0;
+  const size_t plane = (size_t)nx * ny;
+  const ptrdiff_t org = (ptrdiff_t)(y0 - 2) * nx + (x0 - 2);
+  const unsigned here = (2u * (unsigned)nx + 2u) * (unsigned)B;  // position (2, 2): always in the grid
+  double s = 0.0;
+  int cnt = 0;
 
-  // u (and a) planes are prefetched into rotating register sets
+  // u (and a) planes: this thread's places of the LDS plane
   struct Ld {
     T u[NLD];
     T a[AR ? NLD : 1];
   };
-  Ld ldA, ldB, ldC;
+  Ld ld[PF + 1];
+  const bool zero = F32 && P.zero;  // uin is one element
+  const T *const ub = zero ? P.uin : P.uin + org;
+  const T *const ab = AR ? P.a + org : nullptr;
+  const size_t uplane = zero ? 0 : plane;
+  unsigned gu[NLD], ga[AR && F32 ? NLD : 1];
+  int lc[NLD];
+#pragma unroll
+  for (int m = 0; m < NLD; m++) {
+    const int q = threadIdx.x + m * NT, lx = q % LX, ly = q / LX, i = x0 - 2 + lx, j = y0 - 2 + ly;
+    const bool ok = q < PL && i >= 0 && i < nx && j >= 0 && j < ny;
+    const unsigned g = ok ? ((unsigned)ly * (unsigned)nx + (unsigned)lx) * (unsigned)B : here;
+    gu[m] = zero ? 0u : g;
+    if constexpr (AR && F32) ga[m] = g;
+    lc[m] = cs_off<LX>(lx, ly) * B;
+  }
   // the last plane the chunk reads: pass 0 also runs on plane z1 (pass 1 on
   // z1-1 needs its updated points) and reads z1+1
   const int kmax = min(z1 + 1, nz - 1);
-  // unconditional loads (positions outside the grid or the chunk read
-  // element 0, never committed): see phase_prefetch_t
-  auto load_issue = [&](Ld &ld, int k) {
+  // unconditional loads: a load behind a branch makes the compiler's wait
+  // counting fall back to waiting for every load in flight.  Places outside
+  // the grid get another's value, which no updatable point reads.
+  auto load_issue = [&](Ld &d, int k) {
+    const int kk = min(max(k, 0), kmax);
 #pragma unroll
     for (int m = 0; m < NLD; m++) {
-      const int q = threadIdx.x + m * NT;
-      const int lx = q % LX, ly = q / LX;
-      const int i = x0 - 2 + lx, j = y0 - 2 + ly;
-      const bool ok = k >= 0 && k <= kmax && q < LX * LY && i >= 0 && i < nx && j >= 0 && j < ny;
-      const size_t p = ok ? ix3(i, j, k, nx, ny) : 0;
-      if constexpr (std::is_same<T, float>::value) ld.u[m] = uin[P.zero ? 0 : p];
-      else ld.u[m] = uin[p];
-      if constexpr (AR) ld.a[m] = ain[p];
-    }
-  };
-  auto load_commit = [&](const Ld &ld, int k) {
-    if (k < 0 || k > kmax) return;
-    T(*S)[LX] = sU[ring_ix<RING>(k)];
-#pragma unroll
-    for (int m = 0; m < NLD; m++) {
-      const int q = threadIdx.x + m * NT;
-      const int lx = q % LX, ly = q / LX;
-      const int i = x0 - 2 + lx, j = y0 - 2 + ly;
-      if (q < LX * LY && i >= 0 && i < nx && j >= 0 && j < ny) {
-        S[ly][csx<LX>(lx)] = ld.u[m];
-        if constexpr (AR) sA[ring_ix<RING>(k)][ly][csx<LX>(lx)] = ld.a[m];
+      d.u[m] = tile_at(ub, uplane, kk, gu[m]);
+      if constexpr (AR) {
+        if constexpr (F32) d.a[m] = tile_at(ab, plane, kk, ga[m]);
+        else d.a[m] = tile_at(ab, plane, kk, gu[m]);
       }
     }
   };
-  // fixed trip count (unrolled): no loop of global stores inside the march
-  constexpr int NST = (TX * TY + NT - 1) / NT;
-  auto store = [&](int k) {
-    T(*S)[LX] = sU[ring_ix<RING>(k)];
+  auto load_commit = [&](const Ld &d, int slot) {
 #pragma unroll
-    for (int m = 0; m < NST; m++) {
-      const int q = threadIdx.x + m * NT;
-      const int tx = q % TX, ty = q / TX;
-      const int i = x0 + tx, j = y0 + ty;
-      if (q < TX * TY && i <= nx - 2 && j <= ny - 2) uout[ix3(i, j, k, nx, ny)] = S[ty + 2][csx<LX>(tx + 2)];
+    for (int m = 0; m < NLD; m++) {
+      if (m == NLD - 1 && PL % NT && (int)threadIdx.x + m * NT >= PL) continue;
+      L(lu, slot * PL * B + lc[m]) = d.u[m];
+      if constexpr (AR) L(la, slot * PL * B + lc[m]) = d.a[m];
     }
   };
+  unsigned go[NST];
+  int ls[NST];
+  bool st[NST];
+#pragma unroll
+  for (int m = 0; m < NST; m++) {
+    const int q = threadIdx.x + m * NT, tx = q % TX, ty = q / TX;
+    st[m] = q < TX * TY && x0 + tx <= nx - 2 && y0 + ty <= ny - 2;
+    go[m] = ((unsigned)(ty + 2) * (unsigned)nx + (unsigned)(tx + 2)) * (unsigned)B;
+    ls[m] = cs_off<LX>(tx + 2, ty + 2) * B;
+  }
+  auto store = [&](int k, int slot) {
+    char *out = reinterpret_cast<char *>(P.uout + org + (ptrdiff_t)(plane * (size_t)k));
+#pragma unroll
+    for (int m = 0; m < NST; m++)
+      if (st[m]) {
+        asm volatile("" : "+v"(go[m]));
+        *reinterpret_cast<T *>(out + go[m]) = L(lu, slot * PL * B + ls[m]);
+      }
+  };
+
+  SlotTab<N0> tab0;
+  SlotTab<N1> tab1;
+  slot_table<T, TX, TY, NT, true, N0>(P, x0, y0, z0, 0, tab0);
+  slot_table<T, TX, TY, NT, false, N1>(P, x0, y0, z0, 1, tab1);
+  auto prefetch = [&](int k, auto &S, int e, auto &R) {
+    constexpr int N = sizeof(R.rho) / sizeof(T);
+    const int kk = min(k, nz - 1);
+#pragma unroll
+    for (int m = 0; m < N; m++) {
+      unsigned &off = S.off[e][m];
+      if constexpr (EX) {
+        unsigned byte = off / (unsigned)B;
+        R.x[m] = tile_at(P.chr + org, plane, kk, byte);
+      }
+      R.rho[m] = tile_at(P.rho + org, plane, kk, off);
+      if constexpr (!RHS0) R.rhs[m] = tile_at(P.rhs + org, plane, kk, off);
+      if constexpr (OP == 1) R.c[m] = tile_at(P.c + org, plane, kk, off);
+    }
+  };
+  // one colour update of the points in table entry e on plane k; s0, sm, sp:
+  // ring slots of planes k, k-1, k+1
+  auto run = [&](int k, int s0, int sm, int sp, const auto &S, int e, const auto &R, bool count) {
+    constexpr int N = sizeof(R.rho) / sizeof(T);
+    if (k < P.bz0 || k > P.bz1) return;
+    const int b0 = s0 * PL * B, bm = sm * PL * B, bp = sp * PL * B;
+#pragma unroll
+    for (int m = 0; m < N; m++) {
+      bool act = S.ok[e][m];
+      if constexpr (EX) act = act && !R.x[m];
+      if (!act) continue;
+      const int lo = S.lo[e][m], ea = S.ea[e][m], we = ea - B;
+      const T uc = L(lu, b0 + lo);
+      T jac, A;
+      if constexpr (OP == 0) {
+        A = lop_poisson<T, P2>(uc, L(lu, b0 + ea), L(lu, b0 + we), L(lu, b0 + lo + LX * B), L(lu, b0 + lo - LX * B),
+                               L(lu, bp + lo), L(lu, bm + lo), R.rho[m], P.sp);
+        jac = P.sp.jac;
+      } else if constexpr (AR) {
+        A = lop_varcoef<T, P2>(uc, L(lu, b0 + ea), L(lu, b0 + we), L(lu, b0 + lo + LX * B), L(lu, b0 + lo - LX * B),
+                               L(lu, bp + lo), L(lu, bm + lo), L(la, b0 + lo), L(la, b0 + ea), L(la, b0 + we),
+                               L(la, b0 + lo + LX * B), L(la, b0 + lo - LX * B), L(la, bp + lo), L(la, bm + lo),
+                               R.c[m], R.rho[m], P.sp, &jac);
+      } else {
+        const T *__restrict__ a = P.a + org + (ptrdiff_t)(plane * (size_t)k);
+        const size_t p = S.off[e][m] / (unsigned)B, sy = (size_t)nx;
+        A = lop_varcoef<T, P2>(uc, L(lu, b0 + ea), L(lu, b0 + we), L(lu, b0 + lo + LX * B), L(lu, b0 + lo - LX * B),
+                               L(lu, bp + lo), L(lu, bm + lo), a[p], a[p + 1], a[p - 1], a[p + sy], a[p - sy],
+                               a[p + plane], (a - plane)[p], R.c[m], R.rho[m], P.sp, &jac);
+      }
+      T res;
+      if constexpr (RHS0) res = A - T(0); else res = A - R.rhs[m];
+      if constexpr (F32 && OP == 0)
+        L(lu, b0 + lo) = uc - res * P.sp.ijac;  // FP32 inner cycles: no IEEE division
+      else
+        L(lu, b0 + lo) = uc - div_jac<T, OP>(res, jac, P.sp);  // FP64: the reference's V - res/Jac, bit for bit
+      if (count && S.in[e][m]) {
+        s += (double)res * (double)res;
+        cnt++;
+      }
+    }
+  };
+  // ring slot of plane z0 + d (d >= -2)
+  auto slot = [](int d) { return (d + 2 * RING) % RING; };
 
   // prologue: planes z0-2 .. z0+2, pass 0 on z0-1 (tile) and z0 (tile+1).
   // Every load of the prologue and of the first march step is requested
   // before any is used (one memory round trip instead of one per plane).
-  SlotTab<N0> tab0;
-  SlotTab<N1> tab1;
-  slot_table<T, TX, TY, NT, true, N0>(P, x0, y0, 0, tab0);
-  slot_table<T, TX, TY, NT, false, N1>(P, x0, y0, 1, tab1);
-  // the rho/rhs prefetch sets alternate with the steps like the u sets (no
-  // register copies of values still in flight)
-  PhaseRegs<T, N0> pa0, pb0, pc0;
-  PhaseRegs<T, N1> pa1, pb1, pc1;
+  // Pass 0 on z0-1 over the tile takes the colours of pass 1 on z0.
+  PhaseRegs<T, OP, N0> r0[2];
+  PhaseRegs<T, OP, N1> r1[2];
   {
     Ld q0, q1, q2, q3, q4;
     load_issue(q0, z0 - 2);
@@ -324,61 +337,53 @@ __device__ __forceinline__ void sweep_tile(const SweepP<T> &P, int x0, int y0, i
     load_issue(q2, z0);
     load_issue(q3, z0 + 1);
     load_issue(q4, z0 + 2);
-    PhaseRegs<T, N1> pro1;  // pass 0 on plane z0-1 over the tile
-    PhaseRegs<T, N0> pro0;  // pass 0 on plane z0 over tile+1
-    phase_prefetch_t<T, EX, RHS0, N1>(P, z0 - 1, tab1, pro1, z0);
-    phase_prefetch_t<T, EX, RHS0, N0>(P, z0, tab0, pro0, z0);
-    load_issue(ldA, z0 + 3);
-    if constexpr (PF == 2) load_issue(ldB, z0 + 4);
-    phase_prefetch_t<T, EX, RHS0, N0>(P, z0 + 1, tab0, pa0, z0 + 1);
-    phase_prefetch_t<T, EX, RHS0, N1>(P, z0, tab1, pa1, z0);
-    load_commit(q0, z0 - 2);
-    load_commit(q1, z0 - 1);
-    load_commit(q2, z0);
-    load_commit(q3, z0 + 1);
+    prefetch(z0 - 1, tab1, 0, r1[1]);
+    prefetch(z0, tab0, 0, r0[1]);
+    load_issue(ld[0], z0 + 3);
+    if constexpr (PF == 2) load_issue(ld[1], z0 + 4);
+    prefetch(z0 + 1, tab0, 1, r0[0]);
+    prefetch(z0, tab1, 0, r1[0]);
+    load_commit(q0, slot(-2));
+    load_commit(q1, slot(-1));
+    load_commit(q2, slot(0));
+    load_commit(q3, slot(1));
     __syncthreads();
-    phase_run<T, OP, P2, RHS0, TX, TY, N1, AR, RING>(P, sU, sA, z0 - 1, pro1, false, s, cnt);
-    phase_run<T, OP, P2, RHS0, TX, TY, N0, AR, RING>(P, sU, sA, z0, pro0, true, s, cnt);
+    run(z0 - 1, slot(-1), slot(-2), slot(0), tab1, 0, r1[1], false);
+    run(z0, slot(0), slot(-1), slot(1), tab0, 0, r0[1], true);
     __syncthreads();
-    load_commit(q4, z0 + 2);
+    load_commit(q4, slot(2));
     __syncthreads();
   }
-  // step k: issue plane k+3+PF and the next step's rho/rhs; pass 0 on k+1;
-  // pass 1 on k; store k; commit plane k+3 (issued PF steps earlier)
-  auto step = [&](int k, const Ld &ldc, Ld &ldi, const PhaseRegs<T, N0> &cur0, const PhaseRegs<T, N1> &cur1,
-                  PhaseRegs<T, N0> &nxt0, PhaseRegs<T, N1> &nxt1) {
-    load_issue(ldi, k + 3 + PF);
-    phase_prefetch_t<T, EX, RHS0, N0>(P, k + 2, tab0, nxt0, k + 2);
-    phase_prefetch_t<T, EX, RHS0, N1>(P, k + 1, tab1, nxt1, k + 1);
-    phase_run<T, OP, P2, RHS0, TX, TY, N0, AR, RING>(P, sU, sA, k + 1, cur0, k + 1 < z1, s, cnt);
+  // step k = z0 + (multiple of U) + J: issue plane k+3+PF and the next step's
+  // rho/rhs; pass 0 on k+1; pass 1 on k; store k; commit plane k+3 (issued PF
+  // steps earlier)
+  auto step = [&](int k, auto j) {
+    constexpr int J = decltype(j)::value;
+    const int d = U % RING == 0 ? J : k - z0;  // the unrolled ring's slots are constants
+    load_issue(ld[(J + PF) % (PF + 1)], k + 3 + PF);
+    prefetch(k + 2, tab0, J & 1, r0[(J + 1) & 1]);
+    prefetch(k + 1, tab1, (J + 1) & 1, r1[(J + 1) & 1]);
+    run(k + 1, slot(d + 1), slot(d), slot(d + 2), tab0, (J + 1) & 1, r0[J & 1], k + 1 < z1);
     __syncthreads();
-    phase_run<T, OP, P2, RHS0, TX, TY, N1, AR, RING>(P, sU, sA, k, cur1, true, s, cnt);
+    run(k, slot(d), slot(d - 1), slot(d + 1), tab1, J & 1, r1[J & 1], true);
     if constexpr (RING == 5) {
-      load_commit(ldc, k + 3);
+      load_commit(ld[J % (PF + 1)], slot(d + 3));
       __syncthreads();
-      store(k);
+      store(k, slot(d));
     } else {
       __syncthreads();
-      store(k);
-      load_commit(ldc, k + 3);
+      store(k, slot(d));
+      load_commit(ld[J % (PF + 1)], slot(d + 3));
       __syncthreads();
     }
   };
-  if constexpr (PF == 1) {
-    for (int k = z0; k < z1; k += 2) {
-      step(k, ldA, ldB, pa0, pa1, pb0, pb1);
-      if (k + 1 < z1) step(k + 1, ldB, ldA, pb0, pb1, pa0, pa1);
-    }
-  } else {
-    // set (k - z0) % 3 holds plane k+3; the set committed one step earlier
-    // takes plane k+5
-    for (int k = z0; k < z1; k += 3) {
-      step(k, ldA, ldC, pa0, pa1, pb0, pb1);
-      if (k + 1 < z1) step(k + 1, ldB, ldA, pb0, pb1, pc0, pc1);
-      if (k + 2 < z1) step(k + 2, ldC, ldB, pc0, pc1, pa0, pa1);
-    }
-  }
-  norm_partial<NT>(s, cnt, P.ws, P.slot, bid, P.nb);
+  for (int k = z0; k < z1; k += U)
+    unrolled(std::make_integer_sequence<int, U>{}, [&](auto j) {
+      if (k + decltype(j)::value >= z1) return false;
+      step(k + decltype(j)::value, j);
+      return true;
+    });
+  norm_partial<NT>(s, (double)cnt, P.ws, P.slot, bid, P.nb);
 }
 
 template <typename T, int OP, bool EX, bool P2, bool RHS0, int TX, int TY, int NT, int PF = 1, int RING = 4>

@@ -14,7 +14,8 @@ namespace pmg {
   X(8, 128, 8, 512, 2, 4) X(9, 128, 16, 1024, 2, 5) X(10, 128, 16, 1024, 1, 5) X(11, 128, 8, 512, 1, 5)
 constexpr int kNumSweepVariants = 12;
 
-// n workgroups beyond cap (the partial-norm workspace): -3, nothing launched
+// n workgroups beyond cap (the partial-norm workspace) or rows too long for a
+// tile's 32-bit offsets (2^24 points): -3, nothing launched
 template <typename T, int OP, bool EX>
 int launch_sweep(hipStream_t stream, int variant, SweepP<T> P, bool p2, bool rhs0);
 
@@ -31,7 +32,7 @@ int launch_sweep_v(hipStream_t stream, int variant, SweepP<T> P) {
   }
   dim3 grid(((P.nx - 2 + tx - 1) / tx) * ((P.ny - 2 + ty - 1) / ty) * ((P.nz - 2 + P.zchunk - 1) / P.zchunk));
   P.nb = (int)grid.x;
-  if (P.nb > P.ws.cap) return -3;
+  if (P.nb > P.ws.cap || P.nx > 1 << 24) return -3;
   switch (variant) {
 #define PMG_LSW(V, TXV, TYV, NTV, PFV, RGV)                                                         \
   case V:                                                                                           \
