@@ -939,6 +939,7 @@ bool can_fuse_resid_restrict(const pmg_solver *S) {
   const Level &F = S->lev[S->nlev - 1], &C = S->lev[S->nlev - 2];
   for (int d = 0; d < 3; d++)
     if (F.n[d] != 2 * C.n[d] - 1) return false;
+  if ((size_t)F.n[0] * F.n[1] * sizeof(T) >= (size_t)1 << 32) return false;  // 32-bit offsets within a plane
   // the residual box must be the whole interior (ZERO semantics off it)
   return F.rbox.ok && F.rbox.lo[0] == 1 && F.rbox.lo[1] == 1 && F.rbox.lo[2] == 1 && F.rbox.hi[0] == F.n[0] - 2 &&
          F.rbox.hi[1] == F.n[1] - 2 && F.rbox.hi[2] == F.n[2] - 2;
