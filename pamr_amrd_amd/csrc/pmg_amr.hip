@@ -1017,8 +1017,8 @@ void cmask_bytes(const pmg_amr *A, int L, int gi, int which, std::vector<uint8_t
   }
 }
 
-// sweep tile shapes (TX, TY, NT); 1 and 2 are the defaults of single-grid
-// and patch levels, the others are for the per-level autotuner
+// sweep tile shapes (TX, TY, NT); 3 is the default (default_tiles), the others
+// are for the per-level autotuner
 #define PMG_AMR_VARIANTS(X) \
   X(0, 128, 16, 1024) X(1, 64, 16, 512) X(2, 32, 16, 512) X(3, 32, 8, 256) X(4, 16, 16, 256)
 constexpr int kAmrVariants = 5;
@@ -1032,6 +1032,28 @@ bool variant_txy(int v, int &tx, int &ty) {
   tx = 32;
   ty = 16;
   return false;
+}
+
+// The sweep tiles of a level that was never tuned: 32 x 8 columns in 256
+// threads, the longest march that leaves three tiles a CU (32 planes: six; the
+// step to 2 planes: one) -- fewer leave CUs idle in the last wave, shorter
+// marches repeat the prologue.  Tiles and us of one FP64 sweep against 64 x 16
+// (one grid) or 32 x 16 columns (patches) of 4 to 32 planes, op 1: 257^3 2048,
+// 252 (259); 129^3 1024, 28 (46); 33 patches of 50^3 1498, 63.5 (71); 35 of
+// 40^3 876, 37.5 (44); 17 of 28^3 608, 15 (18); 13 of 20^3 339, 9.6 (17); one
+// of 9^3 4, 8 (14).
+void default_tiles(ALevel &Lv) {
+  Lv.variant = 3;
+  int tx, ty, z = 32;
+  variant_txy(Lv.variant, tx, ty);
+  auto tiles = [&] {
+    long long n = 0;
+    for (const HGrid &g : Lv.g)
+      n += (long long)((g.n[0] - 2 + tx - 1) / tx) * ((g.n[1] - 2 + ty - 1) / ty) * ((g.n[2] - 2 + z - 1) / z);
+    return n;
+  };
+  while (z > 2 && tiles() < (z == 32 ? 1500 : z == 4 ? 300 : 750)) z /= 2;
+  Lv.zchunk = z;
 }
 
 int build_tiles(pmg_amr *A, ALevel &Lv) {
@@ -1668,15 +1690,7 @@ int setup_levels(pmg_amr *A, int op) {
     }
     if (hipMalloc(&Lv.child, pool) != hipSuccess) return -1;
     (void)hipMemcpy(Lv.child, child.data(), pool, hipMemcpyHostToDevice);
-    // sweep tiles: single-grid levels use the wide tile, patch levels 32 x 16
-    const HGrid &g0 = Lv.g[0];
-    if (Lv.g.size() == 1) {
-      Lv.variant = 1;
-      Lv.zchunk = g0.n[2] >= 257 ? 32 : g0.n[2] >= 129 ? 16 : g0.n[2] >= 65 ? 8 : 4;
-    } else {
-      Lv.variant = 2;
-      Lv.zchunk = 8;
-    }
+    default_tiles(Lv);
     if (build_tiles(A, Lv)) return -1;
     cap = std::max(cap, std::max(Lv.nstiles, Lv.nptiles) + 64);
   }
