@@ -43,23 +43,6 @@ struct SweepP {
   bool zero = false;
 };
 
-// Position of colour-slot q of a sweep phase on plane k.  HALO (pass 0):
-// tile + 1 ring; otherwise (pass 1) the tile.  Returns false when the slot
-// falls outside the region.  (lx, ly) index the LDS plane, whose origin is
-// the global point (x0-2, y0-2).
-template <int TX, int TY, bool HALO>
-__device__ __forceinline__ bool sweep_pos(int q, int x0, int y0, int k, int pass, int &lx,
-                                          int &ly) {
-  constexpr int W = HALO ? TX + 2 : TX, H = HALO ? TY + 2 : TY, OFF = HALO ? 1 : 2;
-  constexpr int W2 = (W + 1) / 2;
-  if (q >= W2 * H) return false;
-  ly = OFF + q / W2;
-  const int j = y0 - 2 + ly;
-  const int want = (j + k + 3 + pass) & 1;  // parity of i: (i+j+k+3+pass) even
-  lx = OFF + ((want - (x0 - 2 + OFF)) & 1) + 2 * (q % W2);
-  return lx <= OFF + W - 1;
-}
-
 // The variable-coefficient sweep keeps the coefficient a in an LDS ring of
 // the same shape as u's when both rings fit (its seven reads per point then
 // come from LDS, like u's); otherwise a is read from global memory.
@@ -106,40 +89,83 @@ __device__ __forceinline__ void unrolled(std::integer_sequence<int, J...>, const
   (void)(f(std::integral_constant<int, J>{}) && ...);
 }
 
-// Per-thread slot table of one phase, computed once per block for both plane
-// parities: LDS byte offsets of the point and of its east neighbour, its byte
-// offset in the tile (a position inside the grid where there is nothing to
-// update), whether there is, and whether the norm counts it (the tile proper).
+// Two neighbouring values, loaded together wherever they lie (four-byte
+// alignment is all a wide load needs).
+template <typename V>
+struct __attribute__((packed, aligned(alignof(V)))) Two {
+  V v[2];
+};
+template <typename V>
+__device__ __forceinline__ Two<V> tile_two(const V *base, size_t plane, int k, unsigned &off) {
+  asm volatile("" : "+v"(off));
+  return *reinterpret_cast<const Two<V> *>(reinterpret_cast<const char *>(base + plane * (size_t)k) + off);
+}
+
+// Per-thread slots of a sweep, computed once per block.  A slot is a pair of
+// neighbours in x, an even and an odd lx: one of each colour.  The tile's pairs
+// come first, then those of the ring (the rows above and below, and of the
+// columns beside it the near place of each pair), so pass 1 takes the first
+// NT1 slots of a thread only.  Entry e says where a step works whose upper plane
+// has the parity of z0 + e: pass 0 on that plane and pass 1 on the one below it
+// update the same place of the pair (`hi`: the second).  lo, ea: LDS byte offsets
+// of the place and its east neighbour; ok: pass 0 updates it; in: so does pass 1
+// (the tile proper), and the norm counts it.
 template <int N>
 struct SlotTab {
   int lo[2][N], ea[2][N];
-  unsigned off[2][N];
-  bool ok[2][N], in[2][N];
+  unsigned off[N];  // byte offset of the pair in the tile (of a pair in the grid where there is none)
+  bool ok[2][N], in[2][N], hi[2][N];
 };
 
-// kz: the plane whose parity is entry 0 of the table
-template <typename T, int TX, int TY, int NT, bool HALO, int N>
-__device__ __forceinline__ void slot_table(const SweepP<T> &P, int x0, int y0, int kz, int pass, SlotTab<N> &S) {
+template <typename T, int TX, int TY, int NT, int N>
+__device__ __forceinline__ void slot_table(const SweepP<T> &P, int x0, int y0, int z0, SlotTab<N> &S) {
+  constexpr int W = TX / 2;
+  static_assert(TX % 2 == 0, "pairs of points");
 #pragma unroll
-  for (int e = 0; e < 2; e++)
+  for (int m = 0; m < N; m++) {
+    const int q = threadIdx.x + m * NT, r = q - W * TY, c = r - 2 * W;
+    bool slot = true;
+    int ly = 2, lx0 = 2;
+    if (r < 0) {  // the tile
+      ly = 2 + q / W;
+      lx0 = 2 + 2 * (q % W);
+    } else if (c < 0) {  // the rows above and below
+      ly = r < W ? 1 : TY + 2;
+      lx0 = 2 + 2 * (r % W);
+    } else if (c < 2 * TY) {  // the columns beside
+      ly = 2 + c % TY;
+      lx0 = c < TY ? 0 : TX + 2;
+    } else {
+      slot = false;
+    }
+    const int j = y0 - 2 + ly, i0 = x0 - 2 + lx0;
+    // a pair may reach over an end of its row, into the neighbouring one's
+    const bool pair = slot && i0 <= P.nx - 1 && j <= P.ny - 2;
+    const int ry = pair ? ly : 2, rx = pair ? lx0 : 2;
+    S.off[m] = ((unsigned)ry * (unsigned)P.nx + (unsigned)rx) * (unsigned)sizeof(T);
 #pragma unroll
-    for (int m = 0; m < N; m++) {
-      int lx = 2, ly = 2;
-      const bool slot = sweep_pos<TX, TY, HALO>(threadIdx.x + m * NT, x0, y0, kz + e, pass, lx, ly);
-      const int i = x0 - 2 + lx, j = y0 - 2 + ly;
-      const bool ok = slot && i >= P.bx0 && i <= P.bx1 && j >= P.by0 && j <= P.by1;
-      if (!ok) lx = ly = 2;
+    for (int e = 0; e < 2; e++) {
+      const int want = (j + z0 + e + 3) & 1;  // parity of i: (i+j+k+3) even
+      const bool hi = ((want - i0) & 1) != 0;
+      const int lx = lx0 + (hi ? 1 : 0), i = i0 + (hi ? 1 : 0);
+      S.hi[e][m] = hi;
+      S.ok[e][m] = slot && lx >= 1 && lx <= TX + 2 && i >= P.bx0 && i <= P.bx1 && j >= P.by0 && j <= P.by1;
+      S.in[e][m] = S.ok[e][m] && lx >= 2 && lx < TX + 2 && ly >= 2 && ly < TY + 2;
       S.lo[e][m] = cs_off<TX + 4>(lx, ly) * (int)sizeof(T);
       S.ea[e][m] = S.lo[e][m] + cs_east<TX + 4>(lx) * (int)sizeof(T);
-      S.off[e][m] = ((unsigned)ly * (unsigned)P.nx + (unsigned)lx) * (unsigned)sizeof(T);
-      S.ok[e][m] = ok;
-      S.in[e][m] = ok && lx >= 2 && lx < TX + 2 && ly >= 2 && ly < TY + 2;
     }
+  }
 }
 
-// What a phase needs of its points beside u (and a): loaded a step before use.
+// What the passes need of a plane's pairs beside u (and a), loaded a step
+// before pass 0 takes its half; pass 1 takes the other half a step later.
 template <typename T, int OP, int N>
-struct PhaseRegs {
+struct PairRegs {
+  Two<T> rho[N], rhs[N], c[OP == 1 ? N : 1];
+  uint8_t x[N][2];
+};
+template <typename T, int OP, int N>
+struct HalfRegs {
   T rho[N], rhs[N], c[OP == 1 ? N : 1];
   uint8_t x[N];
 };
@@ -165,7 +191,8 @@ struct PhaseRegs {
 // So the march is unrolled over the ring (slots and parities become constants,
 // LDS offsets immediate fields) and an address is a scalar plane plus an offset
 // from the block's tables: 67 a step, and 63 registers instead of 100, two
-// blocks of 1024 threads a CU.  One sweep: FP32 257^3 with variable coefficient
+// blocks of 1024 threads a CU.  rho (rhs, c) comes in pairs, each read once for
+// both colours instead of once for each, a step apart.  One sweep: FP32 257^3 with variable coefficient
 // and excision 141 -> 100 us, FP32 257^3 77 -> 70 and 129^3 17.6 -> 13.7, FP64
 // 129^3 20.5 -> 19.2.  The largest stay with memory: FP64 257^3 93 -> 92 (4.5
 // TB/s), FP32 513^3 475 -> 455 (3.6 TB/s).
@@ -175,8 +202,7 @@ __device__ __forceinline__ void sweep_tile(const SweepP<T> &P, int x0, int y0, i
   static_assert(RING == 4 || RING == 5, "LDS ring");
   constexpr int LX = TX + 4, LY = TY + 4, PL = LX * LY;
   constexpr int NLD = (PL + NT - 1) / NT, NST = (TX * TY + NT - 1) / NT;
-  constexpr int N0 = (((TX + 3) / 2) * (TY + 2) + NT - 1) / NT;
-  constexpr int N1 = (((TX + 1) / 2) * TY + NT - 1) / NT;
+  constexpr int N = (TX / 2 * TY + TX + 2 * TY + NT - 1) / NT, NT1 = (TX / 2 * TY + NT - 1) / NT;
   constexpr bool AR = sweep_a_ring<T, OP, TX, TY, RING>();
   constexpr bool F32 = std::is_same<T, float>::value;
   constexpr int B = (int)sizeof(T);
@@ -260,37 +286,47 @@ __device__ __forceinline__ void sweep_tile(const SweepP<T> &P, int x0, int y0, i
       }
   };
 
-  SlotTab<N0> tab0;
-  SlotTab<N1> tab1;
-  slot_table<T, TX, TY, NT, true, N0>(P, x0, y0, z0, 0, tab0);
-  slot_table<T, TX, TY, NT, false, N1>(P, x0, y0, z0, 1, tab1);
-  auto prefetch = [&](int k, auto &S, int e, auto &R) {
-    constexpr int N = sizeof(R.rho) / sizeof(T);
+  SlotTab<N> tab;
+  slot_table<T, TX, TY, NT, N>(P, x0, y0, z0, tab);
+  auto prefetch = [&](int k, auto &R) {
     const int kk = min(k, nz - 1);
 #pragma unroll
     for (int m = 0; m < N; m++) {
-      unsigned &off = S.off[e][m];
       if constexpr (EX) {
-        unsigned byte = off / (unsigned)B;
-        R.x[m] = tile_at(P.chr + org, plane, kk, byte);
+        unsigned byte = tab.off[m] / (unsigned)B;
+        const Two<uint8_t> x = tile_two(P.chr + org, plane, kk, byte);
+        R.x[m][0] = x.v[0];
+        R.x[m][1] = x.v[1];
       }
-      R.rho[m] = tile_at(P.rho + org, plane, kk, off);
-      if constexpr (!RHS0) R.rhs[m] = tile_at(P.rhs + org, plane, kk, off);
-      if constexpr (OP == 1) R.c[m] = tile_at(P.c + org, plane, kk, off);
+      R.rho[m] = tile_two(P.rho + org, plane, kk, tab.off[m]);
+      if constexpr (!RHS0) R.rhs[m] = tile_two(P.rhs + org, plane, kk, tab.off[m]);
+      if constexpr (OP == 1) R.c[m] = tile_two(P.c + org, plane, kk, tab.off[m]);
     }
   };
-  // one colour update of the points in table entry e on plane k; s0, sm, sp:
-  // ring slots of planes k, k-1, k+1
-  auto run = [&](int k, int s0, int sm, int sp, const auto &S, int e, const auto &R, bool count) {
-    constexpr int N = sizeof(R.rho) / sizeof(T);
+  // a pair's half that pass 0 takes with entry e, or the other
+  auto half = [&](const auto &R, int e, bool other, auto &H) {
+#pragma unroll
+    for (int m = 0; m < N; m++) {
+      if (other && m >= NT1) break;
+      const bool hi = tab.hi[e][m] != other;
+      H.rho[m] = hi ? R.rho[m].v[1] : R.rho[m].v[0];
+      if constexpr (!RHS0) H.rhs[m] = hi ? R.rhs[m].v[1] : R.rhs[m].v[0];
+      if constexpr (OP == 1) H.c[m] = hi ? R.c[m].v[1] : R.c[m].v[0];
+      if constexpr (EX) H.x[m] = hi ? R.x[m][1] : R.x[m][0];
+    }
+  };
+  // one colour update on plane k at entry e's places: of the tile, with the ring
+  // around it too (ring); s0, sm, sp: LDS slots of planes k, k-1, k+1
+  auto run = [&](int k, int s0, int sm, int sp, int e, bool ring, const auto &R, bool count) {
     if (k < P.bz0 || k > P.bz1) return;
     const int b0 = s0 * PL * B, bm = sm * PL * B, bp = sp * PL * B;
 #pragma unroll
     for (int m = 0; m < N; m++) {
-      bool act = S.ok[e][m];
+      if (!ring && m >= NT1) break;
+      bool act = ring ? tab.ok[e][m] : tab.in[e][m];
       if constexpr (EX) act = act && !R.x[m];
       if (!act) continue;
-      const int lo = S.lo[e][m], ea = S.ea[e][m], we = ea - B;
+      const int lo = tab.lo[e][m], ea = tab.ea[e][m], we = ea - B;
       const T uc = L(lu, b0 + lo);
       T jac, A;
       if constexpr (OP == 0) {
@@ -304,7 +340,7 @@ __device__ __forceinline__ void sweep_tile(const SweepP<T> &P, int x0, int y0, i
                                R.c[m], R.rho[m], P.sp, &jac);
       } else {
         const T *__restrict__ a = P.a + org + (ptrdiff_t)(plane * (size_t)k);
-        const size_t p = S.off[e][m] / (unsigned)B, sy = (size_t)nx;
+        const size_t p = tab.off[m] / (unsigned)B + (tab.hi[e][m] ? 1 : 0), sy = (size_t)nx;
         A = lop_varcoef<T, P2>(uc, L(lu, b0 + ea), L(lu, b0 + we), L(lu, b0 + lo + LX * B), L(lu, b0 + lo - LX * B),
                                L(lu, bp + lo), L(lu, bm + lo), a[p], a[p + 1], a[p - 1], a[p + sy], a[p - sy],
                                a[p + plane], (a - plane)[p], R.c[m], R.rho[m], P.sp, &jac);
@@ -315,7 +351,7 @@ __device__ __forceinline__ void sweep_tile(const SweepP<T> &P, int x0, int y0, i
         L(lu, b0 + lo) = uc - res * P.sp.ijac;  // FP32 inner cycles: no IEEE division
       else
         L(lu, b0 + lo) = uc - div_jac<T, OP>(res, jac, P.sp);  // FP64: the reference's V - res/Jac, bit for bit
-      if (count && S.in[e][m]) {
+      if (count && tab.in[e][m]) {
         s += (double)res * (double)res;
         cnt++;
       }
@@ -327,9 +363,9 @@ __device__ __forceinline__ void sweep_tile(const SweepP<T> &P, int x0, int y0, i
   // prologue: planes z0-2 .. z0+2, pass 0 on z0-1 (tile) and z0 (tile+1).
   // Every load of the prologue and of the first march step is requested
   // before any is used (one memory round trip instead of one per plane).
-  // Pass 0 on z0-1 over the tile takes the colours of pass 1 on z0.
-  PhaseRegs<T, OP, N0> r0[2];
-  PhaseRegs<T, OP, N1> r1[2];
+  // Pass 0 on z0-1 over the tile takes the places of pass 0 on z0+1.
+  PairRegs<T, OP, N> pr[2];  // plane z0 + d in pr[d & 1]
+  HalfRegs<T, OP, N> now, left;
   {
     Ld q0, q1, q2, q3, q4;
     load_issue(q0, z0 - 2);
@@ -337,35 +373,37 @@ __device__ __forceinline__ void sweep_tile(const SweepP<T> &P, int x0, int y0, i
     load_issue(q2, z0);
     load_issue(q3, z0 + 1);
     load_issue(q4, z0 + 2);
-    prefetch(z0 - 1, tab1, 0, r1[1]);
-    prefetch(z0, tab0, 0, r0[1]);
+    prefetch(z0 - 1, pr[1]);
+    prefetch(z0, pr[0]);
     load_issue(ld[0], z0 + 3);
     if constexpr (PF == 2) load_issue(ld[1], z0 + 4);
-    prefetch(z0 + 1, tab0, 1, r0[0]);
-    prefetch(z0, tab1, 0, r1[0]);
     load_commit(q0, slot(-2));
     load_commit(q1, slot(-1));
     load_commit(q2, slot(0));
     load_commit(q3, slot(1));
     __syncthreads();
-    run(z0 - 1, slot(-1), slot(-2), slot(0), tab1, 0, r1[1], false);
-    run(z0, slot(0), slot(-1), slot(1), tab0, 0, r0[1], true);
+    half(pr[1], 1, false, now);
+    run(z0 - 1, slot(-1), slot(-2), slot(0), 1, false, now, false);
+    prefetch(z0 + 1, pr[1]);
+    half(pr[0], 0, false, now);
+    half(pr[0], 0, true, left);
+    run(z0, slot(0), slot(-1), slot(1), 0, true, now, true);
     __syncthreads();
     load_commit(q4, slot(2));
     __syncthreads();
   }
-  // step k = z0 + (multiple of U) + J: issue plane k+3+PF and the next step's
-  // rho/rhs; pass 0 on k+1; pass 1 on k; store k; commit plane k+3 (issued PF
-  // steps earlier)
+  // step k = z0 + (multiple of U) + J: issue plane k+3+PF and the pairs of k+2;
+  // pass 0 on k+1; pass 1 on k; store k; commit plane k+3 (issued PF steps earlier)
   auto step = [&](int k, auto j) {
-    constexpr int J = decltype(j)::value;
+    constexpr int J = decltype(j)::value, E = (J + 1) & 1;
     const int d = U % RING == 0 ? J : k - z0;  // the unrolled ring's slots are constants
     load_issue(ld[(J + PF) % (PF + 1)], k + 3 + PF);
-    prefetch(k + 2, tab0, J & 1, r0[(J + 1) & 1]);
-    prefetch(k + 1, tab1, (J + 1) & 1, r1[(J + 1) & 1]);
-    run(k + 1, slot(d + 1), slot(d), slot(d + 2), tab0, (J + 1) & 1, r0[J & 1], k + 1 < z1);
+    prefetch(k + 2, pr[J & 1]);
+    half(pr[E], E, false, now);
+    run(k + 1, slot(d + 1), slot(d), slot(d + 2), E, true, now, k + 1 < z1);
     __syncthreads();
-    run(k, slot(d), slot(d - 1), slot(d + 1), tab1, J & 1, r1[J & 1], true);
+    run(k, slot(d), slot(d - 1), slot(d + 1), E, false, left, true);
+    half(pr[E], E, true, left);
     if constexpr (RING == 5) {
       load_commit(ld[J % (PF + 1)], slot(d + 3));
       __syncthreads();
@@ -592,12 +630,16 @@ __global__ __launch_bounds__(NT) void k_sweep2(SweepP<T> P) {
 // z: the u plane k (tile + 1-point ring) sits in LDS for the x/y
 // neighbours, u(k-1), u(k), u(k+1) of the own column in registers, so each
 // u value is read from HBM once (plus the ring); the coefficient a of the
-// variable-coefficient operator likewise.  Every load is unconditional
-// (positions outside read element 0).  With the variable coefficient the next
-// step's values are requested a whole step ahead (257^3: FP64 173 -> 119 us
-// with u in FP32, FP32 110 -> 91); with the plain operator the registers this
-// takes cost more wavefronts in flight than it gains (96 -> 104 us), and the
-// loads stay within the step.
+// variable-coefficient operator likewise.  Every load is unconditional, and the
+// next step's values are requested a whole step ahead.
+// The addresses are a scalar plane plus an offset in the tile: 42 registers with
+// the plain operator, so that four blocks a CU stay resident with the values in
+// flight, and one barrier a plane (two LDS planes in turn).  257^3 with the
+// variable coefficient: FP64 of an FP32 u 173 -> 111 us, FP32 110 -> 85.  The
+// plain operator is bound by what neighbouring tiles fetch twice (1.4 times its
+// bytes at 513^3, where they have left the L2 in between); tiles of 64 x 16 and
+// marches of 32 planes measured the same or slower there (451 and 468 us over
+// 257^3 and 513^3) and slower on small grids (161 x 97 x 129: 15.6 -> 18.9).
 // UT: the type u is stored in (FP32 for the Krylov solver's preconditioned
 // vectors, whose values are FP32).
 // ---------------------------------------------------------------------------
@@ -622,8 +664,8 @@ constexpr int kResRing = 2 * RTX + 2 * RTY + 4;
 
 template <typename T, int OP, bool EX, bool P2, bool RHS0, bool ZERO, bool OUT32, typename UT = T>
 __global__ __launch_bounds__(RTX * RTY) void k_residual(ResidP<T, UT> P) {
-  __shared__ T sP[RTY + 2][RTX + 2];
-  __shared__ T sA[OP == 1 ? RTY + 2 : 1][RTX + 2];
+  __shared__ T bP[2][RTY + 2][RTX + 2];
+  __shared__ T bA[2][OP == 1 ? RTY + 2 : 1][RTX + 2];
   const int nx = P.nx, ny = P.ny, nz = P.nz;
   const size_t sz = (size_t)nx * ny;
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
@@ -647,19 +689,24 @@ __global__ __launch_bounds__(RTX * RTY) void k_residual(ResidP<T, UT> P) {
   }
   const int hi = x0 - 1 + hx, hj = y0 - 1 + hy;
   const bool hvalid = hx >= 0 && hi <= nx - 1 && hj <= ny - 1;
-  const UT *__restrict__ u = P.u;
-  const T *__restrict__ ca = P.a;
-  constexpr bool AHEAD = OP == 1;
-  const size_t pxy = inside ? (size_t)i + (size_t)nx * j : 0, hxy = hvalid ? (size_t)hi + (size_t)nx * hj : 0;
-  double s = 0.0, cnt = 0.0;
-  T um = (T)u[pxy + (z0 - 1) * sz], uc = (T)u[pxy + z0 * sz], up = T(0);
-  if constexpr (AHEAD) up = (T)u[pxy + (z0 + 1) * sz];
-  T hv = (T)u[hxy + z0 * sz], am = T(0), ac = T(0), ap = T(0), ha = T(0);
+  // addresses as in the sweep: a scalar plane plus an offset within the tile,
+  // places outside the grid reading position (1, 1), which is in it
+  const ptrdiff_t org = (ptrdiff_t)(y0 - 1) * nx + (x0 - 1);
+  auto place = [&](bool ok, int px, int py) { return ok ? (unsigned)py * (unsigned)nx + (unsigned)px : (unsigned)nx + 1u; };
+  const unsigned own_e = place(inside, lx + 1, ly + 1), ring_e = place(hvalid, hx, hy);
+  unsigned own_u = own_e * (unsigned)sizeof(UT), ring_u = ring_e * (unsigned)sizeof(UT);
+  unsigned own_t = own_e * (unsigned)sizeof(T), ring_t = ring_e * (unsigned)sizeof(T), own_x = own_e;
+  auto u_at = [&](int k, unsigned &o) { return (T)tile_at(P.u + org, sz, k, o); };
+  auto a_at = [&](int k, unsigned &o) { return tile_at(P.a + org, sz, k, o); };
+  double s = 0.0;
+  int cnt = 0;
+  T um = u_at(z0 - 1, own_u), uc = u_at(z0, own_u), up = u_at(z0 + 1, own_u), hv = u_at(z0, ring_u);
+  T am = T(0), ac = T(0), ap = T(0), ha = T(0);
   if constexpr (OP == 1) {
-    am = ca[pxy + (z0 - 1) * sz];
-    ac = ca[pxy + z0 * sz];
-    ap = ca[pxy + (z0 + 1) * sz];
-    ha = ca[hxy + z0 * sz];
+    am = a_at(z0 - 1, own_t);
+    ac = a_at(z0, own_t);
+    ap = a_at(z0 + 1, own_t);
+    ha = a_at(z0, ring_t);
   }
   // the point's own data of one step
   struct Own {
@@ -667,41 +714,34 @@ __global__ __launch_bounds__(RTX * RTY) void k_residual(ResidP<T, UT> P) {
     uint8_t x;
   };
   auto own = [&](int k) {
-    const size_t p = pxy + k * sz;
     Own o{T(0), T(0), T(0), 0};
-    if (P.rho) o.rho = P.rho[p];  // no source array: a zero source (FGMRES's operator)
-    if constexpr (!RHS0) o.rhs = P.rhs[p];
-    if constexpr (OP == 1) o.c = P.c[p];
-    if constexpr (EX) o.x = P.chr[p];
+    if (P.rho) o.rho = tile_at(P.rho + org, sz, k, own_t);  // no source array: a zero source (FGMRES's operator)
+    if constexpr (!RHS0) o.rhs = tile_at(P.rhs + org, sz, k, own_t);
+    if constexpr (OP == 1) o.c = tile_at(P.c + org, sz, k, own_t);
+    if constexpr (EX) o.x = tile_at(P.chr + org, sz, k, own_x);
     return o;
   };
-  Own cur{};
-  if constexpr (AHEAD) cur = own(z0);
+  Own cur = own(z0);
   for (int k = z0; k < z1; k++) {
-    const size_t p = pxy + k * sz;
-    T un = T(0), an = T(0), han = T(0);
-    Own nxt{};
-    if constexpr (AHEAD) {
-      const int k2 = min(k + 2, nz - 1);
-      un = (T)u[pxy + k2 * sz];
-      an = ca[pxy + k2 * sz];
-      han = ca[hxy + (k + 1) * sz];
-      nxt = own(k + 1);
-    } else {
-      up = (T)u[pxy + (k + 1) * sz];
-      cur = own(k);
+    const size_t p = sz * (size_t)k + (size_t)(org + (ptrdiff_t)own_e);
+    const int k2 = min(k + 2, nz - 1);
+    const T un = u_at(k2, own_u), hn = u_at(k + 1, ring_u);
+    T an = T(0), han = T(0);
+    if constexpr (OP == 1) {
+      an = a_at(k2, own_t);
+      han = a_at(k + 1, ring_t);
     }
-    const T hn = (T)u[hxy + (k + 1) * sz];
+    const Own nxt = own(k + 1);
     bool on = inxy && k >= P.bz0 && k <= P.bz1;
     if constexpr (EX) on = on && !cur.x;
-    __syncthreads();  // the previous plane's readers are done
+    T(*sP)[RTX + 2] = bP[(k - z0) & 1], (*sA)[RTX + 2] = bA[(k - z0) & 1];
     sP[ly + 1][lx + 1] = uc;
     if (hvalid) sP[hy][hx] = hv;
     if constexpr (OP == 1) {
       sA[ly + 1][lx + 1] = ac;
       if (hvalid) sA[hy][hx] = ha;
     }
-    __syncthreads();
+    __syncthreads();  // the next plane goes to the other buffer
     if (on) {
       T L;
       if constexpr (OP == 0) {
@@ -716,7 +756,7 @@ __global__ __launch_bounds__(RTX * RTY) void k_residual(ResidP<T, UT> P) {
       if constexpr (RHS0) r = L - T(0); else r = L - cur.rhs;
       if constexpr (OUT32) P.neg32[p] = (float)(-r); else P.res[p] = r;
       s += (double)r * (double)r;
-      cnt += 1.0;
+      cnt++;
     } else if constexpr (ZERO) {
       if (interior) {
         if constexpr (OUT32) P.neg32[p] = 0.0f; else P.res[p] = T(0);
@@ -724,17 +764,17 @@ __global__ __launch_bounds__(RTX * RTY) void k_residual(ResidP<T, UT> P) {
     }
     um = uc;
     uc = up;
+    up = un;
     hv = hn;
-    if constexpr (AHEAD) {
-      up = un;
+    if constexpr (OP == 1) {
       am = ac;
       ac = ap;
       ap = an;
       ha = han;
-      cur = nxt;
     }
+    cur = nxt;
   }
-  norm_partial<RTX * RTY>(s, cnt, P.ws, P.slot, blockIdx.x, P.nb);
+  norm_partial<RTX * RTY>(s, (double)cnt, P.ws, P.slot, blockIdx.x, P.nb);
 }
 
 // ---------------------------------------------------------------------------

@@ -431,10 +431,10 @@ int settle(pmg_solver *S, int L) {
 // processed one after another)
 template <typename P>
 int residual_grid(pmg_solver *S, P &p) {
-  p.zchunk = std::max(1, std::min(std::min(RZC, std::max(2, (p.nz - 2) / 16)), p.nz - 2));
+  p.zchunk = std::max(1, std::min(std::min(RZC, std::max(2, (p.nz - 2 + 15) / 16)), p.nz - 2));
   const int nzc = (p.nz - 2 + p.zchunk - 1) / p.zchunk;
   p.nb = ((p.nx - 2 + RTX - 1) / RTX) * ((p.ny - 2 + RTY - 1) / RTY) * nzc;
-  return p.nb > S->ws.cap ? -3 : 0;
+  return p.nb > S->ws.cap || p.nx > 1 << 24 ? -3 : 0;  // partial norms; 32-bit offsets within a tile
 }
 
 template <typename T, int OP, bool EX, bool P2>
