@@ -89,8 +89,9 @@ def autotune(n, zchunks=(2, 4, 8, 16, 32, 64), nrep=20, write=True, verbose=True
     else:
         S.apply_tuning()
     if write:
+        # every solver reads the table: the choices only, not the rows behind them
         tab = load_table()
-        tab[key] = results
+        tab[key] = {name: {k: r[k] for k in ("variant", "zchunk", "ms")} for name, r in results.items()}
         with open(TABLE, "w") as f:
             json.dump(tab, f, indent=1)
     return results
