@@ -1077,46 +1077,92 @@ __device__ __forceinline__ void wave_wait_all() {
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
 }
 
-// one sweep by lanes 0..63 of wave 0; returns the RMS of the residuals
-// (lane-uniform) and writes the norm partial
+// sqrt(s / n) > tol for the sum s of n squares: decided on s alone while it is
+// clearly above (1e-9 against a rounding of 1e-15), by the quotient and the root
+// only near the line, which ends their 300 cycles in nearly every sweep of the
+// coarsest loop
+struct AboveTol {
+  double n, tol, hi;
+  __device__ __forceinline__ AboveTol(double count, double t) : n(count), tol(t) {
+    hi = n * tol * tol * (1.0 + 1e-9);
+    if (!(hi > 1e-280 && hi < 1e280)) hi = __builtin_inf();
+  }
+  __device__ __forceinline__ bool operator()(double s) const { return s > hi || sqrt(s / n) > tol; }
+};
+
+__device__ __forceinline__ double first_lane(double v) {
+  return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(v)),
+                          __builtin_amdgcn_readfirstlane(__double2loint(v)));
+}
+
+// Sweeps by lanes 0..63 of wave 0, one point a lane: where it lies, its source
+// and its coefficients are fetched once, u alone is read from LDS.  A half sweep
+// was index arithmetic, a dozen reads and the wait for the previous sweep's norm
+// on its way to memory: the single-workgroup bottom of a 33^3 solve 32.3 -> 30.0
+// us, the block form below on 11 x 7 x 9 points 68.5 -> 47.0.
 template <typename T, int OP, bool EX, bool P2, bool IJAC>
-__device__ double wave_sweep(const WaveCoarse<T> &W) {
-  const int lane = (int)threadIdx.x;
-  double s = 0.0, cnt = 0.0;
-  const size_t sy = W.nx, sz = (size_t)W.nx * W.ny;
-  const FastDiv dmi = make_fdiv(W.mi), dmj = make_fdiv(W.mj);
-  for (int pass = 0; pass <= 1; pass++) {
+struct WaveRelax {
+  using Lds = __attribute__((address_space(3))) T *;
+  Lds u;
+  int p = 0, sy, sz;
+  bool even = false, odd = false;  // the pass that updates this lane's point
+  T rho = T(0), rhs = T(0), cc = T(0), a[7];
+  Spacing<T> sp;
+  double cnt;
+
+  __device__ __forceinline__ WaveRelax(const WaveCoarse<T> &W) : u((Lds)W.u), sy(W.nx), sz(W.nx * W.ny), sp(W.sp) {
+    const int lane = (int)threadIdx.x;
     if (lane < W.npts) {
+      const FastDiv dmi = make_fdiv(W.mi), dmj = make_fdiv(W.mj);
       int i, j, k;
       box_ijk(lane, dmi, dmj, i, j, k);
       i += W.bx0; j += W.by0; k += W.bz0;
-      const size_t p = ix3(i, j, k, W.nx, W.ny);
-      if (((i + j + k + 3 + pass) & 1) == 0 && !(EX && W.chr[p])) {
-        T jac;
-        const T r = lop_at<T, OP, P2>(W.u, W.rho, W.a, W.c, p, sy, sz, W.sp, &jac) - W.rhs[p];
-        if constexpr (IJAC) W.u[p] = W.u[p] - r * W.sp.ijac;
-        else W.u[p] = W.u[p] - div_jac<T, OP>(r, jac, W.sp);
-        s += (double)r * (double)r;
-        cnt += 1.0;
+      p = (int)ix3(i, j, k, W.nx, W.ny);
+      if (!(EX && W.chr[p])) {
+        even = ((i + j + k + 3) & 1) == 0;
+        odd = !even;
+      }
+      rho = W.rho[p];
+      rhs = W.rhs[p];
+      if constexpr (OP == 1) {
+        cc = W.c[p];
+        a[0] = W.a[p];
+        a[1] = W.a[p + 1];
+        a[2] = W.a[p - 1];
+        a[3] = W.a[p + sy];
+        a[4] = W.a[p - sy];
+        a[5] = W.a[p + sz];
+        a[6] = W.a[p - sz];
       }
     }
-    wave_wait_all();
+    cnt = (double)__popcll(__ballot(even || odd));
   }
-  for (int off = kWave / 2; off > 0; off >>= 1) {
-    s += __shfl_down(s, off, kWave);
-    cnt += __shfl_down(cnt, off, kWave);
-  }
-  double res = 0.0;
-  if (lane == 0) {
-    res = sqrt(s / cnt);
-    if (W.slot) {
-      W.slot[0] = s;
-      W.slot[1] = cnt;
-      *W.slot_nb = 1;
+
+  // returns the sum of the squared residuals, the same in every lane
+  __device__ __forceinline__ double sweep() {
+    double s = 0.0;
+#pragma unroll
+    for (int pass = 0; pass <= 1; pass++) {
+      if (pass == 0 ? even : odd) {
+        const T uc = u[p], ue = u[p + 1], uw = u[p - 1], un = u[p + sy], us = u[p - sy], ut = u[p + sz], ub = u[p - sz];
+        T jac, L;
+        if constexpr (OP == 0) {
+          L = lop_poisson<T, P2>(uc, ue, uw, un, us, ut, ub, rho, sp);
+          jac = sp.jac;
+        } else {
+          L = lop_varcoef<T, P2>(uc, ue, uw, un, us, ut, ub, a[0], a[1], a[2], a[3], a[4], a[5], a[6], cc, rho, sp, &jac);
+        }
+        const T r = L - rhs;
+        if constexpr (IJAC) u[p] = uc - r * sp.ijac;
+        else u[p] = uc - div_jac<T, OP>(r, jac, sp);
+        s = (double)r * (double)r;
+      }
+      wave_wait_all();
     }
+    for (int off = kWave / 2; off > 0; off >>= 1) s += __shfl_down(s, off, kWave);
+    return first_lane(s);
   }
-  return __shfl(res, 0, kWave);
-}
+};
 
 // cycle_watch for one wave (the saved state in global memory; each lane
 // reads back only what it wrote)
@@ -1149,26 +1195,36 @@ __device__ int cycle_watch_wave(const WaveCoarse<T> &W, CycleWatch &cw, int iter
 // sets iter and the pre-loop residual
 template <typename T, int OP, bool EX, bool P2, bool IJAC>
 __device__ double wave_coarsest(const WaveCoarse<T> &W, int &iter_out, double &res_pre) {
-  double res = 0.0;
-  for (int it = 0; it < W.npre; it++) res = wave_sweep<T, OP, EX, P2, IJAC>(W);
-  const double ctol = res * W.crtol;
-  res_pre = res;
+  WaveRelax<T, OP, EX, P2, IJAC> R(W);
+  double s = 0.0;
+  for (int it = 0; it < W.npre; it++) s = R.sweep();
+  res_pre = W.npre > 0 ? sqrt(s / R.cnt) : 0.0;
+  const double ctol = res_pre * W.crtol;
   int iter;
-  for (iter = 0; iter < W.npst; iter++) res = wave_sweep<T, OP, EX, P2, IJAC>(W);
-  res = ctol + 1;
+  for (iter = 0; iter < W.npst; iter++) s = R.sweep();
+  double res = ctol + 1;
+  const AboveTol above(R.cnt, ctol);
   CycleWatch cw;
   int wit = 0;
-  while (iter < W.max_citer && res > ctol) {
-    res = wave_sweep<T, OP, EX, P2, IJAC>(W);
+  bool go = res > ctol;
+  while (iter < W.max_citer && go) {
+    s = R.sweep();
+    go = above(s);
     iter++;
-    if (W.snap && ++wit >= kWatchStart && res > ctol && iter < W.max_citer) {
+    if (W.snap && ++wit >= kWatchStart && go && iter < W.max_citer) {
       const int r = cycle_watch_wave<T>(W, cw, iter);
       if (r >= 0) {
-        for (int k = 0; k < r; k++) res = wave_sweep<T, OP, EX, P2, IJAC>(W);
+        for (int k = 0; k < r; k++) s = R.sweep();
         iter = W.max_citer;
         break;
       }
     }
+  }
+  if (iter > W.npst) res = sqrt(s / R.cnt);
+  if (threadIdx.x == 0 && W.slot && (W.npre > 0 || iter > 0)) {
+    W.slot[0] = s;
+    W.slot[1] = R.cnt;
+    *W.slot_nb = 1;
   }
   iter_out = iter;
   return res;
@@ -1197,31 +1253,6 @@ __global__ __launch_bounds__(NT) void k_coarse_solve(CoarseP<T> P) {
   }
   const int mi = P.bx1 - P.bx0 + 1, mj = P.by1 - P.by0 + 1, mk = P.bz1 - P.bz0 + 1;
   const int npts = (mi > 0 && mj > 0 && mk > 0) ? mi * mj * mk : 0;
-  const FastDiv dmi = make_fdiv(mi), dmj = make_fdiv(mj);
-  __shared__ double bres;
-  auto sweep = [&]() -> double {
-    double s = 0.0, cnt = 0.0;
-    for (int pass = 0; pass <= 1; pass++) {
-      for (int q = threadIdx.x; q < npts; q += NT) {
-        int i, j, k;
-        box_ijk(q, dmi, dmj, i, j, k);
-        i += P.bx0; j += P.by0; k += P.bz0;
-        if (((i + j + k + 3 + pass) & 1) != 0) continue;
-        const size_t p = ix3(i, j, k, nx, ny);
-        if constexpr (EX) { if (P.chr[p]) continue; }
-        T jac;
-        const T r = lop_at<T, OP, P2>(u, rho, a, c, p, sy, sz, P.sp, &jac) - rhs[p];
-        u[p] = u[p] - div_jac<T, OP>(r, jac, P.sp);
-        s += (double)r * (double)r;
-        cnt += 1.0;
-      }
-      __syncthreads();
-    }
-    block_reduce2<NT>(s, cnt);
-    if (threadIdx.x == 0) bres = sqrt(s / cnt);
-    __syncthreads();
-    return bres;
-  };
   if constexpr (LDS) {
     if (npts <= kWave) {  // one wave, same bits (see wave_coarsest)
       if (threadIdx.x < kWave) {
@@ -1241,27 +1272,106 @@ __global__ __launch_bounds__(NT) void k_coarse_solve(CoarseP<T> P) {
       return;
     }
   }
-  double res = 0.0;
-  for (int it = 0; it < P.npre; it++) res = sweep();
+  // The points of a thread, found once for up to kOwn of them: element and
+  // colour; the number of updatable points, which every sweep counts alike.
+  constexpr int kOwn = 4, NW = NT / kWave;
+  const FastDiv dmi = make_fdiv(mi), dmj = make_fdiv(mj);
+  auto point = [&](int q, int &pass) -> size_t {
+    int i, j, k;
+    box_ijk(q, dmi, dmj, i, j, k);
+    i += P.bx0; j += P.by0; k += P.bz0;
+    const size_t p = ix3(i, j, k, nx, ny);
+    pass = (i + j + k + 3) & 1;
+    if constexpr (EX) { if (P.chr[p]) pass = -1; }
+    return p;
+  };
+  unsigned at[kOwn];
+  int by[kOwn];
+#pragma unroll
+  for (int m = 0; m < kOwn; m++) {
+    by[m] = -1;
+    at[m] = 0;
+    const int q = (int)threadIdx.x + m * NT;
+    if (q < npts) at[m] = (unsigned)point(q, by[m]);
+  }
+  double count = 0.0;
+  {
+    double none = 0.0;
+    for (int q = threadIdx.x; q < npts; q += NT) {
+      int pass;
+      point(q, pass);
+      if (pass >= 0) count += 1.0;
+    }
+    block_reduce2<NT>(none, count);
+    __shared__ double bcount;
+    if (threadIdx.x == 0) bcount = count;
+    __syncthreads();
+    count = bcount;
+  }
+  __shared__ double wsum[2][NW];
+  int turn = 0;
+  // one sweep; returns the sum of the squared residuals, the same in every
+  // thread: each wave's by its shuffle tree, those in every thread alike (two
+  // barriers a sweep: the half sweep's, and the one that publishes the sums)
+  auto sweep = [&]() -> double {
+    double s = 0.0;
+    auto relax = [&](size_t p) {
+      T jac;
+      const T r = lop_at<T, OP, P2>(u, rho, a, c, p, sy, sz, P.sp, &jac) - rhs[p];
+      u[p] = u[p] - div_jac<T, OP>(r, jac, P.sp);
+      s += (double)r * (double)r;
+    };
+    for (int pass = 0; pass <= 1; pass++) {
+#pragma unroll
+      for (int m = 0; m < kOwn; m++)
+        if (by[m] == pass) relax(at[m]);
+      for (int q = threadIdx.x + kOwn * NT; q < npts; q += NT) {
+        int mine;
+        const size_t p = point(q, mine);
+        if (mine == pass) relax(p);
+      }
+      if (pass == 0) __syncthreads();
+    }
+    for (int off = kWave / 2; off > 0; off >>= 1) s += __shfl_down(s, off, kWave);
+    double *w = wsum[turn ^= 1];
+    if (threadIdx.x % kWave == 0) w[threadIdx.x / kWave] = s;
+    __syncthreads();
+    double v[NW];
+#pragma unroll
+    for (int m = 0; m < NW; m++) v[m] = w[m];
+#pragma unroll
+    for (int off = NW / 2; off > 0; off >>= 1)
+#pragma unroll
+      for (int m = 0; m < NW; m++)
+        if (m < off) v[m] += v[m + off];
+    return v[0];
+  };
+  double s = 0.0, res = 0.0;
+  for (int it = 0; it < P.npre; it++) s = sweep();
+  if (P.npre > 0) res = sqrt(s / count);
   const double ctol = res * P.crtol;
   if (threadIdx.x == 0 && P.norm_pre) P.norm_pre[0] = res;
   int iter = 0;
-  for (iter = 0; iter < P.npst; iter++) res = sweep();
+  for (iter = 0; iter < P.npst; iter++) s = sweep();
   res = ctol + 1;
+  const AboveTol above(count, ctol);
   CycleWatch cw;
   int wit = 0;
-  while (iter < P.max_citer && res > ctol) {
-    res = sweep();
+  bool go = res > ctol;
+  while (iter < P.max_citer && go) {
+    s = sweep();
+    go = above(s);
     iter++;
-    if (P.snap && ++wit >= kWatchStart && res > ctol && iter < P.max_citer) {
+    if (P.snap && ++wit >= kWatchStart && go && iter < P.max_citer) {
       const int r = cycle_watch<T, NT>(u, n, P.snap, cw, iter, P.max_citer);
       if (r >= 0) {
-        for (int k = 0; k < r; k++) res = sweep();
+        for (int k = 0; k < r; k++) s = sweep();
         iter = P.max_citer;
         break;
       }
     }
   }
+  if (iter > P.npst) res = sqrt(s / count);
   if constexpr (LDS) {
     for (size_t q = threadIdx.x; q < n; q += NT) P.u[q] = u[q];
   }
