@@ -868,7 +868,11 @@ __global__ __launch_bounds__(256) void k_lop_rhs(LopRhsP<T> P, BoxPts bp) {
 //
 // One thread per coarse point (ci, cj, ck): it reads the (up to) 8 corners
 // of its coarse cell once and updates the fine points 2c + r, r in {0,1}^3
-// inside the grid, with the per-point expression of the x/y/z phases.
+// inside the grid, with the per-point expression of the x/y/z phases.  The eight
+// values of u are read before one is written: a store between two loads of the
+// same array orders them, and each point waited for the one before.
+// Average over the levels of a cycle: FP64 257^3 and 129^3 48 -> 38 us, FP32
+// 513^3 to 129^3 118 -> 100.
 template <typename T>
 __global__ __launch_bounds__(256) void k_cgc(T *__restrict__ u, T *__restrict__ alt, const T *__restrict__ uc,
                                              const T *__restrict__ lopc, T *__restrict__ Rc, T w0_i, int nx, int ny,
@@ -892,25 +896,40 @@ __global__ __launch_bounds__(256) void k_cgc(T *__restrict__ u, T *__restrict__ 
       for (int q = 0; q < 8; q++) r[q / 4][(q / 2) % 2][q % 2] = r[q / 4][(q / 2) % 2][q % 2] / w0_i;
     }
     Rc[ix3(ci, cj, ck, cnx, cny)] = r[0][0][0];
+    // u's pairs along x, all requested before any is written (a pair at the end
+    // of an odd row holds its last two points)
+    Two<T> *pu[2][2];
+    Two<T> uv[2][2];
+#pragma unroll
+    for (int rk = 0; rk < 2; rk++)
+#pragma unroll
+      for (int rj = 0; rj < 2; rj++) {
+        const size_t q = ix3(2 * ci, 2 * cj + (yi ? rj : 0), 2 * ck + (zi ? rk : 0), nx, ny);
+        pu[rk][rj] = reinterpret_cast<Two<T> *>(u + q - (xi ? 0 : 1));
+        uv[rk][rj] = *pu[rk][rj];
+      }
 #pragma unroll
     for (int rk = 0; rk < 2; rk++) {
       if (rk == 1 && !zi) continue;
 #pragma unroll
       for (int rj = 0; rj < 2; rj++) {
         if (rj == 1 && !yi) continue;
+        const int j = 2 * cj + rj, k = 2 * ck + rk;
+        const size_t q = ix3(2 * ci, j, k, nx, ny);
+        T nu[2];
 #pragma unroll
         for (int ri = 0; ri < 2; ri++) {
-          if (ri == 1 && !xi) continue;
-          const int i = 2 * ci + ri, j = 2 * cj + rj, k = 2 * ck + rk;
           auto X = [&](int b, int c) -> T { return ri == 0 ? r[c][b][0] : c0 * r[c][b][0] + c1 * r[c][b][1]; };
           auto Y = [&](int c) -> T { return rj == 0 ? X(0, c) : c0 * X(0, c) + c1 * X(1, c); };
           T v = rk == 0 ? Y(0) : c0 * Y(0) + c1 * Y(1);
-          const size_t q = ix3(i, j, k, nx, ny);
-          if (chr && chr[q]) v = T(0);
-          const T nu = u[q] + v;
-          u[q] = nu;
-          if (i == 0 || j == 0 || k == 0 || i == nx - 1 || j == ny - 1 || k == nz - 1) alt[q] = nu;
+          if (chr && chr[q + (xi ? ri : 0)]) v = T(0);
+          nu[ri] = (ri == 0 && !xi ? uv[rk][rj].v[1] : uv[rk][rj].v[ri]) + v;
         }
+        if (xi) *pu[rk][rj] = Two<T>{{nu[0], nu[1]}};
+        else u[q] = nu[0];
+        const bool face = j == 0 || k == 0 || j == ny - 1 || k == nz - 1;
+        if (face || ci == 0 || !xi) alt[q] = nu[0];
+        if (xi && (face || 2 * ci + 1 == nx - 1)) alt[q + 1] = nu[1];
       }
     }
   });
