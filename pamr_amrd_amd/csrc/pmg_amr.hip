@@ -78,6 +78,9 @@ __device__ __forceinline__ bool job_point(const XJob &J, int idx, int &i, int &j
   return true;
 }
 
+// A block moves one field (blockIdx.y): one after another, five fields of a
+// small level were five rounds of memory latency (restriction onto 5^3 .. 33^3:
+// 12-17 us -> 7; onto 129^3 and 50^3 patches 39 -> 32).
 // sync copies (local_transfer, delta = 0)
 template <typename T>
 __global__ __launch_bounds__(kXT) void k_xfer_copy(XFields<T> F, const GridGeo *gs, const GridGeo *gd,
@@ -89,11 +92,10 @@ __global__ __launch_bounds__(kXT) void k_xfer_copy(XFields<T> F, const GridGeo *
   const GridGeo S = gs[J.sg], D = gd[J.dg];
   const size_t qd = D.off + ix3(i, j, k, D.nx, D.ny);
   const size_t qs = S.off + ix3(i + J.sh[0], j + J.sh[1], k + J.sh[2], S.nx, S.ny);
-  for (int f = 0; f < F.nf; f++) {
-    const T v = F.src[f][qs];
-    F.dst[f][qd] = v;
-    if (F.alt[f]) F.alt[f][qd] = v;
-  }
+  const int f = blockIdx.y;
+  const T v = F.src[f][qs];
+  F.dst[f][qd] = v;
+  if (F.alt[f]) F.alt[f][qd] = v;
 }
 
 // inject (local_transfer, delta = 1): dmcopy3d / dmhwr3d / dmfwr3d at
@@ -109,15 +111,14 @@ __global__ __launch_bounds__(kXT) void k_xfer_restrict(XFields<T> F, const GridG
   const GridGeo S = gs[J.sg], D = gd[J.dg];
   const size_t qd = D.off + ix3(i, j, k, D.nx, D.ny);
   const int i0 = 2 * i + J.sh[0] + 1, j0 = 2 * j + J.sh[1] + 1, k0 = 2 * k + J.sh[2] + 1;  // 1-based fine
-  for (int f = 0; f < F.nf; f++) {
-    const T *u1 = F.src[f] + S.off;
-    T v;
-    if constexpr (KIND == 1) v = u1[ix3(i0 - 1, j0 - 1, k0 - 1, S.nx, S.ny)];
-    else if constexpr (KIND == 2) v = hw_point<T, false>(u1, nullptr, T(0), S.nx, S.ny, S.nz, i0, j0, k0);
-    else v = fw_point<T>(u1, S.nx, S.ny, S.nz, i0, j0, k0);
-    F.dst[f][qd] = v;
-    if (F.alt[f]) F.alt[f][qd] = v;
-  }
+  const int f = blockIdx.y;
+  const T *u1 = F.src[f] + S.off;
+  T v;
+  if constexpr (KIND == 1) v = u1[ix3(i0 - 1, j0 - 1, k0 - 1, S.nx, S.ny)];
+  else if constexpr (KIND == 2) v = hw_point<T, false>(u1, nullptr, T(0), S.nx, S.ny, S.nz, i0, j0, k0);
+  else v = fw_point<T>(u1, S.nx, S.ny, S.nz, i0, j0, k0);
+  F.dst[f][qd] = v;
+  if (F.alt[f]) F.alt[f][qd] = v;
 }
 
 // interp (local_transfer, delta = -1): dminterp3d second order
@@ -135,15 +136,14 @@ __global__ __launch_bounds__(kXT) void k_xfer_interp(XFields<T> F, const GridGeo
   const int Fx = i + J.sh[0], Fy = j + J.sh[1], Fz = k + J.sh[2];
   const int ai = Fx >> 1, ri = Fx & 1, aj = Fy >> 1, rj = Fy & 1, ak = Fz >> 1, rk = Fz & 1;
   const T c0 = T(1 - (1 * 1.0) / 2), c1 = T((1 * 1.0) / 2);
-  for (int f = 0; f < F.nf; f++) {
-    const T *uc = F.src[f] + S.off;
-    auto R = [&](int a, int bb, int c) -> T { return uc[ix3(a, bb, c, S.nx, S.ny)]; };
-    auto X = [&](int bb, int c) -> T { return ri == 0 ? R(ai, bb, c) : c0 * R(ai, bb, c) + c1 * R(ai + 1, bb, c); };
-    auto Y = [&](int c) -> T { return rj == 0 ? X(aj, c) : c0 * X(aj, c) + c1 * X(aj + 1, c); };
-    const T v = rk == 0 ? Y(ak) : c0 * Y(ak) + c1 * Y(ak + 1);
-    F.dst[f][qd] = v;
-    if (F.alt[f]) F.alt[f][qd] = v;
-  }
+  const int f = blockIdx.y;
+  const T *uc = F.src[f] + S.off;
+  auto R = [&](int a, int bb, int c) -> T { return uc[ix3(a, bb, c, S.nx, S.ny)]; };
+  auto X = [&](int bb, int c) -> T { return ri == 0 ? R(ai, bb, c) : c0 * R(ai, bb, c) + c1 * R(ai + 1, bb, c); };
+  auto Y = [&](int c) -> T { return rj == 0 ? X(aj, c) : c0 * X(aj, c) + c1 * X(aj + 1, c); };
+  const T v = rk == 0 ? Y(ak) : c0 * Y(ak) + c1 * Y(ak + 1);
+  F.dst[f][qd] = v;
+  if (F.alt[f]) F.alt[f][qd] = v;
 }
 
 // interp at fourth order: dminterp3d ord 4 (src/m_util_r8.f:473-637, dvi4q1d
@@ -162,23 +162,22 @@ __global__ __launch_bounds__(kXT) void k_xfer_interp4(XFields<T> F, const GridGe
   const GridGeo S = gs[J.sg], D = gd[J.dg];
   const size_t qd = D.off + ix3(i, j, k, D.nx, D.ny);
   const int fx = i + J.sh[0] - 2 * J.t0[0], fy = j + J.sh[1] - 2 * J.t0[1], fz = k + J.sh[2] - 2 * J.t0[2];
-  for (int f = 0; f < F.nf; f++) {
-    const T *uc = F.src[f] + S.off;
-    auto line = [&](int d, int fd, const auto &A) -> T {
-      if ((fd & 1) == 0) return A(fd >> 1);
-      return vi4_point(J.tn[d], 2, 1, 2 * J.tn[d] - 1, fd, A);
+  const int f = blockIdx.y;
+  const T *uc = F.src[f] + S.off;
+  auto line = [&](int d, int fd, const auto &A) -> T {
+    if ((fd & 1) == 0) return A(fd >> 1);
+    return vi4_point(J.tn[d], 2, 1, 2 * J.tn[d] - 1, fd, A);
+  };
+  auto Y = [&](int c) -> T {
+    auto X = [&](int bb) -> T {
+      auto R = [&](int a) -> T { return uc[ix3(J.t0[0] + a, J.t0[1] + bb, J.t0[2] + c, S.nx, S.ny)]; };
+      return line(0, fx, R);
     };
-    auto Y = [&](int c) -> T {
-      auto X = [&](int bb) -> T {
-        auto R = [&](int a) -> T { return uc[ix3(J.t0[0] + a, J.t0[1] + bb, J.t0[2] + c, S.nx, S.ny)]; };
-        return line(0, fx, R);
-      };
-      return line(1, fy, X);
-    };
-    const T v = line(2, fz, Y);
-    F.dst[f][qd] = v;
-    if (F.alt[f]) F.alt[f][qd] = v;
-  }
+    return line(1, fy, X);
+  };
+  const T v = line(2, fz, Y);
+  F.dst[f][qd] = v;
+  if (F.alt[f]) F.alt[f][qd] = v;
 }
 
 // compute_cgc fused (amrd/mg.c:323-355), for levels whose interp plan writes
@@ -198,16 +197,27 @@ __global__ __launch_bounds__(kXT) void k_xfer_cgc(const T *__restrict__ cu, cons
   const size_t qd = D.off + ix3(i, j, k, D.nx, D.ny);
   auto C = [&](int a, int bb, int c) -> T {
     const size_t q = S.off + ix3(a, bb, c, S.nx, S.ny);
-    return (cu[q] - clop[q]) / w0_i;
+    const T d = cu[q] - clop[q];
+    return w0_i == T(1) ? d : d / w0_i;  // x / 1 is x
   };
   T v;
   if constexpr (ORD == 2) {
     const int Fx = i + J.sh[0], Fy = j + J.sh[1], Fz = k + J.sh[2];
     const int ai = Fx >> 1, ri = Fx & 1, aj = Fy >> 1, rj = Fy & 1, ak = Fz >> 1, rk = Fz & 1;
     const T c0 = T(1 - (1 * 1.0) / 2), c1 = T((1 * 1.0) / 2);
-    auto X = [&](int bb, int c) -> T { return ri == 0 ? C(ai, bb, c) : c0 * C(ai, bb, c) + c1 * C(ai + 1, bb, c); };
-    auto Y = [&](int c) -> T { return rj == 0 ? X(aj, c) : c0 * X(aj, c) + c1 * X(aj + 1, c); };
-    v = rk == 0 ? Y(ak) : c0 * Y(ak) + c1 * Y(ak + 1);
+    // the (up to) eight corners at once, a point on a coarse line, plane or
+    // corner reading the same ones again: no load waits for a branch, and the
+    // eight divisions by w0_i = 1 go (33 patches of 50^3: 54 -> 40 us)
+    T d[2][2][2];
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+#pragma unroll
+      for (int b2 = 0; b2 < 2; b2++)
+#pragma unroll
+        for (int a = 0; a < 2; a++) d[c][b2][a] = C(ai + a * ri, aj + b2 * rj, ak + c * rk);
+    auto X = [&](int bb, int c) -> T { return ri == 0 ? d[c][bb][0] : c0 * d[c][bb][0] + c1 * d[c][bb][1]; };
+    auto Y = [&](int c) -> T { return rj == 0 ? X(0, c) : c0 * X(0, c) + c1 * X(1, c); };
+    v = rk == 0 ? Y(0) : c0 * Y(0) + c1 * Y(1);
   } else {
     const int fx = i + J.sh[0] - 2 * J.t0[0], fy = j + J.sh[1] - 2 * J.t0[1], fz = k + J.sh[2] - 2 * J.t0[2];
     auto line = [&](int d, int fd, const auto &A) -> double {
@@ -281,6 +291,69 @@ struct PtsBatchP {
   int slot;
 };
 
+// One thread's column of a point tile, marched in z: u (and a) of the planes
+// k-1, k, k+1 in registers, the x and y neighbours from the L1, every address a
+// scalar plane plus one of five offsets worked out once.  33 patches of 50^3
+// points with op 1: 47.6 -> 44.9 us, 35 of 40^3 30.2 -> 28.6.  (L_op with the
+// child mask is quicker point by point, 29 against 39 us: most points of a patch
+// level have no child above them, and skip the operator.)
+template <typename T, int OP, bool P2>
+struct TileCol {
+  const T *u, *rho, *a, *c;  // from the place west and south of the tile's corner
+  size_t plane;
+  int nz;
+  unsigned own, east, west, north, south;  // byte offsets; the own place for a column on the rim
+  T um, uc, up, am, ac, ap;
+  __device__ __forceinline__ TileCol(const PtsBatchP<T> &B, const GridGeo &G, const BTile &tl, int i, int j, bool inner) {
+    const ptrdiff_t org = (ptrdiff_t)G.off + (ptrdiff_t)(tl.y0 - 1) * G.nx + (tl.x0 - 1);
+    u = B.u + org;
+    rho = B.rho + org;
+    a = OP == 1 ? B.a + org : nullptr;
+    c = OP == 1 ? B.c + org : nullptr;
+    plane = (size_t)G.nx * G.ny;
+    nz = G.nz;
+    const int d = inner ? 1 : 0;
+    i = min(i, G.nx - 1) - (tl.x0 - 1);
+    j = min(j, G.ny - 1) - (tl.y0 - 1);
+    auto at = [&](int x, int y) { return ((unsigned)y * (unsigned)G.nx + (unsigned)x) * (unsigned)sizeof(T); };
+    own = at(i, j);
+    east = at(i + d, j);
+    west = at(i - d, j);
+    north = at(i, j + d);
+    south = at(i, j - d);
+    const int k = tl.z0;
+    uc = get(u, k - 1, own);
+    up = get(u, k, own);
+    if constexpr (OP == 1) {
+      ac = get(a, k - 1, own);
+      ap = get(a, k, own);
+    }
+  }
+  __device__ __forceinline__ T get(const T *f, int k, unsigned &o) const {
+    return tile_at(f, plane, min(max(k, 0), nz - 1), o);
+  }
+  __device__ __forceinline__ void step(int k) {  // to plane k
+    um = uc;
+    uc = up;
+    up = get(u, k + 1, own);
+    if constexpr (OP == 1) {
+      am = ac;
+      ac = ap;
+      ap = get(a, k + 1, own);
+    }
+  }
+  __device__ __forceinline__ T lop(int k, const Spacing<T> &sp) {
+    const T ue = get(u, k, east), uw = get(u, k, west), un = get(u, k, north), us = get(u, k, south);
+    const T r = get(rho, k, own);
+    if constexpr (OP == 0) {
+      return lop_poisson<T, P2>(uc, ue, uw, un, us, up, um, r, sp);
+    } else {
+      const T ae = get(a, k, east), aw = get(a, k, west), an = get(a, k, north), as = get(a, k, south);
+      return lop_varcoef<T, P2>(uc, ue, uw, un, us, up, um, ac, ae, aw, an, as, ap, am, get(c, k, own), r, sp, nullptr);
+    }
+  }
+};
+
 // residual hook (w/examples/nps/num_w.f:59-90) on the interior of every grid
 template <typename T, int OP, bool P2, bool RHS0>
 __global__ __launch_bounds__(PTX * PTY) void k_resid_batch(PtsBatchP<T> B) {
@@ -288,26 +361,25 @@ __global__ __launch_bounds__(PTX * PTY) void k_resid_batch(PtsBatchP<T> B) {
   const BTile tl = B.tiles[t];
   const GridGeo G = B.grids[tl.g];
   const int i = tl.x0 + (int)(threadIdx.x % PTX), j = tl.y0 + (int)(threadIdx.x / PTX);
-  const size_t sy = G.nx, sz = (size_t)G.nx * G.ny;
-  double s = 0.0, cnt = 0.0;
-  if (i >= 1 && i <= G.nx - 2 && j >= 1 && j <= G.ny - 2) {
-    const T *u = B.u + G.off, *rho = B.rho + G.off, *rhs = B.rhs + G.off;
-    const T *a = B.a ? B.a + G.off : nullptr, *c = B.c ? B.c + G.off : nullptr;
-    T *res = B.res + G.off;
+  const bool inner = i >= 1 && i <= G.nx - 2 && j >= 1 && j <= G.ny - 2;
+  double s = 0.0;
+  int cnt = 0;
+  const size_t p0 = G.off + ix3(i, j, 0, G.nx, G.ny);
+  TileCol<T, OP, P2> C(B, G, tl, i, j, inner);
 #pragma unroll
-    for (int kk = 0; kk < PTZ; kk++) {
-      const int k = tl.z0 + kk;
-      if (k < 1 || k > G.nz - 2) continue;
-      const size_t p = ix3(i, j, k, G.nx, G.ny);
-      const T L = lop_at<T, OP, P2>(u, rho, a, c, p, sy, sz, B.sp, nullptr);
-      T r;
-      if constexpr (RHS0) r = L - T(0); else r = L - rhs[p];
-      res[p] = r;
-      s += (double)r * (double)r;
-      cnt += 1.0;
-    }
+  for (int kk = 0; kk < PTZ; kk++) {
+    const int k = tl.z0 + kk;
+    C.step(k);
+    const T L = C.lop(k, B.sp);
+    if (!inner || k < 1 || k > G.nz - 2) continue;
+    const size_t p = p0 + C.plane * k;
+    T r;
+    if constexpr (RHS0) r = L - T(0); else r = L - B.rhs[p];
+    B.res[p] = r;
+    s += (double)r * (double)r;
+    cnt++;
   }
-  norm_partial<PTX * PTY>(s, cnt, B.ws, B.slot, t, gridDim.x);
+  norm_partial<PTX * PTY>(s, (double)cnt, B.ws, B.slot, t, gridDim.x);
 }
 
 // L_op + compute_MG_rhs (amrd/mg.c:124-126, 271-304) with the child mask
@@ -357,29 +429,26 @@ __global__ __launch_bounds__(PTX * PTY) void k_defect32_batch(PtsBatchP<double> 
   const BTile tl = B.tiles[t];
   const GridGeo G = B.grids[tl.g];
   const int i = tl.x0 + (int)(threadIdx.x % PTX), j = tl.y0 + (int)(threadIdx.x / PTX);
-  const size_t sy = G.nx, sz = (size_t)G.nx * G.ny;
-  double s = 0.0, cnt = 0.0;
-  if (i < G.nx && j < G.ny) {
-    const double *u = B.u + G.off, *rho = B.rho + G.off;
-    const double *a = B.a ? B.a + G.off : nullptr, *c = B.c ? B.c + G.off : nullptr;
-    float *out = src32 + G.off;
-    const bool ixy = i >= 1 && i <= G.nx - 2 && j >= 1 && j <= G.ny - 2;
+  const bool in = i < G.nx && j < G.ny, inner = i >= 1 && i <= G.nx - 2 && j >= 1 && j <= G.ny - 2;
+  double s = 0.0;
+  int cnt = 0;
+  const size_t p0 = G.off + ix3(i, j, 0, G.nx, G.ny);
+  TileCol<double, OP, P2> C(B, G, tl, i, j, inner);
 #pragma unroll
-    for (int kk = 0; kk < PTZ; kk++) {
-      const int k = tl.z0 + kk;
-      if (k >= G.nz) break;
-      const size_t p = ix3(i, j, k, G.nx, G.ny);
-      float v = 0.0f;
-      if (ixy && k >= 1 && k <= G.nz - 2) {
-        const double r = lop_at<double, OP, P2>(u, rho, a, c, p, sy, sz, B.sp, nullptr) - 0.0;
-        v = (float)(-r);
-        s += r * r;
-        cnt += 1.0;
-      }
-      out[p] = v;
+  for (int kk = 0; kk < PTZ; kk++) {
+    const int k = tl.z0 + kk;
+    if (k >= G.nz) break;
+    C.step(k);
+    const double r = C.lop(k, B.sp) - 0.0;
+    float v = 0.0f;
+    if (inner && k >= 1 && k <= G.nz - 2) {
+      v = (float)(-r);
+      s += r * r;
+      cnt++;
     }
+    if (in) src32[p0 + C.plane * k] = v;
   }
-  norm_partial<PTX * PTY>(s, cnt, B.ws, B.slot, t, gridDim.x);
+  norm_partial<PTX * PTY>(s, (double)cnt, B.ws, B.slot, t, gridDim.x);
 }
 
 // u += e in FP64 over a level's pool, both ping-pong buffers
@@ -1163,7 +1232,7 @@ int run_plan(pmg_amr *A, const XPlan &P, int Ls, int Ld, int kind, const int *wh
     F.nf++;
   }
   if (F.nf == 0) return 0;
-  const dim3 grid(P.nblocks), blk(kXT);
+  const dim3 grid(P.nblocks, F.nf), blk(kXT);
   switch (kind) {
     case 0: hipLaunchKernelGGL(k_xfer_copy<T>, grid, blk, 0, A->stream, F, S.d_geo, D.d_geo, P.d_jobs, P.d_blks); break;
     case 1: hipLaunchKernelGGL((k_xfer_restrict<T, 1>), grid, blk, 0, A->stream, F, S.d_geo, D.d_geo, P.d_jobs, P.d_blks); break;
