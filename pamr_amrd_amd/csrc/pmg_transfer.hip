@@ -100,9 +100,10 @@ __global__ __launch_bounds__(NT) void k_interp3d(const T *u1, T *u2, int nx1, in
 // anchor lattice of its axis and reads only points on it (inside or just
 // outside the segment), so its points are independent; phases run in the
 // reference's order x, y, z on u2 after the common points were copied.
-template <int AX>
+template <int AX, bool R2>
 __global__ __launch_bounds__(NT) void k_interp4(double *u2, int nx2, int ny2, int nz2, int i2, int j2, int k2, int ni,
                                                 int nj, int nk, int irho, int jrho, int krho, BoxPts bp) {
+  if (R2) irho = jrho = krho = 2;
   const int mi = (ni - 1) * irho + 1, mj = (nj - 1) * jrho + 1, mk = (nk - 1) * krho + 1;
   // offsets from (i2, j2, k2); axes behind the phase's own are still coarse
   for_box(bp, [&](int fi, int fj, int fk) {
@@ -301,11 +302,14 @@ __device__ __forceinline__ bool anchor_ex(const T *v, long long i10, long long n
 #undef LC
 }
 
-template <typename T, int AX>
+// R2: all ratios are 2, as between PAMR's levels; the divisions by them are
+// then shifts (six a point; 161 x 97 x 129: 28 + 15 + 11 -> 21 + 14 + 9 us).
+template <typename T, int AX, bool R2>
 __global__ __launch_bounds__(NT) void k_interp_ex2(T *u2, const T *chr1, T ex, int nx1, int ny1, int nx2, int ny2,
                                                    int nz2, int i1, int j1, int k1, int i2, int j2, int k2, int ni,
                                                    int nj, int nk, int si1, int sj1, int sk1, int irho, int jrho,
                                                    int krho, BoxPts bp) {
+  if (R2) irho = jrho = krho = 2;
   const int mi = (ni - 1) * irho + 1, mj = (nj - 1) * jrho + 1, mk = (nk - 1) * krho + 1;
   for_box(bp, [&](int fi, int fj, int fk) {
     if (AX < 1) fj *= jrho;
@@ -495,14 +499,15 @@ int pmg_dminterp3d(double *u1, double *u2, int nx1, int ny1, int nz1, int nx2, i
   }
   if (ni < 1 || nj < 1 || nk < 1) return 0;
   const int mi = (ni - 1) * irho + 1, mj = (nj - 1) * jrho + 1, mk = (nk - 1) * krho + 1;
+  const bool r2 = irho == 2 && jrho == 2 && krho == 2;
   if (ord == 4 && do_ex != 1) {
     int rc = pmg_dmcopy3d(u1, u2, nx1, ny1, nz1, nx2, ny2, nz2, i1, j1, k1, i2, j2, k2, ni, nj, nk, si1, sj1, sk1,
                           irho, jrho, krho, stream);
     if (rc) return rc;
 #define PMG_I4(AX, M1, M2)                                                                                         \
   box_launch(mi, M1, M2, [&](dim3 grid, const BoxPts &b) {                                                         \
-    hipLaunchKernelGGL(k_interp4<AX>, grid, dim3(NT), 0, stream, u2, nx2, ny2, nz2, i2, j2, k2, ni, nj, nk, irho, \
-                       jrho, krho, b);                                                                             \
+    hipLaunchKernelGGL((r2 ? k_interp4<AX, true> : k_interp4<AX, false>), grid, dim3(NT), 0, stream, u2, nx2, ny2, \
+                       nz2, i2, j2, k2, ni, nj, nk, irho, jrho, krho, b);                                          \
   })
     if ((rc = PMG_I4(0, nj, nk)) || (nj == 1 && nk == 1)) return rc;
     if ((rc = PMG_I4(1, mj, nk)) || nk == 1) return rc;
@@ -510,7 +515,6 @@ int pmg_dminterp3d(double *u1, double *u2, int nx1, int ny1, int nz1, int nx2, i
 #undef PMG_I4
   }
   if (do_ex != 1) {
-    const bool r2 = irho == 2 && jrho == 2 && krho == 2;
     return box_launch(mi, mj, mk, [&](dim3 grid, const BoxPts &b) {
       hipLaunchKernelGGL((r2 ? k_interp3d<double, true> : k_interp3d<double, false>), grid, dim3(NT), 0, stream, u1, u2,
                          nx1, ny1, nx2, ny2, i1, j1, k1, i2, j2, k2, ni, nj, nk, si1, sj1, sk1, irho, jrho, krho, b);
@@ -524,8 +528,9 @@ int pmg_dminterp3d(double *u1, double *u2, int nx1, int ny1, int nz1, int nx2, i
   if (ord == 2) {
 #define PMG_IX2(AX, M1, M2)                                                                                            \
   box_launch(mi, M1, M2, [&](dim3 grid, const BoxPts &b) {                                                             \
-    hipLaunchKernelGGL((k_interp_ex2<double, AX>), grid, dim3(NT), 0, stream, u2, chr1, ex, nx1, ny1, nx2, ny2, nz2,  \
-                       i1, j1, k1, i2, j2, k2, ni, nj, nk, si1, sj1, sk1, irho, jrho, krho, b);                        \
+    hipLaunchKernelGGL((r2 ? k_interp_ex2<double, AX, true> : k_interp_ex2<double, AX, false>), grid, dim3(NT), 0,    \
+                       stream, u2, chr1, ex, nx1, ny1, nx2, ny2, nz2, i1, j1, k1, i2, j2, k2, ni, nj, nk, si1, sj1,   \
+                       sk1, irho, jrho, krho, b);                                                                      \
   })
     if ((rc = PMG_IX2(0, nj, nk)) || (nj == 1 && nk == 1)) return rc;
     if ((rc = PMG_IX2(1, mj, nk)) || nk == 1) return rc;
