@@ -41,6 +41,9 @@ struct SweepP {
   // FP32 only: u is zero everywhere, uin one element holding 0 -- a correction
   // cycle's first sweep neither reads its guess nor needs it cleared
   bool zero = false;
+  // u's new values go past the caches: set where the arrays of a sweep do not fit
+  // the 256 MB behind the L2 (stream_stores)
+  bool nt = false;
 };
 
 // The variable-coefficient sweep keeps the coefficient a in an LDS ring of
@@ -282,7 +285,15 @@ __device__ __forceinline__ void sweep_tile(const SweepP<T> &P, int x0, int y0, i
     for (int m = 0; m < NST; m++)
       if (st[m]) {
         asm volatile("" : "+v"(go[m]));
-        *reinterpret_cast<T *>(out + go[m]) = L(lu, slot * PL * B + ls[m]);
+        T *const to = reinterpret_cast<T *>(out + go[m]);
+        const T v = L(lu, slot * PL * B + ls[m]);
+        if (P.nt) {  // the asms: or the two stores become one, without the hint
+          asm volatile("");
+          __builtin_nontemporal_store(v, to);
+          asm volatile("");
+        } else {
+          *to = v;
+        }
       }
   };
 

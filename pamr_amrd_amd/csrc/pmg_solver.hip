@@ -356,6 +356,18 @@ void default_sweep(const int *n, int op, int pi, int *variant, int *zchunk) {
   *zchunk = z;
 }
 
+// Whether a sweep's stores bypass the caches: where its arrays (u twice, rho, rhs,
+// a, c) exceed the 256 MB behind the L2, a line it writes is gone before the next
+// kernel reads it, and in the L2 it pushes out the rows neighbouring tiles
+// share.  257^3 FP64 (407 MB) 84.7 -> 82.2 us, and the residual that follows
+// 92.5 -> 85.4; 513^3 FP32 421 -> 398; where they fit, streaming every store cost
+// the next kernel its hits: the 257^3 FP32 cycles (204 MB) 2 %.  The residual's
+// stores and the loads of rho lost by it at any size.
+template <typename T>
+bool stream_stores(const pmg_solver *S, const Level &Lv, bool rhs0) {
+  return Lv.size * sizeof(T) * (3 + (rhs0 ? 0 : 1) + (S->op == 1 ? 2 : 0)) > (size_t)256 << 20;
+}
+
 // n red-black sweeps on level L (ping-pong u <-> ua; odd counts copy back)
 // zero: u counts as zero, whatever its buffer holds (can_sweep_zero)
 template <typename T>
@@ -376,6 +388,7 @@ int sweeps(pmg_solver *S, int L, int n, int slot, bool rhs0, bool zero = false) 
   P.sp = spacing<T>(Lv);
   P.ws = S->ws;
   P.slot = slot;
+  P.nt = stream_stores<T>(S, Lv, rhs0);
   const bool p2 = P.sp.pow2 != 0;
   const bool two = use_sweep2(S, Lv);
   int done = 0, launches = 0;
