@@ -189,10 +189,11 @@ int pmg_set_level_sweep_config(pmg_solver *S, int L, int variant, int zchunk);
 int pmg_set_level_sweep_config_prec(pmg_solver *S, int L, int prec, int variant, int zchunk);
 int pmg_num_sweep_variants(void);
 int pmg_set_graph(pmg_solver *S, int on);
-/* run the small bottom levels (all dimensions <= 17 points, below the
- * finest level, no excision) as one single-workgroup kernel (default on);
- * on = 0 off, 1 the default, 2..17 the largest side fused (9: only the
- * levels of 9 points and below); results are identical either way */
+/* run the small bottom levels (below the finest level, no excision) as one
+ * single-workgroup kernel (default on); on = 0 off, 1 the default -- levels
+ * of at most 9 points a side in V(2,2) cycles, whose larger levels take one
+ * launch a leg, of 17 otherwise and where an FP32 cycle solves a 17^3 level
+ * exactly --, 2..17 the largest side fused; results are identical either way */
 int pmg_set_bottom_fusion(pmg_solver *S, int on);
 /* keep every array of the fused bottom levels in LDS for the whole bottom V
  * when they fit in one workgroup's LDS (on = 1, the default) or run it from
@@ -222,8 +223,8 @@ int pmg_set_restrict_fusion(pmg_solver *S, int on);
  * workspace holds (small values on large grids) */
 int pmg_set_resid_restrict_zchunk(pmg_solver *S, int prec, int czchunk);
 /* run pairs of red-black sweeps on levels of at least 65 points per side as
- * one temporally blocked pass (default off: at 257^3 a pair takes 0.26 ms
- * against 2 x 0.11 ms for single sweeps; zchunk > 0 sets its z depth);
+ * one temporally blocked pass (default off: at 257^3 a pair takes 0.23 ms
+ * against 2 x 0.08 ms for single sweeps; zchunk > 0 sets its z depth);
  * results are identical either way */
 int pmg_set_sweep_blocking(pmg_solver *S, int on, int zchunk);
 void *pmg_stream(pmg_solver *S);
