@@ -66,20 +66,24 @@ __device__ __forceinline__ bool hook_on(const double *cmask, const double *chr, 
 }
 
 // The hooks' points: the interior box -- for a colour pass the points of its
-// colour, (mi + 1) / 2 places a row -- by one linear index, kPPT places per
-// thread a block's width apart.  With 64-bit divisions for the index and, in a
+// colour, (mi + 1) / 2 places a row -- by one linear index, per thread `ppt`
+// places a block's width apart.  With 64-bit divisions for the index and, in a
 // colour pass, half of the lanes idle, the kernels waited on arithmetic; now on
 // memory (seven arrays read: 3.9 TB/s).  At 150 x 121 x 97 with op 1: a colour
 // pass 32.6 -> 28.6 us, the residual 29.2 -> 27.9, the operator 26.5 -> 25.2,
 // the fold of a quarter of the partials 6.5 -> 4.8.
-constexpr int kPPT = 2;
+constexpr int kTwoFrom = 4 * 256 * 2 * NT;
+// places a thread takes: two where that still makes four blocks a CU, for half
+// of the partial norms; one below, where a thread's second place waits for its
+// first (two sweeps, the residual and the operator on 97 x 65 x 80 points 59 us
+// against 62, 60 x 50 x 40 35 against 40)
+inline int hook_ppt(int ni, int nj, int nk) { return (long long)ni * nj * nk >= kTwoFrom ? 2 : 1; }
 static_assert(NT == kPtsThreads);
 template <typename F>
-__device__ __forceinline__ void hook_points(const BoxPts &b, const F &f) {
-#pragma unroll
-  for (int r = 0; r < kPPT; r++) {
-    const unsigned q = (blockIdx.x * kPPT + r) * NT + threadIdx.x;
-    if (q >= (unsigned)b.n) continue;
+__device__ __forceinline__ void hook_points(const BoxPts &b, int ppt, const F &f) {
+  for (int r = 0; r < ppt; r++) {
+    const unsigned q = (blockIdx.x * ppt + r) * NT + threadIdx.x;
+    if (q >= (unsigned)b.n) return;
     int i, j;
     const int t = b.di.div((int)q, i), k = b.dj.div(t, j);
     f(i + 1, j + b.j0 + 1, k + b.k0 + 1);
@@ -94,9 +98,9 @@ __global__ __launch_bounds__(NT) void k_hook_relax_pass(double *V, const double 
                                                         const double *c, const double *cmask,
                                                         const double *chr, double ex, HookGeom g,
                                                         Spacing<double> sp, int pass, NormWs ws,
-                                                        BoxPts b, int bid0, int nb) {
+                                                        BoxPts b, int ppt, int bid0, int nb) {
   double s = 0.0, cnt = 0.0;
-  hook_points(b, [&](int h, int j, int k) {
+  hook_points(b, ppt, [&](int h, int j, int k) {
     const int i = 2 * h - 1 + ((j + k + pass) & 1);  // i + j + k + pass odd, 0-based
     if (i > g.nx - 2) return;
     const size_t p = ix3(i, j, k, g.nx, g.ny);
@@ -114,8 +118,8 @@ template <int OP, bool P2>
 __global__ __launch_bounds__(NT) void k_hook_lop(double *LV, const double *V, const double *rho,
                                                  const double *a, const double *c,
                                                  const double *cmask, const double *chr,
-                                                 double ex, HookGeom g, Spacing<double> sp, BoxPts b) {
-  hook_points(b, [&](int i, int j, int k) {
+                                                 double ex, HookGeom g, Spacing<double> sp, BoxPts b, int ppt) {
+  hook_points(b, ppt, [&](int i, int j, int k) {
     const size_t p = ix3(i, j, k, g.nx, g.ny);
     if (hook_on(cmask, chr, ex, p)) LV[p] = lop_at<double, OP, P2>(V, rho, a, c, p, g.sy, g.sz, sp, nullptr);
   });
@@ -128,9 +132,9 @@ __global__ __launch_bounds__(NT) void k_hook_residual(double *res, const double 
                                                       const double *a, const double *c,
                                                       const double *cmask, const double *chr,
                                                       double ex, HookGeom g, Spacing<double> sp,
-                                                      NormWs ws, BoxPts b, int bid0, int nb) {
+                                                      NormWs ws, BoxPts b, int ppt, int bid0, int nb) {
   double s = 0.0, cnt = 0.0;
-  hook_points(b, [&](int i, int j, int k) {
+  hook_points(b, ppt, [&](int i, int j, int k) {
     const size_t p = ix3(i, j, k, g.nx, g.ny);
     if (!hook_on(cmask, chr, ex, p)) return;
     const double r = lop_at<double, OP, P2>(V, rho, a, c, p, g.sy, g.sz, sp, nullptr) - rhs[p];
@@ -183,22 +187,23 @@ int ensure_ws(int nb) {
   return 0;
 }
 
-// launch(grid, points, first block) over an ni x nj x nk box in blocks of
-// kPPT * NT places
+// launch(grid, points, places a thread, first block) over an ni x nj x nk box
 template <typename L>
 int hook_launch(int ni, int nj, int nk, const L &launch) {
+  const int ppt = hook_ppt(ni, nj, nk);
   int bid0 = 0;
   box_slabs(ni, nj, nk, [&](const BoxPts &b) {
-    const int nb = (int)(((long long)b.n + kPPT * NT - 1) / (kPPT * NT));
-    launch(dim3(nb), b, bid0);
+    const int nb = (int)(((long long)b.n + ppt * NT - 1) / (ppt * NT));
+    launch(dim3(nb), b, ppt, bid0);
     bid0 += nb;
   });
   PMG_HOST_CHECK(hipGetLastError());
   return 0;
 }
 int hook_blocks(int ni, int nj, int nk) {
+  const int ppt = hook_ppt(ni, nj, nk);
   int nb = 0;
-  box_slabs(ni, nj, nk, [&](const BoxPts &b) { nb += (int)(((long long)b.n + kPPT * NT - 1) / (kPPT * NT)); });
+  box_slabs(ni, nj, nk, [&](const BoxPts &b) { nb += (int)(((long long)b.n + ppt * NT - 1) / (ppt * NT)); });
   return nb;
 }
 
@@ -208,10 +213,10 @@ int relax_launch(int op, double *V, const double *rhs, const double *rho, const 
                  const double *cmask, const double *chr, double ex, const HookGeom &g, const Spacing<double> &sp,
                  int nb, NormWs ws, double *norm_dev, hipStream_t stream) {
   for (int pass = 0; pass <= 1; pass++) {
-    if (hook_launch((g.nx - 1) / 2, g.ny - 2, g.nz - 2, [&](dim3 grid, const BoxPts &b, int bid0) {
+    if (hook_launch((g.nx - 1) / 2, g.ny - 2, g.nz - 2, [&](dim3 grid, const BoxPts &b, int ppt, int bid0) {
 #define PMG_HR(OPV, P2V)                                                                      \
   hipLaunchKernelGGL((k_hook_relax_pass<OPV, P2V>), grid, dim3(NT), 0, stream, V, rhs, rho, \
-                     a, c, cmask, chr, ex, g, sp, pass, ws, b, bid0, nb)
+                     a, c, cmask, chr, ex, g, sp, pass, ws, b, ppt, bid0, nb)
           if (op == 0) { if (sp.pow2) PMG_HR(0, true); else PMG_HR(0, false); }
           else { if (sp.pow2) PMG_HR(1, true); else PMG_HR(1, false); }
 #undef PMG_HR
@@ -259,8 +264,7 @@ int pmg_hook_relax_noalloc(int op, double *V, const double *rhs, const double *r
   NormWs ws{base, reinterpret_cast<int *>(base + kScratchPartials), kScratchBlocks, 2};
   HookGeom g{nx, ny, nz, (size_t)nx, (size_t)nx * ny};
   Spacing<double> sp = make_spacing(dx, dy, dz);
-  // (one place a row more than half of its points, kPPT places a thread: never more
-  // blocks than that)
+  // (a colour's places a row are at most its points: never more blocks than that)
   const int nb = hook_blocks((nx - 1) / 2, ny - 2, nz - 2);
   return relax_launch(op, V, rhs, rho, a, c, cmask, chr, ex, g, sp, nb, ws, norm_dev, stream);
 }
@@ -275,10 +279,10 @@ int pmg_hook_residual(int op, double *res, const double *rhs, const double *V, c
   Spacing<double> sp = make_spacing(dx, dy, dz);
   const int nb = hook_blocks(nx - 2, ny - 2, nz - 2);
   if (ensure_ws(nb)) return -1;
-  if (hook_launch(nx - 2, ny - 2, nz - 2, [&](dim3 grid, const BoxPts &b, int bid0) {
+  if (hook_launch(nx - 2, ny - 2, nz - 2, [&](dim3 grid, const BoxPts &b, int ppt, int bid0) {
 #define PMG_HS(OPV, P2V)                                                                    \
   hipLaunchKernelGGL((k_hook_residual<OPV, P2V>), grid, dim3(NT), 0, stream, res, rhs, V, \
-                     rho, a, c, cmask, chr, ex, g, sp, g_ws, b, bid0, nb)
+                     rho, a, c, cmask, chr, ex, g, sp, g_ws, b, ppt, bid0, nb)
         if (op == 0) { if (sp.pow2) PMG_HS(0, true); else PMG_HS(0, false); }
         else { if (sp.pow2) PMG_HS(1, true); else PMG_HS(1, false); }
 #undef PMG_HS
@@ -298,10 +302,10 @@ int pmg_hook_lop(int op, double *LV, const double *V, const double *rho, const d
   if (op == 1 && (!a || !c)) return -1;
   HookGeom g{nx, ny, nz, (size_t)nx, (size_t)nx * ny};
   Spacing<double> sp = make_spacing(dx, dy, dz);
-  return hook_launch(nx - 2, ny - 2, nz - 2, [&](dim3 grid, const BoxPts &b, int) {
+  return hook_launch(nx - 2, ny - 2, nz - 2, [&](dim3 grid, const BoxPts &b, int ppt, int) {
 #define PMG_HL(OPV, P2V)                                                                \
   hipLaunchKernelGGL((k_hook_lop<OPV, P2V>), grid, dim3(NT), 0, stream, LV, V, rho, a, \
-                     c, cmask, chr, ex, g, sp, b)
+                     c, cmask, chr, ex, g, sp, b, ppt)
     if (op == 0) { if (sp.pow2) PMG_HL(0, true); else PMG_HL(0, false); }
     else { if (sp.pow2) PMG_HL(1, true); else PMG_HL(1, false); }
 #undef PMG_HL

@@ -1,7 +1,8 @@
 """The application hooks over the grids where their index can go wrong: one
 interior point, rows of one point, even and odd rows (the colours then hold
-different counts), sizes around one block's places, no point active -- grid
-functions bit for bit against the oracle."""
+different counts), sizes around one block's places and around the change from
+one to two places a thread, no point active -- grid functions bit for bit
+against the oracle."""
 import numpy as np
 import pytest
 
@@ -12,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("shape", [(3, 3, 3), (4, 3, 3), (3, 40, 3), (3, 3, 1030), (514, 3, 3), (515, 4, 3),
-                                   (1027, 3, 4), (10, 66, 4), (67, 18, 34)])
+                                   (1027, 3, 4), (10, 66, 4), (67, 18, 34), (130, 66, 66),
+                                   (263, 67, 66)])
 @pytest.mark.parametrize("op,on", [(0, 1.0), (1, 0.7), (1, 0.0)])
 def test_hook_forms(torch_cuda, shape, op, on):
     torch = torch_cuda
