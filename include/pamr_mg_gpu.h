@@ -356,7 +356,8 @@ int pmg_band_sample(pmg_solver *S, const double *ustar, double xs, double ts, in
  * preconditioner form (FP32 u against the FP32 source) */
 int pmg_band_correct(pmg_solver *S, int which);
 /* FP32 arrays of the mixed-precision cycles: which 0 u, 1 rho (the source),
- * 2 rhs, 3 res, 4 lop (download); 0 and 1 (upload) */
+ * 2 rhs, 3 res, 4 lop (download); 0 and 1 (upload).  Solves start their
+ * cycles from zero whatever was uploaded as u */
 int pmg_download32(pmg_solver *S, int L, int which, float *host);
 int pmg_upload32(pmg_solver *S, int L, int which, const float *host);
 /* weighted forms of pmg_net_loss_grad / pmg_net_train_step: the mean runs

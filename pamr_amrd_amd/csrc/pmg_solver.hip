@@ -150,6 +150,7 @@ struct pmg_solver {
   int sweep2_zchunk = 32;
   hipGraphExec_t g64 = nullptr;   // captured FP64 V-cycle
   float *zero32 = nullptr;        // one element, 0: the FP32 cycles' initial guess
+  bool corr_faces = false;        // the finest FP32 u may hold nonzero face values (see ready32)
   hipGraphExec_t g32 = nullptr;   // captured mixed-precision outer iteration
   bool fp32_ready = false;
   int last_citer = 0;
@@ -1161,6 +1162,19 @@ int ensure_fp32(pmg_solver *S) {
   return 0;
 }
 
+// Before FP32 cycles that start from zero: they clear no face of the finest u
+// (can_sweep_zero), so what an upload may have left there goes now.
+int ready32(pmg_solver *S) {
+  if (ensure_fp32(S)) return -1;
+  if (!S->corr_faces) return 0;
+  Level &F = S->lev[S->nlev - 1];
+  for (float *p : {F.f.u, F.f.ua})
+    hipLaunchKernelGGL(k_fill<float>, dim3(nblk256(F.size)), dim3(256), 0, S->stream, p, 0.0f, F.size);
+  PMG_HOST_CHECK(hipGetLastError());
+  S->corr_faces = false;
+  return 0;
+}
+
 // The learned band correction of the defect-correction iteration: on entry
 // the FP32 source of the finest level holds -r and d_norms[NS_OUTER] its
 // RMS norm; u += ts * ||r|| * N(r / ||r||) at the band points, then -r is
@@ -1683,7 +1697,7 @@ int pmg_solve_rel(pmg_solver *S, int mode, double rtol, int max_iter, double *hi
   if (mode == 1 || mode == 2 || mode == 3) {
     // the FP64 defect of the initial u: its norm is r0 and, in FP32, it is
     // the source of the first inner cycle
-    if ((rc = ensure_fp32(S))) return rc;
+    if ((rc = ready32(S))) return rc;
     Level &F = S->lev[S->nlev - 1];
     if ((rc = residual<double>(S, S->nlev, NS_OUTER, true, true, F.f.rho))) return rc;
     if ((rc = fold_norms(S, NS_OUTER, 1))) return rc;
@@ -2409,7 +2423,7 @@ extern "C" {
 int pmg_solve_fgmres(pmg_solver *S, int m, double rtol, int max_iter, double *hist, int *iters, double *r0_out) {
   if (!S || m < 1 || m > kKryMax - 1 || max_iter < 0) return -1;
   int rc;
-  if ((rc = ensure_fp32(S))) return rc;
+  if ((rc = ready32(S))) return rc;
   if ((rc = ensure_krylov(S, m))) return rc;
   Level &F = S->lev[S->nlev - 1];
   const size_t n = F.size;
@@ -2761,6 +2775,7 @@ int pmg_band_sample_inner(pmg_solver *S, const double *ustar, int ncrop, unsigne
   if (!S || !ustar || !x || !t || !w || ncrop < 1 || !S->fp32_ready) return -1;
   auto &B = S->band;
   if (B.h_pts.empty()) return -1;
+  if (ready32(S)) return -1;
   Level &F = S->lev[S->nlev - 1];
   const int nx = F.n[0], ny = F.n[1];
   std::vector<int> org(3 * (size_t)ncrop);
@@ -2899,6 +2914,7 @@ int pmg_upload32(pmg_solver *S, int L, int which, const float *host) {
     case 1: dst = Lv.f.rho; break;
     default: return -1;
   }
+  if (which == 0 && L == S->nlev) S->corr_faces = true;
   PMG_HOST_CHECK(hipMemcpyAsync(dst, host, Lv.size * sizeof(float), hipMemcpyHostToDevice, S->stream));
   PMG_HOST_CHECK(hipStreamSynchronize(S->stream));
   return 0;
