@@ -151,6 +151,7 @@ struct pmg_solver {
   hipGraphExec_t g64 = nullptr;   // captured FP64 V-cycle
   float *zero32 = nullptr;        // one element, 0: the FP32 cycles' initial guess
   bool corr_faces = false;        // the finest FP32 u may hold nonzero face values (see ready32)
+  bool corr_spent = false;        // the finest FP32 u holds a correction already added: it counts as 0
   hipGraphExec_t g32 = nullptr;   // captured mixed-precision outer iteration
   bool fp32_ready = false;
   int last_citer = 0;
@@ -1140,6 +1141,11 @@ int enq_mixed(pmg_solver *S) {
   return fold_norms(S, 0, 2 * kNormSlots);
 }
 
+int run_mixed(pmg_solver *S, hipGraphExec_t *cache, int (*enq)(pmg_solver *)) {
+  S->corr_spent = true;
+  return capture_or_run(S, cache, enq);
+}
+
 int ensure_fp32(pmg_solver *S) {
   if (S->fp32_ready) return 0;
   if (!S->zero32) {
@@ -1172,6 +1178,18 @@ int ready32(pmg_solver *S) {
     hipLaunchKernelGGL(k_fill<float>, dim3(nblk256(F.size)), dim3(256), 0, S->stream, p, 0.0f, F.size);
   PMG_HOST_CHECK(hipGetLastError());
   S->corr_faces = false;
+  return 0;
+}
+
+// For readers of the finest FP32 u between solves: a mixed iteration leaves
+// there the correction it has added (the next one starts from zero without
+// reading it), which is cleared when somebody looks.
+int settle_corr(pmg_solver *S) {
+  if (!S->corr_spent) return 0;
+  Level &F = S->lev[S->nlev - 1];
+  hipLaunchKernelGGL(k_fill<float>, dim3(nblk256(F.size)), dim3(256), 0, S->stream, ucur<float>(F), 0.0f, F.size);
+  PMG_HOST_CHECK(hipGetLastError());
+  S->corr_spent = false;
   return 0;
 }
 
@@ -1720,7 +1738,7 @@ int pmg_solve_rel(pmg_solver *S, int mode, double rtol, int max_iter, double *hi
     }
   } else if (mode == 1) {
     while (it < max_iter && r > rtol * r0) {
-      if ((rc = capture_or_run(S, &S->g32, enq_mixed))) return rc;
+      if ((rc = run_mixed(S, &S->g32, enq_mixed))) return rc;
       PMG_HOST_CHECK(hipMemcpyAsync(S->h_pinned, S->d_norms + NS_OUTER, sizeof(double), hipMemcpyDeviceToHost, S->stream));
       PMG_HOST_CHECK(hipStreamSynchronize(S->stream));
       r = S->h_pinned[0];
@@ -1789,7 +1807,7 @@ int pmg_solve_rel(pmg_solver *S, int mode, double rtol, int max_iter, double *hi
         S->net_retry_period = std::min(2 * S->net_retry_period, 1280);
       }
       PMG_HOST_CHECK(hipEventRecord(e0, S->stream));
-      if ((rc = capture_or_run(S, &S->g32, enq_mixed))) return rc;
+      if ((rc = run_mixed(S, &S->g32, enq_mixed))) return rc;
       PMG_HOST_CHECK(hipEventRecord(e1, S->stream));
       double rn;
       if ((rc = read_outer(&rn))) return rc;
@@ -1826,10 +1844,10 @@ int pmg_solve_rel(pmg_solver *S, int mode, double rtol, int max_iter, double *hi
       else fresh = !S->g32;
       PMG_HOST_CHECK(hipEventRecord(ev.e0, S->stream));
       if (with_net && B.inner) {
-        if ((rc = capture_or_run(S, &B.g32i, enq_mixed_inner))) return rc;
+        if ((rc = run_mixed(S, &B.g32i, enq_mixed_inner))) return rc;
       } else {
         if (with_net && (rc = capture_or_run(S, &B.gdc, enq_band_dc))) return rc;
-        if ((rc = capture_or_run(S, &S->g32, enq_mixed))) return rc;
+        if ((rc = run_mixed(S, &S->g32, enq_mixed))) return rc;
       }
       PMG_HOST_CHECK(hipEventRecord(ev.e1, S->stream));
       PMG_HOST_CHECK(hipMemcpyAsync(S->h_pinned, S->d_norms + NS_OUTER, sizeof(double), hipMemcpyDeviceToHost,
@@ -2487,6 +2505,7 @@ int pmg_solve_fgmres(pmg_solver *S, int m, double rtol, int max_iter, double *hi
     for (int j = 0; j < m && it < max_iter; j++) {
       // V_j normalised, and Z_j = M V_j: the FP32 V-cycle from zero with V_j as
       // its source
+      S->corr_spent = false;
       hipLaunchKernelGGL(k_kry_next, dim3(nb), dim3(256), 0, S->stream, V[j], j == 0 ? w : V[j], next, F.f.rho, n);
       PMG_HOST_CHECK(hipGetLastError());
       // prec_cycles FP32 V-cycles on the source V_j, the first from zero;
@@ -2605,6 +2624,7 @@ int pmg_time_kernel(pmg_solver *S, int which, int L, int prec, int nrep, double 
   // to its buffer), 1 = residual.  prec: 0 FP64, 1 FP32.
   if (!S || L < 1 || L > S->nlev || nrep < 2 || !ms_avg) return -1;
   if (prec == 1 && ensure_fp32(S)) return -1;
+  if (prec == 1 && L == S->nlev && settle_corr(S)) return -1;
   if (which == 3) {
     // the finest FP64 sweep inside nrep ungraphed V-cycles: events around
     // each pre- and post-smoothing group, the average per launch
@@ -2802,6 +2822,7 @@ int pmg_band_sample_inner(pmg_solver *S, const double *ustar, int ncrop, unsigne
   B.samp_w = w;
   B.enq_inner = true;
   B.cur_norm = S->d_norms + NS_OUTER;
+  S->corr_spent = true;
   int rc = enq_mixed(S);
   B.enq_inner = false;
   B.samp_x = B.samp_t = B.samp_w = nullptr;
@@ -2880,6 +2901,7 @@ int pmg_band_correct(pmg_solver *S, int which) {
   auto &B = S->band;
   int rc;
   if ((rc = pmg_net_reserve(B.net, (long long)B.ncore * B.side * B.side * B.side))) return rc;
+  if (which != 0 && (rc = settle_corr(S))) return rc;
   rc = which == 0 ? enq_band_dc(S) : enq_band_pc(S);
   if (rc) return rc;
   PMG_HOST_CHECK(hipStreamSynchronize(S->stream));
@@ -2889,6 +2911,7 @@ int pmg_band_correct(pmg_solver *S, int which) {
 // FP32 arrays of a level (mixed precision): which as pmg_field (u, rho, rhs, res, lop)
 int pmg_download32(pmg_solver *S, int L, int which, float *host) {
   if (!S || L < 1 || L > S->nlev || !host || !S->fp32_ready) return -1;
+  if (which == 0 && L == S->nlev && settle_corr(S)) return -1;
   Level &Lv = S->lev[L - 1];
   const float *src = nullptr;
   switch (which) {
@@ -2914,7 +2937,10 @@ int pmg_upload32(pmg_solver *S, int L, int which, const float *host) {
     case 1: dst = Lv.f.rho; break;
     default: return -1;
   }
-  if (which == 0 && L == S->nlev) S->corr_faces = true;
+  if (which == 0 && L == S->nlev) {
+    S->corr_faces = true;
+    S->corr_spent = false;
+  }
   PMG_HOST_CHECK(hipMemcpyAsync(dst, host, Lv.size * sizeof(float), hipMemcpyHostToDevice, S->stream));
   PMG_HOST_CHECK(hipStreamSynchronize(S->stream));
   return 0;

@@ -44,3 +44,18 @@ def test_uploaded_correction_is_not_a_guess(torch_cuda, n, op, fgmres):
         S.close()
     assert np.array_equal(out[0][1], out[1][1])
     assert np.array_equal(out[0][0], out[1][0])
+
+
+@pytest.mark.parametrize("n", [33, 81])
+def test_correction_reads_as_zero_once_added(torch_cuda, n):
+    """a mixed iteration's correction belongs to the FP64 u; what FGMRES's
+    preconditioner returned last stays readable until the next cycle"""
+    print(f"case u32 after solves n={n}", flush=True)
+    S = solver(n, 0)
+    solve(S, False)
+    assert not S.download32(S.nlev, 0).any()
+    solve(S, True)
+    z = S.download32(S.nlev, 0)
+    assert z.any()
+    assert np.array_equal(S.download32(S.nlev, 0), z)
+    S.close()
