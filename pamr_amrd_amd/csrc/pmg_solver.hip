@@ -1169,15 +1169,20 @@ int ensure_fp32(pmg_solver *S) {
 }
 
 // Before FP32 cycles that start from zero: they clear no face of the finest u
-// (can_sweep_zero), so what an upload may have left there goes now.
+// (can_sweep_zero), so what an upload or a weight w0_i that divides a face's 0
+// into a NaN may have left there goes now.
 int ready32(pmg_solver *S) {
   if (ensure_fp32(S)) return -1;
-  if (!S->corr_faces) return 0;
+  const bool nan_faces = !(0.0f / (float)S->w0_i == 0.0f);
+  if (!S->corr_faces) {
+    S->corr_faces = nan_faces;
+    return 0;
+  }
   Level &F = S->lev[S->nlev - 1];
   for (float *p : {F.f.u, F.f.ua})
     hipLaunchKernelGGL(k_fill<float>, dim3(nblk256(F.size)), dim3(256), 0, S->stream, p, 0.0f, F.size);
   PMG_HOST_CHECK(hipGetLastError());
-  S->corr_faces = false;
+  S->corr_faces = nan_faces;
   return 0;
 }
 
@@ -1446,11 +1451,6 @@ int pmg_set_params(pmg_solver *S, int pre, int pst, int max_citer, double crtol,
   S->w0_r = w0_r; S->w0_i = w0_i; S->rop_u = rop_u; S->rop_res = rop_res; S->rop_src = rop_src;
   S->iord = interp_ord;
   invalidate_graphs(S);
-  // weights that are no numbers may have left some on the faces of the FP32
-  // correction, which are not cleared otherwise
-  Level &F = S->lev[S->nlev - 1];
-  for (float *p : {F.f.u, F.f.ua})
-    if (p) PMG_HOST_CHECK(hipMemsetAsync(p, 0, F.size * sizeof(float), S->stream));
   return 0;
 }
 

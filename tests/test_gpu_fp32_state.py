@@ -59,3 +59,32 @@ def test_correction_reads_as_zero_once_added(torch_cuda, n):
     assert z.any()
     assert np.array_equal(S.download32(S.nlev, 0), z)
     S.close()
+
+
+def test_set_params_leaves_the_correction(torch_cuda):
+    print("case u32 after set_params", flush=True)
+    S = solver(81, 0)
+    solve(S, True)
+    z = S.download32(S.nlev, 0)
+    S.set_params(pre=2, pst=2)
+    assert z.any() and np.array_equal(S.download32(S.nlev, 0), z)
+    S.close()
+
+
+@pytest.mark.parametrize("fgmres", [False, True])
+@pytest.mark.parametrize("w0_i", [0.0, float("nan")])
+def test_solve_after_weights_that_give_nan(torch_cuda, w0_i, fgmres):
+    """faces of the correction are 0 / w0_i: what a solve with such a weight
+    leaves there is gone when the weight is a number again"""
+    print(f"case w0_i={w0_i} fgmres={fgmres}", flush=True)
+    out = []
+    for bad in (False, True):
+        S = solver(81, 0)
+        if bad:
+            S.set_params(pre=2, pst=2, w0_i=w0_i)
+            S.solve_rel(1, 1e-9, 2)
+            S.set_params(pre=2, pst=2)
+        out.append(solve(S, fgmres))
+        S.close()
+    assert np.array_equal(out[0][1], out[1][1])
+    assert np.array_equal(out[0][0], out[1][0])
