@@ -204,19 +204,24 @@ __global__ __launch_bounds__(256) void k_conv16_tile(const uint16_t *__restrict_
   const uint16_t *Xb = X + (size_t)T.b * box * NC;
   const int lane = threadIdx.x & 63, w = wave_ix(), m = lane & 15, grp = lane >> 4;
   uint4 reg[CLOAD];
-  int off[CLOAD];  // element offset of this thread's chunks within a plane, or -1
+  // element offset of this thread's chunks within a plane (64 bits: a plane of 16
+  // channels may hold more than 2^31 elements), 0 for those outside the box
+  size_t off[CLOAD];
+  unsigned in = 0;
 #pragma unroll
   for (int q = 0; q < CLOAD; q++) {
     const int idx = (int)threadIdx.x + q * 256;
     const int ly = idx / (CLX * 2), rem = idx % (CLX * 2), lx = rem >> 1, h = rem & 1;
     const int gx = x0 - 1 + lx, gy = y0 - 1 + ly;
-    off[q] = (idx < CCHUNK && gx >= 0 && gx < g.nx && gy >= 0 && gy < g.ny) ? (gy * g.nx + gx) * NC + 8 * h : -1;
+    const bool ok = idx < CCHUNK && gx >= 0 && gx < g.nx && gy >= 0 && gy < g.ny;
+    off[q] = ok ? ((size_t)gy * g.nx + gx) * NC + 8 * h : 0;
+    in |= (unsigned)ok << q;
   }
   const size_t plane = (size_t)g.nx * g.ny * NC;
   auto fetch = [&](int k) {
     const uint16_t *Xk = Xb + (k >= 0 && k < g.nz ? (size_t)k * plane : 0);
 #pragma unroll
-    for (int q = 0; q < CLOAD; q++) reg[q] = *(const uint4 *)(Xk + (off[q] < 0 ? 0 : off[q]));
+    for (int q = 0; q < CLOAD; q++) reg[q] = *(const uint4 *)(Xk + off[q]);
   };
   auto store = [&](int k) {
     uint4 *S = &sX[k & 3][0][0][0];
@@ -224,7 +229,7 @@ __global__ __launch_bounds__(256) void k_conv16_tile(const uint16_t *__restrict_
 #pragma unroll
     for (int q = 0; q < CLOAD; q++) {
       const int idx = (int)threadIdx.x + q * 256;
-      if (idx < CCHUNK) S[idx] = kin && off[q] >= 0 ? reg[q] : make_uint4(0u, 0u, 0u, 0u);
+      if (idx < CCHUNK) S[idx] = kin && ((in >> q) & 1) ? reg[q] : make_uint4(0u, 0u, 0u, 0u);
     }
   };
   // the 14 weight fragments stay in registers for the whole march
@@ -301,12 +306,16 @@ __global__ __launch_bounds__(256) void k_conv_in_tile(const TIN *__restrict__ x,
   const int lane = threadIdx.x & 63, w = wave_ix(), m = lane & 15, grp = lane >> 4;
   constexpr int NPT = CLY * CLX, NLD = (NPT + 255) / 256;
   TIN reg[NLD];
-  int off[NLD], lds[NLD];
+  size_t off[NLD];
+  unsigned in = 0;
+  int lds[NLD];
 #pragma unroll
   for (int q = 0; q < NLD; q++) {
     const int idx = (int)threadIdx.x + q * 256;
     const int ly = idx / CLX, lx = idx % CLX, gx = x0 - 1 + lx, gy = y0 - 1 + ly;
-    off[q] = (idx < NPT && gx >= 0 && gx < g.nx && gy >= 0 && gy < g.ny) ? gy * g.nx + gx : -1;
+    const bool ok = idx < NPT && gx >= 0 && gx < g.nx && gy >= 0 && gy < g.ny;
+    off[q] = ok ? (size_t)gy * g.nx + gx : 0;
+    in |= (unsigned)ok << q;
     lds[q] = idx < NPT ? ly * LXW + lx : -1;
   }
   for (int q = (int)threadIdx.x; q < 4 * (CLY + 1) * LXW; q += 256) (&sx[0][0][0])[q] = 0u;
@@ -315,7 +324,7 @@ __global__ __launch_bounds__(256) void k_conv_in_tile(const TIN *__restrict__ x,
   auto fetch = [&](int k) {
     const TIN *xk = xb + (k >= 0 && k < g.nz ? (size_t)k * plane : 0);
 #pragma unroll
-    for (int q = 0; q < NLD; q++) reg[q] = xk[off[q] < 0 ? 0 : off[q]];
+    for (int q = 0; q < NLD; q++) reg[q] = xk[off[q]];
   };
   auto store = [&](int k) {
     uint16_t *S = (uint16_t *)&sx[k & 3][0][0];
@@ -326,7 +335,7 @@ __global__ __launch_bounds__(256) void k_conv_in_tile(const TIN *__restrict__ x,
       uint16_t v;
       if constexpr (std::is_same<TIN, float>::value) v = (uint16_t)pk_bf16(reg[q] * scale, 0.f);
       else v = reg[q];
-      if (!(kin && off[q] >= 0)) v = 0;
+      if (!(kin && ((in >> q) & 1))) v = 0;
       S[2 * lds[q]] = v;                              // low half of its own word
       if (lds[q] % LXW > 0) S[2 * lds[q] - 1] = v;    // high half of the west neighbour's
     }
@@ -395,17 +404,20 @@ __global__ __launch_bounds__(256) void k_conv_out_tile(const uint16_t *__restric
   const int lane = threadIdx.x & 63, w = wave_ix(), m = lane & 15, grp = lane >> 4;
   // input segment s of this wave: 16 points of row (w * OSEG + s) / 2
   uint2 regA[OSEG], regB[OSEG];
-  int off[OSEG];
+  size_t off[OSEG];
+  unsigned in = 0;
 #pragma unroll
   for (int s = 0; s < OSEG; s++) {
     const int seg = w * OSEG + s, gy = T.y0 - 1 + seg / 2, gx = T.x0 - 1 + 16 * (seg & 1) + m;
-    off[s] = gx >= 0 && gx < g.nx && gy >= 0 && gy < g.ny ? (gy * g.nx + gx) * NC + 4 * grp : -1;
+    const bool ok = gx >= 0 && gx < g.nx && gy >= 0 && gy < g.ny;
+    off[s] = ok ? ((size_t)gy * g.nx + gx) * NC + 4 * grp : 0;
+    in |= (unsigned)ok << s;
   }
   const size_t plane = (size_t)g.nx * g.ny * NC;
   auto fetch = [&](int k, uint2 (&reg)[OSEG]) {
     const uint16_t *Xk = Xb + (k >= 0 && k < g.nz ? (size_t)k * plane : 0);
 #pragma unroll
-    for (int s = 0; s < OSEG; s++) reg[s] = *(const uint2 *)(Xk + (off[s] < 0 ? 0 : off[s]));
+    for (int s = 0; s < OSEG; s++) reg[s] = *(const uint2 *)(Xk + off[s]);
   };
   const bf16x4 w0 = *(const bf16x4 *)(Wo + (size_t)lane * 4), w1 = *(const bf16x4 *)(Wo + (size_t)(64 + lane) * 4);
   // output columns of this thread
@@ -423,7 +435,7 @@ __global__ __launch_bounds__(256) void k_conv_out_tile(const uint16_t *__restric
     bf16x4 a[OSEG];
 #pragma unroll
     for (int s = 0; s < OSEG; s++) {
-      const uint2 v = kin && off[s] >= 0 ? reg[s] : make_uint2(0u, 0u);
+      const uint2 v = kin && ((in >> s) & 1) ? reg[s] : make_uint2(0u, 0u);
       __builtin_memcpy(&a[s], &v, 8);
     }
     if (k + 1 < T.z1) fetch(k + 2, reg);
