@@ -7,6 +7,7 @@
 // Poisson, 1 variable coefficient) and on excision.
 #pragma once
 #include "pmg_ops.h"
+#include "pmg_rules.h"
 #include <type_traits>
 
 namespace pmg {
@@ -670,7 +671,6 @@ struct ResidP {
   int nb;
 };
 
-constexpr int RTX = 64, RTY = 8, RZC = 16;
 constexpr int kResRing = 2 * RTX + 2 * RTY + 4;
 
 template <typename T, int OP, bool EX, bool P2, bool RHS0, bool ZERO, bool OUT32, typename UT = T>

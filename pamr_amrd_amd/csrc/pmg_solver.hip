@@ -447,14 +447,12 @@ int settle(pmg_solver *S, int L) {
   return 0;
 }
 
-// z depth per block of a residual and its grid: long marches on big levels
-// (HBM reuse), short ones on small levels (latency: a block's planes are
-// processed one after another)
+// z depth per block of a residual and its grid
 template <typename P>
 int residual_grid(pmg_solver *S, P &p) {
-  p.zchunk = std::max(1, std::min(std::min(RZC, std::max(2, (p.nz - 2 + 15) / 16)), p.nz - 2));
-  const int nzc = (p.nz - 2 + p.zchunk - 1) / p.zchunk;
-  p.nb = ((p.nx - 2 + RTX - 1) / RTX) * ((p.ny - 2 + RTY - 1) / RTY) * nzc;
+  const int n[3] = {p.nx, p.ny, p.nz};
+  p.zchunk = residual_planes(n, S->ws.cap);
+  p.nb = residual_blocks(n, p.zchunk);
   return p.nb > S->ws.cap || p.nx > 1 << 24 ? -3 : 0;  // partial norms; 32-bit offsets within a tile
 }
 
@@ -1371,12 +1369,7 @@ pmg_solver *pmg_create(int nx, int ny, int nz, const double *bbox, int min_cwidt
       S->rr_czchunk[pi] = cz;
     }
   }
-  // norm workspace sized for the largest launch
-  // partial-norm capacity: the largest launch over the finest level
-  const Level &F = S->lev[nl - 1];
-  const int rblk = ((F.n[0] + RTX - 1) / RTX) * ((F.n[1] + RTY - 1) / RTY) * ((F.n[2] + RZC - 1) / RZC);
-  const int sblk = ((F.n[0] + 61) / 64) * ((F.n[1] + 5) / 8) * ((F.n[2] + 5) / 8);
-  int cap = std::max(1 << 14, std::max(rblk, sblk) + 64);
+  const int cap = norm_room(S->lev[nl - 1].n);
   S->ws.cap = cap;
   S->ws.nslots = 2 * kNormSlots;
   if (hipMalloc(&S->ws.partials, sizeof(double) * 2 * (size_t)cap * S->ws.nslots) != hipSuccess ||
