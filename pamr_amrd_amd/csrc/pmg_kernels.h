@@ -1600,7 +1600,6 @@ __device__ __forceinline__ T fw_plane_chain(T acc, bool first, const V &v, T c) 
 // usual 2^m + 1 grids that is a whole number of tiles, with no tail tile
 // marching for a single column.  The last column and row are x/y faces
 // (point formula, no march) and go to the tiles at the high edges.
-inline __host__ __device__ int rr_tiles(int cn, int c) { return cn > 1 ? (cn - 1 + c - 1) / c : 1; }
 
 template <typename T, int OP, bool P2, int CX, int CY, int NT, int PF>
 __global__ __launch_bounds__(NT) void k_resid_restrict_s(ResRestrP<T> P) {

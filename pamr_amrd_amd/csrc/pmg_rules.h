@@ -22,6 +22,28 @@ inline int residual_planes(const int *n, int cap) {
   return z;
 }
 
+// Fused finest residual + injection (streamed): kRrCX x kRrCY coarse columns a
+// block ([0] FP64, [1] FP32), columns 0 .. cn-2 -- the last ones lie on a face.
+constexpr int kRrCX[2] = {16, 32}, kRrCY = 8;
+constexpr int rr_tiles(int cn, int c) { return cn > 1 ? (cn - 1 + c - 1) / c : 1; }
+inline int rr_blocks(const int *cn, int pi, int cz) {
+  return rr_tiles(cn[0], kRrCX[pi]) * rr_tiles(cn[1], kRrCY) * ((cn[2] + cz - 1) / cz);
+}
+// Coarse planes a block marches: 6 (FP64) and 4 (FP32) on a coarse level of 129
+// planes, 8 from 257 planes on, the fastest measured.  On smaller grids a block's
+// march is the time: halved while it makes fewer than 1000 blocks, down to two
+// planes, and to one where those make fewer than 500.  FP64, us with 6, 3, 2 and
+// 1 (blocks with 2): 161 x 97 x 129 fine points 47 with 8, 18 with 2 (990);
+// 81 x 49 x 257 24.8, 17.9, 16.5, 18.2 (585); 65 x 65 x 257 19.8, 14.6, 12.8, 15.5
+// (520); 97^3 25.1, 17.8, 14.5, 14.0 (450); 33 x 65 x 257 19.7, 12.1, 11.4, 9.9
+// (260).  FP32, with 4, 2 and 1: 65 x 65 x 257 17.9, 12.8, 11.2 (260).
+inline int resid_restrict_planes(const int *cn, int pi) {
+  if (cn[2] >= 257) return 8;
+  int cz = cn[2] < 129 ? 8 : pi ? 4 : 6;
+  while (cz > 2 && rr_blocks(cn, pi, cz) < 1000) cz = std::max(2, cz / 2);
+  return cz == 2 && rr_blocks(cn, pi, cz) < 500 ? 1 : cz;
+}
+
 // Room for the partial norms of the launches over a finest level of n points:
 // its residual in the longest march, and 64 x 8 x 8 points a block.
 inline int norm_room(const int *n) {

@@ -969,15 +969,14 @@ bool can_fuse_resid_restrict(const pmg_solver *S) {
 // coarse column, the streamed one columns 0 .. cn-2 (never more workgroups)
 template <typename T>
 int resid_restrict_blocks(const int *cn, int czchunk, bool streamed = false) {
-  constexpr int CX = std::is_same<T, double>::value ? 16 : 32, CY = 8;
-  const int tx = streamed ? rr_tiles(cn[0], CX) : (cn[0] + CX - 1) / CX;
-  const int ty = streamed ? rr_tiles(cn[1], CY) : (cn[1] + CY - 1) / CY;
-  return tx * ty * ((cn[2] + czchunk - 1) / czchunk);
+  constexpr int pi = std::is_same<T, double>::value ? 0 : 1, CX = kRrCX[pi], CY = kRrCY;
+  if (streamed) return rr_blocks(cn, pi, czchunk);
+  return ((cn[0] + CX - 1) / CX) * ((cn[1] + CY - 1) / CY) * ((cn[2] + czchunk - 1) / czchunk);
 }
 
 template <typename T, int OP, bool P2>
 int launch_resid_restrict_t(pmg_solver *S, ResRestrP<T> P) {
-  constexpr int CX = std::is_same<T, double>::value ? 16 : 32, CY = 8, NT = 256;
+  constexpr int CX = kRrCX[std::is_same<T, double>::value ? 0 : 1], CY = kRrCY, NT = 256;
   const int cn[3] = {P.cnx, P.cny, P.cnz};
   const dim3 grid(resid_restrict_blocks<T>(cn, P.czchunk, S->use_fused_restrict >= 2));
   P.nb = (int)grid.x;
@@ -1353,22 +1352,8 @@ pmg_solver *pmg_create(int nx, int ny, int nz, const double *bbox, int min_cwidt
   }
   for (int L = 1; L <= nl; L++)
     for (int pi = 0; pi < 2; pi++) default_sweep(S->lev[L - 1].n, op, pi, &S->lv_variant[pi][L - 1], &S->lv_zchunk[pi][L - 1]);
-  // coarse planes per block of the fused finest residual + injection
-  // (streamed kernel), the fastest measured: 6 (FP64) and 4 (FP32) on a
-  // coarse level of 129 planes, 8 and 8 from 257 planes.  On smaller grids a
-  // block's march is the time: as many planes as still make 1000 blocks, at
-  // least 2 (161 x 97 x 129 fine points, FP64: 47 us with 8, 18 with 2)
-  if (nl >= 2) {
-    const int *cn = S->lev[nl - 2].n;
-    for (int pi = 0; pi < 2; pi++) {
-      int cz = cn[2] >= 257 ? 8 : (pi ? 4 : 6);
-      if (cn[2] < 129) cz = 8;
-      while (cn[2] < 257 && cz > 2 &&
-             (pi ? resid_restrict_blocks<float>(cn, cz, true) : resid_restrict_blocks<double>(cn, cz, true)) < 1000)
-        cz /= 2;
-      S->rr_czchunk[pi] = cz;
-    }
-  }
+  if (nl >= 2)
+    for (int pi = 0; pi < 2; pi++) S->rr_czchunk[pi] = resid_restrict_planes(S->lev[nl - 2].n, pi);
   const int cap = norm_room(S->lev[nl - 1].n);
   S->ws.cap = cap;
   S->ws.nslots = 2 * kNormSlots;

@@ -44,3 +44,17 @@ def test_residual_fits_the_norm_workspace(tmp_path):
       for (int d = 0; d < 3; d++) c[d] = std::max(3, (c[d] - 1) / 2 + 1);
     }
   });""")
+
+
+def test_resid_restrict_march(tmp_path):
+    """one plane a block only where two make fewer than 500 blocks"""
+    run(tmp_path, r"""
+  shapes([&](const int *n) {
+    if (n[0] % 2 == 0 || n[1] % 2 == 0 || n[2] % 2 == 0) return;
+    const int c[3] = {(n[0] + 1) / 2, (n[1] + 1) / 2, (n[2] + 1) / 2};
+    for (int pi = 0; pi < 2; pi++) {
+      const int z = resid_restrict_planes(c, pi);
+      all++;
+      if (z < 1 || (z == 1) != (c[2] < 257 && rr_blocks(c, pi, 2) < 500)) bad++;
+    }
+  });""")
