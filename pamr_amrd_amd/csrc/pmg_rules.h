@@ -44,6 +44,42 @@ inline int resid_restrict_planes(const int *cn, int pi) {
   return cz == 2 && rr_blocks(cn, pi, cz) < 500 ? 1 : cz;
 }
 
+// Tile variant and z chunk of a level that was never tuned, from what the
+// tuned sizes show.  From 200^3 points on, where memory is the bound: 128 x 16
+// columns, 64 x 16 where 128 would leave more than a sixth of the tile outside;
+// with the variable coefficient, whose LDS ring doubles the block's LDS, 64 x 16
+// in FP64 (257^3: 170 us, 32 x 16 181, 128 x 16 without the ring 211) and the
+// five-plane 128 x 8 in FP32 (92 us, 128 x 16 103).  The longest march that
+// leaves a block a CU; in FP32, where a CU holds two of them, at most 16 planes
+// (32 with the coefficient): neighbours drift apart on a long march and no
+// longer find each other's rows in the L2 (513^3: 453 us with 16 planes, 484
+// with 32, 503 with 64).  Below 200^3: 32 x 16 columns, the longest march of 64
+// .. 2 planes that makes 400 workgroups -- fewer leave CUs without work, shorter
+// marches repeat the prologue (129^3: 14.9 us at 8 planes and 512 workgroups;
+// 65^3: 6.6 us at 2 planes, 7.6 at 4).
+inline void default_sweep(const int *n, int op, int pi, int *variant, int *zchunk) {
+  const size_t size = (size_t)n[0] * n[1] * n[2];
+  int tx = 32, ty = 16, want = 400, z = 64;
+  *variant = 2;
+  if (size >= 8000000) {
+    const int w = n[0] - 2, w128 = (w + 127) / 128 * 128;
+    const bool ring64 = op == 1 && pi == 0;
+    tx = ring64 || 6 * (w128 - w) > w128 ? 64 : 128;
+    *variant = tx == 64 ? 1 : (op == 1 ? 11 : 5);
+    if (*variant == 11) ty = 8;
+    want = tx == 64 && !ring64 ? 400 : 256;
+    if (pi == 1) z = op == 1 ? 32 : 16;
+  }
+  auto columns = [&] { return ((n[0] - 2 + tx - 1) / tx) * ((n[1] - 2 + ty - 1) / ty); };
+  if (columns() > 1 << 14) {  // a thin grid: narrow columns alone outnumber the partial norms (norm_room)
+    tx = std::max(tx, 64);
+    *variant = *variant == 2 ? 1 : *variant;
+  }
+  const int cols = columns();
+  while (z > 2 && cols * ((n[2] - 2 + z - 1) / z) < want) z /= 2;
+  *zchunk = z;
+}
+
 // Room for the partial norms of the launches over a finest level of n points:
 // its residual in the longest march, and 64 x 8 x 8 points a block.
 inline int norm_room(const int *n) {
