@@ -918,6 +918,16 @@ int bottom(pmg_solver *S, int Lb, int norm_base, double *cnorm, int *citer) {
   return 0;
 }
 
+// workgroups of the fused kernel for a coarse level of cn points and a
+// given number of coarse planes per workgroup: the ring kernel tiles every
+// coarse column, the streamed one columns 0 .. cn-2 (never more workgroups)
+template <typename T>
+int resid_restrict_blocks(const int *cn, int czchunk, bool streamed = false) {
+  constexpr int pi = std::is_same<T, double>::value ? 0 : 1, CX = kRrCX[pi], CY = kRrCY;
+  if (streamed) return rr_blocks(cn, pi, czchunk);
+  return ((cn[0] + CX - 1) / CX) * ((cn[1] + CY - 1) / CY) * ((cn[2] + czchunk - 1) / czchunk);
+}
+
 // finest-level residual + full-weight injection of u and f_res in one pass
 // (no excision, full weighting for both, fine = 2 coarse - 1), in the FP64
 // cycle and in the FP32 inner cycle; the finest f_res is then never stored
@@ -928,19 +938,11 @@ bool can_fuse_resid_restrict(const pmg_solver *S) {
   for (int d = 0; d < 3; d++)
     if (F.n[d] != 2 * C.n[d] - 1) return false;
   if ((size_t)F.n[0] * F.n[1] * sizeof(T) >= (size_t)1 << 32) return false;  // 32-bit offsets within a plane
+  const int cz = std::max(1, std::min(S->rr_czchunk[std::is_same<T, double>::value ? 0 : 1], C.n[2]));
+  if (resid_restrict_blocks<T>(C.n, cz, S->use_fused_restrict >= 2) > S->ws.cap) return false;  // a thin grid
   // the residual box must be the whole interior (ZERO semantics off it)
   return F.rbox.ok && F.rbox.lo[0] == 1 && F.rbox.lo[1] == 1 && F.rbox.lo[2] == 1 && F.rbox.hi[0] == F.n[0] - 2 &&
          F.rbox.hi[1] == F.n[1] - 2 && F.rbox.hi[2] == F.n[2] - 2;
-}
-
-// workgroups of the fused kernel for a coarse level of cn points and a
-// given number of coarse planes per workgroup: the ring kernel tiles every
-// coarse column, the streamed one columns 0 .. cn-2 (never more workgroups)
-template <typename T>
-int resid_restrict_blocks(const int *cn, int czchunk, bool streamed = false) {
-  constexpr int pi = std::is_same<T, double>::value ? 0 : 1, CX = kRrCX[pi], CY = kRrCY;
-  if (streamed) return rr_blocks(cn, pi, czchunk);
-  return ((cn[0] + CX - 1) / CX) * ((cn[1] + CY - 1) / CY) * ((cn[2] + czchunk - 1) / czchunk);
 }
 
 template <typename T, int OP, bool P2>

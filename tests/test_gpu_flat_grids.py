@@ -1,6 +1,6 @@
-"""A grid with so many (x, y) tiles that the residual's short marches would
-need more blocks than the norm workspace holds: two cycles bit for bit against
-the oracle."""
+"""Grids with so many (x, y) tiles that a launch would need more blocks than the
+norm workspace holds -- the residual's short marches on a flat one, the fused
+residual + injection on a thin one: two cycles bit for bit against the oracle."""
 import numpy as np
 import pytest
 
@@ -10,9 +10,10 @@ import pamr_amrd_amd as pm
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("op", [0, 1])
-def test_flat_grid_cycles(torch_cuda, op):
-    shape, bbox = (9, 8209, 33), (0.0, 1.0, 0.0, 1026.0, 0.0, 4.0)
+@pytest.mark.parametrize("shape,bbox,op", [((9, 8209, 33), (0.0, 1.0, 0.0, 1026.0, 0.0, 4.0), 0),
+                                           ((9, 8209, 33), (0.0, 1.0, 0.0, 1026.0, 0.0, 4.0), 1),
+                                           ((1048577, 5, 5), (0.0, 262144.0, 0.0, 1.0, 0.0, 1.0), 0)])
+def test_flat_grid_cycles(torch_cuda, shape, bbox, op):
     print(f"case flat grid {shape} op={op}", flush=True)
     rng = np.random.default_rng(op)
     m = O.UniformMG(0, bbox=bbox, mcw=3, op=op, shape=shape)
