@@ -254,7 +254,7 @@ struct SweepBatchP {
   int slot;
 };
 
-template <typename T, int OP, bool P2, bool RHS0, int TX, int TY, int NT>
+template <typename T, int OP, bool P2, bool RHS0, int TX, int TY, int NT, typename O = unsigned>
 __global__ __launch_bounds__(NT) void k_sweep_batch(SweepBatchP<T> B) {
   const int t = xcd_tile(blockIdx.x, gridDim.x);
   const BTile tl = B.tiles[t];
@@ -275,7 +275,7 @@ __global__ __launch_bounds__(NT) void k_sweep_batch(SweepBatchP<T> B) {
   P.ws = B.ws;
   P.slot = B.slot;
   P.nb = gridDim.x;
-  sweep_tile<T, OP, false, P2, RHS0, TX, TY, NT>(P, tl.x0, tl.y0, tl.z0, min(tl.z0 + B.zchunk, G.nz - 1), t);
+  sweep_tile<T, OP, false, P2, RHS0, TX, TY, NT, 1, 4, O>(P, tl.x0, tl.y0, tl.z0, min(tl.z0 + B.zchunk, G.nz - 1), t);
 }
 
 template <typename T>
@@ -297,13 +297,14 @@ struct PtsBatchP {
 // points with op 1: 47.6 -> 44.9 us, 35 of 40^3 30.2 -> 28.6.  (L_op with the
 // child mask is quicker point by point, 29 against 39 us: most points of a patch
 // level have no child above them, and skip the operator.)
-template <typename T, int OP, bool P2>
+template <typename T, int OP, bool P2, typename O>
 struct TileCol {
   const T *u, *rho, *a, *c;  // from the place west and south of the tile's corner
   size_t plane;
   int nz;
-  unsigned own, east, west, north, south;  // byte offsets; the own place for a column on the rim
+  O own, east, west, north, south;  // byte offsets; the own place for a column on the rim
   T um, uc, up, am, ac, ap;
+  static_assert(sizeof(O) > 4 || (PTY + 2) * (size_t)kLongRow * sizeof(T) < (size_t)1 << 32, "offsets within a tile");
   __device__ __forceinline__ TileCol(const PtsBatchP<T> &B, const GridGeo &G, const BTile &tl, int i, int j, bool inner) {
     const ptrdiff_t org = (ptrdiff_t)G.off + (ptrdiff_t)(tl.y0 - 1) * G.nx + (tl.x0 - 1);
     u = B.u + org;
@@ -315,7 +316,7 @@ struct TileCol {
     const int d = inner ? 1 : 0;
     i = min(i, G.nx - 1) - (tl.x0 - 1);
     j = min(j, G.ny - 1) - (tl.y0 - 1);
-    auto at = [&](int x, int y) { return ((unsigned)y * (unsigned)G.nx + (unsigned)x) * (unsigned)sizeof(T); };
+    auto at = [&](int x, int y) { return ((O)y * (O)G.nx + (O)x) * (O)sizeof(T); };
     own = at(i, j);
     east = at(i + d, j);
     west = at(i - d, j);
@@ -329,7 +330,7 @@ struct TileCol {
       ap = get(a, k, own);
     }
   }
-  __device__ __forceinline__ T get(const T *f, int k, unsigned &o) const {
+  __device__ __forceinline__ T get(const T *f, int k, O &o) const {
     return tile_at(f, plane, min(max(k, 0), nz - 1), o);
   }
   __device__ __forceinline__ void step(int k) {  // to plane k
@@ -355,7 +356,7 @@ struct TileCol {
 };
 
 // residual hook (w/examples/nps/num_w.f:59-90) on the interior of every grid
-template <typename T, int OP, bool P2, bool RHS0>
+template <typename T, int OP, bool P2, bool RHS0, typename O>
 __global__ __launch_bounds__(PTX * PTY) void k_resid_batch(PtsBatchP<T> B) {
   const int t = xcd_tile(blockIdx.x, gridDim.x);
   const BTile tl = B.tiles[t];
@@ -365,7 +366,7 @@ __global__ __launch_bounds__(PTX * PTY) void k_resid_batch(PtsBatchP<T> B) {
   double s = 0.0;
   int cnt = 0;
   const size_t p0 = G.off + ix3(i, j, 0, G.nx, G.ny);
-  TileCol<T, OP, P2> C(B, G, tl, i, j, inner);
+  TileCol<T, OP, P2, O> C(B, G, tl, i, j, inner);
 #pragma unroll
   for (int kk = 0; kk < PTZ; kk++) {
     const int k = tl.z0 + kk;
@@ -423,7 +424,7 @@ __global__ __launch_bounds__(256) void k_add_alt(T *u, T *alt, const T *r, size_
 // 0 on every AMR level's own points) of every grid of a level, written
 // negated in FP32 as the source of the FP32 correction cycle (0 off the
 // interior), with the RMS partials of the level's grids
-template <int OP, bool P2>
+template <int OP, bool P2, typename O>
 __global__ __launch_bounds__(PTX * PTY) void k_defect32_batch(PtsBatchP<double> B, float *src32) {
   const int t = xcd_tile(blockIdx.x, gridDim.x);
   const BTile tl = B.tiles[t];
@@ -433,7 +434,7 @@ __global__ __launch_bounds__(PTX * PTY) void k_defect32_batch(PtsBatchP<double> 
   double s = 0.0;
   int cnt = 0;
   const size_t p0 = G.off + ix3(i, j, 0, G.nx, G.ny);
-  TileCol<double, OP, P2> C(B, G, tl, i, j, inner);
+  TileCol<double, OP, P2, O> C(B, G, tl, i, j, inner);
 #pragma unroll
   for (int kk = 0; kk < PTZ; kk++) {
     const int k = tl.z0 + kk;
@@ -607,6 +608,7 @@ struct ALevel {
   double *sres = nullptr;
   float *sres32 = nullptr;
   int variant = 2, zchunk = 16;
+  bool long_rows = false;  // a grid with more than kLongRow points along x
   BTile *d_stiles = nullptr;
   int nstiles = 0;
   int *d_sstart = nullptr;
@@ -1127,6 +1129,9 @@ void default_tiles(ALevel &Lv) {
 
 int build_tiles(pmg_amr *A, ALevel &Lv) {
   int tx, ty;
+  Lv.long_rows = false;
+  for (const HGrid &g : Lv.g) Lv.long_rows = Lv.long_rows || g.n[0] > kLongRow;
+  if (Lv.long_rows) Lv.variant = 3;  // the only tile with 64-bit offsets
   variant_txy(Lv.variant, tx, ty);
   std::vector<BTile> st, pt;
   std::vector<int> ss{0}, ps{0};
@@ -1336,6 +1341,11 @@ int clear_res(pmg_amr *A, int L) {
 template <typename T, int OP, bool P2, bool RHS0>
 int launch_sweep_batch(pmg_amr *A, ALevel &Lv, const SweepBatchP<T> &B) {
   const dim3 grid(Lv.nstiles);
+  if (Lv.long_rows) {  // build_tiles has made tiles of variant 3
+    hipLaunchKernelGGL((k_sweep_batch<T, OP, P2, RHS0, 32, 8, 256, size_t>), grid, dim3(256), 0, A->stream, B);
+    PMG_HOST_CHECK(hipGetLastError());
+    return 0;
+  }
   switch (Lv.variant) {
 #define PMG_LSB(V, TXV, TYV, NTV) \
   case V: hipLaunchKernelGGL((k_sweep_batch<T, OP, P2, RHS0, TXV, TYV, NTV>), grid, dim3(NTV), 0, A->stream, B); break;
@@ -1410,7 +1420,11 @@ int residual(pmg_amr *A, int L, int slot) {
   B.slot = slot;
   const bool rhs0 = L == A->nlev, p2 = B.sp.pow2 != 0;
   const dim3 grid(Lv.nptiles), blk(PTX * PTY);
-#define PMG_RB(OPV, P2V, R0) hipLaunchKernelGGL((k_resid_batch<T, OPV, P2V, R0>), grid, blk, 0, A->stream, B)
+#define PMG_RB(OPV, P2V, R0)                                                                                     \
+  do {                                                                                                           \
+    if (Lv.long_rows) hipLaunchKernelGGL((k_resid_batch<T, OPV, P2V, R0, size_t>), grid, blk, 0, A->stream, B); \
+    else hipLaunchKernelGGL((k_resid_batch<T, OPV, P2V, R0, unsigned>), grid, blk, 0, A->stream, B);            \
+  } while (0)
   if (A->op == 0) {
     if (p2) { if (rhs0) PMG_RB(0, true, true); else PMG_RB(0, true, false); }
     else { if (rhs0) PMG_RB(0, false, true); else PMG_RB(0, false, false); }
@@ -1622,13 +1636,14 @@ int enqueue_defect(pmg_amr *A) {
     const bool p2 = Lv.sp.pow2 != 0;
     const dim3 grid(Lv.nptiles), blk(PTX * PTY);
     float *src = Lv.f32[PMG_F_RHO];
-    if (A->op == 0) {
-      if (p2) hipLaunchKernelGGL((k_defect32_batch<0, true>), grid, blk, 0, A->stream, B, src);
-      else hipLaunchKernelGGL((k_defect32_batch<0, false>), grid, blk, 0, A->stream, B, src);
-    } else {
-      if (p2) hipLaunchKernelGGL((k_defect32_batch<1, true>), grid, blk, 0, A->stream, B, src);
-      else hipLaunchKernelGGL((k_defect32_batch<1, false>), grid, blk, 0, A->stream, B, src);
-    }
+#define PMG_DB(OPV, P2V)                                                                                         \
+  do {                                                                                                           \
+    if (Lv.long_rows) hipLaunchKernelGGL((k_defect32_batch<OPV, P2V, size_t>), grid, blk, 0, A->stream, B, src); \
+    else hipLaunchKernelGGL((k_defect32_batch<OPV, P2V, unsigned>), grid, blk, 0, A->stream, B, src);            \
+  } while (0)
+    if (A->op == 0) { if (p2) PMG_DB(0, true); else PMG_DB(0, false); }
+    else { if (p2) PMG_DB(1, true); else PMG_DB(1, false); }
+#undef PMG_DB
     PMG_HOST_CHECK(hipGetLastError());
   }
   return fold(A);
@@ -1715,7 +1730,7 @@ int setup_levels(pmg_amr *A, int op) {
     // all grids of a level share one spacing (dyadic boxes); check it
     for (const HGrid &g : Lv.g)
       for (int d = 0; d < 3; d++)
-        if (g.hdx[d] != Lv.g[0].hdx[d] || g.n[d] < 3 || g.n[0] > 1 << 24) return -1;
+        if (g.hdx[d] != Lv.g[0].hdx[d] || g.n[d] < 3) return -1;
     Lv.sp = spacing_of(Lv.g[0].hdx);
     Lv.sp32 = spacing_of32(Lv.g[0].hdx);
     size_t pool = 0;

@@ -80,9 +80,10 @@ __device__ __forceinline__ int cs_east(int lx) { return (lx & 1) ? 1 - LX / 2 : 
 // outside the grid is ever read -- and 32-bit byte offsets within the tile are
 // added to it, so that a load is a scalar address plus a register and no plane
 // of the march computes one (the empty asm keeps the compiler from widening
-// the offsets to register pairs ahead of the march).
-template <typename V>
-__device__ __forceinline__ V tile_at(const V *base, size_t plane, int k, unsigned &off) {
+// the offsets to register pairs ahead of the march).  O: unsigned for rows of
+// at most kLongRow points, size_t for longer ones.
+template <typename V, typename O>
+__device__ __forceinline__ V tile_at(const V *base, size_t plane, int k, O &off) {
   asm volatile("" : "+v"(off));
   return *reinterpret_cast<const V *>(reinterpret_cast<const char *>(base + plane * (size_t)k) + off);
 }
@@ -99,8 +100,8 @@ template <typename V>
 struct __attribute__((packed, aligned(alignof(V)))) Two {
   V v[2];
 };
-template <typename V>
-__device__ __forceinline__ Two<V> tile_two(const V *base, size_t plane, int k, unsigned &off) {
+template <typename V, typename O>
+__device__ __forceinline__ Two<V> tile_two(const V *base, size_t plane, int k, O &off) {
   asm volatile("" : "+v"(off));
   return *reinterpret_cast<const Two<V> *>(reinterpret_cast<const char *>(base + plane * (size_t)k) + off);
 }
@@ -114,15 +115,15 @@ __device__ __forceinline__ Two<V> tile_two(const V *base, size_t plane, int k, u
 // update the same place of the pair (`hi`: the second).  lo, ea: LDS byte offsets
 // of the place and its east neighbour; ok: pass 0 updates it; in: so does pass 1
 // (the tile proper), and the norm counts it.
-template <int N>
+template <int N, typename O>
 struct SlotTab {
   int lo[2][N], ea[2][N];
-  unsigned off[N];  // byte offset of the pair in the tile (of a pair in the grid where there is none)
+  O off[N];  // byte offset of the pair in the tile (of a pair in the grid where there is none)
   bool ok[2][N], in[2][N], hi[2][N];
 };
 
-template <typename T, int TX, int TY, int NT, int N>
-__device__ __forceinline__ void slot_table(const SweepP<T> &P, int x0, int y0, int z0, SlotTab<N> &S) {
+template <typename T, int TX, int TY, int NT, int N, typename O>
+__device__ __forceinline__ void slot_table(const SweepP<T> &P, int x0, int y0, int z0, SlotTab<N, O> &S) {
   constexpr int W = TX / 2;
   static_assert(TX % 2 == 0, "pairs of points");
 #pragma unroll
@@ -146,7 +147,7 @@ __device__ __forceinline__ void slot_table(const SweepP<T> &P, int x0, int y0, i
     // a pair may reach over an end of its row, into the neighbouring one's
     const bool pair = slot && i0 <= P.nx - 1 && j <= P.ny - 2;
     const int ry = pair ? ly : 2, rx = pair ? lx0 : 2;
-    S.off[m] = ((unsigned)ry * (unsigned)P.nx + (unsigned)rx) * (unsigned)sizeof(T);
+    S.off[m] = ((O)ry * (O)P.nx + (O)rx) * (O)sizeof(T);
 #pragma unroll
     for (int e = 0; e < 2; e++) {
       const int want = (j + z0 + e + 3) & 1;  // parity of i: (i+j+k+3) even
@@ -200,10 +201,12 @@ struct HalfRegs {
 // and excision 141 -> 100 us, FP32 257^3 77 -> 70 and 129^3 17.6 -> 13.7, FP64
 // 129^3 20.5 -> 19.2.  The largest stay with memory: FP64 257^3 93 -> 92 (4.5
 // TB/s), FP32 513^3 475 -> 455 (3.6 TB/s).
-template <typename T, int OP, bool EX, bool P2, bool RHS0, int TX, int TY, int NT, int PF = 1, int RING = 4>
+template <typename T, int OP, bool EX, bool P2, bool RHS0, int TX, int TY, int NT, int PF = 1, int RING = 4,
+          typename O = unsigned>
 __device__ __forceinline__ void sweep_tile(const SweepP<T> &P, int x0, int y0, int z0, int z1, int bid) {
   static_assert(PF == 1 || PF == 2, "prefetch depth");
   static_assert(RING == 4 || RING == 5, "LDS ring");
+  static_assert(sizeof(O) > 4 || (TY + 4) * (size_t)kLongRow * sizeof(T) < (size_t)1 << 32, "offsets within a tile");
   constexpr int LX = TX + 4, LY = TY + 4, PL = LX * LY;
   constexpr int NLD = (PL + NT - 1) / NT, NST = (TX * TY + NT - 1) / NT;
   constexpr int N = (TX / 2 * TY + TX + 2 * TY + NT - 1) / NT, NT1 = (TX / 2 * TY + NT - 1) / NT;
@@ -220,7 +223,7 @@ __device__ __forceinline__ void sweep_tile(const SweepP<T> &P, int x0, int y0, i
   const int nx = P.nx, ny = P.ny, nz = P.nz;
   const size_t plane = (size_t)nx * ny;
   const ptrdiff_t org = (ptrdiff_t)(y0 - 2) * nx + (x0 - 2);
-  const unsigned here = (2u * (unsigned)nx + 2u) * (unsigned)B;  // position (2, 2): always in the grid
+  const O here = ((O)2 * (O)nx + 2) * B;  // position (2, 2): always in the grid
   double s = 0.0;
   int cnt = 0;
 
@@ -234,14 +237,14 @@ __device__ __forceinline__ void sweep_tile(const SweepP<T> &P, int x0, int y0, i
   const T *const ub = zero ? P.uin : P.uin + org;
   const T *const ab = AR ? P.a + org : nullptr;
   const size_t uplane = zero ? 0 : plane;
-  unsigned gu[NLD], ga[AR && F32 ? NLD : 1];
+  O gu[NLD], ga[AR && F32 ? NLD : 1];
   int lc[NLD];
 #pragma unroll
   for (int m = 0; m < NLD; m++) {
     const int q = threadIdx.x + m * NT, lx = q % LX, ly = q / LX, i = x0 - 2 + lx, j = y0 - 2 + ly;
     const bool ok = q < PL && i >= 0 && i < nx && j >= 0 && j < ny;
-    const unsigned g = ok ? ((unsigned)ly * (unsigned)nx + (unsigned)lx) * (unsigned)B : here;
-    gu[m] = zero ? 0u : g;
+    const O g = ok ? ((O)ly * (O)nx + (O)lx) * B : here;
+    gu[m] = zero ? 0 : g;
     if constexpr (AR && F32) ga[m] = g;
     lc[m] = cs_off<LX>(lx, ly) * B;
   }
@@ -270,14 +273,14 @@ __device__ __forceinline__ void sweep_tile(const SweepP<T> &P, int x0, int y0, i
       if constexpr (AR) L(la, slot * PL * B + lc[m]) = d.a[m];
     }
   };
-  unsigned go[NST];
+  O go[NST];
   int ls[NST];
   bool st[NST];
 #pragma unroll
   for (int m = 0; m < NST; m++) {
     const int q = threadIdx.x + m * NT, tx = q % TX, ty = q / TX;
     st[m] = q < TX * TY && x0 + tx <= nx - 2 && y0 + ty <= ny - 2;
-    go[m] = ((unsigned)(ty + 2) * (unsigned)nx + (unsigned)(tx + 2)) * (unsigned)B;
+    go[m] = ((O)(ty + 2) * (O)nx + (O)(tx + 2)) * B;
     ls[m] = cs_off<LX>(tx + 2, ty + 2) * B;
   }
   auto store = [&](int k, int slot) {
@@ -298,14 +301,14 @@ __device__ __forceinline__ void sweep_tile(const SweepP<T> &P, int x0, int y0, i
       }
   };
 
-  SlotTab<N> tab;
+  SlotTab<N, O> tab;
   slot_table<T, TX, TY, NT, N>(P, x0, y0, z0, tab);
   auto prefetch = [&](int k, auto &R) {
     const int kk = min(k, nz - 1);
 #pragma unroll
     for (int m = 0; m < N; m++) {
       if constexpr (EX) {
-        unsigned byte = tab.off[m] / (unsigned)B;
+        O byte = tab.off[m] / B;
         const Two<uint8_t> x = tile_two(P.chr + org, plane, kk, byte);
         R.x[m][0] = x.v[0];
         R.x[m][1] = x.v[1];
@@ -352,7 +355,7 @@ __device__ __forceinline__ void sweep_tile(const SweepP<T> &P, int x0, int y0, i
                                R.c[m], R.rho[m], P.sp, &jac);
       } else {
         const T *__restrict__ a = P.a + org + (ptrdiff_t)(plane * (size_t)k);
-        const size_t p = tab.off[m] / (unsigned)B + (tab.hi[e][m] ? 1 : 0), sy = (size_t)nx;
+        const size_t p = tab.off[m] / B + (tab.hi[e][m] ? 1 : 0), sy = (size_t)nx;
         A = lop_varcoef<T, P2>(uc, L(lu, b0 + ea), L(lu, b0 + we), L(lu, b0 + lo + LX * B), L(lu, b0 + lo - LX * B),
                                L(lu, bp + lo), L(lu, bm + lo), a[p], a[p + 1], a[p - 1], a[p + sy], a[p - sy],
                                a[p + plane], (a - plane)[p], R.c[m], R.rho[m], P.sp, &jac);
@@ -436,14 +439,15 @@ __device__ __forceinline__ void sweep_tile(const SweepP<T> &P, int x0, int y0, i
   norm_partial<NT>(s, (double)cnt, P.ws, P.slot, bid, P.nb);
 }
 
-template <typename T, int OP, bool EX, bool P2, bool RHS0, int TX, int TY, int NT, int PF = 1, int RING = 4>
+template <typename T, int OP, bool EX, bool P2, bool RHS0, int TX, int TY, int NT, int PF = 1, int RING = 4,
+          typename O = unsigned>
 __global__ __launch_bounds__(NT) void k_sweep(SweepP<T> P) {
   const int tile = xcd_tile(blockIdx.x, gridDim.x);
   const int nty = (P.ny - 2 + TY - 1) / TY, ntx = (P.nx - 2 + TX - 1) / TX;
   const int ty = tile % nty, tx = (tile / nty) % ntx, tz = tile / (nty * ntx);
   const int z0 = 1 + tz * P.zchunk;
-  sweep_tile<T, OP, EX, P2, RHS0, TX, TY, NT, PF, RING>(P, 1 + tx * TX, 1 + ty * TY, z0,
-                                                        min(z0 + P.zchunk, P.nz - 1), blockIdx.x);
+  sweep_tile<T, OP, EX, P2, RHS0, TX, TY, NT, PF, RING, O>(P, 1 + tx * TX, 1 + ty * TY, z0,
+                                                           min(z0 + P.zchunk, P.nz - 1), blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -673,7 +677,8 @@ struct ResidP {
 
 constexpr int kResRing = 2 * RTX + 2 * RTY + 4;
 
-template <typename T, int OP, bool EX, bool P2, bool RHS0, bool ZERO, bool OUT32, typename UT = T>
+template <typename T, int OP, bool EX, bool P2, bool RHS0, bool ZERO, bool OUT32, typename UT = T,
+          typename O = unsigned>
 __global__ __launch_bounds__(RTX * RTY) void k_residual(ResidP<T, UT> P) {
   __shared__ T bP[2][RTY + 2][RTX + 2];
   __shared__ T bA[2][OP == 1 ? RTY + 2 : 1][RTX + 2];
@@ -703,12 +708,13 @@ __global__ __launch_bounds__(RTX * RTY) void k_residual(ResidP<T, UT> P) {
   // addresses as in the sweep: a scalar plane plus an offset within the tile,
   // places outside the grid reading position (1, 1), which is in it
   const ptrdiff_t org = (ptrdiff_t)(y0 - 1) * nx + (x0 - 1);
-  auto place = [&](bool ok, int px, int py) { return ok ? (unsigned)py * (unsigned)nx + (unsigned)px : (unsigned)nx + 1u; };
-  const unsigned own_e = place(inside, lx + 1, ly + 1), ring_e = place(hvalid, hx, hy);
-  unsigned own_u = own_e * (unsigned)sizeof(UT), ring_u = ring_e * (unsigned)sizeof(UT);
-  unsigned own_t = own_e * (unsigned)sizeof(T), ring_t = ring_e * (unsigned)sizeof(T), own_x = own_e;
-  auto u_at = [&](int k, unsigned &o) { return (T)tile_at(P.u + org, sz, k, o); };
-  auto a_at = [&](int k, unsigned &o) { return tile_at(P.a + org, sz, k, o); };
+  static_assert(sizeof(O) > 4 || (RTY + 2) * (size_t)kLongRow * sizeof(double) < (size_t)1 << 32, "offsets within a tile");
+  auto place = [&](bool ok, int px, int py) { return ok ? (O)py * (O)nx + (O)px : (O)nx + 1; };
+  const O own_e = place(inside, lx + 1, ly + 1), ring_e = place(hvalid, hx, hy);
+  O own_u = own_e * (O)sizeof(UT), ring_u = ring_e * (O)sizeof(UT);
+  O own_t = own_e * (O)sizeof(T), ring_t = ring_e * (O)sizeof(T), own_x = own_e;
+  auto u_at = [&](int k, O &o) { return (T)tile_at(P.u + org, sz, k, o); };
+  auto a_at = [&](int k, O &o) { return tile_at(P.a + org, sz, k, o); };
   double s = 0.0;
   int cnt = 0;
   T um = u_at(z0 - 1, own_u), uc = u_at(z0, own_u), up = u_at(z0 + 1, own_u), hv = u_at(z0, ring_u);

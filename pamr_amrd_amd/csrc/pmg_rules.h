@@ -6,6 +6,11 @@
 
 namespace pmg {
 
+// Rows of at most this many points: byte offsets within a tile of up to 36 rows
+// of doubles fit 32 bits.  Longer ones take kernels with 64-bit offsets, on the
+// narrowest tiles (no one has them in earnest; they run, that is all).
+constexpr int kLongRow = 1 << 23;
+
 // Residual: RTX x RTY columns a block.  z planes a block marches: long marches
 // on big levels (HBM reuse), a sixteenth of the planes on small ones (latency:
 // a block's planes are processed one after another).

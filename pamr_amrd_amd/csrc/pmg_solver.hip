@@ -422,18 +422,20 @@ int residual_grid(pmg_solver *S, P &p) {
   const int n[3] = {p.nx, p.ny, p.nz};
   p.zchunk = residual_planes(n, S->ws.cap);
   p.nb = residual_blocks(n, p.zchunk);
-  return p.nb > S->ws.cap || p.nx > 1 << 24 ? -3 : 0;  // partial norms; 32-bit offsets within a tile
+  return p.nb > S->ws.cap ? -3 : 0;
 }
 
 template <typename T, int OP, bool EX, bool P2>
 int launch_residual_t(pmg_solver *S, ResidP<T> P, bool rhs0, bool zero) {
   if (residual_grid(S, P)) return -3;
   const dim3 grid(P.nb);
-#define PMG_LR(R0, Z0, O32) hipLaunchKernelGGL((k_residual<T, OP, EX, P2, R0, Z0, O32>), grid, dim3(RTX * RTY), 0, S->stream, P)
+#define PMG_LRO(R0, Z0, O32, O) hipLaunchKernelGGL((k_residual<T, OP, EX, P2, R0, Z0, O32, T, O>), grid, dim3(RTX * RTY), 0, S->stream, P)
+#define PMG_LR(R0, Z0, O32) do { if (P.nx > kLongRow) PMG_LRO(R0, Z0, O32, size_t); else PMG_LRO(R0, Z0, O32, unsigned); } while (0)
   if (P.neg32) { PMG_LR(true, true, true); }
   else if (rhs0) { if (zero) PMG_LR(true, true, false); else PMG_LR(true, false, false); }
   else { if (zero) PMG_LR(false, true, false); else PMG_LR(false, false, false); }
 #undef PMG_LR
+#undef PMG_LRO
   PMG_HOST_CHECK(hipGetLastError());
   return 0;
 }
@@ -2283,12 +2285,14 @@ int resid_vec(pmg_solver *S, const UT *u, const double *rho, double *res, int sl
   P.slot = slot;
   if (residual_grid(S, P)) return -3;
   const dim3 grid(P.nb);
-#define PMG_RV(OPV, EXV, P2V) hipLaunchKernelGGL((k_residual<double, OPV, EXV, P2V, true, true, false, UT>), grid, dim3(RTX * RTY), 0, S->stream, P)
+#define PMG_RVO(OPV, EXV, P2V, O) hipLaunchKernelGGL((k_residual<double, OPV, EXV, P2V, true, true, false, UT, O>), grid, dim3(RTX * RTY), 0, S->stream, P)
+#define PMG_RV(OPV, EXV, P2V) do { if (P.nx > kLongRow) PMG_RVO(OPV, EXV, P2V, size_t); else PMG_RVO(OPV, EXV, P2V, unsigned); } while (0)
 #define PMG_RV2(OPV, EXV) do { if (P.sp.pow2) PMG_RV(OPV, EXV, true); else PMG_RV(OPV, EXV, false); } while (0)
   if (S->op == 0) { if (S->do_ex) PMG_RV2(0, true); else PMG_RV2(0, false); }
   else { if (S->do_ex) PMG_RV2(1, true); else PMG_RV2(1, false); }
 #undef PMG_RV2
 #undef PMG_RV
+#undef PMG_RVO
   PMG_HOST_CHECK(hipGetLastError());
   return 0;
 }

@@ -14,8 +14,7 @@ namespace pmg {
   X(8, 128, 8, 512, 2, 4) X(9, 128, 16, 1024, 2, 5) X(10, 128, 16, 1024, 1, 5) X(11, 128, 8, 512, 1, 5)
 constexpr int kNumSweepVariants = 12;
 
-// n workgroups beyond cap (the partial-norm workspace) or rows too long for a
-// tile's 32-bit offsets (2^24 points): -3, nothing launched
+// n workgroups beyond cap (the partial-norm workspace): -3, nothing launched
 template <typename T, int OP, bool EX>
 int launch_sweep(hipStream_t stream, int variant, SweepP<T> P, bool p2, bool rhs0);
 
@@ -24,7 +23,8 @@ template <typename T, int OP, bool EX, bool P2, bool RHS0>
 int launch_sweep_v(hipStream_t stream, int variant, SweepP<T> P) {
   P.zchunk = std::max(1, std::min(P.zchunk, P.nz - 2));
   int tx = 64, ty = 8;
-  switch (variant) {
+  const bool wide = P.nx > kLongRow;  // 64-bit offsets, in the tile of variant 0
+  switch (wide ? 0 : variant) {
 #define PMG_TXY(V, TXV, TYV, NTV, PFV, RGV) case V: tx = TXV; ty = TYV; break;
     PMG_SWEEP_VARIANTS(PMG_TXY)
 #undef PMG_TXY
@@ -32,7 +32,12 @@ int launch_sweep_v(hipStream_t stream, int variant, SweepP<T> P) {
   }
   dim3 grid(((P.nx - 2 + tx - 1) / tx) * ((P.ny - 2 + ty - 1) / ty) * ((P.nz - 2 + P.zchunk - 1) / P.zchunk));
   P.nb = (int)grid.x;
-  if (P.nb > P.ws.cap || P.nx > 1 << 24) return -3;
+  if (P.nb > P.ws.cap) return -3;
+  if (wide) {
+    hipLaunchKernelGGL((k_sweep<T, OP, EX, P2, RHS0, 64, 8, 256, 1, 4, size_t>), grid, dim3(256), 0, stream, P);
+    PMG_HOST_CHECK(hipGetLastError());
+    return 0;
+  }
   switch (variant) {
 #define PMG_LSW(V, TXV, TYV, NTV, PFV, RGV)                                                         \
   case V:                                                                                           \
