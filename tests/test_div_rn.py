@@ -1,7 +1,7 @@
-"""The division-free FP64 relaxation quotient (div_rn in csrc/pmg_ops.h):
+"""The division-free FP64 relaxation quotient (div_rn in csrc/pmg_div.h):
 RN(a y) followed by two FMA corrections with the exact remainder returns the
-IEEE quotient a / b when y = RN(1/b).  The same five operations are run on
-the host (C99 fma is correctly rounded, like the GPU's v_fma_f64) for the
+IEEE quotient a / b when y = RN(1/b).  That function is compiled for
+the host (fma is correctly rounded there, like the GPU's v_fma_f64) and run for the
 Jacobians of every dyadic grid size the solver uses, random divisors and
 tens of millions of random dividends across many binades, and compared with
 the division bit for bit."""
@@ -11,11 +11,14 @@ import tempfile
 
 import pytest
 
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "pamr_amrd_amd", "csrc")
+
 SRC = r"""
 #include <math.h>
 #include <stdint.h>
 #include <stdio.h>
 #include <string.h>
+#include "pmg_div.h"
 static uint64_t s = 0x9E3779B97F4A7C15ull;
 static uint64_t next(void) {
   uint64_t z = (s += 0x9E3779B97F4A7C15ull);
@@ -23,13 +26,7 @@ static uint64_t next(void) {
   z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
   return z ^ (z >> 31);
 }
-static double div_rn(double a, double b, double y) {
-  double q0 = a * y;
-  double r0 = fma(-b, q0, a);
-  double q1 = fma(r0, y, q0);
-  double r1 = fma(-b, q1, a);
-  return fma(r1, y, q1);
-}
+using pmg::div_rn;
 static double rnd(int lo, int hi) {  /* random sign, significand and exponent in [lo, hi) */
   uint64_t u = next();
   double m = 1.0 + (double)(u >> 12) * 0x1p-52;
@@ -63,14 +60,14 @@ int main(void) {
 
 def test_div_rn_equals_ieee_division():
     with tempfile.TemporaryDirectory() as d:
-        c = os.path.join(d, "t.c")
+        c = os.path.join(d, "t.cpp")
         exe = os.path.join(d, "t")
         with open(c, "w") as f:
             f.write(SRC)
-        r = subprocess.run(["gcc", "-O2", "-std=c99", "-ffp-contract=off", "-mfma", c, "-o", exe, "-lm"],
+        r = subprocess.run(["g++", "-O2", "-std=c++17", f"-I{CSRC}", "-ffp-contract=off", "-mfma", c, "-o", exe, "-lm"],
                            capture_output=True, text=True)
         if r.returncode != 0:
-            r = subprocess.run(["gcc", "-O2", "-std=c99", "-ffp-contract=off", c, "-o", exe, "-lm"],
+            r = subprocess.run(["g++", "-O2", "-std=c++17", f"-I{CSRC}", "-ffp-contract=off", c, "-o", exe, "-lm"],
                                capture_output=True, text=True)
         if r.returncode != 0:
             pytest.skip("no C compiler: " + r.stderr[-300:])
