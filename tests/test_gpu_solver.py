@@ -38,9 +38,9 @@ def _pair(pm, n, rho, op=0, a=None, c=None, pre=2, pst=2, variant=1, zchunk=32, 
 
 @pytest.mark.parametrize("variant,zchunk", [(v, 32) for v in range(12)] + [(6, 5), (7, 4), (8, 7), (9, 5), (11, 3)])
 def test_c1_ten_cycles_65(pm, variant, zchunk):
-    """65^3 Poisson, seeded Gaussian source, V(2,2), FW, 10 cycles, every
-    sweep tile variant (z-chunks that leave every remainder of the
-    three-step march of the two-planes-in-flight variants)."""
+    """65^3 Poisson, seeded Gaussian source, V(2,2), FW, 10 cycles, whatever
+    sweep tile is set (levels of this size take the one-launch legs in V(2,2);
+    the tiles themselves are compared in test_gpu_sweep_tiles.py)."""
     print(f"case c1 65^3 variant={variant} zchunk={zchunk}", flush=True)
     n = 65
     rho = -pm.gaussian_source(n, seed=1234)
@@ -73,9 +73,8 @@ def test_cycles_other_sizes(pm, n):
 @pytest.mark.parametrize("n,variant,zchunk", [(33, 1, 32), (65, 5, 32), (65, 6, 5), (65, 9, 7), (65, 10, 32),
                                                (65, 11, 3), (65, 2, 8)])
 def test_varcoef_cycles(pm, n, variant, zchunk):
-    """Variable-coefficient cycles, the coefficient a in its LDS ring (4 or 5
-    planes) where both rings fit, read from global memory otherwise (the
-    FP64 128 x 16 tiles)."""
+    """Variable-coefficient V(2,2) cycles, whatever sweep tile is set (levels of
+    these sizes take the one-launch legs; test_gpu_sweep_tiles.py has the tiles)."""
     print(f"case varcoef {n} variant={variant} zchunk={zchunk}", flush=True)
     rng = np.random.default_rng(5)
     rho = -pm.gaussian_source(n, seed=5)
