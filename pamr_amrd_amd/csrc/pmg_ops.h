@@ -140,10 +140,8 @@ __device__ __forceinline__ int w3d_kbranch(int i, int kk) {
 template <typename T>
 __device__ __forceinline__ T fw_point_ex(const T *u1, const T *chr1, T ex, int nx1, int ny1,
                                          int nz1, int i0, int j0, int k0, int iloop) {
-  const int im = i0 - 1, jm = j0 - 1, km = k0 - 1, ip = i0 + 1, jp = j0 + 1, kp = k0 + 1;
   const bool xi = i0 > 1 && i0 <= nx1 - 1, yi = j0 > 1 && j0 <= ny1 - 1,
              zi = k0 > 1 && k0 <= nz1 - 1;
-  (void)im; (void)jm; (void)km; (void)ip; (void)jp; (void)kp;
   if (!xi && !yi && !zi) return PMG_CH(i0, j0, k0) == ex ? T(0) : PMG_U1(i0, j0, k0);
   // The full, plane and line stencils are one product of weights: an axis
   // that does not take part has the point itself with weight 1.  All 54

@@ -72,7 +72,6 @@ __global__ __launch_bounds__(NT) void k_interp3d(const T *u1, T *u2, int nx1, in
                                                  int si1, int sj1, int sk1, int irho, int jrho,
                                                  int krho, BoxPts bp) {
   if (R2) irho = jrho = krho = 2;
-  const int mi = (ni - 1) * irho + 1, mj = (nj - 1) * jrho + 1, mk = (nk - 1) * krho + 1;
   for_box(bp, [&](int fi, int fj, int fk) {
     const int ai = fi / irho, ri = fi % irho, aj = fj / jrho, rj = fj % jrho, ak = fk / krho, rk = fk % krho;
     auto U = [&](int a, int b, int c) -> T {
@@ -104,7 +103,6 @@ template <int AX, bool R2>
 __global__ __launch_bounds__(NT) void k_interp4(double *u2, int nx2, int ny2, int nz2, int i2, int j2, int k2, int ni,
                                                 int nj, int nk, int irho, int jrho, int krho, BoxPts bp) {
   if (R2) irho = jrho = krho = 2;
-  const int mi = (ni - 1) * irho + 1, mj = (nj - 1) * jrho + 1, mk = (nk - 1) * krho + 1;
   // offsets from (i2, j2, k2); axes behind the phase's own are still coarse
   for_box(bp, [&](int fi, int fj, int fk) {
     if (AX < 1) fj *= jrho;
@@ -310,7 +308,6 @@ __global__ __launch_bounds__(NT) void k_interp_ex2(T *u2, const T *chr1, T ex, i
                                                    int nj, int nk, int si1, int sj1, int sk1, int irho, int jrho,
                                                    int krho, BoxPts bp) {
   if (R2) irho = jrho = krho = 2;
-  const int mi = (ni - 1) * irho + 1, mj = (nj - 1) * jrho + 1, mk = (nk - 1) * krho + 1;
   for_box(bp, [&](int fi, int fj, int fk) {
     if (AX < 1) fj *= jrho;
     if (AX < 2) fk *= krho;
