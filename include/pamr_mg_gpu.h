@@ -218,7 +218,10 @@ int pmg_set_fp32_exact_bottom(pmg_solver *S, int on);
 int pmg_set_restrict_fusion(pmg_solver *S, int on);
 /* coarse planes per workgroup of that fused kernel (prec 0 FP64 cycle, 1 FP32
  * inner cycle; 1..64; default 6 / 4 when the coarse level has 129 to 256
- * planes, else 8 / 8); results are identical for every value.  -3 (value kept)
+ * planes, else 8 / 8, and fewer, down to 1, where these make too few
+ * workgroups on a coarse level of up to 256 planes; a grid for which even the
+ * default makes more than the workspace below holds runs the separate
+ * kernels); results are identical for every value.  -3 (value kept)
  * when the launch would need more workgroups than the solver's partial-norm
  * workspace holds (small values on large grids) */
 int pmg_set_resid_restrict_zchunk(pmg_solver *S, int prec, int czchunk);

@@ -69,7 +69,9 @@ __device__ __forceinline__ bool hook_on(const double *cmask, const double *chr, 
 // colour, (mi + 1) / 2 places a row -- by one linear index, per thread `ppt`
 // places a block's width apart.  With 64-bit divisions for the index and, in a
 // colour pass, half of the lanes idle, the kernels waited on arithmetic; now on
-// memory (seven arrays read: 3.9 TB/s).  At 150 x 121 x 97 with op 1: a colour
+// memory: V and a are fetched three times, the planes above and below by blocks of
+// other XCDs, 166 MB for the 99 MB of a colour pass's arrays, 165-179 MB for the
+// operator and the residual, all at 5.7-6.2 TB/s.  At 150 x 121 x 97 with op 1: a colour
 // pass 32.6 -> 28.6 us, the residual 29.2 -> 27.9, the operator 26.5 -> 25.2,
 // the fold of a quarter of the partials 6.5 -> 4.8.
 constexpr int kTwoFrom = 4 * 256 * 2 * NT;

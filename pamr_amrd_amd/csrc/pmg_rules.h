@@ -61,7 +61,11 @@ inline int resid_restrict_planes(const int *cn, int pi) {
 // with 32, 503 with 64).  Below 200^3: 32 x 16 columns, the longest march of 64
 // .. 2 planes that makes 400 workgroups -- fewer leave CUs without work, shorter
 // marches repeat the prologue (129^3: 14.9 us at 8 planes and 512 workgroups;
-// 65^3: 6.6 us at 2 planes, 7.6 at 4).
+// 65^3: 6.6 us at 2 planes, 7.6 at 4).  Not the best of a full search where a
+// side is no 2^m + 1 (back to back): 225^3 FP64 81 us against 73 on 32 x 16 x 32,
+// FP32 58 against 47 on 64 x 32 x 16, FP64 with the coefficient 186 against 140 on 32
+// x 16 x 16; 321 x 257 x 257 FP64 132 against 118 on 64 x 16 x 16; nor at 257^3 FP64,
+// 80 against 75 on the five-plane 128 x 8 x 64, which the tuned table has.
 inline void default_sweep(const int *n, int op, int pi, int *variant, int *zchunk) {
   const size_t size = (size_t)n[0] * n[1] * n[2];
   int tx = 32, ty = 16, want = 400, z = 64;

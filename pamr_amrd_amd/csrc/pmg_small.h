@@ -33,7 +33,13 @@ constexpr int kSmT = 8, kSmH = 4, kSmR = kSmT + 2 * kSmH, kSmL = kSmR + 2;
 constexpr int kSmNT = kSmR * kSmR * 2, kSmP = kSmR / 2;  // threads; points per thread
 constexpr int kSmC = kSmR / 2 + 2;                       // coarse points per axis around a tile
 
-// the largest level whose legs run as one launch each
+// The largest level whose legs run as one launch each.  A cycle with separate
+// kernels and with legs on every level, us (FP64 plain / FP64 variable coefficient
+// / FP32 iteration plain / variable): 33^3 146 -> 124, 169 -> 143, 85 -> 75, 141 ->
+// 117; 65^3 187 -> 163, 231 -> 221, 125 -> 107, 189 -> 162; 81^3 663 -> 653, 430 ->
+// 467, 224 -> 206, 296 -> 270; 97^3 1417 -> 1426, 1957 -> 2100, 300 -> 299, 327 ->
+// 341.  The line is FP64's with the variable coefficient, the first to lose: the
+// others would still gain at 81^3.
 constexpr size_t kSmallPoints = 300000;
 
 template <typename T>
