@@ -136,6 +136,12 @@ struct Spacing {
   int pow2;  // 1 when inv_* are exact
 };
 
+// the same, with its quotients by division (div3 in pmg_div.h)
+template <typename T>
+struct ByDivision : Spacing<T> {
+  using divides = void;
+};
+
 // Wave64 + LDS block reduction of (sum, count) pairs; result valid in
 // thread 0.  Fixed tree order: deterministic for a fixed launch shape.
 template <int NT>

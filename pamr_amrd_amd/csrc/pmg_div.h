@@ -57,13 +57,24 @@ PMG_DIV_FN bool mid_range(float v) {
 // (FP32: 60 and 30) keep every remainder's last bit above the smallest
 // subnormal.  Anything else (zeros, tiny, infinite) takes the division itself.
 // 15 FP64 operations for the three instead of about 36: the sweep of a
-// 161 x 97 x 129 grid with 1/160 spacing 33 -> 24 us.
+// 161 x 97 x 129 grid with 1/160 spacing 33 -> 24 us.  The test is a branch,
+// though, that waits for all three: where a thread works on one point after
+// another with nothing beside it, the divisions overlap better.  A spacing of a
+// type with a member type `divides` asks for them (ByDivision in pmg_common.h).
+template <typename S, typename = void>
+struct divides : std::false_type {};
+template <typename S>
+struct divides<S, std::void_t<typename S::divides>> : std::true_type {};
 template <typename T, bool P2, typename S>
 PMG_DIV_FN void div3(T &x, T &y, T &z, const S &sp) {
   if constexpr (P2) {
     x = x * sp.idx2;
     y = y * sp.idy2;
     z = z * sp.idz2;
+  } else if constexpr (divides<S>::value) {
+    x = x / sp.dx2;
+    y = y / sp.dy2;
+    z = z / sp.dz2;
   } else {
     constexpr int EQ = std::is_same<T, double>::value ? 600 : 60, EI = std::is_same<T, double>::value ? 200 : 30;
     const bool inv = mid_range<EI>(sp.idx2) && mid_range<EI>(sp.idy2) && mid_range<EI>(sp.idz2);

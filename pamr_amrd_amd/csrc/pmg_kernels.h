@@ -1346,6 +1346,11 @@ __global__ __launch_bounds__(NT) void k_coarse_solve(CoarseP<T> P) {
   }
   __shared__ double wsum[2][NW];
   int turn = 0;
+  // A thread's points follow one another, and a sweep is the latency of each: the
+  // divisions overlap, division-free quotients wait for their guard (spacing 1/33
+  // ..., us a sweep: 11 x 7 x 9 points in LDS 2.0 -> 1.6; from memory 18^3 20.5 ->
+  // 15.2, 34 x 50 x 66 489 -> 360, with the variable coefficient 895 -> 591).
+  const ByDivision<T> sp{P.sp};
   // one sweep; returns the sum of the squared residuals, the same in every
   // thread: each wave's by its shuffle tree, those in every thread alike (two
   // barriers a sweep: the half sweep's, and the one that publishes the sums)
@@ -1353,7 +1358,7 @@ __global__ __launch_bounds__(NT) void k_coarse_solve(CoarseP<T> P) {
     double s = 0.0;
     auto relax = [&](size_t p) {
       T jac;
-      const T r = lop_at<T, OP, P2>(u, rho, a, c, p, sy, sz, P.sp, &jac) - rhs[p];
+      const T r = lop_at<T, OP, P2>(u, rho, a, c, p, sy, sz, sp, &jac) - rhs[p];
       u[p] = u[p] - div_jac<T, OP>(r, jac, P.sp);
       s += (double)r * (double)r;
     };

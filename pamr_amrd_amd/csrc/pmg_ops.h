@@ -21,9 +21,9 @@ __device__ __forceinline__ T div_jac(T r, T jac, const Spacing<T> &sp) {
 // Plain Poisson operator L[V] = lap_h V - rho at one point
 // (w/examples/nps/num_w.f:42-45; relax/residual terms at :136-140).
 // Neighbour naming: e/w = i+1/i-1, n/s = j+1/j-1, t/b = k+1/k-1.
-template <typename T, bool P2>
+template <typename T, bool P2, typename S>
 __device__ __forceinline__ T lop_poisson(T uc, T ue, T uw, T un, T us, T ut, T ub,
-                                         T rho, const Spacing<T> &sp) {
+                                         T rho, const S &sp) {
   T lx = (ue - 2 * uc) + uw, ly = (un - 2 * uc) + us, lz = (ut - 2 * uc) + ub;
   div3<T, P2>(lx, ly, lz, sp);
   return ((lx + ly) + lz) - rho;
@@ -32,10 +32,10 @@ __device__ __forceinline__ T lop_poisson(T uc, T ue, T uw, T un, T us, T ut, T u
 // Variable-coefficient operator L[V] = div(a grad V) + c V - rho with
 // arithmetic-mean face coefficients (project-defined hook in the nps style;
 // the reference ships only constant-coefficient hooks).
-template <typename T, bool P2>
+template <typename T, bool P2, typename S>
 __device__ __forceinline__ T lop_varcoef(T uc, T ue, T uw, T un, T us, T ut, T ub,
                                          T ac, T ae, T aw, T an, T as, T at, T ab,
-                                         T cc, T rho, const Spacing<T> &sp, T *jac) {
+                                         T cc, T rho, const S &sp, T *jac) {
   T fe = T(0.5) * (ac + ae), fw = T(0.5) * (ac + aw);
   T fn = T(0.5) * (ac + an), fs = T(0.5) * (ac + as);
   T ft = T(0.5) * (ac + at), fb = T(0.5) * (ac + ab);
@@ -50,9 +50,9 @@ __device__ __forceinline__ T lop_varcoef(T uc, T ue, T uw, T un, T us, T ut, T u
 }
 
 // L at point p of a plain array (global memory neighbours).
-template <typename T, int OP, bool P2>
+template <typename T, int OP, bool P2, typename S>
 __device__ __forceinline__ T lop_at(const T *V, const T *rho, const T *a, const T *c,
-                                    size_t p, size_t sy, size_t sz, const Spacing<T> &sp,
+                                    size_t p, size_t sy, size_t sz, const S &sp,
                                     T *jac) {
   if constexpr (OP == 0) {
     if (jac) *jac = sp.jac;

@@ -26,6 +26,7 @@ static uint64_t next() {
   return z ^ (z >> 31);
 }
 template <typename T> struct Sp { T dx2, dy2, dz2, idx2, idy2, idz2; };
+template <typename T> struct By : Sp<T> { using divides = void; };
 template <typename T> static T any(int e) {  // random significand, exponent in [-e, e)
   return (T)std::ldexp(1 + (double)(next() >> 12) * 0x1p-52, (int)(next() % (2 * e)) - e);
 }
@@ -49,9 +50,12 @@ template <typename T> static long run(int se, int ae, int edge, long n) {
     const Sp<T> sp{d[0], d[1], d[2], 1 / d[0], 1 / d[1], 1 / d[2]};
     for (int k = 0; k < 3; k++) q[k] = a[k];
     pmg::div3<T, false>(q[0], q[1], q[2], sp);
+    T e[3] = {a[0], a[1], a[2]};
+    pmg::div3<T, false>(e[0], e[1], e[2], By<T>{sp});
     for (int k = 0; k < 3; k++) {
       const T x = a[k] / d[k];
       if (!(std::isnan(x) && std::isnan(q[k])) && std::memcmp(&x, &q[k], sizeof x)) bad++;
+      if (!(std::isnan(x) && std::isnan(e[k])) && std::memcmp(&x, &e[k], sizeof x)) bad++;
     }
   }
   return bad;
